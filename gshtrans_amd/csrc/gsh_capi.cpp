@@ -239,14 +239,13 @@ struct NData {
   // null when there are none: sseed * 2^-skexp.
   double* sseed = nullptr;
   int* skexp = nullptr;
-  bool ck_restart = false;  // some such order rises to significance: the FP64
-                            // synthesis restarts from the checkpoints
   double4* rec = nullptr;  // {a, b, c, 0} per (m, l), see gsh_internal.h
   long* roff = nullptr;
   // Recurrence checkpoints at the start of every analysis pass k >= 1
   // (built on the first analysis with this upper index).
   double2* ck = nullptr;
   long* ckoff = nullptr;
+  unsigned short* kf = nullptr;  // first checkpoint that matters per (order, 16 rows)
 };
 
 // Analysis work list on the device (see gsh::work_item).
@@ -483,20 +482,19 @@ int ensure_ck(gsh_grid_s* g, NData* d, int n, hipStream_t s) {
   }
   double2* ck = nullptr;
   long* ckoff = nullptr;
-  int* flag = nullptr;
+  unsigned short* kf = nullptr;
+  const int nrt = (nt + 15) / 16;
   auto release = [&](int status) {
     if (ck) (void)hipFree(ck);
     if (ckoff) (void)hipFree(ckoff);
-    if (flag) (void)hipFree(flag);
+    if (kf) (void)hipFree(kf);
     return status;
   };
   if (hipMalloc(&ck, std::max(rows, 1L) * nt * sizeof(double2)) != hipSuccess ||
       hipMalloc(&ckoff, off.size() * sizeof(long)) != hipSuccess ||
-      (d->sseed && hipMalloc(&flag, sizeof(int)) != hipSuccess))
+      hipMalloc(&kf, off.size() * nrt * sizeof(unsigned short)) != hipSuccess)
     return release(GSH_ERR_OUT_OF_MEMORY);
-  if (hipMemcpy(ckoff, off.data(), off.size() * sizeof(long), hipMemcpyHostToDevice) !=
-          hipSuccess ||
-      (flag && hipMemset(flag, 0, sizeof(int)) != hipSuccess))
+  if (hipMemcpy(ckoff, off.data(), off.size() * sizeof(long), hipMemcpyHostToDevice) != hipSuccess)
     return release(GSH_ERR_DEVICE);
   LegParams p{};
   p.L = L;
@@ -511,16 +509,13 @@ int ensure_ck(gsh_grid_s* g, NData* d, int n, hipStream_t s) {
   p.ckoff = ckoff;
   p.sseed = d->sseed;
   p.skexp = d->skexp;
-  p.ck_flag = flag;
+  p.kf_out = kf;
+  p.nrt = nrt;
   if (gsh::launch_rec_checkpoints(p, s) != hipSuccess || hipStreamSynchronize(s) != hipSuccess)
     return release(GSH_ERR_DEVICE);
-  int rose = 0;
-  if (flag && hipMemcpy(&rose, flag, sizeof(int), hipMemcpyDeviceToHost) != hipSuccess)
-    return release(GSH_ERR_DEVICE);
-  if (flag) (void)hipFree(flag);
   d->ck = ck;
   d->ckoff = ckoff;
-  d->ck_restart = rose != 0;
+  d->kf = kf;
   return GSH_OK;
 }
 
@@ -630,6 +625,92 @@ int ensure_synth_worklist(gsh_grid_s* g, int family, int lmax, int real, int ngr
   }
   WorkList w;
   w.per = static_cast<int>(items.size() / 8);
+  GSH_HIP(hipMalloc(&w.d, items.size() * sizeof(uint2)));
+  GSH_HIP(hipMemcpy(w.d, items.data(), items.size() * sizeof(uint2), hipMemcpyHostToDevice));
+  g->worklists.emplace(key, w);
+  *out = w;
+  return GSH_OK;
+}
+
+// Work list of a paired-order FP64 launch (gsh_pair.hip): items (m, sub | group
+// << 16) for m >= 0 and groups of t.cols virtual columns; sub is the row
+// block of a synthesis (dir 0) or the pass of an analysis (dir 1).  Units of 8
+// neighbouring orders and one group go whole to the least loaded XCD, heaviest
+// first: the coefficients of neighbouring orders at a degree share cache
+// lines, and a unit's items (sub by sub, 8 orders each) run there together.
+// The weight of a degree is the share of rows at which it matters (sin t >
+// m / l).  gl[g] bounds the degrees of group g (empty: lmax); orders past it
+// have no items.
+int ensure_pair_worklist(gsh_grid_s* g, int dir, int lmax, int n, int pair, int ncol,
+                         const gsh::PairTile& t, const std::vector<int>* f_lmax, WorkList* out) {
+  std::vector<int> shape{t.cols, t.nblk, t.vint, ncol};
+  if (f_lmax) shape.insert(shape.end(), f_lmax->begin(), f_lmax->end());
+  auto key = std::make_tuple(40 + dir, lmax, n, pair, shape);
+  auto it = g->worklists.find(key);
+  if (it != g->worklists.end()) {
+    *out = it->second;
+    return GSH_OK;
+  }
+  constexpr int kBand = 8;
+  struct Unit {
+    double w;
+    std::vector<uint2> items;
+  };
+  std::vector<Unit> units;
+  for (int b0 = 0; b0 <= lmax; b0 += kBand) {
+    const int b1 = std::min(b0 + kBand, lmax + 1);
+    for (int v0 = 0, grp = 0; v0 < t.vcols; v0 += t.cols, grp++) {
+      Unit u{0.0, {}};
+      std::vector<int> subs(b1 - b0, 0);
+      int smax = 0;
+      for (int m = b0; m < b1; m++) {
+        // the kernels' vcol and vcol_lmax
+        int col = v0;
+        if (t.vint && pair)
+          col = v0 / 32 * 16;
+        else if (pair && m > 0 && v0 < ncol && v0 + t.cols > ncol)
+          col = 0;
+        else if (pair && m == 0 && v0 >= ncol)
+          continue;
+        else
+          col = v0 % ncol;
+        const int lw = f_lmax ? (*f_lmax)[std::min(col, ncol - 1) / 2] : lmax;
+        const int l0 = std::max(m, std::abs(n));
+        if (l0 > lw) continue;
+        const int nu = (lw - l0 + 32) / 32;
+        subs[m - b0] = dir == 0 ? t.nblk : (nu + t.nblk - 1) / t.nblk;
+        smax = std::max(smax, subs[m - b0]);
+        for (int k = 0; k < nu; k++)
+          u.w += 0.1 + 1.0 - 0.64 * std::asin(m / (l0 + 32.0 * k + 32.0));
+      }
+      for (int sub = 0; sub < smax; sub++)
+        for (int m = b0; m < b1; m++)
+          if (sub < subs[m - b0])
+            u.items.push_back(make_uint2(static_cast<unsigned>(m),
+                                         static_cast<unsigned>(sub) |
+                                             (static_cast<unsigned>(grp) << 16)));
+      if (!u.items.empty()) units.push_back(std::move(u));
+    }
+  }
+  std::stable_sort(units.begin(), units.end(),
+                   [](const Unit& a, const Unit& b) { return a.w > b.w; });
+  std::vector<uint2> xcd[8];
+  double load[8] = {};
+  for (const Unit& u : units) {
+    const int x = static_cast<int>(std::min_element(load, load + 8) - load);
+    load[x] += u.w;
+    xcd[x].insert(xcd[x].end(), u.items.begin(), u.items.end());
+  }
+  size_t per = 1;
+  for (const auto& v : xcd) per = std::max(per, v.size());
+  std::vector<uint2> items;
+  items.reserve(8 * per);
+  for (auto& v : xcd) {
+    v.resize(per, make_uint2(~0u, 0u));
+    items.insert(items.end(), v.begin(), v.end());
+  }
+  WorkList w;
+  w.per = static_cast<int>(per);
   GSH_HIP(hipMalloc(&w.d, items.size() * sizeof(uint2)));
   GSH_HIP(hipMemcpy(w.d, items.data(), items.size() * sizeof(uint2), hipMemcpyHostToDevice));
   g->worklists.emplace(key, w);
@@ -955,6 +1036,7 @@ int gsh_grid_destroy(gsh_grid_t g) {
     (void)hipFree(kv.second.roff);
     if (kv.second.ck) (void)hipFree(kv.second.ck);
     if (kv.second.ckoff) (void)hipFree(kv.second.ckoff);
+    if (kv.second.kf) (void)hipFree(kv.second.kf);
     if (kv.second.sseed) (void)hipFree(kv.second.sseed);
     if (kv.second.skexp) (void)hipFree(kv.second.skexp);
   }
@@ -1014,8 +1096,8 @@ struct RunOpts {
   const int* f_lmax = nullptr;   // device: truncation degree per column field
   const int* cg_lmax = nullptr;  // device: max f_lmax per 16-column group
   std::vector<int> cg_lmax_host;  // the same on the host (work lists)
+  const std::vector<int>* f_lmax_host = nullptr;  // f_lmax on the host
   int f32 = 0;                   // fields stored in FP32
-  int synth_tiles = 0;           // FP64 synthesis: 16-column tiles per workgroup (0: auto)
   int fft = 0;                   // 0: auto, 1: wavefront-per-ring kernel, 2: LDS kernel
   int anal_pass = 0;             // split-BF16 analysis degrees per pass: 64, 128 (0: auto)
   const void* field2 = nullptr;  // analysis of a pointwise expression: second operand
@@ -1027,6 +1109,25 @@ struct RunOpts {
 bool use_wave_fft(const FFTParams& q, const RunOpts& o) {
   return q.twa != nullptr && o.fft != 2;
 }
+// Columns per group of the bins: calls of at most 8 columns whose bins no
+// kernel reads in 16-column tiles (FP64 on the paired-order kernels) keep
+// them together, so a bin's line holds no padding columns.
+int bin_columns(int ncol, int precision) {
+  if (precision != GSH_FP64) return 16;
+  int cw = 2;
+  while (cw < ncol && cw < 16) cw *= 2;
+  return cw;
+}
+// Ring FFTs of a call.  The wavefront kernels (N = 512, 1024, 2048) move bins
+// for 8 complex rings (16 real ones) of a colatitude at a time; calls of at
+// most 4 fields, other lengths and o.fft = 2 take the ring kernels, and
+// transforms of fewer than 64 or more than 4096 points the general ones.
+hipError_t run_fft(const FFTParams& q, const RunOpts& o, bool anal, hipStream_t s) {
+  if (use_wave_fft(q, o) && q.nfield > 4 && q.cw == 16)
+    return anal ? gsh::launch_fft_anal_wave(q, s) : gsh::launch_fft_synth_wave(q, s);
+  if (gsh::ring_fft_supported(q.M)) return gsh::launch_fft_ring(q, anal, s);
+  return anal ? gsh::launch_fft_anal(q, s) : gsh::launch_fft_synth(q, s);
+}
 
 // Synthesis of `batch` column fields with lmax >= 1 (no argument checks; the
 // caller holds the grid lock and has prepared n).
@@ -1035,16 +1136,18 @@ int run_inverse(gsh_grid_s* g, NData* d, int lmax, int n, int real, int precisio
                 const RunOpts& o) {
   int st;
   const int nslot = real ? lmax + 1 : 2 * lmax + 1;
-  const size_t ncg16 = (2 * (size_t)batch + 15) / 16;
-  if ((st = ensure_work(g, sizeof(double) * g->ntheta() * nslot * 16 * ncg16))) return st;
+  const int cw = bin_columns(2 * batch, precision);
+  const size_t ncg = (2 * (size_t)batch + cw - 1) / cw;
+  if ((st = ensure_work(g, sizeof(double) * g->ntheta() * nslot * cw * ncg))) return st;
   LegParams p = base_params(g, d, lmax, n, real, batch);
   p.cin = cin;
   p.cstride = cstride;
   p.fmap = o.fmap;
   p.f_lmax = o.f_lmax;
   p.cg_lmax = o.cg_lmax;
-  const int ntsb = (g->ntheta() + 255) / 256;
   FFTParams q = fft_params(g, lmax, real, batch);
+  p.cw = q.cw = cw;
+  q.f_lmax = o.f_lmax;
   q.fout = field;
   q.fstride = fstride;
   q.f32 = o.f32;
@@ -1055,26 +1158,24 @@ int run_inverse(gsh_grid_s* g, NData* d, int lmax, int n, int real, int precisio
   const bool f32bins = precision != GSH_FP64 && precision != GSH_FP32 && use_wave_fft(q, o);
   p.f32out = q.fa32 = f32bins ? 1 : 0;
   if (precision == GSH_FP64 || precision == GSH_FP32) {
-    // Orders whose seeds underflow but whose values rise to significance
-    // before L: the synthesis takes its state from the scaled checkpoints.
-    if (d->sseed) {
-      if ((st = ensure_ck(g, d, n, s))) return st;
-      if (d->ck_restart) {
-        p.ck = d->ck;
-        p.ckoff = d->ckoff;
-        p.ck_restart = 1;
-      }
-    }
-    const int T = o.synth_tiles == 1 || o.synth_tiles == 2 ? o.synth_tiles : (p.ncol > 16 ? 2 : 1);
+    // Orders m and -m together; upper index 0 over the northern rows by
+    // parity (not in FP32, whose sums keep the order of the degrees).
+    const int sym = n == 0 && precision == GSH_FP64 ? 1 : 0;
+    p.pair = real ? 0 : 1;
+    if ((st = ensure_ck(g, d, n, s))) return st;
+    p.ck = d->ck;
+    p.ckoff = d->ckoff;
+    p.kf = d->kf;
+    p.nrt = (p.ntheta + 15) / 16;
+    const gsh::PairTile t = gsh::pair_synth_tile(p.ncol, p.pair, sym, precision == GSH_FP32,
+                                                 o.f_lmax != nullptr, sym ? (p.ntheta + 1) / 2 : p.ntheta);
     WorkList w;
-    if ((st = ensure_synth_worklist(g, 10 + T, lmax, real, (p.ncol + 16 * T - 1) / (16 * T), ntsb,
-                                    &w)))
+    if ((st = ensure_pair_worklist(g, 0, lmax, n, p.pair, p.ncol, t, o.f_lmax_host, &w)))
       return st;
     p.items = w.d;
     p.items_per = w.per;
-    GSH_HIP(timed(g, GSH_KERNEL_LEGENDRE_SYNTHESIS, s, [&] {
-      return gsh::launch_leg_synth_f64(p, s, T, precision == GSH_FP32);
-    }));
+    GSH_HIP(timed(g, GSH_KERNEL_LEGENDRE_SYNTHESIS, s,
+                  [&] { return gsh::launch_leg_synth_pair(p, t, sym, s); }));
   } else {
     // Upper index 0 is synthesized over the northern colatitudes (items of
     // 128 of them; each writes the mirror rows too), the coefficients in the
@@ -1151,7 +1252,7 @@ int run_inverse(gsh_grid_s* g, NData* d, int lmax, int n, int real, int precisio
     }));
   }
   GSH_HIP(timed(g, GSH_KERNEL_FFT_SYNTHESIS, s, [&] {
-    return use_wave_fft(q, o) ? gsh::launch_fft_synth_wave(q, s) : gsh::launch_fft_synth(q, s);
+    return run_fft(q, o, false, s);
   }));
   return GSH_OK;
 }
@@ -1176,6 +1277,7 @@ int run_forward(gsh_grid_s* g, NData* d, int lmax, int n, int real, int precisio
   q.fstride = fstride;
   q.f32 = o.f32;
   q.fmap = o.fmap;
+  q.f_lmax = o.f_lmax;
   if (adjoint) {
     q.wq = g->d_one;
     q.adjoint = 1;
@@ -1194,7 +1296,9 @@ int run_forward(gsh_grid_s* g, NData* d, int lmax, int n, int real, int precisio
   // floats into the buffer: the paired-order kernel's mirrored reads of the
   // last chunk reach up to 31 rows of 16 floats before a block.
   const bool mixed = precision == GSH_BF16X6 || precision == GSH_BF16X3;
-  const size_t fa = (size_t)nslot * ((ncol + 15) / 16) * ((g->ntheta() + 3) / 4) * 64 + 8 * 64 +
+  const int cw = bin_columns(ncol, precision);
+  p.cw = q.cw = cw;
+  const size_t fa = (size_t)nslot * ((ncol + cw - 1) / cw) * ((g->ntheta() + 3) / 4) * 4 * cw + 8 * 64 +
                     (mixed ? gsh::kFAFrontPad : 0);
   if ((st = ensure_work(g, (mixed ? sizeof(float) : sizeof(double)) * fa))) return st;
   q.F = p.F = mixed ? reinterpret_cast<double*>(reinterpret_cast<float*>(g->work) + gsh::kFAFrontPad)
@@ -1206,15 +1310,30 @@ int run_forward(gsh_grid_s* g, NData* d, int lmax, int n, int real, int precisio
   p.ckoff = d->ckoff;
   const int ncg16 = (ncol + 15) / 16;
   GSH_HIP(timed(g, GSH_KERNEL_FFT_ANALYSIS, s, [&] {
-    return use_wave_fft(q, o) ? gsh::launch_fft_anal_wave(q, s) : gsh::launch_fft_anal(q, s);
+    return run_fft(q, o, true, s);
   }));
-  if (precision == GSH_FP64 || precision == GSH_FP32) {
+  if (precision == GSH_FP64) {
+    const int sym = n == 0 ? 1 : 0;
+    p.pair = real ? 0 : 1;
+    p.kf = d->kf;
+    p.nrt = (p.ntheta + 15) / 16;
+    const gsh::PairTile t = gsh::pair_anal_tile(p.ncol, p.pair, o.f_lmax != nullptr);
+    WorkList w;
+    if ((st = ensure_pair_worklist(g, 1, lmax, n, p.pair, p.ncol, t, o.f_lmax_host, &w)))
+      return st;
+    p.items = w.d;
+    p.items_per = w.per;
+    GSH_HIP(timed(g, GSH_KERNEL_LEGENDRE_ANALYSIS, s,
+                  [&] { return gsh::launch_leg_anal_pair(p, t, sym, s); }));
+    return GSH_OK;
+  }
+  if (precision == GSH_FP32) {
     WorkList w;
     if ((st = ensure_worklist(g, 0, lmax, n, real, ncg16, o.cg_lmax_host, &w))) return st;
     p.items = w.d;
     p.items_per = w.per;
     GSH_HIP(timed(g, GSH_KERNEL_LEGENDRE_ANALYSIS, s, [&] {
-      return gsh::launch_leg_anal_f64(p, s, precision == GSH_FP32);
+      return gsh::launch_leg_anal_f32(p, s);
     }));
     return GSH_OK;
   }
@@ -1579,7 +1698,7 @@ struct PlanGroup {
   int* d_flmax = nullptr;
   int* d_cglmax = nullptr;
   NData* nd = nullptr;
-  int synth_tiles = 0;  // FP64 synthesis column tiles (0: not tuned)
+  int synth_tiles = 0;  // FP64 / FP32 synthesis column tiles per wave (0: not tuned)
   int fft_inv = 0;      // 1: wavefront FFT, 2: LDS FFT (0: not tuned)
   int fft_fwd = 0;
   int anal_pass = 0;    // split-BF16 analysis degrees per pass, 64 or 128 (0: not tuned)
@@ -1683,8 +1802,8 @@ RunOpts group_opts(const gsh_plan_s* P, const PlanGroup& G, int dir) {
   o.f_lmax = G.d_flmax;
   o.cg_lmax = G.d_cglmax;
   o.cg_lmax_host = G.cglmax;
+  o.f_lmax_host = &G.flmax;
   o.f32 = P->storage == GSH_STORE_FP32;
-  o.synth_tiles = G.synth_tiles;
   o.fft = dir == 0 ? G.fft_inv : G.fft_fwd;
   o.anal_pass = dir == 0 ? 0 : G.anal_pass;
   return o;
@@ -1742,7 +1861,8 @@ int run_plan(gsh_plan_s* P, int dir, const void* in, long istride, void* out, lo
 // appended to that file (one "key tiles fft pass" line per shape;
 // unreadable lines are skipped).
 std::mutex tune_mu;
-// Choices per shape: synthesis tiles, FFT family, analysis pass length.
+// Choices per shape: synthesis column tiles (reported only), FFT family,
+// analysis pass length.
 struct TuneChoice {
   int tiles = 0, fft = 0, pass = 0;
 };
@@ -1797,10 +1917,10 @@ void tune_store(const std::string& key, const TuneChoice& v) {
   if (f) f << key << " " << v.tiles << " " << v.fft << " " << v.pass << "\n";
 }
 
-// Autotuner: per group, run each candidate (FP64 synthesis tiles, FFT family,
-// and for the split-BF16 analysis 64- or 128-degree passes) once to warm up
-// and once timed with events, and keep the fastest; a shape tuned before
-// (this process, or the GSH_TUNE_CACHE file) is not timed again.
+// Autotuner: per group, run each candidate (FFT family, and for the
+// split-BF16 analysis 64- or 128-degree passes) once to warm up and once timed
+// with events, and keep the fastest; a shape tuned before (this process, or
+// the GSH_TUNE_CACHE file) is not timed again.
 int tune_plan(gsh_plan_s* P, int dir, const void* in, long istride, void* out, long ostride,
               hipStream_t s) {
   int st;
@@ -1834,17 +1954,14 @@ int tune_plan(gsh_plan_s* P, int dir, const void* in, long istride, void* out, l
     std::vector<TuneChoice> cands;
     const bool wave_ok = P->g->d_twa != nullptr;
     const bool fp = P->precision == GSH_FP64 || P->precision == GSH_FP32;
-    const bool tiles2 = dir == 0 && fp && G.count > 8;
     const std::vector<int> passes =
         dir == 1 && !fp ? std::vector<int>{gsh::kPass, gsh::kWideAnalPass} : std::vector<int>{0};
-    for (int t : tiles2 ? std::vector<int>{1, 2} : std::vector<int>{0})
-      for (int f : wave_ok ? std::vector<int>{1, 2} : std::vector<int>{2})
-        for (int pl : passes) cands.push_back(TuneChoice{t, f, pl});
+    for (int f : wave_ok ? std::vector<int>{1, 2} : std::vector<int>{2})
+      for (int pl : passes) cands.push_back(TuneChoice{0, f, pl});
     float best = 1e30f;
     TuneChoice pick = cands[0];
     for (const auto& c : cands) {
       RunOpts o = group_opts(P, G, dir);
-      o.synth_tiles = c.tiles;
       o.fft = c.fft;
       o.anal_pass = c.pass;
       for (int rep = 0; rep < 2; rep++) {
@@ -1865,6 +1982,13 @@ int tune_plan(gsh_plan_s* P, int dir, const void* in, long istride, void* out, l
       }
     }
     if (dir == 0) {
+      // Reported with the choices, not timed: the synthesis's column tiles.
+      if (fp && G.count > 8) {
+        const int pair = P->kind == GSH_REAL ? 0 : 1;
+        pick.tiles = gsh::pair_synth_tile(2 * G.count, pair, G.n == 0 && P->precision == GSH_FP64,
+                                          P->precision == GSH_FP32, true, P->g->ntheta())
+                         .nj;
+      }
       G.synth_tiles = pick.tiles;
       G.fft_inv = pick.fft;
     } else {

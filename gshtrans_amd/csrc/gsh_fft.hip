@@ -170,7 +170,7 @@ __global__ __launch_bounds__(kFFTThreads) void fft_synth(FFTParams p) {
   const int theta = blockIdx.x / p.nfg;
   const int fg = blockIdx.x % p.nfg;
   const int N = p.N, M = p.M, R = p.rings;
-  const int ncg16 = (p.ncol + 15) >> 4;
+  const int cw = p.cw, ncg = (p.ncol + cw - 1) / cw;
   // Fill: consecutive threads read consecutive fields of one bin.
   for (int idx = threadIdx.x; idx < R * M; idx += kFFTThreads) {
     const int q = idx % R;
@@ -178,23 +178,24 @@ __global__ __launch_bounds__(kFFTThreads) void fft_synth(FFTParams p) {
     const int f = fg * R + q;
     double2 X = make_double2(0.0, 0.0);
     if (f < p.nfield && k < N) {
-      // slot s of this field at Fp[16 s] (F[theta][col/16][slot][16])
-      const double* Fp = p.F + f_index(theta, 0, 2 * f, p.nslot, ncg16);
+      // slot s of this field at Fp[cw s]
+      const double* Fp = p.F + f_index(theta, 0, 2 * f, p.nslot, ncg, cw);
+      const int lf = ring_lmax(p, f);
       if (!p.real) {
-        if (k <= p.lmax) {
+        if (k <= lf) {
           const int s = k - p.m_first;
-          X = make_double2(Fp[16 * (long)s], Fp[16 * (long)s + 1]);
+          X = make_double2(Fp[cw * (long)s], Fp[cw * (long)s + 1]);
         }
-        if (k >= N - p.lmax) {
+        if (k >= N - lf) {
           const int s = (k - N) - p.m_first;
-          X = cadd(X, make_double2(Fp[16 * (long)s], Fp[16 * (long)s + 1]));
+          X = cadd(X, make_double2(Fp[cw * (long)s], Fp[cw * (long)s + 1]));
         }
       } else {
         // Hermitian spectrum from bins 0..N/2 (c2r semantics).
         const int kk = k <= N / 2 ? k : N - k;
-        if (kk <= p.lmax) {
+        if (kk <= lf) {
           const int s = kk - p.m_first;
-          X = make_double2(Fp[16 * (long)s], Fp[16 * (long)s + 1]);
+          X = make_double2(Fp[cw * (long)s], Fp[cw * (long)s + 1]);
           if (kk == 0 || kk == N / 2) X.y = 0.0;
           else if (k > N / 2) X.y = -X.y;
         }
@@ -268,6 +269,7 @@ __global__ __launch_bounds__(kFFTThreads) void fft_anal(FFTParams p) {
     const int f = fg * R + q;
     if (f >= p.nfield) continue;
     const int m = s + p.m_first;
+    if (abs(m) > ring_lmax(p, f)) continue;
     const int k = m >= 0 ? m : N + m;
     double2 X = buf[q * M + k];
     if (p.adjoint && p.real) {
@@ -275,7 +277,7 @@ __global__ __launch_bounds__(kFFTThreads) void fft_anal(FFTParams p) {
       if (k == 0 || 2 * k == N) X.y = 0.0;
       else X = make_double2(2.0 * X.x, 2.0 * X.y);
     }
-    const long fi = fa_index(s, 2 * f, theta, p.n_cg, p.nquad);
+    const long fi = fa_index(s, 2 * f, theta, p.n_cg, p.nquad, p.cw);
     if (p.fa32) {
       float* Fp = reinterpret_cast<float*>(p.F) + fi;
       Fp[0] = (float)(X.x * w);
@@ -287,7 +289,7 @@ __global__ __launch_bounds__(kFFTThreads) void fft_anal(FFTParams p) {
     // The last ring also zeroes the padding rows of the last colatitude
     // quad, which the Legendre contraction reads as B operands.
     for (int tp = theta + 1; theta == p.ntheta - 1 && tp < 4 * p.nquad; tp++) {
-      const long zi = fa_index(s, 2 * f, tp, p.n_cg, p.nquad);
+      const long zi = fa_index(s, 2 * f, tp, p.n_cg, p.nquad, p.cw);
       if (p.fa32) {
         reinterpret_cast<float*>(p.F)[zi] = 0.0f;
         reinterpret_cast<float*>(p.F)[zi + 1] = 0.0f;
@@ -354,7 +356,7 @@ hipError_t launch_fft_synth(const FFTParams& p0, hipStream_t s) {
 
 hipError_t launch_fft_anal(const FFTParams& p0, hipStream_t s) {
   FFTParams p = p0;
-  p.n_cg = (p.ncol + 15) / 16;
+  p.n_cg = (p.ncol + p.cw - 1) / p.cw;
   p.nquad = (p.ntheta + 3) / 4;
   if (p.M > kFFTElemsMax) return hipErrorInvalidValue;
   const bool big = p.M > kFFTElems;

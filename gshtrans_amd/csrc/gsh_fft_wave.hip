@@ -23,6 +23,7 @@
 // complex ring x_a + i x_b.
 #include <type_traits>
 
+#include "gsh_fft_dev.h"
 #include "gsh_internal.h"
 
 namespace gsh {
@@ -44,81 +45,6 @@ constexpr int lds_per_wave(int R) { return (R >= 32 ? R / 2 : R) * 64; }
 // at 8 (0.83 against 1.07 ms).
 constexpr int synth_waves(int R) { return R >= 32 ? 4 : 8; }
 constexpr int anal_waves(int R, int real) { return R >= 32 && real ? 4 : 8; }
-
-// cos(pi k / 16) and sin(pi k / 16), k = 0..16.
-constexpr double kCos16[17] = {
-    1.0,                     0.98078528040323044913, 0.92387953251128675613,
-    0.83146961230254523708,  0.70710678118654752440, 0.55557023301960222474,
-    0.38268343236508977173,  0.19509032201612826785, 0.0,
-    -0.19509032201612826785, -0.38268343236508977173, -0.55557023301960222474,
-    -0.70710678118654752440, -0.83146961230254523708, -0.92387953251128675613,
-    -0.98078528040323044913, -1.0};
-constexpr double kSin16[17] = {
-    0.0,                    0.19509032201612826785, 0.38268343236508977173,
-    0.55557023301960222474, 0.70710678118654752440, 0.83146961230254523708,
-    0.92387953251128675613, 0.98078528040323044913, 1.0,
-    0.98078528040323044913, 0.92387953251128675613, 0.83146961230254523708,
-    0.70710678118654752440, 0.55557023301960222474, 0.38268343236508977173,
-    0.19509032201612826785, 0.0};
-
-__device__ __forceinline__ double2 cadd(double2 a, double2 b) {
-  return make_double2(a.x + b.x, a.y + b.y);
-}
-__device__ __forceinline__ double2 csub(double2 a, double2 b) {
-  return make_double2(a.x - b.x, a.y - b.y);
-}
-__device__ __forceinline__ double2 cmul(double2 a, double2 b) {
-  return make_double2(a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x);
-}
-// a * conj(b)
-__device__ __forceinline__ double2 cmulc(double2 a, double2 b) {
-  return make_double2(a.x * b.x + a.y * b.y, a.y * b.x - a.x * b.y);
-}
-
-// a * exp(i SIGN pi K / 16); K is a constant after unrolling.
-template <int SIGN>
-__device__ __forceinline__ double2 rot16(double2 a, int K) {
-  if (K == 0) return a;
-  if (K == 8) return SIGN > 0 ? make_double2(-a.y, a.x) : make_double2(a.y, -a.x);
-  // exp(i SIGN pi / 4) = h (1 + SIGN i), exp(i SIGN 3 pi / 4) = h (-1 + SIGN i)
-  const double h = kCos16[4];
-  if (K == 4) return make_double2(h * (a.x - SIGN * a.y), h * (a.y + SIGN * a.x));
-  if (K == 12) return make_double2(h * (-a.x - SIGN * a.y), h * (SIGN * a.x - a.y));
-  const double c = kCos16[K], s = SIGN * kSin16[K];
-  return make_double2(a.x * c - a.y * s, a.x * s + a.y * c);
-}
-
-constexpr int bitrev(int x, int bits) {
-  int r = 0;
-  for (int i = 0; i < bits; i++) r |= ((x >> i) & 1) << (bits - 1 - i);
-  return r;
-}
-constexpr int log2c(int x) { return x <= 1 ? 0 : 1 + log2c(x >> 1); }
-
-// In-register DFT of length R (radix-2 decimation in frequency); on return
-// v[bitrev(k)] holds X[k] = sum_j v_in[j] exp(i SIGN 2 pi j k / R).
-template <int R, int SIGN>
-__device__ __forceinline__ void dft_reg(double2* v) {
-#pragma unroll
-  for (int h = R / 2; h >= 1; h >>= 1) {
-#pragma unroll
-    for (int base = 0; base < R; base += 2 * h) {
-#pragma unroll
-      for (int j = 0; j < h; j++) {
-        const double2 a = v[base + j], b = v[base + j + h];
-        v[base + j] = cadd(a, b);
-        // twiddle exp(i SIGN 2 pi j / (2h)) = exp(i SIGN pi (16 j / h) / 16)
-        v[base + j + h] = rot16<SIGN>(csub(a, b), 16 * j / h);
-      }
-    }
-  }
-}
-
-__device__ __forceinline__ void wave_sync() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
 
 // Transform the ring held as v[n1] = x[64 n1 + lane]; on return v[t] =
 // X[lane + 64 t] = sum_n x[n] exp(i SIGN 2 pi n (lane + 64 t) / N).
@@ -226,60 +152,6 @@ __device__ __forceinline__ void wave_fft(double2 (&v)[R], double2* lds,
     for (int d = 0; d < 8; d++) v[cq + G * d] = o[cq][bitrev(d, 3)];
 }
 
-// Field element access for FP64 or FP32 storage (index in elements).
-template <int F32>
-__device__ __forceinline__ double2 ld_cplx(const void* b, long i) {
-  if (F32) {
-    const float2 v = static_cast<const float2*>(b)[i];
-    return make_double2(v.x, v.y);
-  }
-  return static_cast<const double2*>(b)[i];
-}
-template <int F32>
-__device__ __forceinline__ double ld_real(const void* b, long i) {
-  if (F32) return static_cast<const float*>(b)[i];
-  return static_cast<const double*>(b)[i];
-}
-template <int F32>
-__device__ __forceinline__ void st_cplx(void* b, long i, double2 v) {
-  if (F32)
-    static_cast<float2*>(b)[i] = make_float2((float)v.x, (float)v.y);
-  else
-    static_cast<double2*>(b)[i] = v;
-}
-template <int F32>
-__device__ __forceinline__ void st_real(void* b, long i, double v) {
-  if (F32)
-    static_cast<float*>(b)[i] = (float)v;
-  else
-    static_cast<double*>(b)[i] = v;
-}
-
-// Two consecutive real samples (elements i, i + 1) of a real field.
-template <int F32>
-__device__ __forceinline__ double2 ld_pair(const void* b, long i) {
-  if (F32) {
-    const float2 v = *reinterpret_cast<const float2*>(static_cast<const float*>(b) + i);
-    return make_double2(v.x, v.y);
-  }
-  return *reinterpret_cast<const double2*>(static_cast<const double*>(b) + i);
-}
-
-// Re (op kExprReal) or Im (kExprImag) of a complex sample, and of the two
-// consecutive complex samples i, i + 1 (FP64 storage).
-__device__ __forceinline__ double cplx_part(double2 z, int op) {
-  return op == kExprImag ? z.y : z.x;
-}
-__device__ __forceinline__ double2 cplx_part2(const void* b, long i, int op) {
-  const double2 z0 = static_cast<const double2*>(b)[i];
-  const double2 z1 = static_cast<const double2*>(b)[i + 1];
-  return make_double2(cplx_part(z0, op), cplx_part(z1, op));
-}
-// A real expression of two consecutive samples of each operand.
-__device__ __forceinline__ double2 expr_pair(int op, double2 a, double2 b, double s) {
-  return make_double2(expr_real(op, a.x, b.x, s), expr_real(op, a.y, b.y, s));
-}
-
 __device__ __forceinline__ double2 ld2(const double* p) {
   return *reinterpret_cast<const double2*>(p);
 }
@@ -350,15 +222,17 @@ __global__ __launch_bounds__(64 * synth_waves(R), 2) void fft_synth_w(FFTParams 
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave-uniform
   int fg, theta;
   if (!xcd_pair_map(p.nfg, p.ntheta, fg, theta)) return;
+  if (fg * W * (REAL ? 2 : 1) >= p.nfield) return;  // nfg is rounded up to an even count
   const int f0 = (fg * W + wave) * (REAL ? 2 : 1);
   const bool fv = f0 < p.nfield;
   const bool f1v = REAL && f0 + 1 < p.nfield;
-  const int lmax = p.lmax, m_first = p.m_first;
+  const int m_first = p.m_first;
   const int ncg16 = (p.ncol + 15) >> 4;
   // This thread's share of the cooperative gather: ring c, bins 64 i + bq.
   const int c = tid % W, bq = tid / W;
   const int cf = (fg * W + c) * (REAL ? 2 : 1);
   const bool cv = cf < p.nfield, cv1 = REAL && cf + 1 < p.nfield;
+  const int lmax = ring_lmax(p, cf), lmax1 = ring_lmax(p, cf + 1);
   // Bin (re, im) at element i of F: FP64, or FP32 (FA32: the same indices in
   // a float array) from the split-BF16 synthesis.  FP32 bins are loaded
   // unconditionally (an absent bin reads element f00, slot 0 and column 0 of
@@ -423,15 +297,16 @@ __global__ __launch_bounds__(64 * synth_waves(R), 2) void fft_synth_w(FFTParams 
       for (int i = 0; i < CPH; i++) {
         const int kk = r * BH + 64 * i + bq;
         aok[r][i] = cv && kk <= lmax;
-        bok[r][i] = cv1 && kk <= lmax;
+        bok[r][i] = cv1 && kk <= lmax1;
         sa[r][i] = ldF(aok[r][i], fc + 16 * (long)kk);
         sb[r][i] = ldF(bok[r][i], fc + 16 * (long)kk + 2);
       }
     // Slot N/2 of this ring's pair (register R/2, lane 0).
     const long fw = f_index(theta, 0, 2 * f0, p.nslot, ncg16);
-    const bool nok = fv && lane == 0 && N / 2 <= lmax;
+    const bool nok = fv && lane == 0 && N / 2 <= ring_lmax(p, f0);
+    const bool nok1 = f1v && lane == 0 && N / 2 <= ring_lmax(p, f0 + 1);
     const Bin na = ldF(nok, fw + 16 * (long)(N / 2));
-    const Bin nb = ldF(nok && f1v, fw + 16 * (long)(N / 2) + 2);
+    const Bin nb = ldF(nok1, fw + 16 * (long)(N / 2) + 2);
 #pragma unroll
     for (int r = 0; r < H; r++) {
       if (r > 0) __syncthreads();
@@ -466,7 +341,7 @@ __global__ __launch_bounds__(64 * synth_waves(R), 2) void fft_synth_w(FFTParams 
         v[n1] = in ? X : keep;
       }
     }
-    if (lane == 0) v[R / 2] = make_double2(d2(nok, na).x, d2(nok && f1v, nb).x);
+    if (lane == 0) v[R / 2] = make_double2(d2(nok, na).x, d2(nok1, nb).x);
   }
   // Each wave now works in its own LDS region only.
   wave_fft<R, +1>(v, lds_all + wave * LPW, p.twa, p.tw, lane);
@@ -545,10 +420,11 @@ __global__ __launch_bounds__(64 * anal_waves(R, REAL), 2) void fft_anal_w(FFTPar
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave-uniform
   int fg, theta;
   if (!xcd_pair_map(p.nfg, p.ntheta, fg, theta)) return;
+  if (fg * W * (REAL ? 2 : 1) >= p.nfield) return;  // nfg is rounded up to an even count
   const int f0 = (fg * W + wave) * (REAL ? 2 : 1);
   const bool fv = f0 < p.nfield;
   const bool f1v = REAL && f0 + 1 < p.nfield;
-  const int lmax = p.lmax, m_first = p.m_first;
+  const int m_first = p.m_first;
   double2 v[R];
   double2* lw = lds_all + wave * LPW;
   if constexpr (REAL && R >= 16) {
@@ -670,6 +546,7 @@ __global__ __launch_bounds__(64 * anal_waves(R, REAL), 2) void fft_anal_w(FFTPar
   const int c = tid % W, bq = tid / W;
   const int cf = (fg * W + c) * (REAL ? 2 : 1);
   const bool cv = cf < p.nfield, cv1 = REAL && cf + 1 < p.nfield;
+  const int lmax = ring_lmax(p, cf), lmax1 = ring_lmax(p, cf + 1);
   if (!REAL) {
     // Bin k goes to order k (k <= lmax) or k - N (k >= N - lmax), at
     // fa_index(slot, 2 cf, theta) = slot * (n_cg nquad 64) + that of slot 0;
@@ -715,19 +592,21 @@ __global__ __launch_bounds__(64 * anal_waves(R, REAL), 2) void fft_anal_w(FFTPar
         const int k = r * BH + b;
         if (cv && k <= lmax) {
           st_bin<FA32>(p.F, fa_index(k, 2 * cf, theta, n_cg, nquad), lds_all[c * LPW + xch<W>(c, b)]);
-          if (cv1)
+        }
+        if (cv1 && k <= lmax1) {
             st_bin<FA32>(p.F, fa_index(k, 2 * cf + 2, theta, n_cg, nquad),
                          lds_all[c * LPW + BH + xch<W>(c, b)]);
         }
       }
     }
     // Bin N/2 (lane 0, register R/2) exists only when lmax = N/2.
-    if (fv && N / 2 <= lmax) {
+    const bool na = fv && N / 2 <= ring_lmax(p, f0), nb = f1v && N / 2 <= ring_lmax(p, f0 + 1);
+    if (na || nb) {
       double2 xa, xb;
       separate<R>(v, R / 2, lane, w, p.adjoint, xa, xb);
       if (lane == 0) {
-        st_bin<FA32>(p.F, fa_index(N / 2, 2 * f0, theta, n_cg, nquad), xa);
-        if (f1v) st_bin<FA32>(p.F, fa_index(N / 2, 2 * f0 + 2, theta, n_cg, nquad), xb);
+        if (na) st_bin<FA32>(p.F, fa_index(N / 2, 2 * f0, theta, n_cg, nquad), xa);
+        if (nb) st_bin<FA32>(p.F, fa_index(N / 2, 2 * f0 + 2, theta, n_cg, nquad), xb);
       }
     }
   }
@@ -798,8 +677,8 @@ hipError_t launch_anal_r(const FFTParams& p, hipStream_t s) {
 bool wave_fft_supported(int N) { return N == 512 || N == 1024 || N == 2048; }
 
 // Field groups of a launch (W rings per workgroup, 2 real fields per ring),
-// rounded up to an even count for xcd_pair_map (the extra group's waves
-// transform zeros and store nothing).
+// rounded up to an even count for xcd_pair_map (the workgroups of the extra
+// group leave at once).
 static int field_groups(const FFTParams& p, int W) {
   const int per = W * (p.real ? 2 : 1);
   return ((p.nfield + per - 1) / per + 1) / 2 * 2;

@@ -35,6 +35,8 @@ static_assert(kPass % kCk == 0, "passes start at checkpoints");
 // Work layouts in HBM.  slot indexes the order m (slot = m - m_first;
 // m_first = -lmax for complex fields, 0 for real fields) and
 // col = 2*field + part (part 0 = real, 1 = imaginary).
+// (Calls of at most 8 columns in FP64 keep groups of 2, 4 or 8 columns in
+// place of 16; see cw.)
 //   synthesis  F[theta][col/16][slot][16]: the Legendre kernel writes
 //              F_m(theta) in 128-byte rows of 16 columns, and the ring FFT of
 //              one colatitude and 16-column group reads one contiguous block
@@ -72,11 +74,6 @@ struct LegParams {
   // Null when every seed of the upper index is a normal double or zero.
   const double* sseed;
   const int* skexp;
-  int* ck_flag;     // rec_checkpoints: set to 1 when a lane that started scaled
-                    // reaches a state of magnitude 2^-60 or more before L
-  int ck_restart;   // FP64 synthesis: take the state from the checkpoint
-                    // table every kPass degrees (the table's scaled states
-                    // carry the orders whose seeds underflow)
   // Recurrence coefficients {a, b, c, 0} per (m, l):
   //   e_l = (a cos - b) e_{l-1} - c e_{l-2}
   // rec[roff[m + L] + (l - l0)], l0 <= l <= L + kRecPad, zero beyond L.
@@ -134,9 +131,16 @@ struct LegParams {
   // |m| at the same rows, and tail_reduce writes their sums to the mirrored
   // rows ntheta-1-t.
   int pm;
+  // Paired-order FP64 kernels (gsh_pair.hip): complex fields take orders m
+  // and -m together; kf[(m + L) * nrt + tile]: first checkpoint (0: the seed)
+  // of order m whose 16 degrees matter at the 16 rows of a tile.
+  int cw;    // columns per group of F / FA (see f_index)
+  int pair;
+  int vint;  // virtual columns in tiles of 16, order m and -m in turn
+  const unsigned short* kf;
+  unsigned short* kf_out;
+  int nrt;  // row tiles, ceil(ntheta / 16)
 };
-
-
 
 // Truncation degree and caller index of column field f.
 __device__ __forceinline__ int field_lmax(const LegParams& p, int f) {
@@ -146,10 +150,11 @@ __device__ __forceinline__ int field_index(const int* fmap, int f) {
   return fmap ? fmap[f] : f;
 }
 
-// Index of (theta, slot, col) in the synthesis work layout F (ncg16 =
-// ceil(ncol / 16) column groups).
-__host__ __device__ inline long f_index(int theta, int slot, int col, int nslot, int ncg16) {
-  return (((long)theta * ncg16 + (col >> 4)) * nslot + slot) * 16 + (col & 15);
+// Index of (theta, slot, col) in the synthesis work layout F with column
+// groups of cw (a power of two), ncg = ceil(ncol / cw) of them.
+__host__ __device__ inline long f_index(int theta, int slot, int col, int nslot, int ncg,
+                                        int cw = 16) {
+  return (((long)theta * ncg + (unsigned)col / (unsigned)cw) * nslot + slot) * cw + (col & (cw - 1));
 }
 
 // Load of a wave-uniform table entry through the constant address space, so
@@ -172,9 +177,10 @@ __device__ __forceinline__ uint2 work_item(const uint2* items, int per) {
 }
 
 // Index of (slot, col, theta) in the analysis work layout FA.
-__host__ __device__ inline long fa_index(int slot, int col, int theta, int n_cg, int nquad) {
-  return (((long)slot * n_cg + (col >> 4)) * nquad + (theta >> 2)) * 64 + 16 * (theta & 3) +
-         (col & 15);
+__host__ __device__ inline long fa_index(int slot, int col, int theta, int n_cg, int nquad,
+                                         int cw = 16) {
+  return (((long)slot * n_cg + (unsigned)col / (unsigned)cw) * nquad * 4 + theta) * cw +
+         (col & (cw - 1));
 }
 
 // Pointwise field expressions that the analysis ring FFTs form as they load
@@ -244,7 +250,9 @@ struct FFTParams {
   int L, ntheta, lmax, nslot, ncol, nfield, real, m_first;
   int rings;        // rings per workgroup, rings * M <= 4096
   int nfg;          // field groups
-  int n_cg;         // analysis: 16-column groups, ceil(ncol / 16)
+  int cw;           // columns per group of the bins F / FA: 16, or for the ring
+                    // kernels (gsh_fft_ring.hip) the power of two >= ncol below it
+  int n_cg;         // analysis: column groups, ceil(ncol / cw)
   int nquad;        // analysis: colatitude quads
   const double2* tw;  // tw[k] = exp(-2 pi i k / M), k < M
   const double2* twa; // wavefront FFT: twa[k1 * 64 + j] = exp(-2 pi i j k1 / N), k1 < N / 64
@@ -269,14 +277,32 @@ struct FFTParams {
   long fstride;       // elements between fields
   int f32;            // fields stored in FP32 (float / complex float)
   const int* fmap;    // column field f -> index of the field in the caller's arrays
+  const int* f_lmax;  // truncation degree of column field f (null: lmax): bins past
+                      // it are zero in the synthesis and not written by the analysis
 };
+__device__ __forceinline__ int ring_lmax(const FFTParams& p, int f) {
+  return p.f_lmax && f < p.nfield ? p.f_lmax[f] : p.lmax;
+}
 
-// tiles: 16-column tiles per workgroup (1 or 2; 0 picks 2 when ncol > 16);
-// f32m: FP32 MFMA on FP32-rounded operands with FP32 accumulation (the
-// recurrence and weights stay FP64).
-hipError_t launch_leg_synth_f64(const LegParams& p, hipStream_t s, int tiles = 0,
-                                bool f32m = false);
-hipError_t launch_leg_anal_f64(const LegParams& p, hipStream_t s, bool f32m = false);
+// FP32-MFMA analysis (the recurrence and weights stay FP64).
+hipError_t launch_leg_anal_f32(const LegParams& p, hipStream_t s);
+// Paired-order kernels (gsh_pair.hip) and the tiles of their launches; sym:
+// upper index 0 over the northern rows.
+struct PairTile {
+  int kind = 0;  // matrix instruction (Mma in gsh_pair.hip)
+  int rt = 8;    // row (synthesis) or degree (analysis) tiles per wave
+  int nj = 1;    // column tiles per wave
+  int cols = 0;  // virtual columns per workgroup
+  int vcols = 0; // virtual columns of an order m > 0
+  int vint = 0;  // see LegParams
+  int nblk = 1;  // synthesis: row blocks; analysis: units of 32 degrees per pass
+};
+PairTile pair_synth_tile(int ncol, int pair, int sym, bool f32m, bool uneven, int nr);
+PairTile pair_anal_tile(int ncol, int pair, bool uneven);
+hipError_t launch_leg_synth_pair(const LegParams& p, const PairTile& t, int sym, hipStream_t s);
+hipError_t launch_leg_anal_pair(const LegParams& p, const PairTile& t, int sym, hipStream_t s);
+// Values below this at every row of a tile are left out of the FP64 sums.
+constexpr double kNegligible = 0x1p-120;
 // Recurrence checkpoints of every order of upper index p.n (uses L, ntheta,
 // nabs, cosv, seeds, rec, roff, ck, ckoff).
 hipError_t launch_rec_checkpoints(const LegParams& p, hipStream_t s);
@@ -286,6 +312,10 @@ hipError_t launch_fft_anal(const FFTParams& p, hipStream_t s);
 bool wave_fft_supported(int N);
 hipError_t launch_fft_synth_wave(const FFTParams& p, hipStream_t s);
 hipError_t launch_fft_anal_wave(const FFTParams& p, hipStream_t s);
+// Ring FFTs of any length (gsh_fft_ring.hip) for transform lengths M in 64 ..
+// 4096.
+bool ring_fft_supported(int M);
+hipError_t launch_fft_ring(const FFTParams& p, bool anal, hipStream_t s);
 // Mixed precision kernels (gsh_mixed.hip); ns = 2 (bf16x3) or 3 (bf16x6).
 hipError_t launch_coef_split(const LegParams& p, int ns, hipStream_t s);
 hipError_t launch_leg_synth_bf16(const LegParams& p, int ns, hipStream_t s);

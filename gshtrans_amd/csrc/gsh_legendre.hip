@@ -1,71 +1,39 @@
-// gsh_legendre.hip -- fused Wigner-d recurrence + Legendre contraction on
-// gfx950 FP64 MFMA (v_mfma_f64_16x16x4_f64).
+// gsh_legendre.hip -- recurrence checkpoints, and the FP32-MFMA Legendre
+// analysis, on gfx950.  (The FP64 contractions and the FP32 synthesis are in
+// gsh_pair.hip.)
 //
 // For one order m and upper index n the reference sums, per colatitude ring,
-//   synthesis  F_m(theta_i) = sum_l c_lm D^l_{mn}(theta_i)
-//              (GSHTrans/src/GaussLegendreGrid.h:288-312)
 //   analysis   c_lm = sum_i D^l_{mn}(theta_i) w_i (2 pi / N) X_m(theta_i)
 //              (GaussLegendreGrid.h:181-207)
 // reading D from a precomputed O(L^3) table (Wigner.h:122-130, 305-314).
 // Here D is generated in registers by the three-term recurrence in l
-// (Wigner.h:427-445), one lane per colatitude, and never touches HBM:
+// (Wigner.h:427-445), one lane per colatitude:
 //   e_l = (a_l cos(theta) - b_l) e_{l-1} - c_l e_{l-2},   e_{l0-1} = 0,
 // with e_{l0} the Ortho-normalised seed of Wigner.h:52-95 (computed on the
 // host with the reference's libm expression) and (a, b, c) the recurrence
 // coefficients with the Ortho factor sqrt(2l+1)/(2 sqrt(pi)) folded in.
 //
-// The sums over l (synthesis) or theta (analysis) are dense contractions per
-// order m: (theta x l) . (l x columns) and (l x theta) . (theta x columns),
-// columns = (real, imaginary) x fields.  Recurrence lanes hold one theta
-// each; a per-wave LDS transpose turns them into MFMA operands.  The loop
-// bodies are branch-free (coefficient tables are zero-padded past L and
-// loads past lmax are masked by selects), which keeps the MFMA accumulators
-// resident in AGPRs across iterations.
+// The sums over theta are dense contractions per order m: (l x theta) .
+// (theta x columns), columns = (real, imaginary) x fields.  Recurrence lanes
+// hold one theta each; a per-wave LDS transpose turns them into MFMA operands.
 #include "gsh_internal.h"
 
 namespace gsh {
 namespace {
 
 typedef double d4 __attribute__((ext_vector_type(4)));
-// Recurrence tables are read through the constant address space: they are
-// never written while a kernel runs, and uniform loads from it become scalar
-// (s_load) loads even when the kernel stores to global memory in the loop.
-typedef const __attribute__((address_space(4))) d4 rec_t;
-
 typedef float f4 __attribute__((ext_vector_type(4)));
-
-// The contraction's MFMA and accumulator: FP64 (v_mfma_f64_16x16x4f64; the
-// lane holding column lane%16 holds C rows lane/16 + 4r) or, for the FP32
-// precision mode, v_mfma_f32_16x16x4f32 on FP32-rounded operands with FP32
-// accumulation (C rows 4 (lane/16) + r).  A operand: row lane%16, k
-// lane/16; B operand: k lane/16, column lane%16 (both instructions).
-template <bool F32M>
-struct Mma {
-  typedef d4 acc_t;
-  static __device__ __forceinline__ acc_t zero() { return d4{0.0, 0.0, 0.0, 0.0}; }
-  static __device__ __forceinline__ acc_t mma(double a, double b, acc_t c) {
-    return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
-  }
-  static __device__ __forceinline__ int row(int q, int r) { return q + 4 * r; }
-};
-template <>
-struct Mma<true> {
-  typedef f4 acc_t;
-  static __device__ __forceinline__ acc_t zero() { return f4{0.f, 0.f, 0.f, 0.f}; }
-  static __device__ __forceinline__ acc_t mma(double a, double b, acc_t c) {
-    return __builtin_amdgcn_mfma_f32_16x16x4f32((float)a, (float)b, c, 0, 0, 0);
-  }
-  static __device__ __forceinline__ int row(int q, int r) { return 4 * q + r; }
-};
-
-__device__ __forceinline__ rec_t* rec_ptr(const double4* rec, long off) {
-  return (rec_t*)(rec) + off;
-}
 
 __device__ __forceinline__ void wave_sync() {
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
   __builtin_amdgcn_wave_barrier();
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// A operand: row lane%16, k lane/16; B operand: k lane/16, column lane%16; the
+// lane holding column lane%16 holds C rows 4 (lane/16) + r.
+__device__ __forceinline__ f4 mma(double a, double b, f4 c) {
+  return __builtin_amdgcn_mfma_f32_16x16x4f32((float)a, (float)b, c, 0, 0, 0);
 }
 
 // Order handled by work index mw: complex fields take m = 0, -1, 1, -2, 2, ...
@@ -91,163 +59,9 @@ __device__ __forceinline__ void rec_step(const d4 q, double cs, double& e0, doub
 }
 
 // ---------------------------------------------------------------------------
-// Synthesis.  Workgroup = 4 waves = 256 colatitudes x (16*T) columns for one
-// order.  Per 4 degrees: each lane advances its recurrence 4 steps, the wave
-// transposes the 4 x 64 block through LDS into four 16x4 A operands (one per
-// 16-colatitude group), the coefficients of those 4 degrees form the 4x16 B
-// operands, and 4*T MFMAs accumulate F[theta][col].  Coefficients of the
-// next 4 degrees are loaded one chunk ahead.
-// ---------------------------------------------------------------------------
-template <int T, int REAL, bool F32M>
-__global__ __launch_bounds__(256) void leg_synth_f64(LegParams p) {
-  typedef Mma<F32M> M;
-  __shared__ double tr[4][4][66];
-  const int lane = threadIdx.x & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // wave-uniform
-  // Work item: (order, column group, colatitude super-block).
-  const uint2 it = work_item(p.items, p.items_per);
-  if (it.x == ~0u) return;
-  const int mw = it.x;
-  const int tsb = it.y & 0xffff;
-  const int cg = it.y >> 16;
-  const int m = order_of(mw, REAL);
-  const int slot = m - p.m_first;
-  const int l0 = max(abs(m), p.nabs);
-  const int lmax = p.lmax;
-  const int t = tsb * 256 + wave * 64 + lane;
-  const bool tv = t < p.ntheta;
-  // Branch-free loads at a clamped colatitude keep the control flow uniform.
-  const int tc = min(t, p.ntheta - 1);
-  const double cs0 = p.cosv[tc], s0 = p.seeds[(long)(m + p.L) * p.ntheta + tc];
-  const double cs = tv ? cs0 : 0.0;
-  double e0 = tv ? s0 : 0.0;
-  double e1 = 0.0;
-  const int krow = lane >> 4;
-  // Recurrence coefficients of one 8-degree iteration (entries l+1 .. l+8,
-  // 256 bytes) are staged through a per-wave LDS slot: lanes 0..15 fetch the
-  // next iteration's 16 bytes each one iteration ahead, so the steps never
-  // wait on scalar loads.  Entries up to L + kRecPad exist.
-  __shared__ uint4 rsw[4][16];
-  const uint4* recq = reinterpret_cast<const uint4*>(p.rec + (ld_uniform(p.roff, m + p.L) - l0));
-  auto fetch = [&](int l) { return lane < 16 ? recq[2 * (l + 1) + lane] : make_uint4(0, 0, 0, 0); };
-  const d4* rl = reinterpret_cast<const d4*>(&rsw[wave][0]);  // rl[j]: entry l + 1 + j
-
-  // B-operand column of this lane per column tile.  Every load reads a valid
-  // address (column and degree clamped); out-of-range values are zeroed by a
-  // select when the operand is used, so loads stay in flight across a chunk.
-  // Each column's own truncation degree lf masks its degrees; a column with
-  // lf < l0 (no degree of this order) reads element 0 and is masked out.
-  const double* cptr[T];
-  bool cv[T];
-  int lf[T];
-#pragma unroll
-  for (int j = 0; j < T; j++) {
-    const int col = cg * 16 * T + 16 * j + (lane & 15);
-    cv[j] = col < p.ncol;
-    const int cc = cv[j] ? col : 0;
-    lf[j] = field_lmax(p, cc >> 1);
-    cptr[j] = p.cin + (long)field_index(p.fmap, cc >> 1) * p.cstride * 2 + (cc & 1);
-  }
-  // Degree loop bound of the workgroup: the largest lf of its column groups.
-  int lwg = lmax;
-  if (p.cg_lmax) {
-    lwg = 0;
-#pragma unroll
-    for (int j = 0; j < T; j++)
-      if ((cg * T + j) * 16 < p.ncol) lwg = max(lwg, ld_uniform(p.cg_lmax, cg * T + j));
-  }
-  auto loadB = [&](int l, double* out) {
-#pragma unroll
-    for (int j = 0; j < T; j++) {
-      const int lk = min(l + krow, lf[j]);
-      const long ci = lf[j] >= l0 ? 2 * coef_index(lk, m, p.nabs, REAL) : 0;
-      out[j] = cptr[j][ci];
-    }
-  };
-
-  typename M::acc_t acc[4][T];
-#pragma unroll
-  for (int g = 0; g < 4; g++)
-#pragma unroll
-    for (int j = 0; j < T; j++) acc[g][j] = M::zero();
-
-  // One 4-degree chunk: recurrence, LDS transpose, B mask, 4*T MFMAs; j0 is
-  // the chunk's first entry in the staged coefficients.
-  auto chunk = [&](int l, int j0, double* B) {
-    const d4 q1 = rl[j0], q2 = rl[j0 + 1], q3 = rl[j0 + 2], q4 = rl[j0 + 3];
-    tr[wave][0][lane] = e0;
-    rec_step(q1, cs, e0, e1);
-    tr[wave][1][lane] = e0;
-    rec_step(q2, cs, e0, e1);
-    tr[wave][2][lane] = e0;
-    rec_step(q3, cs, e0, e1);
-    tr[wave][3][lane] = e0;
-    rec_step(q4, cs, e0, e1);
-    wave_sync();
-    double A[4];
-#pragma unroll
-    for (int g = 0; g < 4; g++) A[g] = tr[wave][krow][g * 16 + (lane & 15)];
-    wave_sync();
-    bool lv[T];
-#pragma unroll
-    for (int j = 0; j < T; j++) lv[j] = cv[j] && l + krow <= lf[j];
-#pragma unroll
-    for (int g = 0; g < 4; g++)
-#pragma unroll
-      for (int j = 0; j < T; j++)
-        acc[g][j] = M::mma(A[g], lv[j] ? B[j] : 0.0, acc[g][j]);
-  };
-
-  // Chunks are processed in pairs with ping-pong operand buffers, so each
-  // load has a full chunk of work to hide behind; an odd final chunk is
-  // paired with an all-zero one.
-  double B0[T], B1[T];
-  loadB(l0, B0);
-  uint4 rq = fetch(l0);
-  // With ck_restart the state is taken from the checkpoint table every kPass
-  // degrees (checkpoint (l - l0) / kCk at degree l <= L), loaded a pass ahead.
-  const int nck = (p.L - l0 + kCk) / kCk;  // checkpoints 1 .. nck - 1 exist
-  const double2* ckm = p.ck_restart ? p.ck + ld_uniform(p.ckoff, m + p.L) * (long)p.ntheta + tc
-                                    : nullptr;
-  double2 ckn = make_double2(0.0, 0.0);
-  if (ckm && kPass / kCk < nck) ckn = ckm[(long)(kPass / kCk - 1) * p.ntheta];
-  for (int l = l0; l <= lwg; l += 8) {
-    if (ckm && l > l0 && ((l - l0) & (kPass - 1)) == 0) {
-      const int k = (l - l0) / kCk;
-      if (k < nck) {
-        e0 = tv ? ckn.x : 0.0;
-        e1 = tv ? ckn.y : 0.0;
-        if (k + kPass / kCk < nck) ckn = ckm[(long)(k + kPass / kCk - 1) * p.ntheta];
-      }
-    }
-    if (lane < 16) rsw[wave][lane] = rq;
-    wave_sync();
-    rq = fetch(l + 8);
-    loadB(l + 4, B1);
-    chunk(l, 0, B0);
-    loadB(l + 8, B0);
-    chunk(l + 4, 4, B1);
-  }
-
-  // C layout: the lane holds column lane%16, rows M::row(lane/16, r).
-#pragma unroll
-  for (int g = 0; g < 4; g++)
-#pragma unroll
-    for (int j = 0; j < T; j++) {
-      const int col = cg * 16 * T + 16 * j + (lane & 15);
-      if (col >= p.ncol) continue;
-#pragma unroll
-      for (int r = 0; r < 4; r++) {
-        const int row = tsb * 256 + wave * 64 + g * 16 + M::row(krow, r);
-        if (row < p.ntheta)
-          p.F[f_index(row, slot, col, p.nslot, (p.ncol + 15) >> 4)] = acc[g][j][r];
-      }
-    }
-}
-
-// ---------------------------------------------------------------------------
-// Analysis.  Workgroup = 4 waves for one (order, 16-column group), covering
-// every colatitude.  The colatitudes are cut into quads (the K=4 of one
+// Analysis in FP32 (v_mfma_f32_16x16x4f32 on FP32-rounded operands with FP32
+// accumulation; the recurrence and weights stay FP64).  Workgroup = 4 waves
+// for one (order, 16-column group), covering every colatitude.  The colatitudes are cut into quads (the K=4 of one
 // MFMA); each wave owns MB full blocks of 16 quads (64 lanes), wave w taking
 // blocks w, w+4, ...; the leftover quads (fewer than 64) are dealt round-robin
 // to the waves as a "tail" block.  Per chunk of 64 degrees each wave walks
@@ -262,9 +76,8 @@ __global__ __launch_bounds__(256) void leg_synth_f64(LegParams p) {
 // ---------------------------------------------------------------------------
 constexpr int kAnalLT = 4;  // 16-degree tiles per chunk
 
-template <int MB, bool F32M>
-__global__ __launch_bounds__(256) void leg_anal_f64(LegParams p) {
-  typedef Mma<F32M> M;
+template <int MB>
+__global__ __launch_bounds__(256) void leg_anal_f32(LegParams p) {
   __shared__ double tr[4][16][66];  // also holds the cross-wave reduction
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // wave-uniform
@@ -358,9 +171,9 @@ __global__ __launch_bounds__(256) void leg_anal_f64(LegParams p) {
 
   (void)lwg;
   {
-    typename M::acc_t acc[kAnalLT];
+    f4 acc[kAnalLT];
 #pragma unroll
-    for (int lt = 0; lt < kAnalLT; lt++) acc[lt] = M::zero();
+    for (int lt = 0; lt < kAnalLT; lt++) acc[lt] = f4{0.f, 0.f, 0.f, 0.f};
 
     double Ba[16], Bb[16];
     if (MB > 0) loadBlk(0, Ba);
@@ -376,16 +189,16 @@ __global__ __launch_bounds__(256) void leg_anal_f64(LegParams p) {
 #pragma unroll
         for (int q = 0; q < 16; q++) {
           const double A = tr[wave][lane & 15][4 * q + krow];
-          acc[lt] = M::mma(A, Bcur[q], acc[lt]);
+          acc[lt] = mma(A, Bcur[q], acc[lt]);
         }
         wave_sync();
       }
     }
 
     if (tq > 0) {
-      typename M::acc_t acct[kAnalLT];
+      f4 acct[kAnalLT];
 #pragma unroll
-      for (int lt = 0; lt < kAnalLT; lt++) acct[lt] = M::zero();
+      for (int lt = 0; lt < kAnalLT; lt++) acct[lt] = f4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int lt = 0; lt < kAnalLT; lt++) {
         steps16(rl, lt, cst, e0t, e1t);
@@ -394,7 +207,7 @@ __global__ __launch_bounds__(256) void leg_anal_f64(LegParams p) {
           const int q = (tail0 >> 2) + 4 * i + wave;  // global quad index
           const double Bv = ldB(q);
           const double A = tr[wave][lane & 15][4 * i + krow];
-          acct[lt] = M::mma(A, Bv, acct[lt]);
+          acct[lt] = mma(A, Bv, acct[lt]);
         }
         wave_sync();
       }
@@ -417,7 +230,7 @@ __global__ __launch_bounds__(256) void leg_anal_f64(LegParams p) {
       s += red[((1 * kAnalLT + lt) * 4 + r) * 64 + lane];
       s += red[((2 * kAnalLT + lt) * 4 + r) * 64 + lane];
       s += red[((3 * kAnalLT + lt) * 4 + r) * 64 + lane];
-      const int l = lc + 16 * lt + M::row(krow, r);
+      const int l = lc + 16 * lt + 4 * krow + r;
       if (cv && l <= lf) {
         const long ci = (cbase + coef_index(l, m, p.nabs, p.real)) * 2 + (col & 1);
         double v = s;
@@ -430,12 +243,8 @@ __global__ __launch_bounds__(256) void leg_anal_f64(LegParams p) {
 }
 
 template <int MB>
-hipError_t launch_anal(const LegParams& p, hipStream_t s, bool f32m) {
-  const dim3 grid(8 * p.items_per);
-  if (f32m)
-    hipLaunchKernelGGL((leg_anal_f64<MB, true>), grid, dim3(256), 0, s, p);
-  else
-    hipLaunchKernelGGL((leg_anal_f64<MB, false>), grid, dim3(256), 0, s, p);
+hipError_t launch_anal(const LegParams& p, hipStream_t s) {
+  hipLaunchKernelGGL((leg_anal_f32<MB>), dim3(8 * p.items_per), dim3(256), 0, s, p);
   return hipGetLastError();
 }
 
@@ -464,8 +273,7 @@ __global__ __launch_bounds__(256) void rec_checkpoints(LegParams p) {
   double e0 = p.seeds[(long)mi * nt + tc], e1 = 0.0;
   int kk = p.skexp ? p.skexp[(long)mi * nt + tc] : 0;
   if (kk > 0) e0 = p.sseed[(long)mi * nt + tc];
-  const bool scaled = kk > 0;
-  bool rose = false;  // a scaled lane reached 2^-60
+  int kfirst = kk == 0 && fabs(e0) >= kNegligible ? 0 : 0x7fff;  // first state that matters
   const int nck = (p.L - l0 + kCk) / kCk;
   __shared__ uint4 rs[128];
   const uint4* recq = reinterpret_cast<const uint4*>(p.rec + (ld_uniform(p.roff, mi) - l0));
@@ -493,24 +301,18 @@ __global__ __launch_bounds__(256) void rec_checkpoints(LegParams p) {
     }
     const double s0 = kk > 0 ? ldexp(e0, -kk) : e0;
     const double s1 = kk > 0 ? ldexp(e1, -kk) : e1;
-    rose = rose || (scaled && fabs(s0) >= 0x1p-60);
+    if (kfirst == 0x7fff && (fabs(s0) >= kNegligible || fabs(s1) >= kNegligible)) kfirst = k;
     if (t < nt) out[(long)(k - 1) * nt + t] = make_double2(s0, s1);
   }
-  if (p.ck_flag && t < nt && rose) atomicOr(p.ck_flag, 1);
-}
-
-template <bool F32M>
-hipError_t launch_synth(const LegParams& p, int T, hipStream_t s) {
-  const dim3 nblocks(8 * p.items_per);  // work list: (order, column group, theta block)
-  if (T == 2 && p.real)
-    hipLaunchKernelGGL((leg_synth_f64<2, 1, F32M>), nblocks, dim3(256), 0, s, p);
-  else if (T == 2)
-    hipLaunchKernelGGL((leg_synth_f64<2, 0, F32M>), nblocks, dim3(256), 0, s, p);
-  else if (p.real)
-    hipLaunchKernelGGL((leg_synth_f64<1, 1, F32M>), nblocks, dim3(256), 0, s, p);
-  else
-    hipLaunchKernelGGL((leg_synth_f64<1, 0, F32M>), nblocks, dim3(256), 0, s, p);
-  return hipGetLastError();
+  // kf: the checkpoint before the first state that matters at any of 16 rows
+  // (the degrees up to it are negligible: below the turning point the values
+  // of an order rise with the degree).
+  if (t >= nt) kfirst = 0x7fff;
+#pragma unroll
+  for (int d = 1; d < 16; d <<= 1) kfirst = min(kfirst, __shfl_xor(kfirst, d));
+  if ((threadIdx.x & 15) == 0 && t < nt)
+    p.kf_out[(long)mi * p.nrt + (t >> 4)] =
+        static_cast<unsigned short>(kfirst == 0x7fff ? kfirst : max(kfirst - 1, 0));
 }
 
 }  // namespace
@@ -521,31 +323,23 @@ hipError_t launch_rec_checkpoints(const LegParams& p, hipStream_t s) {
   return hipGetLastError();
 }
 
-hipError_t launch_leg_synth_f64(const LegParams& p0, hipStream_t s, int tiles, bool f32m) {
-  LegParams p = p0;
-  p.n_tsb = (p.ntheta + 255) / 256;
-  const int T = tiles == 1 || tiles == 2 ? tiles : (p.ncol > 16 ? 2 : 1);
-  p.n_cg = (p.ncol + 16 * T - 1) / (16 * T);
-  return f32m ? launch_synth<true>(p, T, s) : launch_synth<false>(p, T, s);
-}
-
-hipError_t launch_leg_anal_f64(const LegParams& p0, hipStream_t s, bool f32m) {
+hipError_t launch_leg_anal_f32(const LegParams& p0, hipStream_t s) {
   if (!p0.ck || !p0.ckoff) return hipErrorInvalidValue;  // checkpoint table required
   LegParams p = p0;
   p.n_cg = (p.ncol + 15) / 16;
   p.nquad = (p.ntheta + 3) / 4;
   const int mb = p.nquad / 64;  // full 16-quad blocks per wave
   switch (mb) {
-    case 0: return launch_anal<0>(p, s, f32m);
-    case 1: return launch_anal<1>(p, s, f32m);
-    case 2: return launch_anal<2>(p, s, f32m);
-    case 3: return launch_anal<3>(p, s, f32m);
-    case 4: return launch_anal<4>(p, s, f32m);
-    case 5: return launch_anal<5>(p, s, f32m);
-    case 6: return launch_anal<6>(p, s, f32m);
-    case 7: return launch_anal<7>(p, s, f32m);
-    case 8: return launch_anal<8>(p, s, f32m);
-    case 9: return launch_anal<9>(p, s, f32m);
+    case 0: return launch_anal<0>(p, s);
+    case 1: return launch_anal<1>(p, s);
+    case 2: return launch_anal<2>(p, s);
+    case 3: return launch_anal<3>(p, s);
+    case 4: return launch_anal<4>(p, s);
+    case 5: return launch_anal<5>(p, s);
+    case 6: return launch_anal<6>(p, s);
+    case 7: return launch_anal<7>(p, s);
+    case 8: return launch_anal<8>(p, s);
+    case 9: return launch_anal<9>(p, s);
     default: return hipErrorInvalidValue;
   }
 }

@@ -1,0 +1,878 @@
+// gsh_pair.hip -- FP64 Legendre contractions (and the FP32-MFMA synthesis)
+// over orders m >= 0, one workgroup for both orders m and -m.
+//
+// The recurrence values of order m >= 0 serve order -m as well, on the
+// equatorially symmetric Gauss-Legendre nodes (Wigner.h:52-95, 386-472):
+//   n = 0   d^l_{-m,0}(t) = (-1)^m d^l_{m,0}(t), and the parity
+//           d^l_{m,0}(pi - t) = (-1)^(l+m) d^l_{m,0}(t): the sums run over the
+//           northern rows only, degrees of even and odd l + m apart (SYM = 1);
+//   n != 0  d^l_{-m,n}(t) = (-1)^(l+n) d^l_{m,n}(pi - t): order -m reads or
+//           writes the mirrored rows with signed coefficients (SYM = 0).
+// So an item's columns are "virtual": 2 nfield columns of order m, then as
+// many of order -m (complex fields, m > 0).
+//
+// What bounds these kernels: on this chip FP64 MFMA and FP64 vector
+// instructions share one pipe (a half-and-half mix of both runs at the sum of
+// their times, 61 of 68 TFLOP/s), so every recurrence step is paid in MFMA
+// time.  The four waves of a workgroup therefore share the recurrence values
+// through LDS: each value is computed once for up to 128 virtual columns
+// (3 FP64 instructions against 128 multiply-adds), 16 degrees at a time from
+// the checkpoint table, one chunk ahead of the MFMAs that use it.
+//
+// Degrees whose values stay below 2^-200 at every row of a tile (near the
+// poles d^l_{mn} is evanescent for l < m / sin t) are left out of the MFMAs:
+// kf[order][row tile] holds the first 16-degree checkpoint that matters.  At
+// lMax = 1024 that is a fifth of the work.  A term of that size changes no
+// sum of doubles unless every other term is below 2^-147 of it; Inf and NaN
+// of the terms left out still reach the result (added as 0 * value).
+#include <algorithm>
+#include <type_traits>
+
+#include "gsh_internal.h"
+
+namespace gsh {
+namespace {
+
+typedef double d4 __attribute__((ext_vector_type(4)));
+typedef float f4 __attribute__((ext_vector_type(4)));
+
+// The matrix instruction: CT columns per tile, 16 rows, K = 4; the lane
+// holding column col(lane) holds the NR rows row(lane, r).  A operand: row
+// lane % 16, k lane / 16; B operand: k lane / 16, column col(lane).
+//   0  v_mfma_f64_16x16x4_f64
+//   1  v_mfma_f32_16x16x4_f32 on FP32-rounded operands
+//   2  v_mfma_f64_4x4x4_4b_f64: four blocks of 4 rows against the same 4
+//      columns, a quarter of the time of 0 (for calls of few columns)
+template <int KIND>
+struct Mma;
+template <>
+struct Mma<0> {
+  typedef double elem;
+  typedef d4 acc;
+  static constexpr int CT = 16, NR = 4;
+  static __device__ __forceinline__ acc mma(double a, double b, acc c) {
+    return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
+  }
+  static __device__ __forceinline__ int row(int lane, int r) { return (lane >> 4) + 4 * r; }
+  static __device__ __forceinline__ double get(const acc& c, int r) { return c[r]; }
+  static __device__ __forceinline__ void add(acc& c, double v) { c += v; }
+};
+template <>
+struct Mma<1> {
+  typedef float elem;
+  typedef f4 acc;
+  static constexpr int CT = 16, NR = 4;
+  static __device__ __forceinline__ acc mma(float a, float b, acc c) {
+    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+  }
+  static __device__ __forceinline__ int row(int lane, int r) { return 4 * (lane >> 4) + r; }
+  static __device__ __forceinline__ double get(const acc& c, int r) { return c[r]; }
+  static __device__ __forceinline__ void add(acc& c, float v) { c += v; }
+};
+template <>
+struct Mma<2> {
+  typedef double elem;
+  typedef double acc;
+  static constexpr int CT = 4, NR = 1;
+  static __device__ __forceinline__ acc mma(double a, double b, acc c) {
+    return __builtin_amdgcn_mfma_f64_4x4x4f64(a, b, c, 0, 0, 0);
+  }
+  static __device__ __forceinline__ int row(int lane, int) {
+    return 4 * ((lane >> 2) & 3) + (lane >> 4);
+  }
+  static __device__ __forceinline__ double get(const acc& c, int) { return c; }
+  static __device__ __forceinline__ void add(acc& c, double v) { c += v; }
+};
+
+// One recurrence step with uniform coefficients {a, b, c} and per-lane cos.
+__device__ __forceinline__ void rec_step(double2 ab, double c, double cs, double& e0, double& e1) {
+  const double t = fma(ab.x, cs, -ab.y);
+  const double en = fma(t, e0, -(c * e1));
+  e1 = e0;
+  e0 = en;
+}
+
+// Coefficient index of (l, m), as in Indexing.h:104-146.
+__device__ __forceinline__ int coef_index(int l, int m, int nabs, int real) {
+  return real ? l * (l + 1) / 2 - nabs * (nabs + 1) / 2 + m : l * l - nabs * nabs + m + l;
+}
+
+// A virtual column of an item: order sign, column, the column's field and its
+// truncation degree.  Columns past the last read column 0 and store nothing.
+struct VCol {
+  bool valid;
+  int sgn;  // 1: order -m
+  int col;  // 2 field + part
+  int lf;   // truncation degree
+  int field;
+};
+// Virtual column v of order m.  Wide launches (vint) interleave tiles of 16
+// columns of order m and of order -m, so that a tile has one order sign and a
+// workgroup's columns belong to few fields; narrow ones append the columns of
+// order -m to those of order m.
+__device__ __forceinline__ VCol vcol(const LegParams& p, int v, int m) {
+  VCol c;
+  const bool two = p.pair && m > 0;
+  if (p.vint) {
+    c.sgn = p.pair ? (v >> 4) & 1 : 0;
+    c.col = p.pair ? (v >> 5) * 16 + (v & 15) : v;
+    c.valid = c.col < p.ncol && (two || !c.sgn);
+  } else {
+    c.valid = v < (two ? 2 * p.ncol : p.ncol);
+    c.sgn = v >= p.ncol ? 1 : 0;
+    c.col = v - c.sgn * p.ncol;
+  }
+  if (!c.valid) c.col = c.sgn = 0;
+  c.lf = field_lmax(p, c.col >> 1);
+  c.field = field_index(p.fmap, c.col >> 1);
+  return c;
+}
+// Largest truncation degree of the virtual columns v0 .. v0 + nv - 1, the
+// first a multiple of 32 when interleaved: the fields of a batch of uneven
+// truncation are ordered by descending degree.
+__device__ __forceinline__ int vcol_lmax(const LegParams& p, int v0, int nv, int m) {
+  int col = v0;
+  if (p.vint && p.pair)
+    col = (v0 >> 5) * 16;
+  else if (p.pair && m > 0 && v0 < p.ncol && v0 + nv > p.ncol)
+    col = 0;
+  else
+    col = v0 % p.ncol;
+  return field_lmax(p, min(col, p.ncol - 1) >> 1);
+}
+// Smallest degree of a wave's columns (wave-uniform).
+__device__ __forceinline__ int wave_min(int v) {
+#pragma unroll
+  for (int d = 1; d < 16; d <<= 1) v = min(v, __shfl_xor(v, d));
+  return __builtin_amdgcn_readfirstlane(v);
+}
+
+
+// Narrow tiles multiply for a few hundred cycles per chunk, which hides
+// neither a load nor the barrier: they keep one D buffer (two barriers per
+// chunk) and run four workgroups per CU instead of two.
+constexpr int nbuf(int kind, int tiles) { return kind == 2 || tiles <= 2 ? 1 : 2; }
+// Workgroups per CU (waves per SIMD) that the registers are cut to.
+constexpr int waves(int kind, int tiles, int nj) {
+  return nbuf(kind, tiles) == 2 ? 2 : kind != 2 && nj == 2 ? 3 : 4;
+}
+
+// ---------------------------------------------------------------------------
+// Synthesis.  An item is (m, row block, group of virtual columns); the 4
+// waves share the D values of (32 degrees) x (RT WR + 1 row tiles) and split
+// the tile: WR row groups of RT row tiles x WC column groups of NJ column
+// tiles.  Wave w produces degrees 16 (w / 2) .. + 15 of each chunk for 64
+// rows; the last row group takes one row tile more where the block has it
+// (ntheta = 2^k + 1 would otherwise leave a block of one row).  SYM: one
+// column tile per wave, the even and odd degrees in accumulators of their own.
+//
+// Beside the MFMAs every vector instruction costs about 3 of an MFMA's 72
+// cycles (measured, two waves per SIMD), so the coefficient loads step one
+// byte offset per 4 degrees and mask nothing until a column's last degrees.
+// ---------------------------------------------------------------------------
+template <int KIND, int SYM, int RT, int NJ>
+__global__ __launch_bounds__(256, waves(KIND, RT, SYM ? 2 : NJ)) void leg_synth_p(LegParams p) {
+  typedef Mma<KIND> M;
+  typedef typename M::elem E;
+  constexpr int WR = RT == 2 ? 4 : RT <= 4 ? 2 : 1;
+  constexpr int WC = 4 / WR;
+  constexpr int TW = RT * WR;      // row tiles of a block without the extra one
+  constexpr int NH = 2;            // 16-degree segments of a chunk
+  constexpr int SC = kCk * NH;     // degrees per chunk
+  // Elements per degree row in LDS: 9 row tiles, padded so that the A operands
+  // of both forms spread over all banks.
+  constexpr int SP = 152;
+  constexpr int NB = SYM ? 2 : NJ; // accumulators per row tile
+  constexpr int NC = SYM ? 1 : NJ; // column tiles per wave
+  constexpr int NBUF = nbuf(KIND, RT);
+  __shared__ E D[NBUF][SC * SP];
+  __shared__ uint4 rs[2][2 * SC];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wr = wave / WC, wc = wave % WC;
+  const uint2 it = work_item(p.items, p.items_per);
+  if (it.x == ~0u) return;
+  const int m = it.x, tb = it.y & 0xffff, cg = it.y >> 16;
+  const int nt = p.ntheta, nr = SYM ? (nt + 1) / 2 : nt;
+  const int rtt = (nr + 15) >> 4;
+  // Blocks 0 .. next - 1 have TW + 1 row tiles, the others TW.
+  const int next = max(0, rtt - p.n_tsb * TW);
+  const int tile0 = tb * TW + min(tb, next);
+  const int ntile = min(TW + (tb < next ? 1 : 0), rtt - tile0);
+  const bool ext = ntile > TW;
+  const int l0 = max(m, p.nabs);
+  const int krow = lane >> 4;
+
+  // Columns of this wave.
+  const int vb = cg * (WC * NC * M::CT);  // first virtual column of the block
+  VCol vc[NC];
+  const char* cbase[NC];  // (l, m) of order m at cbase + 16 coef_index(l, m)
+  int lmin = 1 << 20;
+#pragma unroll
+  for (int j = 0; j < NC; j++) {
+    vc[j] = vcol(p, vb + (wc * NC + j) * M::CT + lane % M::CT, m);
+    cbase[j] = reinterpret_cast<const char*>(p.cin + (long)vc[j].field * p.cstride * 2 +
+                                             (vc[j].col & 1)) -
+               (vc[j].sgn ? 32l * m : 0);
+    lmin = min(lmin, vc[j].lf);
+  }
+  lmin = wave_min(lmin);
+  const int lwg = vcol_lmax(p, vb, WC * NC * M::CT, m);
+
+  // First checkpoint that matters for the block's rows.
+  int ks = 1 << 20;
+  {
+    const unsigned short* kf = p.kf + (long)(m + p.L) * p.nrt + tile0;
+    for (int i = 0; i < ntile; i++) ks = min(ks, (int)ld_uniform(kf, i));
+  }
+  ks = min(ks, max(0, lwg - l0 + kCk) / kCk);
+  const int ls = l0 + kCk * ks;
+  const int nchunk = ls > lwg ? 0 : (lwg - ls + SC) / SC;
+
+  // Coefficient loads: accumulator b reads degree l + d (d = krow, or SYM
+  // 2 krow + b) of every ST-th degree l, GB loads per 16 degrees.  A group
+  // of 16 degrees from l with l + 15 <= lmin is inside every column's degrees
+  // (plain()); its byte offset off[b] steps by an arithmetic progression.  The
+  // others clamp each load to a valid address, and operand() masks them.
+  constexpr int ST = SYM ? 8 : 4;
+  constexpr int GB = SYM ? 2 : 4;
+  constexpr int NO = SYM ? 2 : 1;  // offsets: order -m shares order m's
+  unsigned off[NO], step[NO];
+  unsigned sgn[NC];  // sign bit of order -m (SYM0: the parity of l is the lane's)
+#pragma unroll
+  for (int b = 0; b < NO; b++) {
+    const int l = l0 + (SYM ? 2 * krow + b : krow);
+    off[b] = 16u * coef_index(l, m, p.nabs, p.real);
+    step[b] = (SYM ? 16 * l + 72 : 8 * l + 20) * (p.real ? 8u : 16u);
+  }
+  const unsigned sinc = (SYM ? 128 : 32) * (p.real ? 8u : 16u);
+#pragma unroll
+  for (int j = 0; j < NC; j++)
+    sgn[j] = vc[j].sgn && ((SYM ? m : l0 + krow + p.n) & 1) ? 0x80000000u : 0u;
+  auto plain = [&](int l) { return l + kCk - 1 <= lmin; };
+  auto load_group = [&](int l, double (&B)[GB][NB]) {
+    if (plain(l)) {
+#pragma unroll
+      for (int g = 0; g < GB; g++) {
+#pragma unroll
+        for (int b = 0; b < NB; b++)
+          B[g][b] = *reinterpret_cast<const double*>(cbase[SYM ? 0 : b] + off[SYM ? b : 0]);
+#pragma unroll
+        for (int b = 0; b < NO; b++) {
+          off[b] += step[b];
+          step[b] += sinc;
+        }
+      }
+    } else {
+#pragma unroll
+      for (int g = 0; g < GB; g++)
+#pragma unroll
+        for (int b = 0; b < NB; b++) {
+          const VCol& c = vc[SYM ? 0 : b];
+          const int ll = min(l + ST * g + (SYM ? 2 * krow + b : krow), c.lf);
+          // A field without a degree of this order reads its element 0.
+          const long o = c.lf >= l0 ? 16l * coef_index(ll, m, p.nabs, p.real) : c.sgn ? 32l * m : 0;
+          B[g][b] = *reinterpret_cast<const double*>(cbase[SYM ? 0 : b] + o);
+        }
+    }
+  };
+  // Operand of accumulator b from the raw load of group g of the 16 degrees
+  // from l (mask: not plain(l)).  SYM: the sign of order -m goes to the result.
+  auto operand = [&](auto mask, double v, int b, int l, int g) -> E {
+    if (!SYM) {
+      uint2 u = __builtin_bit_cast(uint2, v);
+      u.y ^= sgn[SYM ? 0 : b];
+      v = __builtin_bit_cast(double, u);
+    }
+    if (decltype(mask)::value && l + ST * g + (SYM ? 2 * krow + b : krow) > vc[SYM ? 0 : b].lf)
+      v = 0.0;
+    return (E)v;
+  };
+
+  // Degrees left out: 0 * value.
+  E pz[NB];
+#pragma unroll
+  for (int b = 0; b < NB; b++) pz[b] = (E)0;
+  for (int l = l0; l < ls; l += kCk) {
+    double t[GB][NB];
+    load_group(l, t);
+#pragma unroll
+    for (int g = 0; g < GB; g++)
+#pragma unroll
+      for (int b = 0; b < NB; b++) pz[b] += (E)0 * operand(std::true_type{}, t[g][b], b, l, g);
+  }
+
+  // Production: wave -> (16-degree segment, 64 rows), and for the extra row
+  // tile lanes 0..15 of waves 0 and 2.
+  const int seg = wave >> 1;
+  const int prow = 64 * (wave & 1) + lane;
+  const bool xprod = ext && TW == 8 && !(wave & 1);
+  constexpr int XR = 16 * TW;  // first row of the extra tile
+  const int t = 16 * tile0 + prow, tx = 16 * tile0 + XR + (lane & 15);
+  const bool tv = t < nr, txv = xprod && lane < 16 && tx < nr;
+  const double cs = tv ? p.cosv[t] : 0.0, csx = txv ? p.cosv[tx] : 0.0;
+  const int nck = (p.L - l0 + kCk) / kCk;  // checkpoints 1 .. nck - 1 exist
+  const double* seedm = p.seeds + (long)(m + p.L) * nt;
+  const double2* ckm = p.ck + ld_uniform(p.ckoff, m + p.L) * (long)nt;
+  auto state = [&](int c, bool v, int row) -> double2 {
+    const int k = ks + NH * c + seg;
+    double2 s = make_double2(0.0, 0.0);
+    if (k < nck && v) {
+      if (k == 0)
+        s.x = seedm[row];
+      else
+        s = ckm[(long)(k - 1) * nt + row];
+    }
+    return s;
+  };
+  const uint4* recq = reinterpret_cast<const uint4*>(p.rec + (ld_uniform(p.roff, m + p.L) - l0));
+  auto fetch_rec = [&](int c) {
+    return tid < 2 * SC ? recq[2 * (ls + SC * c + 1) + tid] : make_uint4(0, 0, 0, 0);
+  };
+  auto produce = [&](int c, double2 s, double csv, int row) {
+    const double2* r = reinterpret_cast<const double2*>(rs[c & 1]) + 2 * kCk * seg;
+    E* d = D[NBUF == 2 ? c & 1 : 0] + (kCk * seg) * SP + row;
+    double e0 = s.x, e1 = s.y;
+#pragma unroll 4
+    for (int j = 0; j < kCk; j++) {
+      d[j * SP] = (E)e0;
+      rec_step(r[2 * j], r[2 * j + 1].x, csv, e0, e1);
+    }
+  };
+
+  typename M::acc acc[RT + 1][NB];
+#pragma unroll
+  for (int i = 0; i <= RT; i++)
+#pragma unroll
+    for (int b = 0; b < NB; b++) acc[i][b] = typename M::acc{};
+  const bool xt = ext && wr == WR - 1;  // this wave has the extra row tile
+
+  double B[NH][GB][NB];
+  // MFMAs of the 16 degrees from l (half h of chunk c) for N row tiles: no
+  // branch inside, so that the LDS reads of later steps overlap the MFMAs.
+  auto mma_group = [&](auto nrow, auto mask, int c, int h, double (&Bh)[GB][NB]) {
+    constexpr int N = decltype(nrow)::value;
+    const int l = ls + SC * c + kCk * h;
+    const E* d = D[NBUF == 2 ? c & 1 : 0] + (kCk * h) * SP + 16 * (wr * RT) + (lane & 15);
+#pragma unroll
+    for (int g = 0; g < GB; g++) {
+      E X[NB];
+#pragma unroll
+      for (int j = 0; j < NB; j++) X[j] = operand(mask, Bh[g][j], j, l, g);
+#pragma unroll
+      for (int b = 0; b < (SYM ? 2 : 1); b++) {
+        const E* dr = d + (SYM ? 8 * g + 2 * krow + b : 4 * g + krow) * SP;
+#pragma unroll
+        for (int i = 0; i < N; i++) {
+          const E A = dr[16 * i];
+          if (SYM) {
+            acc[i][b] = M::mma(A, X[b], acc[i][b]);
+          } else {
+#pragma unroll
+            for (int j = 0; j < NB; j++) acc[i][j] = M::mma(A, X[j], acc[i][j]);
+          }
+        }
+      }
+    }
+  };
+
+  if (nchunk > 0) {
+#pragma unroll
+    for (int h = 0; h < NH; h++) load_group(ls + kCk * h, B[h]);
+    double2 st = state(0, tv, t), sx = state(0, txv, tx);
+    if (tid < 2 * SC) rs[0][tid] = fetch_rec(0);
+    uint4 rq = make_uint4(0, 0, 0, 0);
+    __syncthreads();
+    // Chunk c + 1 is produced (NBUF 1: chunk c) while its state and
+    // recurrence coefficients for the chunk after it are on their way.
+    auto advance = [&](int c) {
+      produce(c, st, cs, prow);
+      if (xprod && lane < 16) produce(c, sx, csx, XR + lane);
+      if (c + 1 < nchunk) {
+        st = state(c + 1, tv, t);
+        sx = state(c + 1, txv, tx);
+        // rs[(c + 1) & 1] was last read producing chunk c - 1, a barrier ago.
+        if (tid < 2 * SC) rs[(c + 1) & 1][tid] = rq;
+        if (c + 2 < nchunk) rq = fetch_rec(c + 2);
+      }
+    };
+    if (nchunk > 1) rq = fetch_rec(1);
+    if (NBUF == 2) advance(0);
+    // The chunks inside every column's degrees, then the others.
+    const int nplain = min(nchunk, max(0, lmin + 1 - ls) / SC);
+    auto run = [&](auto nrow, auto mask, int ca, int cb) {
+      for (int c = ca; c < cb; c++) {
+        __syncthreads();
+        if (NBUF == 2) {
+          if (c + 1 < nchunk) advance(c + 1);
+        } else {
+          advance(c);
+          __syncthreads();
+        }
+#pragma unroll
+        for (int h = 0; h < NH; h++) {
+          if (!decltype(mask)::value || ls + SC * c + kCk * h <= lwg)
+            mma_group(nrow, mask, c, h, B[h]);
+          if (c + 1 < nchunk) load_group(ls + SC * (c + 1) + kCk * h, B[h]);
+        }
+      }
+    };
+    if (xt) {
+      run(std::integral_constant<int, RT + 1>{}, std::false_type{}, 0, nplain);
+      run(std::integral_constant<int, RT + 1>{}, std::true_type{}, nplain, nchunk);
+    } else {
+      run(std::integral_constant<int, RT>{}, std::false_type{}, 0, nplain);
+      run(std::integral_constant<int, RT>{}, std::true_type{}, nplain, nchunk);
+    }
+  }
+
+  // 0 * (degrees left out), summed over the operand rows of each column.
+  if (ls > l0) {
+#pragma unroll
+    for (int b = 0; b < NB; b++) {
+      E z = pz[b];
+      z += __shfl_xor(z, 16);
+      z += __shfl_xor(z, 32);
+#pragma unroll
+      for (int i = 0; i <= RT; i++) M::add(acc[i][b], z);
+    }
+  }
+
+  // Store: order m at row t, order -m at the mirrored row (n != 0).
+  const int ncg = (p.ncol + p.cw - 1) / p.cw;
+#pragma unroll
+  for (int i = 0; i <= RT; i++) {
+    if (i == RT && !xt) continue;
+#pragma unroll
+    for (int j = 0; j < NC; j++) {
+      if (!vc[j].valid) continue;
+      const int slot = (vc[j].sgn ? -m : m) - p.m_first;
+#pragma unroll
+      for (int r = 0; r < M::NR; r++) {
+        const int tr = 16 * (wr * RT + i) + M::row(lane, r);
+        const int row = 16 * tile0 + tr;
+        if (tr >= 16 * ntile || row >= nr) continue;
+        if (SYM) {
+          double e = M::get(acc[i][0], r), o = M::get(acc[i][1], r);
+          if (sgn[j]) {
+            e = -e;
+            o = -o;
+          }
+          p.F[f_index(row, slot, vc[j].col, p.nslot, ncg, p.cw)] = e + o;
+          if (nt - 1 - row != row)
+            p.F[f_index(nt - 1 - row, slot, vc[j].col, p.nslot, ncg, p.cw)] = e - o;
+        } else {
+          p.F[f_index(vc[j].sgn ? nt - 1 - row : row, slot, vc[j].col, p.nslot, ncg, p.cw)] =
+              M::get(acc[i][j], r);
+        }
+      }
+    }
+  }
+}
+
+// ---------------------------------------------------------------------------
+// Analysis.  An item is (m, pass, group of virtual columns): a pass covers up
+// to 128 degrees (nu units of 32), walking the rows in chunks of 32.  Thread
+// (seg, row) produces 16 degrees of the next chunk from its checkpoint.  The 4 waves
+// split the pass: WR degree groups of LT tiles x WC column groups of NJ tiles.
+// SYM: the rows run over the north, a degree tile holds 16 degrees of one
+// parity, multiplied with X(t) +- X(nt-1-t).
+// ---------------------------------------------------------------------------
+template <int KIND, int SYM, int LT, int NJ>
+__global__ __launch_bounds__(256, waves(KIND, LT, NJ)) void leg_anal_p(LegParams p) {
+  typedef Mma<KIND> M;
+  constexpr int WR = 8 / LT, WC = 4 / WR;
+  constexpr int NBUF = nbuf(KIND, LT);
+  constexpr int PD = 128;             // degrees per pass
+  constexpr int PU = PD / 32;         // units per pass
+  constexpr int CR = 32;              // rows per chunk
+  constexpr int AP = CR + 2;          // elements per degree row in LDS
+  constexpr int NQ = CR / 4;          // quads per chunk
+  __shared__ double D[NBUF][PD * AP];
+  __shared__ uint4 rs[2 * PD];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wr = wave / WC, wc = wave % WC;
+  const uint2 it = work_item(p.items, p.items_per);
+  if (it.x == ~0u) return;
+  const int m = it.x, pass = it.y & 0xffff, cg = it.y >> 16;
+  const int nt = p.ntheta, nr = SYM ? (nt + 1) / 2 : nt;
+  const int l0 = max(m, p.nabs);
+  const int krow = lane >> 4;
+  const int vb = cg * (WC * NJ * M::CT);
+  // B operands: row 4 q + krow (mirrored for order -m; SYM: the row and its
+  // mirror) of a column of FA, whose rows are cw elements apart.
+  constexpr int NL = SYM ? 2 * NJ : NJ;
+  const int cw = KIND == 0 && NJ == 2 ? 16 : p.cw;  // more than 8 columns: 16
+  VCol vc[NJ];
+  const double* fb[NL];  // lane's row of quad 0
+  int fs[NL];            // elements per quad
+  int lw = -1;           // largest degree of this wave's columns
+#pragma unroll
+  for (int j = 0; j < NJ; j++) {
+    vc[j] = vcol(p, vb + (wc * NJ + j) * M::CT + lane % M::CT, m);
+    const int slot = (vc[j].sgn ? -m : m) - p.m_first;
+    const double* f0 = p.F + fa_index(slot, vc[j].col, 0, p.n_cg, p.nquad, cw);
+    if (SYM) {
+      fb[2 * j] = f0 + cw * krow;
+      fs[2 * j] = 4 * cw;
+      fb[2 * j + 1] = f0 + cw * (nt - 1 - krow);
+      fs[2 * j + 1] = -4 * cw;
+    } else {
+      fb[j] = vc[j].sgn ? f0 + cw * (nt - 1 - krow) : f0 + cw * krow;
+      fs[j] = vc[j].sgn ? -4 * cw : 4 * cw;
+    }
+    lw = max(lw, vc[j].valid ? vc[j].lf : -1);
+  }
+  lw = -wave_min(-lw);
+  const int lwg = vcol_lmax(p, vb, WC * NJ * M::CT, m);
+  if (l0 > lwg) return;
+  // Units of 32 degrees, PU to a pass (the last pass takes what is left).
+  const int U = (lwg - l0 + 32) >> 5;
+  const int u0 = PU * pass, nu = min(U - u0, PU);
+  if (nu <= 0) return;
+  const int lp = l0 + 32 * u0;
+
+  // Rows that matter: chunks c0 .. c1 (chunks past 64 always run).
+  const int nch = (nr + CR - 1) / CR;
+  const int nrt = (nr + 15) >> 4;
+  const unsigned short* kf = p.kf + (long)(m + p.L) * p.nrt;
+  int c0, c1 = nch - 1;
+  {
+    const int kend = 2 * u0 + 2 * nu;
+    bool live = false;
+    if (lane < nch)
+#pragma unroll
+      for (int i = 0; i < CR / 16; i++) live = live || kf[min(CR / 16 * lane + i, nrt - 1)] < kend;
+    const unsigned long long b = __ballot(live);
+    c0 = b ? __builtin_ctzll(b) : min(nch, 64);
+    if (nch <= 64 && b) c1 = 63 - __builtin_clzll(b);
+  }
+
+  if (tid < 64 * nu)
+    rs[tid] = reinterpret_cast<const uint4*>(p.rec + (ld_uniform(p.roff, m + p.L) - l0))
+        [2 * (lp + 1) + tid];
+
+  // Production: thread -> (16-degree segment, row of the chunk).
+  const int seg = tid / CR, prow = tid % CR;
+  const int nck = (p.L - l0 + kCk) / kCk;
+  const int kk = 2 * u0 + seg;
+  const bool pv = seg < 2 * nu && kk < nck;
+  const double* seedm = p.seeds + (long)(m + p.L) * nt;
+  const double2* ckm = p.ck + (ld_uniform(p.ckoff, m + p.L) + kk - 1) * (long)nt;
+  double cs = 0.0;
+  auto state = [&](int c) -> double2 {
+    const int row = CR * c + prow;
+    double2 s = make_double2(0.0, 0.0);
+    cs = 0.0;
+    if (pv && row < nr) {
+      cs = p.cosv[row];
+      if (kk == 0)
+        s.x = seedm[row];
+      else
+        s = ckm[row];
+    }
+    return s;
+  };
+  // Row of degree 16 seg + j of the pass in LDS: SYM keeps the two parities
+  // of a unit of 32 degrees apart.
+  auto produce = [&](int buf, double2 s) {
+    if ((64 / CR) * wave >= 2 * nu) return;  // the wave's segments are past the pass
+    const double2* r = reinterpret_cast<const double2*>(rs) + 2 * kCk * seg;
+    double* d = D[buf] + (SYM ? 32 * (seg >> 1) + 8 * (seg & 1) : 16 * seg) * AP + prow;
+    double e0 = s.x, e1 = s.y;
+#pragma unroll 4
+    for (int j = 0; j < kCk; j++) {
+      d[(SYM ? 16 * (j & 1) + (j >> 1) : j) * AP] = e0;
+      rec_step(r[2 * j], r[2 * j + 1].x, cs, e0, e1);
+    }
+  };
+
+  // Quads q .. of full() groups lie strictly inside the rows (SYM: of the
+  // north, without the equator); the last ones are clamped to valid rows (rows
+  // past the last have D = 0, and SYM takes the equator once).
+  const int nfull = (SYM ? nt / 2 : nt) >> 2;
+  auto load_quads = [&](int q, auto& B) {
+    constexpr int N = sizeof(B) / sizeof(B[0]);
+    if (q + N <= nfull) {
+#pragma unroll
+      for (int j = 0; j < NL; j++)
+#pragma unroll
+        for (int g = 0; g < N; g++) B[g][j] = fb[j][(q + g) * fs[j]];
+    } else {
+#pragma unroll
+      for (int g = 0; g < N; g++) {
+        const int back = max(0, 4 * (q + g) + krow - (nt - 1));  // rows past the last
+#pragma unroll
+        for (int j = 0; j < NL; j++)
+          B[g][j] = fb[j][(q + g) * fs[j] + (fs[j] > 0 ? -cw : cw) * back];
+      }
+    }
+  };
+
+  typename M::acc acc[LT][NJ];
+#pragma unroll
+  for (int i = 0; i < LT; i++)
+#pragma unroll
+    for (int j = 0; j < NJ; j++) acc[i][j] = typename M::acc{};
+
+  const int nq = (nr + 3) >> 2;
+  // Rows left out: 0 * value.
+  double pz[NJ];
+#pragma unroll
+  for (int j = 0; j < NJ; j++) pz[j] = 0.0;
+  for (int c = 0; c < nch; c++) {
+    if (c == c0) c = c1 + 1;
+    if (c >= nch) break;
+    double b[4][NL];
+#pragma unroll
+    for (int h = 0; h < NQ / 4; h++) {
+      load_quads(NQ * c + 4 * h, b);
+#pragma unroll
+      for (int q = 0; q < 4; q++)
+#pragma unroll
+        for (int j = 0; j < NL; j++) pz[SYM ? j >> 1 : j] += 0.0 * b[q][j];
+    }
+  }
+
+  constexpr int GQ = SYM ? 2 : 4;  // quads per group of loads
+  constexpr int NG = NQ / GQ;
+  // This wave's units: those of its degree group, up to its columns' degrees.
+  constexpr int WU = LT / 2;
+  const int mine = min(min(nu, (lw - lp + 32) >> 5) - wr * WU, WU);
+  double Bq[2][GQ][NL];
+  // All degree tiles of the wave (whole), or those of its units: tiles past
+  // the pass are skipped in pairs.
+  auto run_group = [&](auto whole, auto full, int buf, int c, int h, double (&B)[GQ][NL]) {
+    const double* d = D[buf] + (16 * LT * wr + (lane & 15)) * AP + 4 * GQ * h + krow;
+#pragma unroll
+    for (int g = 0; g < GQ; g++) {
+      double X[2][NJ];
+#pragma unroll
+      for (int j = 0; j < NJ; j++) {
+        if (SYM) {
+          const double a = B[g][2 * j];
+          double b = B[g][2 * j + 1];
+          if (!decltype(full)::value) {
+            const int row = 4 * (NQ * c + GQ * h + g) + krow;
+            b = nt - 1 - row > row ? b : 0.0;
+          }
+          X[0][j] = a + b;
+          X[1][j] = a - b;
+        } else {
+          X[0][j] = B[g][j];
+        }
+      }
+      double A[LT];
+#pragma unroll
+      for (int i = 0; i < LT; i++) A[i] = d[16 * i * AP + 4 * g];
+#pragma unroll
+      for (int u = 0; u < WU; u++)
+        if (decltype(whole)::value || u < mine) {
+#pragma unroll
+          for (int i = 2 * u; i < 2 * u + 2; i++)
+#pragma unroll
+            for (int j = 0; j < NJ; j++) acc[i][j] = M::mma(A[i], X[SYM ? i & 1 : 0][j], acc[i][j]);
+        }
+    }
+  };
+
+  __syncthreads();
+  if (c0 <= c1) {
+    load_quads(NQ * c0, Bq[0]);
+    double2 st = state(c0);
+    if (NBUF == 2) {
+      produce(0, st);
+      if (c0 < c1) st = state(c0 + 1);
+    }
+    // The chunks whose rows lie strictly inside, then the last.
+    const int cfull = min(c1 + 1, nfull / NQ);
+    auto run = [&](auto whole, auto full, int ca, int cb) {
+      for (int c = ca; c < cb; c++) {
+        const int buf = NBUF == 2 ? (c - c0) & 1 : 0;
+        __syncthreads();
+        load_quads(NQ * c + GQ, Bq[1]);
+        if (NBUF == 2) {
+          if (c < c1) {
+            produce(buf ^ 1, st);
+            if (c + 1 < c1) st = state(c + 2);
+          }
+        } else {
+          produce(0, st);
+          if (c < c1) st = state(c + 1);
+          __syncthreads();
+        }
+#pragma unroll
+        for (int h = 0; h < NG; h++) {
+          if (decltype(full)::value || NQ * c + GQ * h < nq)
+            run_group(whole, full, buf, c, h, Bq[h & 1]);
+          if (h + 2 < NG)
+            load_quads(NQ * c + GQ * (h + 2), Bq[h & 1]);
+          else if (h + 2 == NG && c < c1)
+            load_quads(NQ * (c + 1), Bq[0]);
+        }
+      }
+    };
+    if (mine == WU) {
+      run(std::true_type{}, std::true_type{}, c0, cfull);
+      run(std::true_type{}, std::false_type{}, max(c0, cfull), c1 + 1);
+    } else {
+      run(std::false_type{}, std::true_type{}, c0, cfull);
+      run(std::false_type{}, std::false_type{}, max(c0, cfull), c1 + 1);
+    }
+  }
+
+#pragma unroll
+  for (int j = 0; j < NJ; j++) {
+    double z = pz[j];
+    z += __shfl_xor(z, 16);
+    z += __shfl_xor(z, 32);
+#pragma unroll
+    for (int i = 0; i < LT; i++) M::add(acc[i][j], z);
+  }
+
+#pragma unroll
+  for (int i = 0; i < LT; i++) {
+    if (i >= 2 * mine) continue;
+#pragma unroll
+    for (int j = 0; j < NJ; j++) {
+      if (!vc[j].valid) continue;
+      const int mo = vc[j].sgn ? -m : m;
+      double* co = p.cout + ((long)vc[j].field * p.cstride) * 2 + (vc[j].col & 1);
+#pragma unroll
+      for (int r = 0; r < M::NR; r++) {
+        const int tile = wr * LT + i, mr = M::row(lane, r);
+        const int l = lp + (SYM ? 32 * (tile >> 1) + 2 * mr + (tile & 1) : 16 * tile + mr);
+        if (l > vc[j].lf) continue;
+        double v = M::get(acc[i][j], r);
+        if (vc[j].sgn && ((SYM ? m : l + p.n) & 1)) v = -v;
+        const long ci = 2 * (long)coef_index(l, mo, p.nabs, p.real);
+        if (p.accumulate) v += co[ci];
+        if (p.zero_last && vc[j].lf == p.L && l == p.L && mo == p.L) v = 0.0;
+        co[ci] = v;
+      }
+    }
+  }
+}
+
+template <int KIND, int SYM, int RT, int NJ>
+hipError_t go_synth(const LegParams& p, hipStream_t s) {
+  hipLaunchKernelGGL((leg_synth_p<KIND, SYM, RT, NJ>), dim3(8 * p.items_per), dim3(256), 0, s, p);
+  return hipGetLastError();
+}
+template <int KIND, int SYM, int LT, int NJ>
+hipError_t go_anal(const LegParams& p, hipStream_t s) {
+  hipLaunchKernelGGL((leg_anal_p<KIND, SYM, LT, NJ>), dim3(8 * p.items_per), dim3(256), 0, s, p);
+  return hipGetLastError();
+}
+
+}  // namespace
+
+// Tile of a launch: ncol columns (twice that many virtual ones when paired),
+// nr rows, uneven: fields of different truncation degrees.  Wider tiles share
+// each recurrence value and each A operand among more columns; the narrow
+// ones keep the matrix unit off padding columns: at most 4 (8) columns take
+// the 4-column instruction, at most 16 (32, 64) one (two, four) tiles of 16;
+// more are interleaved by order sign.  Uneven batches stop at 64, whose 16
+// fields have neighbouring degrees.  The rows of a block are 6 or 8 tiles,
+// whichever covers the launch's row tiles with less left over.
+static PairTile pair_tile(int ncol, int pair, bool f32m, bool uneven) {
+  PairTile t;
+  const int V = ncol * (pair ? 2 : 1);
+  t.kind = f32m ? 1 : V <= 8 ? 2 : 0;
+  t.vint = V > 32 ? 1 : 0;
+  t.vcols = t.vint ? (ncol + 15) / 16 * 16 * (pair ? 2 : 1) : V;
+  t.rt = t.kind == 2 || V <= 32 ? 2 : t.vcols <= 64 || uneven ? 4 : 8;
+  t.nj = V <= 16 ? 1 : 2;
+  return t;
+}
+PairTile pair_synth_tile(int ncol, int pair, int sym, bool f32m, bool uneven, int nr) {
+  PairTile t = pair_tile(ncol, pair, f32m, uneven);
+  if (t.kind == 2) {
+    t.nj = 1;
+    if (t.vcols > 4) t.rt = 4;
+  } else if (sym) {  // one column tile per wave
+    if (t.vcols <= 16) t.rt = 2;
+    else if (t.vcols <= 32) t.rt = 4;
+    else t.rt = 8;
+    t.nj = 1;
+  }
+  const int rtt = (nr + 15) / 16;
+  const int wr = 8 / t.rt, wc = 4 / wr;
+  t.cols = wc * t.nj * (t.kind == 2 ? 4 : 16);
+  // Blocks of tw row tiles, each with room for one more.
+  auto blocks = [rtt](int tw) { return std::max(1, (rtt + tw) / (tw + 1)); };
+  t.nblk = blocks(8);
+  if (t.kind == 0 && t.rt >= 4) {
+    const int n6 = blocks(6), n8 = blocks(8);
+    const int c6 = std::max(6 * n6, rtt), c8 = std::max(8 * n8, rtt);
+    if (c6 < c8) {
+      t.rt = t.rt == 8 ? 6 : 3;
+      t.nblk = n6;
+    }
+  }
+  return t;
+}
+PairTile pair_anal_tile(int ncol, int pair, bool uneven) {
+  PairTile t = pair_tile(ncol, pair, false, uneven);
+  if (t.kind == 2) t.nj = t.vcols <= 4 ? 1 : 2;
+  t.nblk = 4;  // units of 32 degrees per pass
+  const int wr = 8 / t.rt, wc = 4 / wr;
+  t.cols = wc * t.nj * (t.kind == 2 ? 4 : 16);
+  return t;
+}
+
+hipError_t launch_leg_synth_pair(const LegParams& p0, const PairTile& t, int sym, hipStream_t s) {
+  if (!p0.ck || !p0.ckoff || !p0.kf) return hipErrorInvalidValue;  // checkpoint table required
+  LegParams p = p0;
+  p.n_tsb = t.nblk;
+  p.vint = t.vint;
+  if (t.kind == 1) {
+    if (sym) return hipErrorInvalidValue;
+    if (t.rt == 8) return go_synth<1, 0, 8, 2>(p, s);
+    if (t.rt == 4) return go_synth<1, 0, 4, 2>(p, s);
+    return t.nj == 2 ? go_synth<1, 0, 2, 2>(p, s) : go_synth<1, 0, 2, 1>(p, s);
+  }
+  if (t.kind == 2) {
+    if (sym) return t.rt == 2 ? go_synth<2, 1, 2, 1>(p, s) : go_synth<2, 1, 4, 1>(p, s);
+    return t.rt == 2 ? go_synth<2, 0, 2, 1>(p, s) : go_synth<2, 0, 4, 1>(p, s);
+  }
+  if (sym) switch (t.rt) {
+      case 8: return go_synth<0, 1, 8, 1>(p, s);
+      case 6: return go_synth<0, 1, 6, 1>(p, s);
+      case 4: return go_synth<0, 1, 4, 1>(p, s);
+      case 3: return go_synth<0, 1, 3, 1>(p, s);
+      default: return go_synth<0, 1, 2, 1>(p, s);
+    }
+  switch (t.rt) {
+    case 8: return go_synth<0, 0, 8, 2>(p, s);
+    case 6: return go_synth<0, 0, 6, 2>(p, s);
+    case 4: return go_synth<0, 0, 4, 2>(p, s);
+    case 3: return go_synth<0, 0, 3, 2>(p, s);
+    default: return t.nj == 2 ? go_synth<0, 0, 2, 2>(p, s) : go_synth<0, 0, 2, 1>(p, s);
+  }
+}
+
+hipError_t launch_leg_anal_pair(const LegParams& p0, const PairTile& t, int sym, hipStream_t s) {
+  if (!p0.ck || !p0.ckoff || !p0.kf) return hipErrorInvalidValue;
+  LegParams p = p0;
+  p.vint = t.vint;
+  p.n_cg = (p.ncol + p.cw - 1) / p.cw;
+  p.nquad = (p.ntheta + 3) / 4;
+  if (t.kind == 2) {
+    if (sym) return t.nj == 1 ? go_anal<2, 1, 2, 1>(p, s) : go_anal<2, 1, 2, 2>(p, s);
+    return t.nj == 1 ? go_anal<2, 0, 2, 1>(p, s) : go_anal<2, 0, 2, 2>(p, s);
+  }
+  if (sym) switch (t.rt) {
+      case 8: return go_anal<0, 1, 8, 2>(p, s);
+      case 4: return go_anal<0, 1, 4, 2>(p, s);
+      default: return t.nj == 2 ? go_anal<0, 1, 2, 2>(p, s) : go_anal<0, 1, 2, 1>(p, s);
+    }
+  switch (t.rt) {
+    case 8: return go_anal<0, 0, 8, 2>(p, s);
+    case 4: return go_anal<0, 0, 4, 2>(p, s);
+    default: return t.nj == 2 ? go_anal<0, 0, 2, 2>(p, s) : go_anal<0, 0, 2, 1>(p, s);
+  }
+}
+
+}  // namespace gsh

@@ -1,0 +1,97 @@
+"""The paired-order FP64 kernels (gsh_pair.hip) and the ring FFTs of any length
+(gsh_fft_ring.hip) at the edges of their tiles, against the CPU oracle.
+
+Bar: relative L2 <= 1e-12, that of the FP64 parity tests (sums of at most a
+few hundred terms of rounding 1.1e-16 each).
+"""
+import sys
+
+import numpy as np
+import pytest
+
+import gshtrans_amd as G
+import oracle
+
+pytestmark = pytest.mark.gpu
+SEED0 = 20261205
+
+
+def say(*a):
+    print(*a, file=sys.stderr, flush=True)
+
+
+def rel(a, b):
+    return float(np.linalg.norm(np.ravel(a - b)) / np.linalg.norm(np.ravel(b)))
+
+
+@pytest.fixture(scope="module")
+def torch():
+    import torch as _t
+    assert _t.cuda.is_available(), "GPU tests need a device"
+    return _t
+
+
+def check(torch, L, lmax, n, real, batch):
+    say(f"[pair] L={L} lmax={lmax} n={n} real={real} batch={batch}")
+    g = G.GaussLegendreGrid(L, min(2, L))
+    og = oracle.OracleGrid(L, min(2, L), table=False)
+    c = G.random_coefficients(lmax, n, real=real, seed=SEED0 + L + batch, grid_lmax=L, batch=batch)
+    f = g.inverse(lmax, n, torch.from_numpy(c).cuda(), real=real)
+    a = g.forward(lmax, n, f, real=real)
+    fh, ah = f.cpu().numpy(), a.cpu().numpy()
+    for i in sorted({0, batch // 2, batch - 1}):  # first, middle and last columns
+        ref = og.inverse(lmax, n, c[i], real=real)
+        assert rel(fh[i], ref) <= 1e-12, i
+        assert rel(ah[i], og.forward(lmax, n, fh[i], real=real)) <= 1e-12, i
+
+
+# Columns: 2 batch (real) or 4 batch (complex) virtual columns, around the
+# tile widths 4, 8, 16, 32, 64 and 128; rows around 16, 96, 112, 128 and 144
+# (n = 0: half of them); degrees around the chunks of 32 and passes of 128.
+@pytest.mark.parametrize("batch", [1, 2, 3, 4, 5, 8, 9, 16, 17, 33])
+@pytest.mark.parametrize("n,real", [(0, True), (0, False), (1, True), (-2, False)])
+def test_column_tiles(torch, n, real, batch):
+    check(torch, 40, 33, n, real, batch)
+
+
+@pytest.mark.parametrize("L,lmax", [(15, 15), (16, 16), (95, 64), (111, 96), (127, 127), (128, 128),
+                                    (143, 129), (144, 144), (255, 250), (287, 160)])
+@pytest.mark.parametrize("n,real,batch", [(0, True, 3), (2, False, 1), (-1, False, 20)])
+def test_row_and_degree_tiles(torch, L, lmax, n, real, batch):
+    check(torch, L, lmax, n, real, batch)
+
+
+# Ring lengths 2 L at the edges of each transform length: powers of two (64 ..
+# 1024 points), and the shortest and longest that Bluestein's convolution of
+# 64 .. 4096 points serves.
+@pytest.mark.parametrize("L", [17, 18, 31, 32, 33, 63, 64, 65, 128, 129, 255, 256, 257, 511, 512,
+                               513])
+@pytest.mark.parametrize("real", [False, True])
+def test_ring_lengths(torch, L, real):
+    check(torch, L, min(L, 40), 0 if real else 1, real, 2)
+    check(torch, L, L, 0 if real else -1, real, 1)
+
+
+@pytest.mark.parametrize("n,real", [(0, True), (0, False), (2, False), (1, True)])
+@pytest.mark.parametrize("bad", [float("nan"), float("inf")])
+def test_left_out_terms_stay_visible(torch, n, real, bad):
+    """Near the poles the high orders' values are negligible and their terms
+    are left out; an Inf or NaN among them still makes the field (the
+    coefficients) it belongs to non-finite, and no other field of the batch."""
+    L = 300
+    g = G.GaussLegendreGrid(L, 2)
+    c = torch.from_numpy(G.random_coefficients(L, n, real=real, seed=SEED0, batch=3)).cuda()
+    f = g.inverse(L, n, c, real=real)
+    a = g.forward(L, n, f, real=real)
+    say(f"[pair] non-finite n={n} real={real} {bad}")
+    c[1, G.coefficient_index(L, n, 150, 149, real)] = bad
+    g.inverse(L, n, c, field=f, real=real)
+    finite = torch.isfinite(torch.view_as_real(f) if f.is_complex() else f).reshape(3, -1)
+    assert finite[0].all() and finite[2].all() and not finite[1].any()
+    f = torch.nan_to_num(f, nan=1.0, posinf=1.0, neginf=1.0)
+    f[1, 1, 5] = bad  # a sample next to the pole
+    g.forward(L, n, f, coeffs=a, real=real)
+    finite = torch.isfinite(torch.view_as_real(a)).reshape(3, -1, 2)
+    assert finite[0].all() and finite[2].all()
+    # (L, L) of a complex field is zeroed
+    assert not finite[1, :-1].all(dim=-1).any()
