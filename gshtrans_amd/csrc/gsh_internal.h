@@ -151,10 +151,11 @@ __device__ __forceinline__ int field_index(const int* fmap, int f) {
 }
 
 // Index of (theta, slot, col) in the synthesis work layout F with column
-// groups of cw (a power of two), ncg = ceil(ncol / cw) of them.
+// groups of cw (16, or a smaller power of two >= ncol), ncg = ceil(ncol / cw)
+// of them.
 __host__ __device__ inline long f_index(int theta, int slot, int col, int nslot, int ncg,
                                         int cw = 16) {
-  return (((long)theta * ncg + (unsigned)col / (unsigned)cw) * nslot + slot) * cw + (col & (cw - 1));
+  return (((long)theta * ncg + (cw == 16 ? col >> 4 : 0)) * nslot + slot) * cw + (col & (cw - 1));
 }
 
 // Load of a wave-uniform table entry through the constant address space, so
@@ -179,7 +180,7 @@ __device__ __forceinline__ uint2 work_item(const uint2* items, int per) {
 // Index of (slot, col, theta) in the analysis work layout FA.
 __host__ __device__ inline long fa_index(int slot, int col, int theta, int n_cg, int nquad,
                                          int cw = 16) {
-  return (((long)slot * n_cg + (unsigned)col / (unsigned)cw) * nquad * 4 + theta) * cw +
+  return (((long)slot * n_cg + (cw == 16 ? col >> 4 : 0)) * nquad * 4 + theta) * cw +
          (col & (cw - 1));
 }
 

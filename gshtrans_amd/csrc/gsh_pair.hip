@@ -189,9 +189,9 @@ __global__ __launch_bounds__(256, waves(KIND, RT, SYM ? 2 : NJ)) void leg_synth_
   __shared__ uint4 rs[2][2 * SC];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int wr = wave / WC, wc = wave % WC;
   const uint2 it = work_item(p.items, p.items_per);
   if (it.x == ~0u) return;
+  const int wr = wave / WC, wc = wave % WC;
   const int m = it.x, tb = it.y & 0xffff, cg = it.y >> 16;
   const int nt = p.ntheta, nr = SYM ? (nt + 1) / 2 : nt;
   const int rtt = (nr + 15) >> 4;
@@ -207,7 +207,7 @@ __global__ __launch_bounds__(256, waves(KIND, RT, SYM ? 2 : NJ)) void leg_synth_
   const int vb = cg * (WC * NC * M::CT);  // first virtual column of the block
   VCol vc[NC];
   const char* cbase[NC];  // (l, m) of order m at cbase + 16 coef_index(l, m)
-  int lmin = 1 << 20;
+  int lmin = 1 << 20, lww = -1;  // smallest and largest degree of the wave's columns
 #pragma unroll
   for (int j = 0; j < NC; j++) {
     vc[j] = vcol(p, vb + (wc * NC + j) * M::CT + lane % M::CT, m);
@@ -215,8 +215,10 @@ __global__ __launch_bounds__(256, waves(KIND, RT, SYM ? 2 : NJ)) void leg_synth_
                                              (vc[j].col & 1)) -
                (vc[j].sgn ? 32l * m : 0);
     lmin = min(lmin, vc[j].lf);
+    lww = max(lww, vc[j].valid ? vc[j].lf : -1);
   }
   lmin = wave_min(lmin);
+  lww = -wave_min(-lww);
   const int lwg = vcol_lmax(p, vb, WC * NC * M::CT, m);
 
   // First checkpoint that matters for the block's rows.
@@ -411,9 +413,9 @@ __global__ __launch_bounds__(256, waves(KIND, RT, SYM ? 2 : NJ)) void leg_synth_
         }
 #pragma unroll
         for (int h = 0; h < NH; h++) {
-          if (!decltype(mask)::value || ls + SC * c + kCk * h <= lwg)
+          if (!decltype(mask)::value || ls + SC * c + kCk * h <= lww)
             mma_group(nrow, mask, c, h, B[h]);
-          if (c + 1 < nchunk) load_group(ls + SC * (c + 1) + kCk * h, B[h]);
+          if (ls + SC * (c + 1) + kCk * h <= lww) load_group(ls + SC * (c + 1) + kCk * h, B[h]);
         }
       }
     };
@@ -439,14 +441,15 @@ __global__ __launch_bounds__(256, waves(KIND, RT, SYM ? 2 : NJ)) void leg_synth_
   }
 
   // Store: order m at row t, order -m at the mirrored row (n != 0).
-  const int ncg = (p.ncol + p.cw - 1) / p.cw;
+  const long frow = f_index(1, 0, 0, p.nslot, (p.ncol + p.cw - 1) / p.cw, p.cw);  // F per row
 #pragma unroll
-  for (int i = 0; i <= RT; i++) {
-    if (i == RT && !xt) continue;
+  for (int j = 0; j < NC; j++) {
+    if (!vc[j].valid) continue;
+    double* f = p.F + f_index(0, (vc[j].sgn ? -m : m) - p.m_first, vc[j].col, p.nslot, 0, p.cw);
+    const bool mirrored = !SYM && vc[j].sgn;
 #pragma unroll
-    for (int j = 0; j < NC; j++) {
-      if (!vc[j].valid) continue;
-      const int slot = (vc[j].sgn ? -m : m) - p.m_first;
+    for (int i = 0; i <= RT; i++) {
+      if (i == RT && !xt) continue;
 #pragma unroll
       for (int r = 0; r < M::NR; r++) {
         const int tr = 16 * (wr * RT + i) + M::row(lane, r);
@@ -458,12 +461,10 @@ __global__ __launch_bounds__(256, waves(KIND, RT, SYM ? 2 : NJ)) void leg_synth_
             e = -e;
             o = -o;
           }
-          p.F[f_index(row, slot, vc[j].col, p.nslot, ncg, p.cw)] = e + o;
-          if (nt - 1 - row != row)
-            p.F[f_index(nt - 1 - row, slot, vc[j].col, p.nslot, ncg, p.cw)] = e - o;
+          f[row * frow] = e + o;
+          if (nt - 1 - row != row) f[(nt - 1 - row) * frow] = e - o;
         } else {
-          p.F[f_index(vc[j].sgn ? nt - 1 - row : row, slot, vc[j].col, p.nslot, ncg, p.cw)] =
-              M::get(acc[i][j], r);
+          f[(mirrored ? nt - 1 - row : row) * frow] = M::get(acc[i][j], r);
         }
       }
     }
@@ -492,9 +493,9 @@ __global__ __launch_bounds__(256, waves(KIND, LT, NJ)) void leg_anal_p(LegParams
   __shared__ uint4 rs[2 * PD];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int wr = wave / WC, wc = wave % WC;
   const uint2 it = work_item(p.items, p.items_per);
   if (it.x == ~0u) return;
+  const int wr = wave / WC, wc = wave % WC;
   const int m = it.x, pass = it.y & 0xffff, cg = it.y >> 16;
   const int nt = p.ntheta, nr = SYM ? (nt + 1) / 2 : nt;
   const int l0 = max(m, p.nabs);
@@ -794,7 +795,7 @@ PairTile pair_synth_tile(int ncol, int pair, int sym, bool f32m, bool uneven, in
   } else if (sym) {  // one column tile per wave
     if (t.vcols <= 16) t.rt = 2;
     else if (t.vcols <= 32) t.rt = 4;
-    else t.rt = 8;
+    else t.rt = uneven ? 4 : 8;
     t.nj = 1;
   }
   const int rtt = (nr + 15) / 16;
@@ -816,6 +817,7 @@ PairTile pair_synth_tile(int ncol, int pair, int sym, bool f32m, bool uneven, in
 PairTile pair_anal_tile(int ncol, int pair, bool uneven) {
   PairTile t = pair_tile(ncol, pair, false, uneven);
   if (t.kind == 2) t.nj = t.vcols <= 4 ? 1 : 2;
+  if (uneven) t.rt = 2;
   t.nblk = 4;  // units of 32 degrees per pass
   const int wr = 8 / t.rt, wc = 4 / wr;
   t.cols = wc * t.nj * (t.kind == 2 ? 4 : 16);
