@@ -633,7 +633,8 @@ int ensure_synth_worklist(gsh_grid_s* g, int family, int lmax, int real, int ngr
 }
 
 // Work list of a paired-order FP64 launch (gsh_pair.hip): items (m, sub | group
-// << 16) for m >= 0 and groups of t.cols virtual columns; sub is the row
+// << 16, the order's offsets in the checkpoint and recurrence tables) for m >= 0
+// and groups of t.cols virtual columns; sub is the row
 // block of a synthesis (dir 0) or the pass of an analysis (dir 1).  Units of 8
 // neighbouring orders and one group go whole to the least loaded XCD, heaviest
 // first: the coefficients of neighbouring orders at a degree share cache
@@ -654,8 +655,24 @@ int ensure_pair_worklist(gsh_grid_s* g, int dir, int lmax, int n, int pair, int 
   constexpr int kBand = 8;
   struct Unit {
     double w;
-    std::vector<uint2> items;
+    std::vector<uint4> items;
   };
+  // The offsets that ensure_ndata (roff) and ensure_ck (ckoff) give orders
+  // 0 .. lmax, in entries and rows.
+  const int L = g->L, na = std::abs(n);
+  std::vector<unsigned> ckrow(lmax + 1), rec0(lmax + 1);
+  {
+    unsigned row = 0, ent = 0;
+    for (int m = -L; m <= lmax; m++) {
+      const int l0 = std::max(std::abs(m), na);
+      if (m >= 0) {
+        ckrow[m] = row;
+        rec0[m] = ent;
+      }
+      row += std::max(0, (L - l0 + gsh::kCk) / gsh::kCk - 1);
+      ent += L - l0 + 1 + gsh::kRecPad;
+    }
+  }
   std::vector<Unit> units;
   for (int b0 = 0; b0 <= lmax; b0 += kBand) {
     const int b1 = std::min(b0 + kBand, lmax + 1);
@@ -686,15 +703,16 @@ int ensure_pair_worklist(gsh_grid_s* g, int dir, int lmax, int n, int pair, int 
       for (int sub = 0; sub < smax; sub++)
         for (int m = b0; m < b1; m++)
           if (sub < subs[m - b0])
-            u.items.push_back(make_uint2(static_cast<unsigned>(m),
+            u.items.push_back(make_uint4(static_cast<unsigned>(m),
                                          static_cast<unsigned>(sub) |
-                                             (static_cast<unsigned>(grp) << 16)));
+                                             (static_cast<unsigned>(grp) << 16),
+                                         ckrow[m], rec0[m]));
       if (!u.items.empty()) units.push_back(std::move(u));
     }
   }
   std::stable_sort(units.begin(), units.end(),
                    [](const Unit& a, const Unit& b) { return a.w > b.w; });
-  std::vector<uint2> xcd[8];
+  std::vector<uint4> xcd[8];
   double load[8] = {};
   for (const Unit& u : units) {
     const int x = static_cast<int>(std::min_element(load, load + 8) - load);
@@ -703,16 +721,16 @@ int ensure_pair_worklist(gsh_grid_s* g, int dir, int lmax, int n, int pair, int 
   }
   size_t per = 1;
   for (const auto& v : xcd) per = std::max(per, v.size());
-  std::vector<uint2> items;
+  std::vector<uint4> items;
   items.reserve(8 * per);
   for (auto& v : xcd) {
-    v.resize(per, make_uint2(~0u, 0u));
+    v.resize(per, make_uint4(~0u, 0u, 0u, 0u));
     items.insert(items.end(), v.begin(), v.end());
   }
   WorkList w;
   w.per = static_cast<int>(per);
-  GSH_HIP(hipMalloc(&w.d, items.size() * sizeof(uint2)));
-  GSH_HIP(hipMemcpy(w.d, items.data(), items.size() * sizeof(uint2), hipMemcpyHostToDevice));
+  GSH_HIP(hipMalloc(&w.d, items.size() * sizeof(uint4)));
+  GSH_HIP(hipMemcpy(w.d, items.data(), items.size() * sizeof(uint4), hipMemcpyHostToDevice));
   g->worklists.emplace(key, w);
   *out = w;
   return GSH_OK;
@@ -949,7 +967,9 @@ int gsh_grid_create(int lmax, int nmax, int mrange, int nrange, gsh_grid_t* grid
     cs[i] = std::cos(g->theta[i]);
     wq[i] = g->weight[i] * scale;
   }
-  const int M = N > 0 ? fft_length(N) : 1;
+  // Rings of fewer than 64 points go through Bluestein's convolution of 64,
+  // the shortest transform of the ring kernels.
+  const int M = N > 0 ? std::max(64, fft_length(N)) : 1;
   g->M = M;
   std::vector<double2> tw(M);
   for (int k = 0; k < M; k++) {
@@ -1121,7 +1141,7 @@ int bin_columns(int ncol, int precision) {
 // Ring FFTs of a call.  The wavefront kernels (N = 512, 1024, 2048) move bins
 // for 8 complex rings (16 real ones) of a colatitude at a time; calls of at
 // most 4 fields, other lengths and o.fft = 2 take the ring kernels, and
-// transforms of fewer than 64 or more than 4096 points the general ones.
+// transforms of more than 4096 points the LDS kernels.
 hipError_t run_fft(const FFTParams& q, const RunOpts& o, bool anal, hipStream_t s) {
   if (use_wave_fft(q, o) && q.nfield > 4 && q.cw == 16)
     return anal ? gsh::launch_fft_anal_wave(q, s) : gsh::launch_fft_synth_wave(q, s);
@@ -1304,6 +1324,7 @@ int run_forward(gsh_grid_s* g, NData* d, int lmax, int n, int real, int precisio
   q.F = p.F = mixed ? reinterpret_cast<double*>(reinterpret_cast<float*>(g->work) + gsh::kFAFrontPad)
                     : g->work;
   q.fa32 = mixed ? 1 : 0;
+  q.zero_pad = precision != GSH_FP64 ? 1 : 0;
   p.FA32 = mixed ? reinterpret_cast<const float*>(q.F) : nullptr;
   if ((st = ensure_ck(g, d, n, s))) return st;
   p.ck = d->ck;

@@ -288,7 +288,7 @@ __global__ __launch_bounds__(kFFTThreads) void fft_anal(FFTParams p) {
     }
     // The last ring also zeroes the padding rows of the last colatitude
     // quad, which the Legendre contraction reads as B operands.
-    for (int tp = theta + 1; theta == p.ntheta - 1 && tp < 4 * p.nquad; tp++) {
+    for (int tp = theta + 1; p.zero_pad && theta == p.ntheta - 1 && tp < 4 * p.nquad; tp++) {
       const long zi = fa_index(s, 2 * f, tp, p.n_cg, p.nquad, p.cw);
       if (p.fa32) {
         reinterpret_cast<float*>(p.F)[zi] = 0.0f;

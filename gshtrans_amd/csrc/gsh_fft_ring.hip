@@ -71,21 +71,40 @@ __device__ __forceinline__ void dft_half(double2* u) {
       }
 }
 
+// The table entries that the passes of one transform start their twiddle
+// powers from, loaded before anything waits (a load inside a pass would add
+// its latency to the chain of exchanges): entry q of pass i >= 1 is
+// exp(-2 pi i (j % Ns) / (Ns R)), j = t + T q.
+template <int M, bool REV>
+struct Twiddles {
+  double2 w[2][4];
+  __device__ __forceinline__ Twiddles(const double2* tw, int t) {
+    int ns = REV ? radix_rev(M, 0) : radix(M, 0);
+#pragma unroll
+    for (int i = 1; i < npass(M); i++) {
+      const int R = REV ? radix_rev(M, i) : radix(M, i);
+#pragma unroll
+      for (int q = 0; q < 16 / R; q++)
+        w[i - 1][q] = tw[((t + M / 16 * q) & (ns - 1)) * (M / (ns * R))];
+      ns *= R;
+    }
+  }
+};
+
 // One Stockham pass of radix R after Ns points are done: butterflies j = t +
 // T q, q < 16 / R, each over v[q + (16 / R) i].  LAST passes leave the result
 // in place; the others go through LDS.
 template <int M, int SIGN, int R, int NS, bool LAST, bool HALF>
-__device__ __forceinline__ void pass(double2 (&v)[16], double2* lds, const double2* tw, int t) {
+__device__ __forceinline__ void pass(double2 (&v)[16], double2* lds, const double2* w1, int t) {
   constexpr int T = M / 16, Q = 16 / R, LR = log2c(R);
 #pragma unroll
   for (int q = 0; q < Q; q++) {
-    const int j = t + T * q;
     double2 u[R];
 #pragma unroll
     for (int i = 0; i < R; i++) u[i] = v[q + Q * i];
     if (NS > 1) {
       double2 w[R];
-      w[1] = tw[(j & (NS - 1)) * (M / (NS * R))];
+      w[1] = w1[q];
 #pragma unroll
       for (int i = 2; i < R; i++) w[i] = cmul(w[i / 2], w[i - i / 2]);
 #pragma unroll
@@ -116,45 +135,43 @@ __device__ __forceinline__ void pass(double2 (&v)[16], double2* lds, const doubl
 // M-point transform of v[e] = x[t + T e]; on return v[e] = X[t + T e].  REV
 // runs the radices in reverse order; HALF: x[k] = 0 for k >= M / 2.
 template <int M, int SIGN, bool REV, bool HALF>
-__device__ __forceinline__ void ring_fft(double2 (&v)[16], double2* lds, const double2* tw, int t) {
+__device__ __forceinline__ void ring_fft(double2 (&v)[16], double2* lds,
+                                         const Twiddles<M, REV>& tw, int t) {
   constexpr int R0 = REV ? radix_rev(M, 0) : radix(M, 0);
   constexpr int R1 = REV ? radix_rev(M, 1) : radix(M, 1);
-  pass<M, SIGN, R0, 1, false, HALF>(v, lds, tw, t);
+  pass<M, SIGN, R0, 1, false, HALF>(v, lds, nullptr, t);
   if constexpr (npass(M) == 2) {
-    pass<M, SIGN, R1, R0, true, false>(v, lds, tw, t);
+    pass<M, SIGN, R1, R0, true, false>(v, lds, tw.w[0], t);
   } else {
     constexpr int R2 = REV ? radix_rev(M, 2) : radix(M, 2);
-    pass<M, SIGN, R1, R0, false, false>(v, lds, tw, t);
-    pass<M, SIGN, R2, R0 * R1, true, false>(v, lds, tw, t);
+    pass<M, SIGN, R1, R0, false, false>(v, lds, tw.w[0], t);
+    pass<M, SIGN, R2, R0 * R1, true, false>(v, lds, tw.w[1], t);
   }
 }
 
 // Unnormalised N-point DFT of the ring held as v[e] = x[t + T e] (zero from N
 // on): direct (BLUE 0, M = N) or Bluestein's.
 template <int M, int BLUE, int SIGN>
-__device__ __forceinline__ void ring_dft(double2 (&v)[16], double2* lds, const FFTParams& p, int t) {
-  if (!BLUE) {
-    ring_fft<M, SIGN, false, false>(v, lds, p.tw, t);
-    return;
-  }
-  constexpr int T = M / 16;
-  const int N = p.N;
-  double2 ch[8];
+__device__ __forceinline__ void ring_dft(double2 (&v)[16], double2* lds, const FFTParams& p,
+                                         const Twiddles<M, false>& tw, int t) {
+  if constexpr (!BLUE) {
+    ring_fft<M, SIGN, false, false>(v, lds, tw, t);
+  } else {
+    constexpr int T = M / 16;
+    auto chirp = [&](int e) {
+      const double2 c = p.chirp[min(t + T * e, p.N - 1)];
+      v[e] = SIGN < 0 ? cmul(v[e], c) : cmulc(v[e], c);
+    };
 #pragma unroll
-  for (int e = 0; e < 8; e++) {
-    const int k = t + T * e;
-    ch[e] = p.chirp[min(k, N - 1)];
-    v[e] = SIGN < 0 ? cmul(v[e], ch[e]) : cmulc(v[e], ch[e]);
-  }
-  ring_fft<M, -1, false, true>(v, lds, p.tw, t);
-  const double2* h = SIGN < 0 ? p.hf : p.hb;
+    for (int e = 0; e < 8; e++) chirp(e);
+    ring_fft<M, -1, false, true>(v, lds, tw, t);
+    const double2* h = SIGN < 0 ? p.hf : p.hb;
+    const Twiddles<M, true> rev(p.tw, t);
 #pragma unroll
-  for (int e = 0; e < 16; e++) v[e] = cmul(v[e], h[t + T * e]);
-  ring_fft<M, +1, true, false>(v, lds, p.tw, t);
+    for (int e = 0; e < 16; e++) v[e] = cmul(v[e], h[t + T * e]);
+    ring_fft<M, +1, true, false>(v, lds, rev, t);
 #pragma unroll
-  for (int e = 0; e < 8; e++) {
-    const double2 c = p.chirp[min(t + T * e, N - 1)];
-    v[e] = SIGN < 0 ? cmul(v[e], c) : cmulc(v[e], c);
+    for (int e = 0; e < 8; e++) chirp(e);
   }
 }
 
@@ -217,6 +234,7 @@ __global__ __launch_bounds__(Ring<M>::kThreads) void fft_synth_r(FFTParams p) {
   const int t = threadIdx.x % T;
   const RingId d = ring_id(p, my_ring<M>());
   const int N = p.N, cw = p.cw, ncg = (p.ncol + cw - 1) / cw;
+  const Twiddles<M, false> tw(p.tw, t);
   double2 v[16];
 #pragma unroll
   for (int e = 0; e < 16; e++) v[e] = make_double2(0.0, 0.0);
@@ -259,7 +277,7 @@ __global__ __launch_bounds__(Ring<M>::kThreads) void fft_synth_r(FFTParams p) {
       }
     }
   }
-  ring_dft<M, BLUE, +1>(v, lds, p, t);
+  ring_dft<M, BLUE, +1>(v, lds, p, tw, t);
   if (!d.a) return;
   const long oa = (long)field_index(p.fmap, d.fa) * p.fstride + (long)d.ta * N;
   if (!p.real) {
@@ -313,6 +331,8 @@ __global__ __launch_bounds__(Ring<M>::kThreads) void fft_anal_r(FFTParams p) {
   const int t = threadIdx.x % T;
   const RingId d = ring_id(p, my_ring<M>());
   const int N = p.N, cw = p.cw;
+  const Twiddles<M, false> tw(p.tw, t);
+  const double wa = d.a ? p.wq[d.ta] : 0.0, wb = d.b ? p.wq[d.tb] : 0.0;
   double2 v[16];
 #pragma unroll
   for (int e = 0; e < 16; e++) v[e] = make_double2(0.0, 0.0);
@@ -344,20 +364,26 @@ __global__ __launch_bounds__(Ring<M>::kThreads) void fft_anal_r(FFTParams p) {
       if (BLUE && t + T * e >= N) v[e] = make_double2(0.0, 0.0);
     }
   }
-  ring_dft<M, BLUE, -1>(v, lds, p, t);
+  ring_dft<M, BLUE, -1>(v, lds, p, tw, t);
   const int n_cg = p.n_cg, nquad = p.nquad;
   if (!p.real) {
     if (d.a) {
-      const double w = p.wq[d.ta];
       const int la = ring_lmax(p, d.fa);
-      const long b0 = fa_index(0, 2 * d.fa, d.ta, n_cg, nquad, cw);
+      const long b0 = fa_index(-p.m_first, 2 * d.fa, d.ta, n_cg, nquad, cw);  // order 0
       const long sst = fa_index(1, 0, 0, n_cg, nquad, cw);
 #pragma unroll
       for (int e = 0; e < EN; e++) {
         const int k = t + T * e;
-        const double2 X = make_double2(v[e].x * w, v[e].y * w);
-        if (k <= la) st_bin(p, b0 + (k - p.m_first) * sst, X);
-        if (k < N && k >= N - la) st_bin(p, b0 + (k - N - p.m_first) * sst, X);
+        const bool lo = k <= la;
+        if (lo || (k >= N - la && k < N))
+          st_bin(p, b0 + (lo ? k : k - N) * sst, make_double2(v[e].x * wa, v[e].y * wa));
+      }
+      // Bin N/2 belongs to orders N/2 and -N/2 when lmax = N/2.
+      if (2 * la >= N && t == (N / 2) % T) {
+#pragma unroll
+        for (int e = 0; e < EN; e++)
+          if (t + T * e == N / 2)
+            st_bin(p, b0 - N / 2 * sst, make_double2(v[e].x * wa, v[e].y * wa));
       }
     }
   } else {
@@ -371,7 +397,6 @@ __global__ __launch_bounds__(Ring<M>::kThreads) void fft_anal_r(FFTParams p) {
     Ring<M>::sync();
     if (d.a) {
       const int la = ring_lmax(p, d.fa), lb = d.b ? ring_lmax(p, d.fb) : -1;
-      const double wa = p.wq[d.ta], wb = d.b ? p.wq[d.tb] : 0.0;
       const long b0 = fa_index(0, 2 * d.fa, d.ta, n_cg, nquad, cw);
       const long b1 = fa_index(0, 2 * d.fb, d.tb, n_cg, nquad, cw);
       const long sst = fa_index(1, 0, 0, n_cg, nquad, cw);
@@ -390,7 +415,8 @@ __global__ __launch_bounds__(Ring<M>::kThreads) void fft_anal_r(FFTParams p) {
     }
   }
   // The ring of the last colatitude zeroes the padding rows of its quad.
-  const bool za = d.a && d.ta == p.ntheta - 1, zb = d.b && d.tb == p.ntheta - 1;
+  const bool za = p.zero_pad && d.a && d.ta == p.ntheta - 1;
+  const bool zb = p.zero_pad && d.b && d.tb == p.ntheta - 1;
   if (za || zb)
     for (int tp = p.ntheta; tp < 4 * nquad; tp++)
       for (int s = t; s < p.nslot; s += T) {

@@ -610,7 +610,7 @@ __global__ __launch_bounds__(64 * anal_waves(R, REAL), 2) void fft_anal_w(FFTPar
       }
     }
   }
-  if (fv && theta == p.ntheta - 1) {
+  if (p.zero_pad && fv && theta == p.ntheta - 1) {
     const int ncw = REAL && f1v ? 4 : 2;
     for (int tp = theta + 1; tp < 4 * nquad; tp++)
       for (int s = lane; s < p.nslot; s += 64)

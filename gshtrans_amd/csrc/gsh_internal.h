@@ -255,6 +255,8 @@ struct FFTParams {
                     // kernels (gsh_fft_ring.hip) the power of two >= ncol below it
   int n_cg;         // analysis: column groups, ceil(ncol / cw)
   int nquad;        // analysis: colatitude quads
+  int zero_pad;     // analysis: zero the padding rows of the last quad (the FP64
+                    // contraction does not read them)
   const double2* tw;  // tw[k] = exp(-2 pi i k / M), k < M
   const double2* twa; // wavefront FFT: twa[k1 * 64 + j] = exp(-2 pi i j k1 / N), k1 < N / 64
   const double2* chirp;  // Bluestein: exp(-i pi k^2 / N), k < N

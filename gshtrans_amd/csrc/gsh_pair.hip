@@ -97,6 +97,16 @@ __device__ __forceinline__ int coef_index(int l, int m, int nabs, int real) {
   return real ? l * (l + 1) / 2 - nabs * (nabs + 1) / 2 + m : l * l - nabs * nabs + m + l;
 }
 
+// Work item of this workgroup: (m, sub | group << 16, first checkpoint row of
+// order m, first recurrence entry of order m).  The offsets travel with the
+// item, so that nothing waits for a table of them.
+__device__ __forceinline__ uint4 pair_item(const LegParams& p) {
+  typedef unsigned u4 __attribute__((ext_vector_type(4)));
+  const int b = blockIdx.x;
+  const u4 v = ld_uniform(reinterpret_cast<const u4*>(p.items), (long)(b & 7) * p.items_per + (b >> 3));
+  return make_uint4(v.x, v.y, v.z, v.w);
+}
+
 // A virtual column of an item: order sign, column, the column's field and its
 // truncation degree.  Columns past the last read column 0 and store nothing.
 struct VCol {
@@ -140,7 +150,7 @@ __device__ __forceinline__ int vcol_lmax(const LegParams& p, int v0, int nv, int
     col = v0 % p.ncol;
   return field_lmax(p, min(col, p.ncol - 1) >> 1);
 }
-// Smallest degree of a wave's columns (wave-uniform).
+// Minimum over the 16 lanes of a row (the four rows alike; wave-uniform).
 __device__ __forceinline__ int wave_min(int v) {
 #pragma unroll
   for (int d = 1; d < 16; d <<= 1) v = min(v, __shfl_xor(v, d));
@@ -189,7 +199,7 @@ __global__ __launch_bounds__(256, waves(KIND, RT, SYM ? 2 : NJ)) void leg_synth_
   __shared__ uint4 rs[2][2 * SC];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const uint2 it = work_item(p.items, p.items_per);
+  const uint4 it = pair_item(p);
   if (it.x == ~0u) return;
   const int wr = wave / WC, wc = wave % WC;
   const int m = it.x, tb = it.y & 0xffff, cg = it.y >> 16;
@@ -222,11 +232,7 @@ __global__ __launch_bounds__(256, waves(KIND, RT, SYM ? 2 : NJ)) void leg_synth_
   const int lwg = vcol_lmax(p, vb, WC * NC * M::CT, m);
 
   // First checkpoint that matters for the block's rows.
-  int ks = 1 << 20;
-  {
-    const unsigned short* kf = p.kf + (long)(m + p.L) * p.nrt + tile0;
-    for (int i = 0; i < ntile; i++) ks = min(ks, (int)ld_uniform(kf, i));
-  }
+  int ks = wave_min(p.kf[(long)(m + p.L) * p.nrt + tile0 + min(lane & 15, ntile - 1)]);
   ks = min(ks, max(0, lwg - l0 + kCk) / kCk);
   const int ls = l0 + kCk * ks;
   const int nchunk = ls > lwg ? 0 : (lwg - ls + SC) / SC;
@@ -315,7 +321,7 @@ __global__ __launch_bounds__(256, waves(KIND, RT, SYM ? 2 : NJ)) void leg_synth_
   const double cs = tv ? p.cosv[t] : 0.0, csx = txv ? p.cosv[tx] : 0.0;
   const int nck = (p.L - l0 + kCk) / kCk;  // checkpoints 1 .. nck - 1 exist
   const double* seedm = p.seeds + (long)(m + p.L) * nt;
-  const double2* ckm = p.ck + ld_uniform(p.ckoff, m + p.L) * (long)nt;
+  const double2* ckm = p.ck + (long)it.z * nt;
   auto state = [&](int c, bool v, int row) -> double2 {
     const int k = ks + NH * c + seg;
     double2 s = make_double2(0.0, 0.0);
@@ -327,7 +333,7 @@ __global__ __launch_bounds__(256, waves(KIND, RT, SYM ? 2 : NJ)) void leg_synth_
     }
     return s;
   };
-  const uint4* recq = reinterpret_cast<const uint4*>(p.rec + (ld_uniform(p.roff, m + p.L) - l0));
+  const uint4* recq = reinterpret_cast<const uint4*>(p.rec + ((long)it.w - l0));
   auto fetch_rec = [&](int c) {
     return tid < 2 * SC ? recq[2 * (ls + SC * c + 1) + tid] : make_uint4(0, 0, 0, 0);
   };
@@ -493,7 +499,7 @@ __global__ __launch_bounds__(256, waves(KIND, LT, NJ)) void leg_anal_p(LegParams
   __shared__ uint4 rs[2 * PD];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const uint2 it = work_item(p.items, p.items_per);
+  const uint4 it = pair_item(p);
   if (it.x == ~0u) return;
   const int wr = wave / WC, wc = wave % WC;
   const int m = it.x, pass = it.y & 0xffff, cg = it.y >> 16;
@@ -551,8 +557,7 @@ __global__ __launch_bounds__(256, waves(KIND, LT, NJ)) void leg_anal_p(LegParams
   }
 
   if (tid < 64 * nu)
-    rs[tid] = reinterpret_cast<const uint4*>(p.rec + (ld_uniform(p.roff, m + p.L) - l0))
-        [2 * (lp + 1) + tid];
+    rs[tid] = reinterpret_cast<const uint4*>(p.rec + ((long)it.w - l0))[2 * (lp + 1) + tid];
 
   // Production: thread -> (16-degree segment, row of the chunk).
   const int seg = tid / CR, prow = tid % CR;
@@ -560,7 +565,7 @@ __global__ __launch_bounds__(256, waves(KIND, LT, NJ)) void leg_anal_p(LegParams
   const int kk = 2 * u0 + seg;
   const bool pv = seg < 2 * nu && kk < nck;
   const double* seedm = p.seeds + (long)(m + p.L) * nt;
-  const double2* ckm = p.ck + (ld_uniform(p.ckoff, m + p.L) + kk - 1) * (long)nt;
+  const double2* ckm = p.ck + ((long)it.z + kk - 1) * nt;
   double cs = 0.0;
   auto state = [&](int c) -> double2 {
     const int row = CR * c + prow;
@@ -825,7 +830,7 @@ PairTile pair_anal_tile(int ncol, int pair, bool uneven) {
 }
 
 hipError_t launch_leg_synth_pair(const LegParams& p0, const PairTile& t, int sym, hipStream_t s) {
-  if (!p0.ck || !p0.ckoff || !p0.kf) return hipErrorInvalidValue;  // checkpoint table required
+  if (!p0.ck || !p0.kf) return hipErrorInvalidValue;  // checkpoint table required
   LegParams p = p0;
   p.n_tsb = t.nblk;
   p.vint = t.vint;
@@ -856,7 +861,7 @@ hipError_t launch_leg_synth_pair(const LegParams& p0, const PairTile& t, int sym
 }
 
 hipError_t launch_leg_anal_pair(const LegParams& p0, const PairTile& t, int sym, hipStream_t s) {
-  if (!p0.ck || !p0.ckoff || !p0.kf) return hipErrorInvalidValue;
+  if (!p0.ck || !p0.kf) return hipErrorInvalidValue;
   LegParams p = p0;
   p.vint = t.vint;
   p.n_cg = (p.ncol + p.cw - 1) / p.cw;
