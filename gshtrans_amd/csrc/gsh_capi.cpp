@@ -1188,7 +1188,8 @@ int run_inverse(gsh_grid_s* g, NData* d, int lmax, int n, int real, int precisio
     p.kf = d->kf;
     p.nrt = (p.ntheta + 15) / 16;
     const gsh::PairTile t = gsh::pair_synth_tile(p.ncol, p.pair, sym, precision == GSH_FP32,
-                                                 o.f_lmax != nullptr, sym ? (p.ntheta + 1) / 2 : p.ntheta);
+                                                 o.f_lmax != nullptr, sym ? (p.ntheta + 1) / 2 : p.ntheta,
+                                                 lmax + 1);
     WorkList w;
     if ((st = ensure_pair_worklist(g, 0, lmax, n, p.pair, p.ncol, t, o.f_lmax_host, &w)))
       return st;
@@ -1338,7 +1339,7 @@ int run_forward(gsh_grid_s* g, NData* d, int lmax, int n, int real, int precisio
     p.pair = real ? 0 : 1;
     p.kf = d->kf;
     p.nrt = (p.ntheta + 15) / 16;
-    const gsh::PairTile t = gsh::pair_anal_tile(p.ncol, p.pair, o.f_lmax != nullptr);
+    const gsh::PairTile t = gsh::pair_anal_tile(p.ncol, p.pair, o.f_lmax != nullptr, lmax + 1);
     WorkList w;
     if ((st = ensure_pair_worklist(g, 1, lmax, n, p.pair, p.ncol, t, o.f_lmax_host, &w)))
       return st;
@@ -1851,7 +1852,7 @@ int run_plan(gsh_plan_s* P, int dir, const void* in, long istride, void* out, lo
     const double* cin = static_cast<const double*>(in);
     if (f32) {
       if ((st = plan_stage(P, istride))) return st;
-      GSH_HIP(gsh::launch_widen_c32(in, P->stage, (long)P->count * istride, s));
+      GSH_HIP(gsh::launch_widen_c32(in, P->stage, istride, P->d_csize, P->cmax, P->count, s));
       cin = P->stage;
     }
     for (const PlanGroup& G : P->groups)
@@ -1950,7 +1951,7 @@ int tune_plan(gsh_plan_s* P, int dir, const void* in, long istride, void* out, l
   double* cout = static_cast<double*>(out);
   if (f32) {
     if ((st = plan_stage(P, dir == 0 ? istride : ostride))) return st;
-    if (dir == 0) GSH_HIP(gsh::launch_widen_c32(in, P->stage, (long)P->count * istride, s));
+    if (dir == 0) GSH_HIP(gsh::launch_widen_c32(in, P->stage, istride, P->d_csize, P->cmax, P->count, s));
     cin = P->stage;
     cout = P->stage;
   }
@@ -2007,7 +2008,7 @@ int tune_plan(gsh_plan_s* P, int dir, const void* in, long istride, void* out, l
       if (fp && G.count > 8) {
         const int pair = P->kind == GSH_REAL ? 0 : 1;
         pick.tiles = gsh::pair_synth_tile(2 * G.count, pair, G.n == 0 && P->precision == GSH_FP64,
-                                          P->precision == GSH_FP32, true, P->g->ntheta())
+                                          P->precision == GSH_FP32, true, P->g->ntheta(), G.lmax + 1)
                          .nj;
       }
       G.synth_tiles = pick.tiles;

@@ -300,8 +300,8 @@ struct PairTile {
   int vint = 0;  // see LegParams
   int nblk = 1;  // synthesis: row blocks; analysis: units of 32 degrees per pass
 };
-PairTile pair_synth_tile(int ncol, int pair, int sym, bool f32m, bool uneven, int nr);
-PairTile pair_anal_tile(int ncol, int pair, bool uneven);
+PairTile pair_synth_tile(int ncol, int pair, int sym, bool f32m, bool uneven, int nr, int norder);
+PairTile pair_anal_tile(int ncol, int pair, bool uneven, int norder);
 hipError_t launch_leg_synth_pair(const LegParams& p, const PairTile& t, int sym, hipStream_t s);
 hipError_t launch_leg_anal_pair(const LegParams& p, const PairTile& t, int sym, hipStream_t s);
 // Values below this at every row of a tile are left out of the FP64 sums.
@@ -335,7 +335,8 @@ hipError_t launch_leg_anal_bf16(const LegParams& p, int ns, hipStream_t s, int f
 
 // FP32 <-> FP64 coefficient staging of batch plans (gsh_batch.hip); strides
 // and sizes in complex elements.
-hipError_t launch_widen_c32(const void* in, double* out, long total, hipStream_t s);
+hipError_t launch_widen_c32(const void* in, double* out, long stride, const long* csize, long cmax,
+                            int count, hipStream_t s);
 hipError_t launch_narrow_c64(const double* in, void* out, long stride, const long* csize,
                              long cmax, int count, hipStream_t s);
 

@@ -836,38 +836,56 @@ hipError_t go_anal(const LegParams& p, hipStream_t s) {
 }  // namespace
 
 // Tile of a launch: ncol columns (twice that many virtual ones when paired),
-// nr rows, uneven: fields of different truncation degrees.  Wider tiles share
-// each recurrence value and each A operand among more columns; the narrow
-// ones keep the matrix unit off padding columns: at most 4 (8) columns take
-// the 4-column instruction, at most 16 (32, 64) one (two, four) tiles of 16;
-// more are interleaved by order sign.  Uneven batches stop at 64, whose 16
-// fields have neighbouring degrees.  The rows of a block are 6 or 8 tiles,
-// whichever covers the launch's row tiles with less left over.
-static PairTile pair_tile(int ncol, int pair, bool f32m, bool uneven) {
+// nr rows, norder orders, uneven: fields of different truncation degrees.
+// Wider tiles share each recurrence value and each A operand among more
+// columns; the narrow ones keep the matrix unit off padding columns: at most 8
+// columns take the 4-column instruction, at most 16 (32) one (two) tiles of
+// 16; more are interleaved by order sign.  Uneven batches stop at 64 (32 in
+// the analysis), whose fields have neighbouring degrees.  A launch of fewer than
+// kFewBlocks workgroups takes narrower tiles (and no 9th row tile): a wave
+// then has fewer MFMAs between two barriers, and idle CUs repeat the recurrence
+// for the other columns.  lMax=256, complex: 8 fields (514 workgroups of 32
+// columns) 42.7 -> 36.0 us synthesis, 38.8 -> 33.8 us analysis; lMax=384 (1155
+// of them) no gain, 69.7 -> 80.7 us analysis.
+constexpr int kFewBlocks = 600;
+static void set_cols(PairTile& t, int cols) {
+  t.cols = cols;
+  t.nj = cols == 16 ? 1 : 2;
+  t.rt = cols <= 32 ? 2 : cols / 16;
+}
+static PairTile pair_tile(int ncol, int pair, bool f32m) {
   PairTile t;
   const int V = ncol * (pair ? 2 : 1);
   t.kind = f32m ? 1 : V <= 8 ? 2 : 0;
   t.vint = V > 32 ? 1 : 0;
   t.vcols = t.vint ? (ncol + 15) / 16 * 16 * (pair ? 2 : 1) : V;
-  t.rt = t.kind == 2 ? 8 : V <= 32 ? 2 : t.vcols <= 64 || uneven ? 4 : 8;
-  t.nj = V <= (t.kind == 2 ? 4 : 16) ? 1 : 2;
+  if (t.kind == 2) {
+    t.rt = 8;
+    t.nj = V <= 4 ? 1 : 2;
+    t.cols = 4 * t.nj;
+  } else {
+    set_cols(t, V <= 16 ? 16 : V <= 32 ? 32 : t.vcols <= 64 ? 64 : 128);
+  }
   return t;
 }
-PairTile pair_synth_tile(int ncol, int pair, int sym, bool f32m, bool uneven, int nr) {
-  PairTile t = pair_tile(ncol, pair, f32m, uneven);
-  if (sym && t.kind != 2) {  // one column tile per wave
-    if (t.vcols <= 16) t.rt = 2;
-    else if (t.vcols <= 32) t.rt = 4;
-    else t.rt = uneven ? 4 : 8;
-    t.nj = 1;
-  }
+PairTile pair_synth_tile(int ncol, int pair, int sym, bool f32m, bool uneven, int nr, int norder) {
+  PairTile t = pair_tile(ncol, pair, f32m);
   const int rtt = (nr + 15) / 16;
-  t.cols = t.kind == 2 ? 4 * t.nj : t.rt / 2 * t.nj * 16;
   // Blocks of tw row tiles, each with room for one more.
   auto blocks = [rtt](int tw) { return std::max(1, (rtt + tw) / (tw + 1)); };
   t.nblk = blocks(8);
+  if (t.kind == 2) return t;
+  if (uneven && t.cols > 64) set_cols(t, 64);
+  auto few = [&] { return norder * t.nblk * ((t.vcols + t.cols - 1) / t.cols) < kFewBlocks; };
+  if (few()) t.nblk = std::max(1, (rtt + 7) / 8);
+  while (t.cols > 16 && few()) set_cols(t, t.cols / 2);
+  if (sym) {  // both parities in a wave: one column tile
+    t.cols = std::min(t.cols, 64);
+    t.rt = t.cols / 8;
+    t.nj = 1;
+  }
   if (t.kind == 0 && t.rt >= 4) {
-    const int n6 = blocks(6), n8 = blocks(8);
+    const int n6 = blocks(6), n8 = t.nblk;
     const int c6 = std::max(6 * n6, rtt), c8 = std::max(8 * n8, rtt);
     if (c6 < c8) {
       t.rt = t.rt == 8 ? 6 : 3;
@@ -876,11 +894,14 @@ PairTile pair_synth_tile(int ncol, int pair, int sym, bool f32m, bool uneven, in
   }
   return t;
 }
-PairTile pair_anal_tile(int ncol, int pair, bool uneven) {
-  PairTile t = pair_tile(ncol, pair, false, uneven);
-  if (uneven && t.kind != 2) t.rt = 2;
+PairTile pair_anal_tile(int ncol, int pair, bool uneven, int norder) {
+  PairTile t = pair_tile(ncol, pair, false);
   t.nblk = 4;  // units of 32 degrees per pass
-  t.cols = t.kind == 2 ? 4 * t.nj : t.rt / 2 * t.nj * 16;
+  if (t.kind == 2) return t;
+  if (uneven && t.cols > 32) set_cols(t, 32);
+  while (t.cols > 16 &&
+         norder * ((norder + 255) / 256) * ((t.vcols + t.cols - 1) / t.cols) < kFewBlocks)
+    set_cols(t, t.cols / 2);
   return t;
 }
 
