@@ -845,8 +845,9 @@ hipError_t go_anal(const LegParams& p, hipStream_t s) {
 // kFewBlocks workgroups takes narrower tiles (and no 9th row tile): a wave
 // then has fewer MFMAs between two barriers, and idle CUs repeat the recurrence
 // for the other columns.  lMax=256, complex: 8 fields (514 workgroups of 32
-// columns) 42.7 -> 36.0 us synthesis, 38.8 -> 33.8 us analysis; lMax=384 (1155
-// of them) no gain, 69.7 -> 80.7 us analysis.
+// columns) 44.0 -> 39.8 us synthesis, 39.2 -> 34.1 us analysis with n=1, 33.8 ->
+// 30.1 and 28.1 -> 24.2 us with n=0; lMax=384 (1155 of them) no gain, 69.7 ->
+// 80.7 us analysis.
 constexpr int kFewBlocks = 600;
 static void set_cols(PairTile& t, int cols) {
   t.cols = cols;
