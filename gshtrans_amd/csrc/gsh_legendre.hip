@@ -304,6 +304,17 @@ __global__ __launch_bounds__(256) void rec_checkpoints(LegParams p) {
     if (kfirst == 0x7fff && (fabs(s0) >= kNegligible || fabs(s1) >= kNegligible)) kfirst = k;
     if (t < nt) out[(long)(k - 1) * nt + t] = make_double2(s0, s1);
   }
+  // The degrees after the last state are stored nowhere, so an order whose
+  // states are all negligible runs them too (entries past L are zero).
+  if (kfirst == 0x7fff) {
+    const d4* rl = reinterpret_cast<const d4*>(recq) + l0 + kCk * (nck - 1) + 1;
+    double big = 0.0;
+    for (int j = 0; j < kCk; j++) {
+      rec_step(rl[j], cs, e0, e1);
+      big = fmax(big, fabs(e0));
+    }
+    if (ldexp(big, -kk) >= kNegligible) kfirst = nck;
+  }
   // kf: the checkpoint before the first state that matters at any of 16 rows
   // (the degrees up to it are negligible: below the turning point the values
   // of an order rise with the degree).

@@ -95,3 +95,32 @@ def test_left_out_terms_stay_visible(torch, n, real, bad):
     assert finite[0].all() and finite[2].all()
     # (L, L) of a complex field is zeroed
     assert not finite[1, :-1].all(dim=-1).any()
+
+
+# Degrees after an order's last stored state: the order L - 12 rises from
+# negligible seeds to 2^-83 at rows near the pole within its last 13 degrees.
+# One field for each such ring, zero elsewhere, so its sums hold nothing larger.
+# FP64: 13 recurrence steps of a few roundings each and one ring FFT, far below
+# 1e-10.  Split BF16: FP32-accurate products of FP32 bins (6e-8), their smallest
+# planes above FP32's underflow for values from 2^-92: 1e-5.
+@pytest.mark.parametrize("precision", ["fp64", "bf16x6"])
+@pytest.mark.parametrize("n", [0, 2])
+def test_last_degrees_of_an_order(torch, n, precision):
+    L, m = 256, 244
+    g = G.GaussLegendreGrid(L, 2)
+    og = oracle.OracleGrid(L, 2, table=False)
+    idx = [G.coefficient_index(L, n, l, m, False) for l in range(m, L + 1)]
+    c = np.zeros(G.coefficient_size(L, n), dtype=np.complex128)
+    c[idx] = 1.0
+    ring = og.inverse(L, n, c)
+    size = np.abs(ring).max(axis=-1)
+    rows = np.flatnonzero((size > 2.0**-92) & (size < 2.0**-83))
+    say(f"[pair] last degrees n={n} {precision} rows={rows}")
+    assert rows.size
+    f = np.zeros((rows.size,) + ring.shape, dtype=np.complex128)
+    f[np.arange(rows.size), rows] = ring[rows] / size[rows, None]
+    a = g.forward(L, n, torch.from_numpy(f).cuda(), precision=precision).cpu().numpy()
+    tol = 1e-10 if precision == "fp64" else 1e-5
+    for i, t in enumerate(rows):
+        ref = og.forward(L, n, f[i])[idx]
+        assert np.linalg.norm(a[i][idx] - ref) <= tol * np.linalg.norm(ref), t
