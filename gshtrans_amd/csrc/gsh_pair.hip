@@ -162,10 +162,6 @@ __device__ __forceinline__ int wave_min(int v) {
 // neither a load nor the barrier: they keep one D buffer (two barriers per
 // chunk) and run four workgroups per CU instead of two.
 constexpr int nbuf(int kind, int tiles) { return kind == 2 || tiles <= 2 ? 1 : 2; }
-// The 4-column tiles leave a wave of 32 rows little to multiply with a loaded
-// coefficient: their waves share the rows (degrees, in the analysis) and split
-// the sum instead, each taking a quarter of the operands, and add up at the end.
-constexpr bool ksplit(int kind) { return kind == 2; }
 // Workgroups per CU (waves per SIMD) that the registers are cut to.
 constexpr int waves(int kind, int tiles, int nj) {
   return nbuf(kind, tiles) == 2 ? 2 : kind != 2 && nj == 2 ? 3 : 4;
@@ -188,18 +184,16 @@ template <int KIND, int SYM, int RT, int NJ>
 __global__ __launch_bounds__(256, waves(KIND, RT, SYM ? 2 : NJ)) void leg_synth_p(LegParams p) {
   typedef Mma<KIND> M;
   typedef typename M::elem E;
-  constexpr bool KS = ksplit(KIND);
-  constexpr int WR = KS ? 1 : RT == 2 ? 4 : RT <= 4 ? 2 : 1;
-  constexpr int WC = KS ? 1 : 4 / WR;
+  constexpr int WR = RT == 2 ? 4 : RT <= 4 ? 2 : 1;
+  constexpr int WC = 4 / WR;
   constexpr int TW = RT * WR;      // row tiles of a block without the extra one
   constexpr int NH = 2;            // 16-degree segments of a chunk
   constexpr int SC = kCk * NH;     // degrees per chunk
   // Elements per degree row in LDS: 9 row tiles, padded so that the A operands
   // of both forms spread over all banks.
   constexpr int SP = 152;
-  constexpr bool S2 = SYM && !KS;  // both parities in one wave
-  constexpr int NB = S2 ? 2 : NJ;  // accumulators per row tile
-  constexpr int NC = S2 ? 1 : NJ;  // column tiles per wave
+  constexpr int NB = SYM ? 2 : NJ; // accumulators per row tile
+  constexpr int NC = SYM ? 1 : NJ; // column tiles per wave
   constexpr int NBUF = nbuf(KIND, RT);
   __shared__ E D[NBUF][SC * SP];
   __shared__ uint4 rs[2][2 * SC];
@@ -207,7 +201,7 @@ __global__ __launch_bounds__(256, waves(KIND, RT, SYM ? 2 : NJ)) void leg_synth_
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const uint4 it = pair_item(p);
   if (it.x == ~0u) return;
-  const int wr = KS ? 0 : wave / WC, wc = KS ? 0 : wave % WC;
+  const int wr = wave / WC, wc = wave % WC;
   const int m = it.x, tb = it.y & 0xffff, cg = it.y >> 16;
   const int nt = p.ntheta, nr = SYM ? (nt + 1) / 2 : nt;
   const int rtt = (nr + 15) >> 4;
@@ -243,29 +237,26 @@ __global__ __launch_bounds__(256, waves(KIND, RT, SYM ? 2 : NJ)) void leg_synth_
   const int ls = l0 + kCk * ks;
   const int nchunk = ls > lwg ? 0 : (lwg - ls + SC) / SC;
 
-  // Coefficient loads: accumulator b reads degrees l + deg(b) of every ST-th
-  // degree l, GB loads per 16 degrees.  A group of 16 degrees from l with l +
-  // 15 <= lmin is inside every column's degrees (plain()); its byte offset
-  // off[b] steps by an arithmetic progression.  The others clamp each load to
-  // a valid address, and operand() masks them.
-  constexpr int ST = KS ? 16 : SYM ? 8 : 4;
-  constexpr int GB = kCk / ST;
-  constexpr int NO = S2 ? 2 : 1;  // offsets: order -m shares order m's
-  // KS: wave w takes the w-th 4 degrees (SYM: 8 (w / 2) + w % 2 + 0, 2, 4, 6).
-  const int kdeg = !KS ? 0 : SYM ? 8 * (wave >> 1) + 2 * krow + (wave & 1) : 4 * wave + krow;
-  auto deg = [&](int b) { return KS ? kdeg : SYM ? 2 * krow + b : krow; };
+  // Coefficient loads: accumulator b reads degree l + d (d = krow, or SYM
+  // 2 krow + b) of every ST-th degree l, GB loads per 16 degrees.  A group
+  // of 16 degrees from l with l + 15 <= lmin is inside every column's degrees
+  // (plain()); its byte offset off[b] steps by an arithmetic progression.  The
+  // others clamp each load to a valid address, and operand() masks them.
+  constexpr int ST = SYM ? 8 : 4;
+  constexpr int GB = SYM ? 2 : 4;
+  constexpr int NO = SYM ? 2 : 1;  // offsets: order -m shares order m's
   unsigned off[NO], step[NO];
   unsigned sgn[NC];  // sign bit of order -m (SYM0: the parity of l is the lane's)
 #pragma unroll
   for (int b = 0; b < NO; b++) {
-    const int l = l0 + deg(b);
+    const int l = l0 + (SYM ? 2 * krow + b : krow);
     off[b] = 16u * coef_index(l, m, p.nabs, p.real);
-    step[b] = (2 * ST * l + ST * ST + ST) * (p.real ? 8u : 16u);
+    step[b] = (SYM ? 16 * l + 72 : 8 * l + 20) * (p.real ? 8u : 16u);
   }
-  const unsigned sinc = 2 * ST * ST * (p.real ? 8u : 16u);
+  const unsigned sinc = (SYM ? 128 : 32) * (p.real ? 8u : 16u);
 #pragma unroll
   for (int j = 0; j < NC; j++)
-    sgn[j] = vc[j].sgn && ((SYM ? m : l0 + deg(0) + p.n) & 1) ? 0x80000000u : 0u;
+    sgn[j] = vc[j].sgn && ((SYM ? m : l0 + krow + p.n) & 1) ? 0x80000000u : 0u;
   auto plain = [&](int l) { return l + kCk - 1 <= lmin; };
   auto load_group = [&](int l, double (&B)[GB][NB]) {
     if (plain(l)) {
@@ -273,7 +264,7 @@ __global__ __launch_bounds__(256, waves(KIND, RT, SYM ? 2 : NJ)) void leg_synth_
       for (int g = 0; g < GB; g++) {
 #pragma unroll
         for (int b = 0; b < NB; b++)
-          B[g][b] = *reinterpret_cast<const double*>(cbase[S2 ? 0 : b] + off[S2 ? b : 0]);
+          B[g][b] = *reinterpret_cast<const double*>(cbase[SYM ? 0 : b] + off[SYM ? b : 0]);
 #pragma unroll
         for (int b = 0; b < NO; b++) {
           off[b] += step[b];
@@ -285,11 +276,11 @@ __global__ __launch_bounds__(256, waves(KIND, RT, SYM ? 2 : NJ)) void leg_synth_
       for (int g = 0; g < GB; g++)
 #pragma unroll
         for (int b = 0; b < NB; b++) {
-          const VCol& c = vc[S2 ? 0 : b];
-          const int ll = min(l + ST * g + deg(b), c.lf);
+          const VCol& c = vc[SYM ? 0 : b];
+          const int ll = min(l + ST * g + (SYM ? 2 * krow + b : krow), c.lf);
           // A field without a degree of this order reads its element 0.
           const long o = c.lf >= l0 ? 16l * coef_index(ll, m, p.nabs, p.real) : c.sgn ? 32l * m : 0;
-          B[g][b] = *reinterpret_cast<const double*>(cbase[S2 ? 0 : b] + o);
+          B[g][b] = *reinterpret_cast<const double*>(cbase[SYM ? 0 : b] + o);
         }
     }
   };
@@ -298,10 +289,10 @@ __global__ __launch_bounds__(256, waves(KIND, RT, SYM ? 2 : NJ)) void leg_synth_
   auto operand = [&](auto mask, double v, int b, int l, int g) -> E {
     if (!SYM) {
       uint2 u = __builtin_bit_cast(uint2, v);
-      u.y ^= sgn[S2 ? 0 : b];
+      u.y ^= sgn[SYM ? 0 : b];
       v = __builtin_bit_cast(double, u);
     }
-    if (decltype(mask)::value && l + ST * g + deg(b) > vc[S2 ? 0 : b].lf)
+    if (decltype(mask)::value && l + ST * g + (SYM ? 2 * krow + b : krow) > vc[SYM ? 0 : b].lf)
       v = 0.0;
     return (E)v;
   };
@@ -377,12 +368,12 @@ __global__ __launch_bounds__(256, waves(KIND, RT, SYM ? 2 : NJ)) void leg_synth_
 #pragma unroll
       for (int j = 0; j < NB; j++) X[j] = operand(mask, Bh[g][j], j, l, g);
 #pragma unroll
-      for (int b = 0; b < (S2 ? 2 : 1); b++) {
-        const E* dr = d + (ST * g + deg(b)) * SP;
+      for (int b = 0; b < (SYM ? 2 : 1); b++) {
+        const E* dr = d + (SYM ? 8 * g + 2 * krow + b : 4 * g + krow) * SP;
 #pragma unroll
         for (int i = 0; i < N; i++) {
           const E A = dr[16 * i];
-          if (S2) {
+          if (SYM) {
             acc[i][b] = M::mma(A, X[b], acc[i][b]);
           } else {
 #pragma unroll
@@ -455,56 +446,34 @@ __global__ __launch_bounds__(256, waves(KIND, RT, SYM ? 2 : NJ)) void leg_synth_
     }
   }
 
-  // Store: order m at row t, order -m at the mirrored row (n != 0); SYM: the
-  // sums of even and odd degrees give the row and its mirror.
+  // Store: order m at row t, order -m at the mirrored row (n != 0).
   const long frow = f_index(1, 0, 0, p.nslot, (p.ncol + p.cw - 1) / p.cw, p.cw);  // F per row
-  double* fcol[NC];
 #pragma unroll
-  for (int j = 0; j < NC; j++)
-    fcol[j] = p.F + f_index(0, (vc[j].sgn ? -m : m) - p.m_first, vc[j].col, p.nslot, 0, p.cw);
-  auto store = [&](int j, int tr, double e, double o) {
-    const int row = 16 * tile0 + tr;
-    if (!vc[j].valid || tr >= 16 * ntile || row >= nr) return;
-    if (SYM) {
-      if (sgn[j]) {
-        e = -e;
-        o = -o;
+  for (int j = 0; j < NC; j++) {
+    if (!vc[j].valid) continue;
+    double* f = p.F + f_index(0, (vc[j].sgn ? -m : m) - p.m_first, vc[j].col, p.nslot, 0, p.cw);
+    const bool mirrored = !SYM && vc[j].sgn;
+#pragma unroll
+    for (int i = 0; i <= RT; i++) {
+      if (i == RT && !xt) continue;
+#pragma unroll
+      for (int r = 0; r < M::NR; r++) {
+        const int tr = 16 * (wr * RT + i) + M::row(lane, r);
+        const int row = 16 * tile0 + tr;
+        if (tr >= 16 * ntile || row >= nr) continue;
+        if (SYM) {
+          double e = M::get(acc[i][0], r), o = M::get(acc[i][1], r);
+          if (sgn[j]) {
+            e = -e;
+            o = -o;
+          }
+          f[row * frow] = e + o;
+          if (nt - 1 - row != row) f[(nt - 1 - row) * frow] = e - o;
+        } else {
+          f[(mirrored ? nt - 1 - row : row) * frow] = M::get(acc[i][j], r);
+        }
       }
-      fcol[j][row * frow] = e + o;
-      if (nt - 1 - row != row) fcol[j][(nt - 1 - row) * frow] = e - o;
-    } else {
-      fcol[j][(vc[j].sgn ? nt - 1 - row : row) * frow] = e;
     }
-  };
-  if constexpr (KS) {
-    // The waves' partial sums meet in LDS; wave w stores row tiles w, w + 4, ..
-    double* red = reinterpret_cast<double*>(D[0]);
-    __syncthreads();
-#pragma unroll
-    for (int i = 0; i <= RT; i++)
-#pragma unroll
-      for (int j = 0; j < NC; j++) red[((wave * (RT + 1) + i) * NC + j) * 64 + lane] = acc[i][j];
-    __syncthreads();
-    for (int i = wave; i < ntile; i += 4)
-#pragma unroll
-      for (int j = 0; j < NC; j++) {
-        double v[4];
-#pragma unroll
-        for (int w = 0; w < 4; w++) v[w] = red[((w * (RT + 1) + i) * NC + j) * 64 + lane];
-        const double e = v[0] + v[2], o = v[1] + v[3];
-        store(j, 16 * i + M::row(lane, 0), SYM ? e : e + o, o);
-      }
-  } else {
-#pragma unroll
-    for (int j = 0; j < NC; j++)
-#pragma unroll
-      for (int i = 0; i <= RT; i++) {
-        if (i == RT && !xt) continue;
-#pragma unroll
-        for (int r = 0; r < M::NR; r++)
-          store(j, 16 * (wr * RT + i) + M::row(lane, r), M::get(acc[i][S2 ? 0 : j], r),
-                S2 ? M::get(acc[i][NB - 1], r) : 0.0);
-      }
   }
 }
 
@@ -519,8 +488,7 @@ __global__ __launch_bounds__(256, waves(KIND, RT, SYM ? 2 : NJ)) void leg_synth_
 template <int KIND, int SYM, int LT, int NJ>
 __global__ __launch_bounds__(256, waves(KIND, LT, NJ)) void leg_anal_p(LegParams p) {
   typedef Mma<KIND> M;
-  constexpr bool KS = ksplit(KIND);
-  constexpr int WR = 8 / LT, WC = KS ? 1 : 4 / WR;
+  constexpr int WR = 8 / LT, WC = 4 / WR;
   constexpr int NBUF = nbuf(KIND, LT);
   constexpr int PD = 128;             // degrees per pass
   constexpr int PU = PD / 32;         // units per pass
@@ -533,7 +501,7 @@ __global__ __launch_bounds__(256, waves(KIND, LT, NJ)) void leg_anal_p(LegParams
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const uint4 it = pair_item(p);
   if (it.x == ~0u) return;
-  const int wr = KS ? 0 : wave / WC, wc = KS ? 0 : wave % WC;
+  const int wr = wave / WC, wc = wave % WC;
   const int m = it.x, pass = it.y & 0xffff, cg = it.y >> 16;
   const int nt = p.ntheta, nr = SYM ? (nt + 1) / 2 : nt;
   const int l0 = max(m, p.nabs);
@@ -662,31 +630,27 @@ __global__ __launch_bounds__(256, waves(KIND, LT, NJ)) void leg_anal_p(LegParams
   for (int c = 0; c < nch; c++) {
     if (c == c0) c = c1 + 1;
     if (c >= nch) break;
-    constexpr int PQ = KS ? 2 : 4;
-    double b[PQ][NL];
+    double b[4][NL];
 #pragma unroll
-    for (int h = 0; h < (KS ? 1 : NQ / PQ); h++) {
-      load_quads(NQ * c + (KS ? 2 * wave : PQ * h), b);
+    for (int h = 0; h < NQ / 4; h++) {
+      load_quads(NQ * c + 4 * h, b);
 #pragma unroll
-      for (int q = 0; q < PQ; q++)
+      for (int q = 0; q < 4; q++)
 #pragma unroll
         for (int j = 0; j < NL; j++) pz[SYM ? j >> 1 : j] += 0.0 * b[q][j];
     }
   }
 
-  // Quads per group of loads and groups per chunk; KS: wave w takes the quads
-  // 2 w, 2 w + 1 of a chunk.
-  constexpr int GQ = SYM || KS ? 2 : 4;
-  constexpr int NG = KS ? 1 : NQ / GQ;
-  const int kq = KS ? 2 * wave : 0;
+  constexpr int GQ = SYM ? 2 : 4;  // quads per group of loads
+  constexpr int NG = NQ / GQ;
   // This wave's units: those of its degree group, up to its columns' degrees.
   constexpr int WU = LT / 2;
   const int mine = min(min(nu, (lw - lp + 32) >> 5) - wr * WU, WU);
-  double Bq[KS ? 1 : 2][GQ][NL];
+  double Bq[2][GQ][NL];
   // All degree tiles of the wave (whole), or those of its units: tiles past
   // the pass are skipped in pairs.
   auto run_group = [&](auto whole, auto full, int buf, int c, int h, double (&B)[GQ][NL]) {
-    const double* d = D[buf] + (16 * LT * wr + (lane & 15)) * AP + 4 * (GQ * h + kq) + krow;
+    const double* d = D[buf] + (16 * LT * wr + (lane & 15)) * AP + 4 * GQ * h + krow;
 #pragma unroll
     for (int g = 0; g < GQ; g++) {
       double X[2][NJ];
@@ -696,7 +660,7 @@ __global__ __launch_bounds__(256, waves(KIND, LT, NJ)) void leg_anal_p(LegParams
           const double a = B[g][2 * j];
           double b = B[g][2 * j + 1];
           if (!decltype(full)::value) {
-            const int row = 4 * (NQ * c + GQ * h + kq + g) + krow;
+            const int row = 4 * (NQ * c + GQ * h + g) + krow;
             b = nt - 1 - row > row ? b : 0.0;
           }
           X[0][j] = a + b;
@@ -721,7 +685,7 @@ __global__ __launch_bounds__(256, waves(KIND, LT, NJ)) void leg_anal_p(LegParams
 
   __syncthreads();
   if (c0 <= c1) {
-    load_quads(NQ * c0 + kq, Bq[0]);
+    load_quads(NQ * c0, Bq[0]);
     double2 st = state(c0);
     if (NBUF == 2) {
       produce(0, st);
@@ -733,7 +697,7 @@ __global__ __launch_bounds__(256, waves(KIND, LT, NJ)) void leg_anal_p(LegParams
       for (int c = ca; c < cb; c++) {
         const int buf = NBUF == 2 ? (c - c0) & 1 : 0;
         __syncthreads();
-        if constexpr (!KS) load_quads(NQ * c + GQ, Bq[1]);
+        load_quads(NQ * c + GQ, Bq[1]);
         if (NBUF == 2) {
           if (c < c1) {
             produce(buf ^ 1, st);
@@ -744,19 +708,14 @@ __global__ __launch_bounds__(256, waves(KIND, LT, NJ)) void leg_anal_p(LegParams
           if (c < c1) st = state(c + 1);
           __syncthreads();
         }
-        if constexpr (KS) {
-          run_group(whole, full, buf, c, 0, Bq[0]);
-          if (c < c1) load_quads(NQ * (c + 1) + kq, Bq[0]);
-        } else {
 #pragma unroll
-          for (int h = 0; h < NG; h++) {
-            if (decltype(full)::value || NQ * c + GQ * h < nq)
-              run_group(whole, full, buf, c, h, Bq[h & 1]);
-            if (h + 2 < NG)
-              load_quads(NQ * c + GQ * (h + 2), Bq[h & 1]);
-            else if (h + 2 == NG && c < c1)
-              load_quads(NQ * (c + 1), Bq[0]);
-          }
+        for (int h = 0; h < NG; h++) {
+          if (decltype(full)::value || NQ * c + GQ * h < nq)
+            run_group(whole, full, buf, c, h, Bq[h & 1]);
+          if (h + 2 < NG)
+            load_quads(NQ * c + GQ * (h + 2), Bq[h & 1]);
+          else if (h + 2 == NG && c < c1)
+            load_quads(NQ * (c + 1), Bq[0]);
         }
       }
     };
@@ -778,46 +737,26 @@ __global__ __launch_bounds__(256, waves(KIND, LT, NJ)) void leg_anal_p(LegParams
     for (int i = 0; i < LT; i++) M::add(acc[i][j], z);
   }
 
-  auto store = [&](int j, int l, double v) {
-    if (!vc[j].valid || l > vc[j].lf) return;
-    const int mo = vc[j].sgn ? -m : m;
-    double* co = p.cout + ((long)vc[j].field * p.cstride + coef_index(l, mo, p.nabs, p.real)) * 2 +
-                 (vc[j].col & 1);
-    if (vc[j].sgn && ((SYM ? m : l + p.n) & 1)) v = -v;
-    if (p.accumulate) v += *co;
-    if (p.zero_last && vc[j].lf == p.L && l == p.L && mo == p.L) v = 0.0;
-    *co = v;
-  };
-  // Degree of row mr of degree tile i of the pass.
-  auto degree = [&](int i, int mr) {
-    return lp + (SYM ? 32 * (i >> 1) + 2 * mr + (i & 1) : 16 * i + mr);
-  };
-  if constexpr (KS) {
-    // The waves' partial sums meet in LDS; wave w stores degree tiles w, w + 4.
-    double* red = D[0];
-    __syncthreads();
 #pragma unroll
-    for (int i = 0; i < LT; i++)
+  for (int i = 0; i < LT; i++) {
+    if (i >= 2 * mine) continue;
 #pragma unroll
-      for (int j = 0; j < NJ; j++) red[((wave * LT + i) * NJ + j) * 64 + lane] = acc[i][j];
-    __syncthreads();
-    for (int i = wave; i < 2 * mine; i += 4)
+    for (int j = 0; j < NJ; j++) {
+      if (!vc[j].valid) continue;
+      const int mo = vc[j].sgn ? -m : m;
+      double* co = p.cout + ((long)vc[j].field * p.cstride) * 2 + (vc[j].col & 1);
 #pragma unroll
-      for (int j = 0; j < NJ; j++) {
-        double v = 0.0;
-#pragma unroll
-        for (int w = 0; w < 4; w++) v += red[((w * LT + i) * NJ + j) * 64 + lane];
-        store(j, degree(i, M::row(lane, 0)), v);
+      for (int r = 0; r < M::NR; r++) {
+        const int tile = wr * LT + i, mr = M::row(lane, r);
+        const int l = lp + (SYM ? 32 * (tile >> 1) + 2 * mr + (tile & 1) : 16 * tile + mr);
+        if (l > vc[j].lf) continue;
+        double v = M::get(acc[i][j], r);
+        if (vc[j].sgn && ((SYM ? m : l + p.n) & 1)) v = -v;
+        const long ci = 2 * (long)coef_index(l, mo, p.nabs, p.real);
+        if (p.accumulate) v += co[ci];
+        if (p.zero_last && vc[j].lf == p.L && l == p.L && mo == p.L) v = 0.0;
+        co[ci] = v;
       }
-  } else {
-#pragma unroll
-    for (int i = 0; i < LT; i++) {
-      if (i >= 2 * mine) continue;
-#pragma unroll
-      for (int j = 0; j < NJ; j++)
-#pragma unroll
-        for (int r = 0; r < M::NR; r++)
-          store(j, degree(wr * LT + i, M::row(lane, r)), M::get(acc[i][j], r));
     }
   }
 }
@@ -840,7 +779,8 @@ hipError_t go_anal(const LegParams& p, hipStream_t s) {
 // Wider tiles share each recurrence value and each A operand among more
 // columns; the narrow ones keep the matrix unit off padding columns: at most 8
 // columns take the 4-column instruction, at most 16 (32) one (two) tiles of
-// 16; more are interleaved by order sign.  Uneven batches stop at 64 (32 in
+// 16; more are interleaved by order sign.  Every tile adds a sum's terms in the
+// same order, so a batch equals its fields one by one.  Uneven batches stop at 64 (32 in
 // the analysis), whose fields have neighbouring degrees.  A launch of fewer than
 // kFewBlocks workgroups takes narrower tiles (and no 9th row tile): a wave
 // then has fewer MFMAs between two barriers, and idle CUs repeat the recurrence
@@ -860,13 +800,10 @@ static PairTile pair_tile(int ncol, int pair, bool f32m) {
   t.kind = f32m ? 1 : V <= 8 ? 2 : 0;
   t.vint = V > 32 ? 1 : 0;
   t.vcols = t.vint ? (ncol + 15) / 16 * 16 * (pair ? 2 : 1) : V;
-  if (t.kind == 2) {
-    t.rt = 8;
-    t.nj = V <= 4 ? 1 : 2;
-    t.cols = 4 * t.nj;
-  } else {
+  if (t.kind == 2)
+    t.rt = 2;
+  else
     set_cols(t, V <= 16 ? 16 : V <= 32 ? 32 : t.vcols <= 64 ? 64 : 128);
-  }
   return t;
 }
 PairTile pair_synth_tile(int ncol, int pair, int sym, bool f32m, bool uneven, int nr, int norder) {
@@ -875,7 +812,12 @@ PairTile pair_synth_tile(int ncol, int pair, int sym, bool f32m, bool uneven, in
   // Blocks of tw row tiles, each with room for one more.
   auto blocks = [rtt](int tw) { return std::max(1, (rtt + tw) / (tw + 1)); };
   t.nblk = blocks(8);
-  if (t.kind == 2) return t;
+  if (t.kind == 2) {
+    t.nj = 1;
+    if (t.vcols > 4) t.rt = 4;
+    t.cols = t.vcols > 4 ? 8 : 4;
+    return t;
+  }
   if (uneven && t.cols > 64) set_cols(t, 64);
   auto few = [&] { return norder * t.nblk * ((t.vcols + t.cols - 1) / t.cols) < kFewBlocks; };
   if (few()) t.nblk = std::max(1, (rtt + 7) / 8);
@@ -898,7 +840,11 @@ PairTile pair_synth_tile(int ncol, int pair, int sym, bool f32m, bool uneven, in
 PairTile pair_anal_tile(int ncol, int pair, bool uneven, int norder) {
   PairTile t = pair_tile(ncol, pair, false);
   t.nblk = 4;  // units of 32 degrees per pass
-  if (t.kind == 2) return t;
+  if (t.kind == 2) {
+    t.nj = t.vcols <= 4 ? 1 : 2;
+    t.cols = 4 * t.nj;
+    return t;
+  }
   if (uneven && t.cols > 32) set_cols(t, 32);
   while (t.cols > 16 &&
          norder * ((norder + 255) / 256) * ((t.vcols + t.cols - 1) / t.cols) < kFewBlocks)
@@ -918,8 +864,8 @@ hipError_t launch_leg_synth_pair(const LegParams& p0, const PairTile& t, int sym
     return t.nj == 2 ? go_synth<1, 0, 2, 2>(p, s) : go_synth<1, 0, 2, 1>(p, s);
   }
   if (t.kind == 2) {
-    if (sym) return t.nj == 1 ? go_synth<2, 1, 8, 1>(p, s) : go_synth<2, 1, 8, 2>(p, s);
-    return t.nj == 1 ? go_synth<2, 0, 8, 1>(p, s) : go_synth<2, 0, 8, 2>(p, s);
+    if (sym) return t.rt == 2 ? go_synth<2, 1, 2, 1>(p, s) : go_synth<2, 1, 4, 1>(p, s);
+    return t.rt == 2 ? go_synth<2, 0, 2, 1>(p, s) : go_synth<2, 0, 4, 1>(p, s);
   }
   if (sym) switch (t.rt) {
       case 8: return go_synth<0, 1, 8, 1>(p, s);
@@ -944,8 +890,8 @@ hipError_t launch_leg_anal_pair(const LegParams& p0, const PairTile& t, int sym,
   p.n_cg = (p.ncol + p.cw - 1) / p.cw;
   p.nquad = (p.ntheta + 3) / 4;
   if (t.kind == 2) {
-    if (sym) return t.nj == 1 ? go_anal<2, 1, 8, 1>(p, s) : go_anal<2, 1, 8, 2>(p, s);
-    return t.nj == 1 ? go_anal<2, 0, 8, 1>(p, s) : go_anal<2, 0, 8, 2>(p, s);
+    if (sym) return t.nj == 1 ? go_anal<2, 1, 2, 1>(p, s) : go_anal<2, 1, 2, 2>(p, s);
+    return t.nj == 1 ? go_anal<2, 0, 2, 1>(p, s) : go_anal<2, 0, 2, 2>(p, s);
   }
   if (sym) switch (t.rt) {
       case 8: return go_anal<0, 1, 8, 2>(p, s);
