@@ -531,12 +531,12 @@ constexpr int kAnalBand = 8;
 
 // Work list of an analysis launch: items (mw, pass | group << 16) in bands
 // of kAnalBand neighbouring order indices mw, each band ordered by group,
-// pass, order; padded to a multiple of 8 with (~0u, 0).  glmax[g] bounds the
+// pass, order; each XCD's eighth padded with (~0u, 0).  glmax[g] bounds the
 // degrees of group g (empty: lmax for every group).  Passes are kPass
 // degrees, or kWideAnalPass for family 3 (the 128-degree split-BF16 kernel);
 // family 5's items are the orders m >= 0 (mw = m) of the paired kernel.
-// An XCD runs a contiguous eighth of the list, so the workgroups on it at
-// one time hold a few passes of each order of a band: the passes of one order
+// An XCD runs whole bands, so the workgroups on it at one time hold a few
+// passes of each order of a band: the passes of one order
 // and group read the same input blocks (from L2 after the first), and the
 // orders of a band write neighbouring 16-byte coefficients of each degree
 // (the coefficient layout runs over m within a degree), which meet in L2 as
@@ -553,22 +553,66 @@ int ensure_worklist(gsh_grid_s* g, int family, int lmax, int n, int real, int ng
   // Family 5 (orders m and -m in one item) lists the orders m >= 0 in turn.
   const int nslot = family == 5 ? lmax + 1 : real ? lmax + 1 : 2 * lmax + 1;
   const int plen = family == 3 ? gsh::kWideAnalPass : gsh::kPass;  // degrees per pass
-  std::vector<uint2> items;
-  for (int b0 = 0; b0 < nslot; b0 += kAnalBand)
+  // Passes of order index mw in group grp.
+  auto passes = [&](int mw, int grp) {
+    const int lw = glmax.empty() ? lmax : glmax[grp];
+    const int m = family == 5 ? mw : order_of_host(mw, real);
+    const int l0 = std::max(std::abs(m), std::abs(n));
+    return l0 <= lw ? (lw - l0 + plen) / plen : 0;
+  };
+  // Every XCD takes its share of the bands of heavy and of light orders.  The
+  // split-BF16 kernels leave out the colatitudes near the poles: about
+  // 2 / pi asin(m / l) of them at degree l (fewer at small lmax, which the
+  // mixture evens out).  With contiguous ranges of equal item counts the XCD
+  // of the lowest orders, which leave nothing out, set the time: lMax=1024, 64
+  // complex fields, n=2, 18% fewer products 2176 -> 2170 us, with this list
+  // 1820 (timed without the rows left out).  Single orders for units took
+  // 2360 us in place of 2094: neighbouring orders' 16-byte coefficients then
+  // leave different XCDs as partial lines.  Narrower bands where there would be
+  // fewer than 64.  Family 0 leaves nothing out, and gains from the mixture too
+  // (FP32, lMax=1000, 32 real fields, n=1: analysis 1677 -> 1592 us).
+  const int bw = std::max(1, std::min<int>(kAnalBand, (long)nslot * ngroups / 64));
+  struct Unit {
+    double w;
+    std::vector<uint2> items;
+  };
+  std::vector<Unit> units;
+  for (int b0 = 0; b0 < nslot; b0 += bw)
     for (int grp = 0; grp < ngroups; grp++) {
-      const int lw = glmax.empty() ? lmax : glmax[grp];
-      for (int k = 0; k <= lw / plen; k++)
-        for (int mw = b0; mw < std::min(nslot, b0 + kAnalBand); mw++) {
-          const int m = family == 5 ? mw : order_of_host(mw, real);
-          const int l0 = std::max(std::abs(m), std::abs(n));
-          if (l0 <= lw && k < (lw - l0 + plen) / plen)
-            items.push_back(make_uint2(static_cast<unsigned>(mw),
+      Unit u{0.0, {}};
+      const int b1 = std::min(nslot, b0 + bw);
+      int np = 0;
+      for (int mw = b0; mw < b1; mw++) np = std::max(np, passes(mw, grp));
+      for (int k = 0; k < np; k++)
+        for (int mw = b0; mw < b1; mw++) {
+          if (k >= passes(mw, grp)) continue;
+          const int m = std::abs(family == 5 ? mw : order_of_host(mw, real));
+          const int l0 = std::max(m, std::abs(n));
+          u.w += family == 0 ? 1.0 : 1.1 - 0.64 * std::asin(m / (l0 + plen * (k + 1.0)));
+          u.items.push_back(make_uint2(static_cast<unsigned>(mw),
                                        static_cast<unsigned>(k) | (static_cast<unsigned>(grp) << 16)));
         }
+      if (!u.items.empty()) units.push_back(std::move(u));
     }
-  while (items.size() % 8 != 0 || items.empty()) items.push_back(make_uint2(~0u, 0u));
+  std::stable_sort(units.begin(), units.end(),
+                   [](const Unit& x, const Unit& y) { return x.w > y.w; });
+  std::vector<uint2> list[8];
+  double load[8] = {};
+  for (const Unit& u : units) {
+    const int x = static_cast<int>(std::min_element(load, load + 8) - load);
+    load[x] += u.w;
+    list[x].insert(list[x].end(), u.items.begin(), u.items.end());
+  }
+  size_t per = 1;
+  for (const auto& v : list) per = std::max(per, v.size());
+  std::vector<uint2> items;
+  items.reserve(8 * per);
+  for (auto& v : list) {
+    v.resize(per, make_uint2(~0u, 0u));
+    items.insert(items.end(), v.begin(), v.end());
+  }
   WorkList w;
-  w.per = static_cast<int>(items.size() / 8);
+  w.per = static_cast<int>(per);
   GSH_HIP(hipMalloc(&w.d, items.size() * sizeof(uint2)));
   GSH_HIP(hipMemcpy(w.d, items.data(), items.size() * sizeof(uint2), hipMemcpyHostToDevice));
   g->worklists.emplace(key, w);
@@ -1227,6 +1271,8 @@ int run_inverse(gsh_grid_s* g, NData* d, int lmax, int n, int real, int precisio
     if ((st = ensure_ck(g, d, n, s))) return st;
     p.ck = d->ck;
     p.ckoff = d->ckoff;
+    p.kf = d->kf;
+    p.nrt = (p.ntheta + 15) / 16;
     long* cso = nullptr;
     long nchunks = 0;
     if ((st = ensure_cso(g, lmax, n, real, sym, &cso, &nchunks))) return st;
@@ -1330,6 +1376,8 @@ int run_forward(gsh_grid_s* g, NData* d, int lmax, int n, int real, int precisio
   if ((st = ensure_ck(g, d, n, s))) return st;
   p.ck = d->ck;
   p.ckoff = d->ckoff;
+  p.kf = d->kf;
+  p.nrt = (p.ntheta + 15) / 16;
   const int ncg16 = (ncol + 15) / 16;
   GSH_HIP(timed(g, GSH_KERNEL_FFT_ANALYSIS, s, [&] {
     return run_fft(q, o, true, s);
@@ -1337,8 +1385,6 @@ int run_forward(gsh_grid_s* g, NData* d, int lmax, int n, int real, int precisio
   if (precision == GSH_FP64) {
     const int sym = n == 0 ? 1 : 0;
     p.pair = real ? 0 : 1;
-    p.kf = d->kf;
-    p.nrt = (p.ntheta + 15) / 16;
     const gsh::PairTile t = gsh::pair_anal_tile(p.ncol, p.pair, o.f_lmax != nullptr, lmax + 1);
     WorkList w;
     if ((st = ensure_pair_worklist(g, 1, lmax, n, p.pair, p.ncol, t, o.f_lmax_host, &w)))

@@ -118,6 +118,67 @@ __device__ __forceinline__ void flush(d4& acc, const f4 c) {
   acc[3] += (double)c[3];
 }
 
+// Near the poles an order's values are negligible (below kNegligible) up to a
+// degree that grows with the order: kf holds, per order and 16 colatitudes, the
+// first checkpoint that matters.  The products of the blocks before it are left
+// out as 0 * value, so a non-finite operand still reaches the sums it would
+// have reached.  lMax=1024, 64 fields, bf16x6: synthesis 1622 -> 1540 us (n=2)
+// and 624 -> 585 us (n=0, real), analysis 2200 -> 2026 us and 955 -> 897 us; the
+// rows left out still have to be read, 180 of the 2026 us.
+//
+// first_checkpoint: of row tiles t0 .. t0 + 7 (tiles past t1 take t1's).
+__device__ __forceinline__ int first_checkpoint(const LegParams& p, int m, int t0, int t1) {
+  int k = p.kf[(long)(m + p.L) * p.nrt + min(t0 + (int)(threadIdx.x & 7), t1)];
+#pragma unroll
+  for (int d = 1; d < 8; d <<= 1) k = min(k, __shfl_xor(k, d));
+  return __builtin_amdgcn_readfirstlane(k);
+}
+// live_tiles: the first and last of tiles 0 .. nrt - 1 whose degrees before
+// checkpoint kend matter (tile 0 if none does).
+__device__ __forceinline__ void live_tiles(const LegParams& p, int m, int nrt, int kend,
+                                           int& first, int& last) {
+  const unsigned short* kf = p.kf + (long)(m + p.L) * p.nrt;
+  const int lane = threadIdx.x & 63;
+  first = -1;
+  last = 0;
+  for (int b = 0; b < nrt; b += 64) {
+    const unsigned long long live = __ballot(b + lane < nrt && kf[min(b + lane, nrt - 1)] < kend);
+    if (!live) continue;
+    if (first < 0) first = b + __builtin_ctzll(live);
+    last = b + 63 - __builtin_clzll(live);
+  }
+  first = max(first, 0);
+}
+
+// left_out: 0 * x summed over rows t0 .. t0 + len - 1 of FP32 bins a (16 columns
+// to a row) and rows u0 .. u0 - len + 1 of bins b, 16 rows a load instruction:
+// lane (r, q) takes columns 4 q .. 4 q + 3 of row r.  column_poison then gives
+// every lane NaN if column lane % 16 met a non-finite value, else 0.  (Read as
+// B operands, 4 bytes a lane, after the sums: 2090 us in place of 2026.  Deeper
+// batches of loads, 8 and 12 for 4, gain nothing.)
+__device__ __forceinline__ void left_out(const float* a, int t0, const float* b, int u0, int len,
+                                         f4& za, f4& zb) {
+  const int lane = threadIdx.x & 63;
+#pragma unroll 4
+  for (int i = 0; i < len; i += 16) {
+    const int r = min(i + (lane >> 2), len - 1);
+    const f4 x = *reinterpret_cast<const f4*>(a + 16l * (t0 + r) + 4 * (lane & 3));
+    const f4 y = *reinterpret_cast<const f4*>(b + 16l * (u0 - r) + 4 * (lane & 3));
+    za += 0.0f * x;
+    zb += 0.0f * y;
+  }
+}
+__device__ __forceinline__ float column_poison(f4 z) {
+  const int lane = threadIdx.x & 63;
+  unsigned long long bad[4];
+#pragma unroll
+  for (int j = 0; j < 4; j++) bad[j] = __ballot(z[j] != z[j]);
+  if (!(bad[0] | bad[1] | bad[2] | bad[3])) return 0.0f;
+  const int j = lane & 3;
+  const unsigned long long m = j == 0 ? bad[0] : j == 1 ? bad[1] : j == 2 ? bad[2] : bad[3];
+  return m & (0x1111111111111111ull << ((lane & 15) >> 2)) ? __builtin_nanf("") : 0.0f;
+}
+
 // Analysis epilogues.  Column 16 tile + lane % 16 of the sums is the real
 // (even column) or imaginary (odd column) part of field col / 2, so the two
 // lanes of a field hold halves of the same coefficients.  trade_halves takes
@@ -535,6 +596,8 @@ __global__ __launch_bounds__(512) void leg_synth_bf16_s(LegParams p) {
   const int nb = 2 * nC;                     // blocks: block 2 c + k is chunk c's class k
   const int rows = min(128, nn - tsb * 128);  // valid colatitudes of the item
   const int par0 = (l0 + m) & 1;             // class of the even offsets from l0
+  // First chunk that matters at the item's rows (tile by tile up to the north's last).
+  const int c0 = min(first_checkpoint(p, m, 8 * tsb, (nn - 1) >> 4) >> 2, nC - 1);
 
   // Producer share: colatitude block pb, degree quarter pq of a chunk.
   const int pb = wave & 1, pq = wave >> 1;
@@ -548,11 +611,11 @@ __global__ __launch_bounds__(512) void leg_synth_bf16_s(LegParams p) {
   auto ck_state = [&](int k) { return ckm[(long)(nck > 1 ? min(k, nck - 1) - 1 : 0) * nt]; };
   double pe0, pe1;
   {
-    // Chunk 0: the seed for quarter 0, checkpoint pq for the others.
+    // Chunk c0: checkpoint 4 c0 + pq, the seed for checkpoint 0.
     const double seed = p.seeds[(long)(m + p.L) * nt + tpc];
-    const double2 c1 = ck_state(max(pq, 1));
-    pe0 = pq == 0 || nck < 2 ? seed : c1.x;
-    pe1 = pq == 0 || nck < 2 ? 0.0 : c1.y;
+    const double2 c1 = ck_state(max(4 * c0 + pq, 1));
+    pe0 = 4 * c0 + pq == 0 || nck < 2 ? seed : c1.x;
+    pe1 = 4 * c0 + pq == 0 || nck < 2 ? 0.0 : c1.y;
   }
 
   const uint4* recq = reinterpret_cast<const uint4*>(p.rec + (ld_uniform(p.roff, m + p.L) - l0));
@@ -584,6 +647,19 @@ __global__ __launch_bounds__(512) void leg_synth_bf16_s(LegParams p) {
     for (int t = 0; t < 2; t++)
 #pragma unroll
       for (int k = 0; k < 2; k++) acc[g][t][k] = d4{0.0, 0.0, 0.0, 0.0};
+  if (c0 > 0) {  // the coefficients left out (plane 0 is non-finite where they are)
+    f4 z[2] = {f4{0.f, 0.f, 0.f, 0.f}, f4{0.f, 0.f, 0.f, 0.f}};
+#pragma unroll 4
+    for (int b = 0; b < 2 * c0; b++) {
+      const uint4* cb = bbase + (long)b * bstride + toff;
+      z[0] = mfma(make_uint4(0u, 0u, 0u, 0u), cb[0], z[0]);
+      z[1] = mfma(make_uint4(0u, 0u, 0u, 0u), cb[NS * 64], z[1]);
+    }
+#pragma unroll
+    for (int g = 0; g < 4; g++)  // E: both F(t) and F(nt-1-t) take it
+#pragma unroll
+      for (int t = 0; t < 2; t++) flush(acc[g][t][0], z[t]);
+  }
 
   // Production: pair i (0..7) of this wave's quarter is steps 2 i, 2 i + 1,
   // degrees d = 16 pq + 2 i (+1) of the chunk.  An even pair keeps its two
@@ -626,14 +702,14 @@ __global__ __launch_bounds__(512) void leg_synth_bf16_s(LegParams p) {
     }
   };
 
-  // Prologue: coefficients of chunks 0 and 1, B operands of block 0,
-  // production of chunk 0.
+  // Prologue: coefficients of chunks c0 and c0 + 1, B operands of c0's first
+  // block, production of c0.
   if (tid < 128) {
-    rsc[0][tid] = fetch_rec(0);
-    rsc[1][tid] = fetch_rec(1);
+    rsc[0][tid] = fetch_rec(c0);
+    rsc[1][tid] = fetch_rec(c0 + 1);
   }
   uint4 Bc[2][NS];
-  fetchB(0, Bc);
+  fetchB(2 * c0, Bc);
   __syncthreads();
   const bool pv = 64 * pb < rows;  // this wave's producer block holds colatitudes
   if (pv) {
@@ -647,10 +723,10 @@ __global__ __launch_bounds__(512) void leg_synth_bf16_s(LegParams p) {
   // of chunk c + 1 (none in the last chunk).  One barrier per chunk, after
   // its class-1 block.  The state of chunk c + 1 (checkpoint 4 (c + 1) + pq)
   // is loaded one chunk before its use.
-  double2 nx = ck_state(4 + pq);
+  double2 nx = ck_state(4 * (c0 + 1) + pq);
   auto block = [&](int c, const int k, const bool next) {
     const int b = 2 * c + k;
-    const int abuf = c & 1;
+    const int abuf = (c ^ c0) & 1;
     const bool prod = pv && c + 1 < nC;
     uint4 Bn[2][NS];
     if (next) fetchB(b + 1, Bn);
@@ -678,12 +754,12 @@ __global__ __launch_bounds__(512) void leg_synth_bf16_s(LegParams p) {
         for (int s = 0; s < NS; s++) Bc[t][s] = Bn[t][s];
     }
     if (k == 1) {
-      // Chunk c + 2's coefficients (rsc[c & 1] was last read in chunk c - 1).
+      // Chunk c + 2's coefficients (its buffer was last read in chunk c - 1).
       if (tid < 128) rsc[abuf][tid] = qr;
       __syncthreads();
     }
   };
-  for (int c = 0; c + 1 < nC; c++) {
+  for (int c = c0; c + 1 < nC; c++) {
     block(c, 0, true);
     block(c, 1, true);
   }
@@ -765,6 +841,8 @@ __global__ __launch_bounds__(512) void leg_synth_bf16_pm(LegParams p) {
   const int nC = (p.lmax - l0 + 64) >> 6;   // 64-degree chunks
   const int n32 = (p.lmax - l0 + 32) >> 5;  // 32-degree coefficient blocks of each order
   const int rows = min(128, nt - tsb * 128);  // valid colatitudes of the item
+  // First chunk that matters at the item's rows.
+  const int c0 = min(first_checkpoint(p, m, 8 * tsb, p.nrt - 1) >> 2, nC - 1);
 
   // Producer share: colatitude block pb, degree quarter pq of a chunk.
   const int pb = wave & 1, pq = wave >> 1;
@@ -776,11 +854,11 @@ __global__ __launch_bounds__(512) void leg_synth_bf16_pm(LegParams p) {
   auto ck_state = [&](int k) { return ckm[(long)(nck > 1 ? min(k, nck - 1) - 1 : 0) * nt]; };
   double pe0, pe1;
   {
-    // Chunk 0: the seed for quarter 0, checkpoint pq for the others.
+    // Chunk c0: checkpoint 4 c0 + pq, the seed for checkpoint 0.
     const double seed = p.seeds[(long)(m + p.L) * nt + tpc];
-    const double2 c1 = ck_state(max(pq, 1));
-    pe0 = pq == 0 || nck < 2 ? seed : c1.x;
-    pe1 = pq == 0 || nck < 2 ? 0.0 : c1.y;
+    const double2 c1 = ck_state(max(4 * c0 + pq, 1));
+    pe0 = 4 * c0 + pq == 0 || nck < 2 ? seed : c1.x;
+    pe1 = 4 * c0 + pq == 0 || nck < 2 ? 0.0 : c1.y;
   }
 
   const uint4* recq = reinterpret_cast<const uint4*>(p.rec + (ld_uniform(p.roff, m + p.L) - l0));
@@ -812,6 +890,19 @@ __global__ __launch_bounds__(512) void leg_synth_bf16_pm(LegParams p) {
   for (int g = 0; g < 8; g++)
 #pragma unroll
     for (int o = 0; o < 2; o++) acc[g][o] = d4{0.0, 0.0, 0.0, 0.0};
+  if (c0 > 0) {  // the coefficients left out (plane 0 is non-finite where they are)
+    f4 z[2] = {f4{0.f, 0.f, 0.f, 0.f}, f4{0.f, 0.f, 0.f, 0.f}};
+#pragma unroll 4
+    for (int b = 0; b < 2 * c0; b++) {
+      const long off = (long)b * bstride + toff;
+      z[0] = mfma(make_uint4(0u, 0u, 0u, 0u), bbp[off], z[0]);
+      z[1] = mfma(make_uint4(0u, 0u, 0u, 0u), bbn[off], z[1]);
+    }
+#pragma unroll
+    for (int g = 0; g < 8; g++)
+#pragma unroll
+      for (int o = 0; o < 2; o++) flush(acc[g][o], z[o]);
+  }
 
   // Production: pair i (0..7) of this wave's quarter is steps 2 i, 2 i + 1,
   // degrees 16 pq + 2 i (+1) of the chunk; every 4 pairs fill the uint4 of
@@ -843,14 +934,14 @@ __global__ __launch_bounds__(512) void leg_synth_bf16_pm(LegParams p) {
     }
   };
 
-  // Prologue: coefficients of chunks 0 and 1, B operands of block 0,
-  // production of chunk 0.
+  // Prologue: coefficients of chunks c0 and c0 + 1, B operands of c0's first
+  // block, production of c0.
   if (tid < 128) {
-    rsc[0][tid] = fetch_rec(0);
-    rsc[1][tid] = fetch_rec(1);
+    rsc[0][tid] = fetch_rec(c0);
+    rsc[1][tid] = fetch_rec(c0 + 1);
   }
   uint4 Bc[2][NS];
-  fetchB(0, 0, Bc);
+  fetchB(c0, 0, Bc);
   __syncthreads();
   const bool pv = 64 * pb < rows;  // this wave's producer block holds colatitudes
   if (pv) {
@@ -866,9 +957,9 @@ __global__ __launch_bounds__(512) void leg_synth_bf16_pm(LegParams p) {
   // coefficients of chunk c + 2 are complete, and chunk c's planes free,
   // after it.  The state of chunk c + 1 (checkpoint 4 (c + 1) + pq) is
   // loaded one chunk before its use.
-  double2 nx = ck_state(4 + pq);
+  double2 nx = ck_state(4 * (c0 + 1) + pq);
   auto block = [&](int c, const int dh, const bool next) {
-    const int abuf = c & 1;
+    const int abuf = (c ^ c0) & 1;
     const bool prod = pv && c + 1 < nC;
     const bool live = 2 * c + dh < n32;
     uint4 Bn[2][NS];
@@ -902,12 +993,12 @@ __global__ __launch_bounds__(512) void leg_synth_bf16_pm(LegParams p) {
         for (int s = 0; s < NS; s++) Bc[o][s] = Bn[o][s];
     }
     if (dh == 1) {
-      // Chunk c + 2's coefficients (rsc[c & 1] was last read in chunk c - 1).
+      // Chunk c + 2's coefficients (its buffer was last read in chunk c - 1).
       if (tid < 128) rsc[abuf][tid] = qr;
       __syncthreads();
     }
   };
-  for (int c = 0; c + 1 < nC; c++) {
+  for (int c = c0; c + 1 < nC; c++) {
     block(c, 0, true);
     block(c, 1, true);
   }
@@ -1208,8 +1299,18 @@ __global__ __launch_bounds__(512) void leg_anal_bf16_pm(LegParams p) {
   const int slot = m - p.m_first, slotn = -m - p.m_first;
   const int l0 = max(m, p.nabs);
   const int nt = p.ntheta;
-  const int ngrp = (nt + 127) >> 7;
   const int lp = l0 + kPass * pass;
+  // Colatitudes that matter to the pass: K chunks kb .. kb + nk - 1 of 32, in
+  // whole pairs (chunk sums are flushed in pairs).
+  int kb, nk;
+  {
+    int first, last;
+    live_tiles(p, m, p.nrt, (kPass / kCk) * (pass + 1), first, last);
+    kb = 2 * (first >> 2);
+    nk = min(p.nkc, 2 * ((last >> 2) + 1)) - kb;
+  }
+  const int tb = 32 * kb;  // first colatitude
+  const int ngrp = (nk + 3) >> 2;
   rec_t* rq = rec_ptr(p.rec, ld_uniform(p.roff, m + p.L) - l0);
 
   // Production (leg_anal_bf16's): block half bh, degree quarter q.
@@ -1221,7 +1322,7 @@ __global__ __launch_bounds__(512) void leg_anal_bf16_pm(LegParams p) {
   double nx_seed, nx_cs;
   double2 nx_ck;
   auto prefetch = [&](int g) {
-    const int tc = min((2 * g + bh) * 64 + lane, nt - 1);
+    const int tc = min(tb + (2 * g + bh) * 64 + lane, nt - 1);
     nx_seed = sdp[tc];
     nx_ck = ckp[tc];
     nx_cs = p.cosv[tc];
@@ -1251,7 +1352,7 @@ __global__ __launch_bounds__(512) void leg_anal_bf16_pm(LegParams p) {
     }
   };
 
-  // B operands: lane (q4, c) of K chunk kc takes colatitudes theta = 32 kc +
+  // B operands: lane (q4, c) of K chunk kb + kc takes colatitudes theta = tb + 32 kc +
   // 8 q4 + e (e = 0..7) of column 16 tile + c.  Order m reads FA row theta
   // (leg_anal_bf16's addresses); order -m reads row nt-1-theta, 16 floats
   // before the previous e within the (slot, column group) block, whose rows
@@ -1264,9 +1365,9 @@ __global__ __launch_bounds__(512) void leg_anal_bf16_pm(LegParams p) {
   const int tile = csg * 8 + wave;
   const int tcl = min(tile, p.n_cg - 1);
   const float* fb =
-      p.FA32 + (((long)slot * p.n_cg + tcl) * p.nquad + 2 * (lane >> 4)) * 64 + (lane & 15);
+      p.FA32 + (((long)slot * p.n_cg + tcl) * p.nquad + 8 * kb + 2 * (lane >> 4)) * 64 + (lane & 15);
   const float* fbn = p.FA32 + ((long)slotn * p.n_cg + tcl) * p.nquad * 64 + (lane & 15);
-  const int rn0 = nt - 1 - 8 * (lane >> 4);  // row of order -m at kc = 0, e = 0
+  const int rn0 = nt - 1 - tb - 8 * (lane >> 4);  // row of order -m at kc = 0, e = 0
   auto loadB = [&](int kc, RawB (&X)[2]) {
 #pragma unroll
     for (int e = 0; e < 8; e++) X[0].x[e] = fb[(long)kc * 512 + 16 * e];
@@ -1276,7 +1377,7 @@ __global__ __launch_bounds__(512) void leg_anal_bf16_pm(LegParams p) {
   };
   auto splitB = [&](const RawB& X, uint4 (&B)[NS], int kc, bool last) {
     unsigned pl[NS][4];
-    const int th = 32 * kc + 8 * (lane >> 4);
+    const int th = tb + 32 * kc + 8 * (lane >> 4);
 #pragma unroll
     for (int e2 = 0; e2 < 4; e2++) {
       float x0 = X.x[2 * e2], x1 = X.x[2 * e2 + 1];
@@ -1332,14 +1433,27 @@ __global__ __launch_bounds__(512) void leg_anal_bf16_pm(LegParams p) {
   };
 
   prefetch(0);
+  // Colatitudes left out, at either end (order -m: their mirrors), here, where
+  // the loads wait together with the first state's.
+  float left[2] = {0.0f, 0.0f};
+  if (nk < p.nkc) {
+    const float* bp = p.FA32 + ((long)slot * p.n_cg + tcl) * p.nquad * 64;
+    const float* bn = p.FA32 + ((long)slotn * p.n_cg + tcl) * p.nquad * 64;
+    const int te = min(tb + 32 * nk, nt);
+    f4 z[2] = {f4{0.f, 0.f, 0.f, 0.f}, f4{0.f, 0.f, 0.f, 0.f}};
+    left_out(bp, 0, bn, nt - 1, tb, z[0], z[1]);
+    left_out(bp, te, bn, nt - 1 - te, nt - te, z[0], z[1]);
+    left[0] = column_poison(z[0]);
+    left[1] = column_poison(z[1]);
+  }
   begin();
 #pragma unroll
   for (int part = 0; part < 4; part++) produce4(0, part);
   prefetch(1);
   __syncthreads();
   // B operands one chunk ahead: chunk c in X[c & 1] (loads clamp to the
-  // last chunk nkc - 1).
-  const int kcl = p.nkc - 1;
+  // last chunk nk - 1).
+  const int kcl = nk - 1;
   RawB X[2][2];
   loadB(0, X[0]);
   for (int g = 0; g + 1 < ngrp; g++) {
@@ -1357,21 +1471,27 @@ __global__ __launch_bounds__(512) void leg_anal_bf16_pm(LegParams p) {
     __syncthreads();
   }
   {
-    // Last group: chunks 4 (ngrp-1) .. nkc-1 (X[0] holds the first).
+    // Last group: chunks 4 (ngrp-1) .. nk-1 (X[0] holds the first).
     const int buf = (ngrp - 1) & 1;
     const int kc0 = 4 * (ngrp - 1);
 #pragma unroll
     for (int j = 0; j < 4; j++)
-      if (kc0 + j < p.nkc) {
-        if (kc0 + j + 1 < p.nkc) loadB(kc0 + j + 1, X[(j + 1) & 1]);
+      if (kc0 + j < nk) {
+        if (kc0 + j + 1 < nk) loadB(kc0 + j + 1, X[(j + 1) & 1]);
         step(buf, kc0 + j, X[j & 1], true, j & 1);
       }
-    const bool lodd = (p.nkc - 1) & 1;
+    const bool lodd = (nk - 1) & 1;
 #pragma unroll
     for (int i = 0; i < 4; i++)
 #pragma unroll
       for (int j = 0; j < 2; j++) flush(acc[i][j], lodd ? pp[i][j] + cp[i][j] : cp[i][j]);
   }
+
+#pragma unroll
+  for (int j = 0; j < 2; j++)
+    if (__ballot(left[j] != 0.0f))
+#pragma unroll
+      for (int i = 0; i < 4; i++) flush(acc[i][j], f4{left[j], left[j], left[j], left[j]});
 
   // Rows l = lp + 16*lt + 4*(lane/16) + r, column 16*tile + lane%16; order
   // -m's sums take the sign (-1)^(l+n).
@@ -1894,9 +2014,17 @@ __global__ __launch_bounds__(512) void leg_anal_bf16_ws(LegParams p) {
   const int l0 = max(abs(m), p.nabs);
   const int nt = p.ntheta;
   const int nts = (nt + 1) >> 1;  // northern colatitudes, the equator included
-  const int ngrp = (nts + 63) >> 6;
-  const int nkc = (nts + 31) >> 5;
   const int lp = l0 + kWidePass * pass;  // first degree of the pass
+  // Colatitudes that matter to the pass: K chunks kb .. kb + nk - 1 of 32.
+  int kb;
+  {
+    int first, last;
+    live_tiles(p, m, (nts + 15) >> 4, (kWidePass / kCk) * (pass + 1), first, last);
+    kb = first >> 1;
+  }
+  const int tb = 32 * kb;  // first colatitude
+  const int nk = ((nts + 31) >> 5) - kb;
+  const int ngrp = (nk + 1) >> 1;
   const int par0 = (lp + m) & 1;         // parity of l + m at the pass's first degree
   // Recurrence coefficients of the pass: entries lp+1 .. lp+128 (entry l for
   // degree l).  Entries up to L + kRecPad exist: kRecPad covers the 128
@@ -1913,7 +2041,7 @@ __global__ __launch_bounds__(512) void leg_anal_bf16_ws(LegParams p) {
   double nx_seed, nx_cs;
   double2 nx_ck;
   auto prefetch = [&](int g) {
-    const int tc = min(64 * g + lane, nts - 1);
+    const int tc = min(tb + 64 * g + lane, nts - 1);
     nx_seed = sdp[tc];
     nx_ck = ckp[tc];
     nx_cs = p.cosv[tc];
@@ -1955,14 +2083,14 @@ __global__ __launch_bounds__(512) void leg_anal_bf16_ws(LegParams p) {
   };
   const int tile = csg * 8 + wave;
   const float* ft = p.FA32 + ((long)slot * p.n_cg + min(tile, p.n_cg - 1)) * p.nquad * 64 + (lane & 15);
-  const float* fb = ft + 2 * (lane >> 4) * 64;
-  // Chunk kc's colatitudes t = 32 kc + 8 (lane / 16) + e (X) and their
+  const float* fb = ft + (8 * kb + 2 * (lane >> 4)) * 64;
+  // Chunk kb + kc's colatitudes t = tb + 32 kc + 8 (lane / 16) + e (X) and their
   // mirrors nt - 1 - t (Y), 16 floats apart per row within the (slot, column
   // group) block.  A mirror row below 0 (t past the north, the last chunk
   // only, at most 31 rows) reads the previous block or the front pad of FA;
   // combine zeroes it.
   auto loadB = [&](int kc, RawB& X, RawB& Y) {
-    const float* fm = ft + 16 * (nt - 1 - 32 * kc - 8 * (lane >> 4));
+    const float* fm = ft + 16 * (nt - 1 - tb - 32 * kc - 8 * (lane >> 4));
 #pragma unroll
     for (int e = 0; e < 8; e++) {
       X.x[e] = fb[(long)kc * 512 + 16 * e];
@@ -1974,7 +2102,7 @@ __global__ __launch_bounds__(512) void leg_anal_bf16_ws(LegParams p) {
   // (+1) and 0 (-1) at the equator, 0 past the north.  Only the chunks of
   // the last group (`last`) hold the equator or rows past the north.
   auto combine = [&](const RawB& X, const RawB& Y, int kc, float sign, RawB& Z, bool last) {
-    const int th = 32 * kc + 8 * (lane >> 4);
+    const int th = tb + 32 * kc + 8 * (lane >> 4);
 #pragma unroll
     for (int e = 0; e < 8; e++) {
       if (!last) {
@@ -1988,7 +2116,7 @@ __global__ __launch_bounds__(512) void leg_anal_bf16_ws(LegParams p) {
   };
   auto splitB = [&](const RawB& X, uint4 (&B)[1][NS], int kc, bool last) {
     unsigned pl[NS][4];
-    const int th = 32 * kc + 8 * (lane >> 4);
+    const int th = tb + 32 * kc + 8 * (lane >> 4);
 #pragma unroll
     for (int e2 = 0; e2 < 4; e2++) {
       float x0 = X.x[2 * e2], x1 = X.x[2 * e2 + 1];
@@ -2042,13 +2170,20 @@ __global__ __launch_bounds__(512) void leg_anal_bf16_ws(LegParams p) {
   };
 
   prefetch(0);
+  float left = 0.0f;  // colatitudes left out, and their mirrors
+  if (kb > 0) {
+    const float* bp = ft - (lane & 15);
+    f4 z = f4{0.f, 0.f, 0.f, 0.f}, y = z;
+    left_out(bp, 0, bp, nt - 1, tb, z, y);
+    left = column_poison(z + y);
+  }
   begin();
   produce8(0, 0);
   produce8(0, 1);
   prefetch(1);
   __syncthreads();
   // B operands one chunk ahead: chunk c in X[c & 1], its mirrors in Y[c & 1].
-  const int kcl = nkc - 1;
+  const int kcl = nk - 1;
   RawB X[2], Y[2];
   loadB(0, X[0], Y[0]);
   for (int g = 0; g + 1 < ngrp; g++) {
@@ -2066,15 +2201,19 @@ __global__ __launch_bounds__(512) void leg_anal_bf16_ws(LegParams p) {
     __syncthreads();
   }
   {
-    // Last group: chunks 2 (ngrp-1) .. nkc-1 (one or two).
+    // Last group: chunks 2 (ngrp-1) .. nk-1 (one or two).
     const int buf = (ngrp - 1) & 1;
     const int kc0 = 2 * (ngrp - 1);
-    if (kc0 + 1 < nkc) loadB(kc0 + 1, X[1], Y[1]);
+    if (kc0 + 1 < nk) loadB(kc0 + 1, X[1], Y[1]);
     step(buf, kc0, X[0], Y[0], true);
-    if (kc0 + 1 < nkc) step(buf, kc0 + 1, X[1], Y[1], true);
+    if (kc0 + 1 < nk) step(buf, kc0 + 1, X[1], Y[1], true);
 #pragma unroll
     for (int i = 0; i < 8; i++) flush(acc[i][0], cp[i]);
   }
+
+  if (__ballot(left != 0.0f))
+#pragma unroll
+    for (int i = 0; i < 8; i++) flush(acc[i][0], f4{left, left, left, left});
 
   const int col = tile * 16 + (lane & 15);
   const bool odd = lane & 1;
@@ -2191,7 +2330,7 @@ hipError_t launch_coef_split(const LegParams& p, int ns, hipStream_t s) {
 }
 
 hipError_t launch_leg_synth_bf16(const LegParams& p0, int ns, hipStream_t s) {
-  if (!p0.ck || !p0.ckoff) return hipErrorInvalidValue;  // checkpoint table required
+  if (!p0.ck || !p0.ckoff || !p0.kf) return hipErrorInvalidValue;  // checkpoint tables required
   LegParams p = p0;
   p.n_tsb = (p.ntheta + 255) / 256;
   p.n_cg = (p.ntile + 7) / 8;  // column super-groups of 8 tiles
@@ -2278,7 +2417,7 @@ hipError_t launch_anal_bf16_w(const LegParams& p0, hipStream_t s, bool sym) {
 }
 
 hipError_t launch_leg_anal_bf16(const LegParams& p, int ns, hipStream_t s, int form) {
-  if (!p.ck || !p.ckoff) return hipErrorInvalidValue;  // checkpoint table required
+  if (!p.ck || !p.ckoff || !p.kf) return hipErrorInvalidValue;  // checkpoint tables required
   if (!p.FA32) return hipErrorInvalidValue;             // FP32 bins required
   if ((form == 2 || form == 3) && p.nabs != 0) return hipErrorInvalidValue;  // n = 0 only
   if (form == 4) {  // orders m and -m together: complex fields

@@ -97,6 +97,37 @@ def test_left_out_terms_stay_visible(torch, n, real, bad):
     assert not finite[1, :-1].all(dim=-1).any()
 
 
+# The split-BF16 kernels leave whole blocks of 128 rows x 64 degrees (synthesis)
+# and pairs of 32 rows x 64 degrees (analysis) out, so a larger grid; the sums
+# kept against FP64: FP32-accurate products and bins, 2^-24 each, 1e-5 for
+# bf16x6 and 2^-16 products, 1e-3 for bf16x3.
+@pytest.mark.parametrize("n,real", [(0, True), (0, False), (2, False)])
+@pytest.mark.parametrize("precision,tol", [("bf16x6", 1e-5), ("bf16x3", 1e-3)])
+@pytest.mark.parametrize("L,lmax", [(1000, 1000), (767, 700)])
+def test_left_out_split_blocks(torch, L, lmax, n, real, precision, tol):
+    say(f"[pair] split L={L} lmax={lmax} n={n} real={real} {precision}")
+    g = G.GaussLegendreGrid(L, 2)
+    c = torch.from_numpy(G.random_coefficients(lmax, n, real=real, seed=SEED0, grid_lmax=L,
+                                               batch=3)).cuda()
+    f = g.inverse(lmax, n, c, real=real)
+    a = g.forward(lmax, n, f, real=real)
+    fp = g.inverse(lmax, n, c, real=real, precision=precision)
+    ap = g.forward(lmax, n, f, real=real, precision=precision)
+    for x, y in ((fp, f), (ap, a)):
+        assert float((x - y).norm() / y.norm()) <= tol
+    c[1, G.coefficient_index(lmax, n, lmax - 100, lmax - 105, real)] = float("nan")
+    g.inverse(lmax, n, c, field=fp, real=real, precision=precision)
+    finite = torch.isfinite(torch.view_as_real(fp) if fp.is_complex() else fp).reshape(3, -1)
+    assert finite[0].all() and finite[2].all() and not finite[1].any()
+    for row in (1, -2):  # a sample next to either pole
+        h = f.clone()
+        h[1, row, 5] = float("inf")
+        g.forward(lmax, n, h, coeffs=ap, real=real, precision=precision)
+        finite = torch.isfinite(torch.view_as_real(ap)).reshape(3, -1, 2)
+        assert finite[0].all() and finite[2].all()
+        assert not finite[1, :-1].all(dim=-1).any()
+
+
 # Degrees after an order's last stored state: the order L - 12 rises from
 # negligible seeds to 2^-83 at rows near the pole within its last 13 degrees.
 # One field for each such ring, zero elsewhere, so its sums hold nothing larger.
