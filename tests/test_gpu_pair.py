@@ -155,3 +155,26 @@ def test_last_degrees_of_an_order(torch, n, precision):
     for i, t in enumerate(rows):
         ref = og.forward(L, n, f[i])[idx]
         assert np.linalg.norm(a[i][idx] - ref) <= tol * np.linalg.norm(ref), t
+
+
+# The analysis allocates its coefficients without a fill: every one is written,
+# at odd sizes, truncations and column counts, in every mode.
+@pytest.mark.parametrize("precision", ["fp64", "fp32", "bf16x3", "bf16x6"])
+@pytest.mark.parametrize("n,real", [(0, True), (0, False), (2, False), (-1, True)])
+def test_every_coefficient_is_written(torch, n, real, precision):
+    for L, lmax, batch in ((2, 2, 1), (3, 2, 3), (40, 33, 17), (129, 128, 5), (300, 300, 2),
+                           (300, 190, 40)):
+        say(f"[pair] written L={L} lmax={lmax} n={n} real={real} B={batch} {precision}")
+        g = G.GaussLegendreGrid(L, 2)
+        size = G.coefficient_size(lmax, n, real)
+        c = torch.from_numpy(G.random_coefficients(lmax, n, real=real, seed=SEED0, grid_lmax=L,
+                                                   batch=batch)).cuda()
+        f = g.inverse(lmax, n, c, real=real, precision=precision)
+        out = torch.full((batch, size), float("nan"), dtype=torch.complex128, device="cuda")
+        g.forward(lmax, n, f, coeffs=out, real=real, precision=precision)
+        assert torch.isfinite(torch.view_as_real(out)).all()
+        assert torch.equal(g.forward(lmax, n, f, real=real, precision=precision), out)
+        out.fill_(float("nan"))
+        g.forward_product(lmax, n, f, torch.ones_like(f), coeffs=out, real=real,
+                          precision=precision)
+        assert torch.isfinite(torch.view_as_real(out)).all()
