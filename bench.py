@@ -48,12 +48,13 @@ TRAFFIC_FILE = os.path.join(ROOT, "profiles", "transform_kernels_lmax1024_b64_co
 # batch), as regular expressions over the summary's kernel names.
 FAMILY_KERNELS = {
     # split-BF16 Legendre kernels: the n=0 batch runs the equatorially
-    # symmetric variants (_ws, _s), the n=2 batch orders m and -m paired (_pm)
-    "legendre_analysis": {"fp64": r"leg_anal_f64<4, false>", "fp32": r"leg_anal_f64<4, true>",
+    # symmetric variants (_ws, _s), the n=2 batch orders m and -m paired (_pm);
+    # FP64: n=0 by parity and n=2 paired are leg_*_p<0, 1, ..> and <0, 0, ..>
+    "legendre_analysis": {"fp64": r"leg_anal_p<0, \d, 8, 2>", "fp32": r"leg_anal_f32<4>",
                           "bf16x3": r"leg_anal_bf16_(ws<2, \d>|pm<2>)",
                           "bf16x6": r"leg_anal_bf16_(ws<3, \d>|pm<3>)"},
-    "legendre_synthesis": {"fp64": r"leg_synth_f64<2, \d, false>",
-                           "fp32": r"leg_synth_f64<2, \d, true>",
+    "legendre_synthesis": {"fp64": r"leg_synth_p<0, \d, 8, \d>",
+                           "fp32": r"leg_synth_p<1, 0, 8, 2>",
                            "bf16x3": r"leg_synth_bf16_(s<2, \d>|pm<2>)",
                            "bf16x6": r"leg_synth_bf16_(s<3, \d>|pm<3>)"},
     # FA in FP64 (fp64, fp32) or FP32 (split-BF16 modes): last template argument
@@ -74,21 +75,15 @@ def log(*a):
 
 def algorithmic_counts():
     """Per-field algorithmic work: Legendre flops 4*ntheta*C (complex) or
-    4*ntheta*R (real); ring-FFT HBM bytes (field read/write + F bins).
-
-    Also the Legendre flops the kernels issue: the n=0 kernels fold each
-    colatitude with its mirror (d^l_{m0}(pi - theta) = (-1)^(l+m) d^l_{m0}(theta)
-    on the equatorially symmetric Gauss-Legendre nodes), so they multiply over
-    the ceil(ntheta/2) northern colatitudes only."""
+    4*ntheta*R (real); ring-FFT HBM bytes (field read/write + F bins)."""
     import gshtrans_amd as G
     nt, N = L + 1, 2 * L
     R0 = G.coefficient_size(L, 0, real=True)
     C2 = G.coefficient_size(L, 2, real=False)
     leg = {"real": 4.0 * nt * R0, "complex": 4.0 * nt * C2}
-    issued = {"real": 4.0 * ((nt + 1) // 2) * R0, "complex": 4.0 * nt * C2}
     fft_bytes = {"real": nt * N * 8 + nt * (L + 1) * 16,
                  "complex": nt * N * 16 + nt * (2 * L + 1) * 16}
-    return leg, fft_bytes, issued
+    return leg, fft_bytes
 
 
 def run_gpu(args):
@@ -226,7 +221,7 @@ def run_gpu(args):
 
 
 def roofline(results, headline):
-    leg, fftb, issued = algorithmic_counts()
+    leg, fftb = algorithmic_counts()
     kt = results[headline]["kernels"]
     # per-step work: real batch + complex batch, one launch each per kernel
     work = {
@@ -248,9 +243,10 @@ def roofline(results, headline):
         achieved = total * PRODUCTS[headline] / sec / 1e12
         peak = PEAK_TFLOPS[headline]
         unit = "TFLOP/s"
-        # the same over the products the kernels issue (n=0: northern half)
-        done = BATCH * (issued["real"] + issued["complex"]) * steps
-        issued_frac = done * PRODUCTS[headline] / sec / 1e12 / peak
+        # the same over the products the kernels issue (n=0: the northern half;
+        # without what is negligible near the poles; with tile padding)
+        done = issued_per_launch(name, headline)
+        issued_frac = done * launches / sec / 1e12 / peak if done else None
     else:
         achieved = total / sec / 1e9
         peak = HBM_GBPS
@@ -263,21 +259,29 @@ def roofline(results, headline):
             "avg_launch_ms": ms / max(launches, 1), "per_kernel": per_kernel}
 
 
+def counter_rows(family, mode):
+    """The committed counter summary's rows of a work family's real and complex
+    instantiations (empty: none)."""
+    from gshtrans_amd.profile_summary import load_table
+    t = load_table(TRAFFIC_FILE)
+    pat = FAMILY_KERNELS.get(family)
+    pat = pat.get(mode) if isinstance(pat, dict) else pat
+    if not t or pat is None:
+        return []
+    return [v for k, v in t["kernels"].items() if re.fullmatch(pat, k)]
+
+
 def traffic_per_launch(family, mode):
     """HBM bytes per launch of a work family (mean over its real and complex
     instantiations) from the committed counter summary, or None."""
-    from gshtrans_amd.profile_summary import load_table
-    t = load_table(TRAFFIC_FILE)
-    if not t:
-        return None
-    pat = FAMILY_KERNELS.get(family)
-    pat = pat.get(mode) if isinstance(pat, dict) else pat
-    if pat is None:
-        return None
-    rows = [v for k, v in t["kernels"].items() if re.fullmatch(pat, k)]
-    if not rows:
-        return None
-    return sum(r["fetch_bytes"] + r["write_bytes"] for r in rows) / len(rows)
+    rows = counter_rows(family, mode)
+    return sum(r["fetch_bytes"] + r["write_bytes"] for r in rows) / len(rows) if rows else None
+
+
+def issued_per_launch(family, mode):
+    """MFMA flops per launch of a work family, likewise, or None."""
+    rows = counter_rows(family, mode)
+    return sum(r["mfma_tflops"] * r["avg_ns"] * 1e3 for r in rows) / len(rows) if rows else None
 
 
 def host_info():
