@@ -1184,8 +1184,10 @@ int bin_columns(int ncol, int precision) {
 }
 // Ring FFTs of a call.  The wavefront kernels (N = 512, 1024, 2048) move bins
 // for 8 complex rings (16 real ones) of a colatitude at a time; calls of at
-// most 4 fields, other lengths and o.fft = 2 take the ring kernels, and
-// transforms of more than 4096 points the LDS kernels.
+// most 4 fields, other lengths and o.fft = 2 take the ring kernels (a group of 8
+// would be half empty), and transforms of more than 4096 points the LDS
+// kernels.  The two families add in another order, so at these three lengths a
+// batch of more than 4 fields and one field alone agree to rounding.
 hipError_t run_fft(const FFTParams& q, const RunOpts& o, bool anal, hipStream_t s) {
   if (use_wave_fft(q, o) && q.nfield > 4 && q.cw == 16)
     return anal ? gsh::launch_fft_anal_wave(q, s) : gsh::launch_fft_synth_wave(q, s);
@@ -1766,8 +1768,8 @@ struct PlanGroup {
   int* d_flmax = nullptr;
   int* d_cglmax = nullptr;
   NData* nd = nullptr;
-  int synth_tiles = 0;  // FP64 / FP32 synthesis column tiles per wave (0: not tuned)
-  int fft_inv = 0;      // 1: wavefront FFT, 2: LDS FFT (0: not tuned)
+  int synth_tiles = 0;  // FP64 / FP32 synthesis column tiles per wave, reported (0: not executed)
+  int fft_inv = 0;      // 1: wavefront FFT, 2: ring kernels of any length (0: not tuned)
   int fft_fwd = 0;
   int anal_pass = 0;    // split-BF16 analysis degrees per pass, 64 or 128 (0: not tuned)
 };

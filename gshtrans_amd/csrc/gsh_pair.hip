@@ -19,11 +19,11 @@
 // (3 FP64 instructions against 128 multiply-adds), 16 degrees at a time from
 // the checkpoint table, one chunk ahead of the MFMAs that use it.
 //
-// Degrees whose values stay below 2^-200 at every row of a tile (near the
+// Degrees whose values stay below 2^-120 at every row of a tile (near the
 // poles d^l_{mn} is evanescent for l < m / sin t) are left out of the MFMAs:
 // kf[order][row tile] holds the first 16-degree checkpoint that matters.  At
 // lMax = 1024 that is a fifth of the work.  A term of that size changes no
-// sum of doubles unless every other term is below 2^-147 of it; Inf and NaN
+// sum of doubles unless every other term is below 2^-67 of it; Inf and NaN
 // of the terms left out still reach the result (added as 0 * value).
 #include <algorithm>
 #include <type_traits>
@@ -179,6 +179,10 @@ constexpr int waves(int kind, int tiles, int nj) {
 // Beside the MFMAs every vector instruction costs about 3 of an MFMA's 72
 // cycles (measured, two waves per SIMD), so the coefficient loads step one
 // byte offset per 4 degrees and mask nothing until a column's last degrees.
+// Bound: FP64 MFMA, 47 of 71 TFLOP/s of the products issued.  lMax=1024, 64
+// fields: 7.21 -> 4.95 ms (complex, n=2) and 3.55 -> 1.56 ms (real, n=0) against
+// a kernel that ran the recurrence of every order for every 32 columns; FP32
+// 3.98 -> 2.52 ms, the mean of both.
 // ---------------------------------------------------------------------------
 template <int KIND, int SYM, int RT, int NJ>
 __global__ __launch_bounds__(256, waves(KIND, RT, SYM ? 2 : NJ)) void leg_synth_p(LegParams p) {
@@ -484,6 +488,9 @@ __global__ __launch_bounds__(256, waves(KIND, RT, SYM ? 2 : NJ)) void leg_synth_
 // split the pass: WR degree groups of LT tiles x WC column groups of NJ tiles.
 // SYM: the rows run over the north, a degree tile holds 16 degrees of one
 // parity, multiplied with X(t) +- X(nt-1-t).
+// Bound: FP64 MFMA, 52 of 71 TFLOP/s of the products issued; without the bin
+// loads it takes 12% less, without the stores 6%, without the recurrence 5%.
+// lMax=1024, 64 fields: mean of complex n=2 and real n=0 5.58 -> 2.86 ms.
 // ---------------------------------------------------------------------------
 template <int KIND, int SYM, int LT, int NJ>
 __global__ __launch_bounds__(256, waves(KIND, LT, NJ)) void leg_anal_p(LegParams p) {

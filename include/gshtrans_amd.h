@@ -217,8 +217,8 @@ int gsh_adjoint_inverse(gsh_grid_t grid, int lmax, int n, int value_kind,
  * upper index n[i]; all share one value kind, precision and storage.  The
  * plan groups the fields by upper index, orders each group by degree so that
  * every 16-column group of a launch carries its own degree bound, and on its
- * first execution in each direction times the candidate tile shapes
- * (synthesis column tiles, ring-FFT kernel family) and keeps the fastest.
+ * first execution in each direction times the candidates (ring-FFT kernel
+ * family; for the split-BF16 analysis degrees per pass) and keeps the fastest.
  *
  * Arrays: coefficients of field i at coeffs + i*coeff_stride (complex
  * elements of the storage type; GSHIndices(lmax[i], lmax[i], n[i]) layout,
@@ -238,8 +238,10 @@ int gsh_plan_inverse(gsh_plan_t plan, const void* coeffs, long coeff_stride, voi
 int gsh_plan_forward(gsh_plan_t plan, const void* field, long field_stride, void* coeffs,
                      long coeff_stride, int graph, void* stream);
 /* Launch groups and the tuned choices: per group g < *ngroups (up to cap),
- * n, lmax, field count, synthesis column tiles (0 = not tuned yet), and the
- * FFT family of synthesis / analysis (1 wavefront-per-ring, 2 LDS). */
+ * n, lmax, field count, column tiles of a wave in the FP64 / FP32 synthesis
+ * (chosen by rule and reported; 0 = not executed yet, or at most 8 fields), and
+ * the FFT family of synthesis / analysis (1 wavefront-per-ring, 2 the ring
+ * kernels of any length). */
 int gsh_plan_info(gsh_plan_t plan, int* ngroups, int cap, int* n, int* lmax, int* count,
                   int* synth_tiles, int* fft_inverse, int* fft_forward);
 /* The tuned degrees per pass of each group's split-BF16 analysis (64 or
