@@ -126,6 +126,12 @@ __device__ __forceinline__ void flush(d4& acc, const f4 c) {
 // and 624 -> 585 us (n=0, real), analysis 2200 -> 2026 us and 955 -> 897 us; the
 // rows left out still have to be read, 180 of the 2026 us.
 //
+// A wave whose columns all lie past the last field (`used` false) takes its
+// share of the production and multiplies nothing: the waves of a SIMD share its
+// matrix unit.  Synthesis and analysis of 20 complex fields (3 of 8 column
+// tiles), lMax=360, bf16x3: 372 -> 348 us; 4 fields, lMax=512, bf16x6: 605 -> 496
+// us; whole super-groups of 64 fields are unchanged.
+//
 // first_checkpoint: of row tiles t0 .. t0 + 7 (tiles past t1 take t1's).
 __device__ __forceinline__ int first_checkpoint(const LegParams& p, int m, int t0, int t1) {
   int k = p.kf[(long)(m + p.L) * p.nrt + min(t0 + (int)(threadIdx.x & 7), t1)];
@@ -640,6 +646,7 @@ __global__ __launch_bounds__(512) void leg_synth_bf16_s(LegParams p) {
   // Consumer role.
   const int h = wave >> 2;
   const int tile0 = csg * 8 + (wave & 3) * 2;
+  const bool used = 16 * tile0 < p.ncol;  // the others only produce (padding columns)
   d4 acc[4][2][2];  // row group, column tile, class
 #pragma unroll
   for (int g = 0; g < 4; g++)
@@ -694,7 +701,7 @@ __global__ __launch_bounds__(512) void leg_synth_bf16_s(LegParams p) {
     for (int s = 0; s < NS; s++) A[0][s] = trb[abuf][s][k][lane >> 4][h * 64 + g * 16 + (lane & 15)];
   };
   auto consume_group = [&](int g, int k, const uint4 (&A)[1][NS], const uint4 (&B)[2][NS]) {
-    if (h * 64 + g * 16 < rows) {
+    if (used && h * 64 + g * 16 < rows) {
       f4 c[1][2];
       split_mma<NS, 1>(A, B, c);
       flush(acc[g][0][k], c[0][0]);
@@ -885,6 +892,7 @@ __global__ __launch_bounds__(512) void leg_synth_bf16_pm(LegParams p) {
 
   // Consumer role: column tile w of both orders, all 128 colatitudes.
   const int tile = csg * 8 + wave;
+  const bool used = 16 * tile < p.ncol;  // the others only produce (padding columns)
   d4 acc[8][2];  // row group, order
 #pragma unroll
   for (int g = 0; g < 8; g++)
@@ -961,7 +969,7 @@ __global__ __launch_bounds__(512) void leg_synth_bf16_pm(LegParams p) {
   auto block = [&](int c, const int dh, const bool next) {
     const int abuf = (c ^ c0) & 1;
     const bool prod = pv && c + 1 < nC;
-    const bool live = 2 * c + dh < n32;
+    const bool live = used && 2 * c + dh < n32;
     uint4 Bn[2][NS];
     if (next) fetchB(c + dh, dh ^ 1, Bn);
     uint4 qr = make_uint4(0u, 0u, 0u, 0u);
@@ -1364,6 +1372,7 @@ __global__ __launch_bounds__(512) void leg_anal_bf16_pm(LegParams p) {
   };
   const int tile = csg * 8 + wave;
   const int tcl = min(tile, p.n_cg - 1);
+  const bool used = tile < p.n_cg;  // the others only produce (padding columns)
   const float* fb =
       p.FA32 + (((long)slot * p.n_cg + tcl) * p.nquad + 8 * kb + 2 * (lane >> 4)) * 64 + (lane & 15);
   const float* fbn = p.FA32 + ((long)slotn * p.n_cg + tcl) * p.nquad * 64 + (lane & 15);
@@ -1436,7 +1445,7 @@ __global__ __launch_bounds__(512) void leg_anal_bf16_pm(LegParams p) {
   // Colatitudes left out, at either end (order -m: their mirrors), here, where
   // the loads wait together with the first state's.
   float left[2] = {0.0f, 0.0f};
-  if (nk < p.nkc) {
+  if (used && nk < p.nkc) {
     const float* bp = p.FA32 + ((long)slot * p.n_cg + tcl) * p.nquad * 64;
     const float* bn = p.FA32 + ((long)slotn * p.n_cg + tcl) * p.nquad * 64;
     const int te = min(tb + 32 * nk, nt);
@@ -1461,15 +1470,21 @@ __global__ __launch_bounds__(512) void leg_anal_bf16_pm(LegParams p) {
     const int kc0 = 4 * g;
     begin();
     prefetch(g + 2);
+    if (used) {
 #pragma unroll
-    for (int j = 0; j < 4; j++) {
-      loadB(min(kc0 + j + 1, kcl), X[(j + 1) & 1]);
-      produce4(buf ^ 1, j);
-      step(buf, kc0 + j, X[j & 1], false, j & 1);
-      __builtin_amdgcn_sched_barrier(0);
+      for (int j = 0; j < 4; j++) {
+        loadB(min(kc0 + j + 1, kcl), X[(j + 1) & 1]);
+        produce4(buf ^ 1, j);
+        step(buf, kc0 + j, X[j & 1], false, j & 1);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    } else {
+#pragma unroll
+      for (int j = 0; j < 4; j++) produce4(buf ^ 1, j);
     }
     __syncthreads();
   }
+  if (!used) return;  // past the last barrier
   {
     // Last group: chunks 4 (ngrp-1) .. nk-1 (X[0] holds the first).
     const int buf = (ngrp - 1) & 1;
@@ -2082,6 +2097,7 @@ __global__ __launch_bounds__(512) void leg_anal_bf16_ws(LegParams p) {
     float x[8];
   };
   const int tile = csg * 8 + wave;
+  const bool used = tile < p.n_cg;  // the others only produce (padding columns)
   const float* ft = p.FA32 + ((long)slot * p.n_cg + min(tile, p.n_cg - 1)) * p.nquad * 64 + (lane & 15);
   const float* fb = ft + (8 * kb + 2 * (lane >> 4)) * 64;
   // Chunk kb + kc's colatitudes t = tb + 32 kc + 8 (lane / 16) + e (X) and their
@@ -2171,7 +2187,7 @@ __global__ __launch_bounds__(512) void leg_anal_bf16_ws(LegParams p) {
 
   prefetch(0);
   float left = 0.0f;  // colatitudes left out, and their mirrors
-  if (kb > 0) {
+  if (used && kb > 0) {
     const float* bp = ft - (lane & 15);
     f4 z = f4{0.f, 0.f, 0.f, 0.f}, y = z;
     left_out(bp, 0, bp, nt - 1, tb, z, y);
@@ -2191,15 +2207,21 @@ __global__ __launch_bounds__(512) void leg_anal_bf16_ws(LegParams p) {
     const int kc0 = 2 * g;
     begin();
     prefetch(g + 2);
+    if (used) {
 #pragma unroll
-    for (int j = 0; j < 2; j++) {
-      loadB(min(kc0 + j + 1, kcl), X[(j + 1) & 1], Y[(j + 1) & 1]);
-      produce8(buf ^ 1, j);
-      step(buf, kc0 + j, X[j], Y[j], false);
-      __builtin_amdgcn_sched_barrier(0);
+      for (int j = 0; j < 2; j++) {
+        loadB(min(kc0 + j + 1, kcl), X[(j + 1) & 1], Y[(j + 1) & 1]);
+        produce8(buf ^ 1, j);
+        step(buf, kc0 + j, X[j], Y[j], false);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    } else {
+#pragma unroll
+      for (int j = 0; j < 2; j++) produce8(buf ^ 1, j);
     }
     __syncthreads();
   }
+  if (!used) return;  // past the last barrier
   {
     // Last group: chunks 2 (ngrp-1) .. nk-1 (one or two).
     const int buf = (ngrp - 1) & 1;
