@@ -417,6 +417,7 @@ __global__ __launch_bounds__(512) void leg_synth_bf16(LegParams p) {
   // Consumer role.
   const int h = wave >> 2;
   const int tile0 = csg * 8 + (wave & 3) * 2;
+  const bool used = 16 * tile0 < p.ncol;  // the others only produce (padding columns)
   d4 acc[8][2];
 #pragma unroll
   for (int g = 0; g < 8; g++)
@@ -455,7 +456,7 @@ __global__ __launch_bounds__(512) void leg_synth_bf16(LegParams p) {
     for (int s = 0; s < NS; s++) A[0][s] = trb[buf][s][lane >> 4][h * 128 + g * 16 + (lane & 15)];
   };
   auto consume_group = [&](int g, const uint4 (&A)[1][NS], const uint4 (&B)[2][NS]) {
-    if (h * 128 + g * 16 < rows) {
+    if (used && h * 128 + g * 16 < rows) {
       f4 c[1][2];
       split_mma<NS, 1>(A, B, c);
       flush(acc[g][0], c[0][0]);
@@ -1147,6 +1148,7 @@ __global__ __launch_bounds__(512) void leg_anal_bf16(LegParams p) {
     float x[8];
   };
   const int tile = csg * 8 + wave;
+  const bool used = tile < p.n_cg;  // the others only produce (padding columns)
   const float* fb =
       p.FA32 + (((long)slot * p.n_cg + min(tile, p.n_cg - 1)) * p.nquad + 2 * (lane >> 4)) * 64 +
       (lane & 15);
@@ -1230,15 +1232,21 @@ __global__ __launch_bounds__(512) void leg_anal_bf16(LegParams p) {
     const int kc0 = 4 * g;
     begin();
     prefetch(g + 2);  // a whole group ahead of its use
+    if (used) {
 #pragma unroll
-    for (int j = 0; j < 4; j++) {
-      loadB(min(kc0 + j + kAhead, kcl), X[(j + kAhead) & 3]);
-      produce4(buf ^ 1, j);
-      step(buf, kc0 + j, X[j], false, j & 1);
-      __builtin_amdgcn_sched_barrier(0);
+      for (int j = 0; j < 4; j++) {
+        loadB(min(kc0 + j + kAhead, kcl), X[(j + kAhead) & 3]);
+        produce4(buf ^ 1, j);
+        step(buf, kc0 + j, X[j], false, j & 1);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    } else {
+#pragma unroll
+      for (int j = 0; j < 4; j++) produce4(buf ^ 1, j);
     }
     __syncthreads();
   }
+  if (!used) return;  // past the last barrier
   {
     // Last group: chunks 4 (ngrp-1) .. nkc-1.
     const int buf = (ngrp - 1) & 1;
@@ -1644,6 +1652,7 @@ __global__ __launch_bounds__(512) void leg_anal_bf16_s(LegParams p) {
     float x[8];
   };
   const int tile = csg * 8 + wave;
+  const bool used = tile < p.n_cg;  // the others only produce (padding columns)
   const float* ft = p.FA32 + ((long)slot * p.n_cg + min(tile, p.n_cg - 1)) * p.nquad * 64 + (lane & 15);
   const float* fb = ft + 2 * (lane >> 4) * 64;
   // Chunk kc's colatitudes t = 32 kc + 8 (lane / 16) + e (X) and their
@@ -1754,15 +1763,21 @@ __global__ __launch_bounds__(512) void leg_anal_bf16_s(LegParams p) {
     const int kc0 = 4 * g;
     begin();
     prefetch(g + 2);  // a whole group ahead of its use
+    if (used) {
 #pragma unroll
-    for (int j = 0; j < 4; j++) {
-      loadB(min(kc0 + j + kAhead, kcl), X[(j + kAhead) & 3], Y[(j + kAhead) & 3]);
-      produce4(buf ^ 1, j);
-      step(buf, kc0 + j, X[j], Y[j], false);
-      __builtin_amdgcn_sched_barrier(0);
+      for (int j = 0; j < 4; j++) {
+        loadB(min(kc0 + j + kAhead, kcl), X[(j + kAhead) & 3], Y[(j + kAhead) & 3]);
+        produce4(buf ^ 1, j);
+        step(buf, kc0 + j, X[j], Y[j], false);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    } else {
+#pragma unroll
+      for (int j = 0; j < 4; j++) produce4(buf ^ 1, j);
     }
     __syncthreads();
   }
+  if (!used) return;  // past the last barrier
   {
     // Last group: chunks 4 (ngrp-1) .. nkc-1.
     const int buf = (ngrp - 1) & 1;
@@ -1814,7 +1829,11 @@ __global__ __launch_bounds__(512) void leg_anal_bf16_s(LegParams p) {
 // ---------------------------------------------------------------------------
 constexpr int kWidePass = kWideAnalPass;
 
-template <int NS, int REAL>
+// PAD: launches of less than a super-group, whose last waves have no column of a
+// field (see `used`).  Wider ones run without the test, whose branch costs the
+// schedule 2%: lMax=1024, 64 real fields, n=1, 1305 us without and 1336 with it;
+// 72 fields, lMax=300, 127.5 and 128.0; 20 fields, lMax=512, 219 and 166.
+template <int NS, int REAL, int PAD>
 __global__ __launch_bounds__(512) void leg_anal_bf16_w(LegParams p) {
   static_assert(kCk == 16 && kWidePass == 8 * kCk, "8 degree tiles of 16 per pass");
   // Rows of 64 colatitudes padded to 72 (144 bytes, 36 banks apart): the 16
@@ -1886,6 +1905,7 @@ __global__ __launch_bounds__(512) void leg_anal_bf16_w(LegParams p) {
     float x[8];
   };
   const int tile = csg * 8 + wave;
+  const bool used = !PAD || tile < p.n_cg;  // the others only produce (padding columns)
   const float* fb =
       p.FA32 + (((long)slot * p.n_cg + min(tile, p.n_cg - 1)) * p.nquad + 2 * (lane >> 4)) * 64 +
       (lane & 15);
@@ -1961,15 +1981,21 @@ __global__ __launch_bounds__(512) void leg_anal_bf16_w(LegParams p) {
     const int kc0 = 2 * g;
     begin();
     prefetch(g + 2);
+    if (used) {
 #pragma unroll
-    for (int j = 0; j < 2; j++) {
-      loadB(min(kc0 + j + 1, kcl), X[(j + 1) & 1]);
-      produce8(buf ^ 1, j);
-      step(buf, kc0 + j, X[j], false, j & 1);
-      __builtin_amdgcn_sched_barrier(0);
+      for (int j = 0; j < 2; j++) {
+        loadB(min(kc0 + j + 1, kcl), X[(j + 1) & 1]);
+        produce8(buf ^ 1, j);
+        step(buf, kc0 + j, X[j], false, j & 1);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    } else {
+#pragma unroll
+      for (int j = 0; j < 2; j++) produce8(buf ^ 1, j);
     }
     __syncthreads();
   }
+  if (!used) return;  // past the last barrier
   {
     // Last group: chunks 2 (ngrp-1) .. nkc-1 (one or two).
     const int buf = (ngrp - 1) & 1;
@@ -2431,10 +2457,14 @@ hipError_t launch_anal_bf16_w(const LegParams& p0, hipStream_t s, bool sym) {
     hipLaunchKernelGGL((leg_anal_bf16_ws<NS, 1>), grid, dim3(512), 0, s, p);
   else if (sym)
     hipLaunchKernelGGL((leg_anal_bf16_ws<NS, 0>), grid, dim3(512), 0, s, p);
+  else if (p.n_cg >= 8 && p.real)
+    hipLaunchKernelGGL((leg_anal_bf16_w<NS, 1, 0>), grid, dim3(512), 0, s, p);
+  else if (p.n_cg >= 8)
+    hipLaunchKernelGGL((leg_anal_bf16_w<NS, 0, 0>), grid, dim3(512), 0, s, p);
   else if (p.real)
-    hipLaunchKernelGGL((leg_anal_bf16_w<NS, 1>), grid, dim3(512), 0, s, p);
+    hipLaunchKernelGGL((leg_anal_bf16_w<NS, 1, 1>), grid, dim3(512), 0, s, p);
   else
-    hipLaunchKernelGGL((leg_anal_bf16_w<NS, 0>), grid, dim3(512), 0, s, p);
+    hipLaunchKernelGGL((leg_anal_bf16_w<NS, 0, 1>), grid, dim3(512), 0, s, p);
   return hipGetLastError();
 }
 
