@@ -886,7 +886,24 @@ FFTParams fft_params(gsh_grid_s* g, int lmax, int real, int batch) {
 
 bool is_pow2(int N) { return N >= 1 && (N & (N - 1)) == 0; }
 
-// LDS transform length for ring length N: N itself when a power of two,
+// exp(-2 pi i k / N), N even, 0 <= k < N, with the symmetries of the circle
+// exact: opposite roots are negatives, and the quarter roots have no rounding.
+double2 root_of_unity(int k, int N) {
+  if (2 * k >= N) {
+    const double2 r = root_of_unity(k - N / 2, N);
+    return make_double2(-r.x, -r.y);
+  }
+  if (4 * k > N) {
+    const double2 r = root_of_unity(N / 2 - k, N);
+    return make_double2(-r.x, r.y);
+  }
+  if (k == 0) return make_double2(1.0, 0.0);
+  if (4 * k == N) return make_double2(0.0, -1.0);
+  const long double a = -2.0L * kPiL * k / N;
+  return make_double2(static_cast<double>(std::cos(a)), static_cast<double>(std::sin(a)));
+}
+
+// Transform length for ring length N: N itself when a power of two,
 // else the Bluestein convolution length (smallest power of two >= 2N - 1).
 int fft_length(int N) {
   if (is_pow2(N)) return N;
@@ -1011,16 +1028,18 @@ int gsh_grid_create(int lmax, int nmax, int mrange, int nrange, gsh_grid_t* grid
     cs[i] = std::cos(g->theta[i]);
     wq[i] = g->weight[i] * scale;
   }
-  // Rings of fewer than 64 points go through Bluestein's convolution of 64,
-  // the shortest transform of the ring kernels.
+  // Rings of at most 32 points are summed directly by the 64-point form of the
+  // ring kernels, from the N-th roots of unity.
+  const bool short_ring = N > 0 && N <= 32;
   const int M = N > 0 ? std::max(64, fft_length(N)) : 1;
   g->M = M;
   std::vector<double2> tw(M);
   for (int k = 0; k < M; k++) {
     const long double a = -2.0L * kPiL * k / M;
-    tw[k] = make_double2(static_cast<double>(std::cos(a)), static_cast<double>(std::sin(a)));
+    tw[k] = short_ring ? root_of_unity(k % N, N)
+                       : make_double2(static_cast<double>(std::cos(a)), static_cast<double>(std::sin(a)));
   }
-  if (N > 0 && M != N) {
+  if (N > 0 && M != N && !short_ring) {
     // Bluestein: chirp w_k = exp(-i pi k^2 / N); forward filter conj(w),
     // backward filter w, both circularly extended to M and transformed.
     std::vector<std::complex<long double>> w(N), hf(M), hb(M);

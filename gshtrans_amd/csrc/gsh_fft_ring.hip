@@ -22,6 +22,9 @@
 // lMax=360 (720-point rings, M = 2048), 20 complex fields: 382 -> 97 us
 // synthesis, 381 -> 92 us analysis against a whole workgroup per ring with every
 // pass in LDS.
+// Rings of at most 32 points are summed directly (direct_dft): a convolution of
+// 64 points rounds up to twice as much as the transform of the ring itself
+// (lMax = 2: 3.7e-16 in place of 1.5e-16 relative to extended precision).
 // Real fields go two rings at a time as x_a + i x_b, two colatitudes of one
 // field (a field's Inf or NaN reaches no other field).
 #include "gsh_fft_dev.h"
@@ -152,13 +155,74 @@ __device__ __forceinline__ void ring_fft(double2 (&v)[16], double2* lds,
   }
 }
 
+// Unnormalised DFT of a ring of N <= 32 points (N even) held by 4 threads as
+// v[e] = x[t + 4 e], e < 8, with one root of unity per term: p.tw[j] = exp(-2 pi
+// i j / N).  The outputs k = t + 4 e of a thread are of one class modulo 4 (modulo
+// 2), so the N / 4 (N / 2) terms left after a radix-4 (radix-2) butterfly are the
+// same for all of them.  Four partial sums per output: less rounding than one
+// chain, and independent multiply-adds.
+template <int SIGN>
+__device__ __forceinline__ void direct_dft(double2 (&v)[16], double2* lds, const FFTParams& p,
+                                           int t) {
+  constexpr int E = 8, ROOT = 34;  // outputs per thread; the roots' place in LDS
+  static_assert(ROOT + 4 * E <= Ring<64>::kStride, "ring and roots share a row");
+  const int N = p.N, four = N % 4 == 0, H = four ? N / 4 : N / 2;
+#pragma unroll
+  for (int e = 0; e < E; e++) {
+    lds[t + 4 * e] = v[e];  // zero from N on
+    lds[ROOT + t + 4 * e] = p.tw[t + 4 * e];
+  }
+  Ring<64>::sync();
+  double2 a[E][4];
+  int j[E], dj[E];  // root of the next term, its step
+#pragma unroll
+  for (int e = 0; e < E; e++) {
+    j[e] = 0;
+    dj[e] = t + 4 * e < N ? t + 4 * e : 0;
+#pragma unroll
+    for (int r = 0; r < 4; r++) a[e][r] = make_double2(0.0, 0.0);
+  }
+  for (int n0 = 0; n0 < H; n0 += 4) {
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+      const int n = n0 + r;
+      double2 x = make_double2(0.0, 0.0);
+      if (n < H) {
+        const double2 x0 = lds[n], x1 = lds[n + H];
+        if (four) {
+          const double2 x2 = lds[n + 2 * H], x3 = lds[n + 3 * H];
+          const double2 s = t & 1 ? csub(x0, x2) : cadd(x0, x2);
+          const double2 d = t & 1 ? rot16<SIGN>(csub(x1, x3), 8) : cadd(x1, x3);
+          x = t & 2 ? csub(s, d) : cadd(s, d);
+        } else {
+          x = t & 1 ? csub(x0, x1) : cadd(x0, x1);
+        }
+      }
+#pragma unroll
+      for (int e = 0; e < E; e++) {
+        double2 w = lds[ROOT + j[e]];
+        if (SIGN > 0) w.y = -w.y;
+        a[e][r].x = fma(x.x, w.x, fma(-x.y, w.y, a[e][r].x));
+        a[e][r].y = fma(x.x, w.y, fma(x.y, w.x, a[e][r].y));
+        j[e] += dj[e];
+        j[e] -= j[e] >= N ? N : 0;
+      }
+    }
+  }
+#pragma unroll
+  for (int e = 0; e < E; e++) v[e] = cadd(cadd(a[e][0], a[e][2]), cadd(a[e][1], a[e][3]));
+}
+
 // Unnormalised N-point DFT of the ring held as v[e] = x[t + T e] (zero from N
-// on): direct (BLUE 0, M = N) or Bluestein's.
+// on): direct (BLUE 0, M = N), or Bluestein's, or for rings of at most 32 points
+// (M = 64 and N < M) the sums themselves.
 template <int M, int BLUE, int SIGN>
 __device__ __forceinline__ void ring_dft(double2 (&v)[16], double2* lds, const FFTParams& p,
                                          const Twiddles<M, false>& tw, int t) {
   if constexpr (!BLUE) {
     ring_fft<M, SIGN, false, false>(v, lds, tw, t);
+  } else if constexpr (M == 64) {
+    direct_dft<SIGN>(v, lds, p, t);
   } else {
     constexpr int T = M / 16;
     auto chirp = [&](int e) {
