@@ -19,12 +19,18 @@
 // (3 FP64 instructions against 128 multiply-adds), 16 degrees at a time from
 // the checkpoint table, one chunk ahead of the MFMAs that use it.
 //
-// Degrees whose values stay below 2^-120 at every row of a tile (near the
-// poles d^l_{mn} is evanescent for l < m / sin t) are left out of the MFMAs:
-// kf[order][row tile] holds the first 16-degree checkpoint that matters.  At
-// lMax = 1024 that is a fifth of the work.  A term of that size changes no
-// sum of doubles unless every other term is below 2^-67 of it; Inf and NaN
-// of the terms left out still reach the result (added as 0 * value).
+// Near the poles d^l_{mn} is evanescent for l < m / sin t.  Values of the 16
+// degrees from a checkpoint count as zero at the 16 rows of a tile where all of
+// them, and all at lower degrees, are below 2^-120: kf[order][row tile] holds the
+// first checkpoint that counts, and blocks of zeros are left out of the MFMAs (at
+// lMax = 1024 a fifth of the work).  So a sum over coefficients c is off by at
+// most 2^-120 sum |c| of the terms left out, which is below the rounding of any
+// larger term; a field of high orders only has zeros near the poles where its
+// values are that small.  What is left out does not depend on how a batch is
+// tiled: a synthesis that starts at an earlier degree for another of its row tiles
+// multiplies by zeros, and an analysis leaves out the rows of a whole pass of 128
+// degrees.  Inf and NaN of the terms left out still reach the result (added as
+// 0 * value).
 #include <algorithm>
 #include <type_traits>
 
@@ -83,6 +89,10 @@ struct Mma<2> {
   static __device__ __forceinline__ double get(const acc& c, int) { return c; }
   static __device__ __forceinline__ void add(acc& c, double v) { c += v; }
 };
+
+__device__ __forceinline__ int ld_uniform_u16(const unsigned short* a, int i) {
+  return __builtin_amdgcn_readfirstlane((int)a[i]);
+}
 
 // One recurrence step with uniform coefficients {a, b, c} and per-lane cos.
 __device__ __forceinline__ void rec_step(double2 ab, double c, double cs, double& e0, double& e1) {
@@ -235,8 +245,9 @@ __global__ __launch_bounds__(256, waves(KIND, RT, SYM ? 2 : NJ)) void leg_synth_
   lww = -wave_min(-lww);
   const int lwg = vcol_lmax(p, vb, WC * NC * M::CT, m);
 
-  // First checkpoint that matters for the block's rows.
-  int ks = wave_min(p.kf[(long)(m + p.L) * p.nrt + tile0 + min(lane & 15, ntile - 1)]);
+  // First checkpoint that counts at any of the block's rows.
+  const unsigned short* kfm = p.kf + (long)(m + p.L) * p.nrt;
+  int ks = wave_min(kfm[tile0 + min(lane & 15, ntile - 1)]);
   ks = min(ks, max(0, lwg - l0 + kCk) / kCk);
   const int ls = l0 + kCk * ks;
   const int nchunk = ls > lwg ? 0 : (lwg - ls + SC) / SC;
@@ -324,12 +335,27 @@ __global__ __launch_bounds__(256, waves(KIND, RT, SYM ? 2 : NJ)) void leg_synth_
   const bool tv = t < nr, txv = xprod && lane < 16 && tx < nr;
   const double cs = tv ? p.cosv[t] : 0.0, csx = txv ? p.cosv[tx] : 0.0;
   const int nck = (p.L - l0 + kCk) / kCk;  // checkpoints 1 .. nck - 1 exist
+  // First checkpoints that count at the wave's four row tiles and at the extra
+  // one, in scalar registers (a per-lane copy of them costs the widest tiles 3%).
+  int kt[5];
+#pragma unroll
+  for (int i = 0; i < 4; i++)
+    kt[i] = ld_uniform_u16(kfm, min(tile0 + 4 * (wave & 1) + i, p.nrt - 1));
+  kt[4] = ld_uniform_u16(kfm, min(tile0 + TW, p.nrt - 1));
+  const unsigned long long rows = __ballot(tv), rowsx = __ballot(txv);
   const double* seedm = p.seeds + (long)(m + p.L) * nt;
   const double2* ckm = p.ck + (long)it.z * nt;
-  auto state = [&](int c, bool v, int row) -> double2 {
+  auto state = [&](int c, bool extra, int row) -> double2 {
     const int k = ks + NH * c + seg;
+    unsigned long long live = k < nck ? extra ? rowsx : rows : 0;
+    if (extra) {
+      live = k < kt[4] ? 0 : live;
+    } else {
+#pragma unroll
+      for (int i = 0; i < 4; i++) live &= k < kt[i] ? ~(0xffffull << (16 * i)) : ~0ull;
+    }
     double2 s = make_double2(0.0, 0.0);
-    if (k < nck && v) {
+    if (__builtin_amdgcn_inverse_ballot_w64(live)) {
       if (k == 0)
         s.x = seedm[row];
       else
@@ -391,7 +417,7 @@ __global__ __launch_bounds__(256, waves(KIND, RT, SYM ? 2 : NJ)) void leg_synth_
   if (nchunk > 0) {
 #pragma unroll
     for (int h = 0; h < NH; h++) load_group(ls + kCk * h, B[h]);
-    double2 st = state(0, tv, t), sx = state(0, txv, tx);
+    double2 st = state(0, false, t), sx = state(0, true, tx);
     if (tid < 2 * SC) rs[0][tid] = fetch_rec(0);
     uint4 rq = make_uint4(0, 0, 0, 0);
     __syncthreads();
@@ -401,8 +427,8 @@ __global__ __launch_bounds__(256, waves(KIND, RT, SYM ? 2 : NJ)) void leg_synth_
       produce(c, st, cs, prow);
       if (xprod && lane < 16) produce(c, sx, csx, XR + lane);
       if (c + 1 < nchunk) {
-        st = state(c + 1, tv, t);
-        sx = state(c + 1, txv, tx);
+        st = state(c + 1, false, t);
+        sx = state(c + 1, true, tx);
         // rs[(c + 1) & 1] was last read producing chunk c - 1, a barrier ago.
         if (tid < 2 * SC) rs[(c + 1) & 1][tid] = rq;
         if (c + 2 < nchunk) rq = fetch_rec(c + 2);
@@ -547,13 +573,14 @@ __global__ __launch_bounds__(256, waves(KIND, LT, NJ)) void leg_anal_p(LegParams
   if (nu <= 0) return;
   const int lp = l0 + 32 * u0;
 
-  // Rows that matter: chunks c0 .. c1 (chunks past 64 always run).
+  // Rows that count for a whole pass, whatever part of it this group's degrees
+  // fill: chunks c0 .. c1 (chunks past 64 always run).
   const int nch = (nr + CR - 1) / CR;
   const int nrt = (nr + 15) >> 4;
   const unsigned short* kf = p.kf + (long)(m + p.L) * p.nrt;
   int c0, c1 = nch - 1;
   {
-    const int kend = 2 * u0 + 2 * nu;
+    const int kend = 2 * (u0 + PU);
     bool live = false;
     if (lane < nch)
 #pragma unroll

@@ -178,3 +178,59 @@ def test_every_coefficient_is_written(torch, n, real, precision):
         g.forward_product(lmax, n, f, torch.ones_like(f), coeffs=out, real=real,
                           precision=precision)
         assert torch.isfinite(torch.view_as_real(out)).all()
+
+
+# Values below 2^-120 near the poles count as zero by rows and degrees alone, so
+# one high order by itself, whose values are that small at many rows, gives the
+# same bits alone, in batches of every tile shape and in plans of uneven degrees.
+# Against the oracle: 1e-12 of the field, and at each row 1e-12 of the sum of the
+# terms' absolute values (alternating terms cancel at a mirror row) and 2^-120
+# for each of at most 301 unit coefficients left out.
+@pytest.mark.parametrize("n,real", [(0, True), (0, False), (1, True), (2, False)])
+def test_one_high_order_in_any_tile(torch, n, real):
+    L = 300
+    orders = [100 + 6 * i for i in range(33)]
+    g = G.GaussLegendreGrid(L, 2)
+    og = oracle.OracleGrid(L, 2, table=False)
+    c = np.zeros((len(orders), G.coefficient_size(L, n, real)), dtype=np.complex128)
+    for i, m in enumerate(orders):
+        c[i, [G.coefficient_index(L, n, l, m, real) for l in range(m, L + 1)]] = 1.0
+    cd = torch.from_numpy(c).cuda()
+    one = torch.cat([g.inverse(L, n, cd[i:i + 1], real=real) for i in range(len(orders))])
+    # samples on the rows near the poles alone, where the order is small
+    polar = one.clone()
+    size = polar.abs().amax(dim=-1, keepdim=True)
+    polar = torch.where((size > 0) & (size < 2.0**-90), polar / size.clamp_min(2.0**-1000), 0 * polar)
+    back = torch.cat([g.forward(L, n, polar[i:i + 1], real=real) for i in range(len(orders))])
+    for batch in (2, 3, 4, 5, 8, 9, 16, 17, 33):
+        say(f"[pair] one order n={n} real={real} batch={batch}")
+        for i in range(0, len(orders) - batch + 1, batch):
+            f = g.inverse(L, n, cd[i:i + batch], real=real)
+            assert torch.equal(f, one[i:i + batch]), batch
+            a = g.forward(L, n, polar[i:i + batch], real=real)
+            assert torch.equal(a, back[i:i + batch]), batch
+    lmax = [L] + [L - 7 * (i % 8) for i in range(1, 33)]
+    plan = G.BatchPlan(g, lmax, [n] * 33, real=real)
+    co = torch.zeros((33, plan.cmax), dtype=torch.complex128, device="cuda")
+    single = []
+    for i, lm in enumerate(lmax):
+        size = G.coefficient_size(lm, n, real)
+        co[i, :size] = cd[i, :size]
+        single.append(g.inverse(lm, n, co[i:i + 1, :size].contiguous(), real=real))
+    f = plan.inverse(co)
+    a = plan.forward(polar)
+    for i, lm in enumerate(lmax):
+        size = G.coefficient_size(lm, n, real)
+        assert torch.equal(f[i], single[i][0]), i
+        assert torch.equal(a[i, :size], g.forward(lm, n, polar[i:i + 1], real=real)[0]), i
+    f = one.cpu().numpy()
+    th = og.nodes()[0]
+    for i in (0, 16, 32):
+        ref = og.inverse(L, n, c[i], real=real)
+        assert rel(f[i], ref) <= 1e-12
+        if real:  # its rings are transformed in pairs, which rounds to the larger of two
+            continue
+        idx = [oracle.gsh_index(L, L, n, l, orders[i]) for l in range(orders[i], L + 1)]
+        terms = [np.abs(oracle.wigner_block(L, L, n, t)[idx]).sum() for t in th]
+        err = np.abs(f[i] - ref).max(axis=1)
+        assert (err <= 301 * 2.0**-120 + 1e-12 * np.array(terms)).all()
