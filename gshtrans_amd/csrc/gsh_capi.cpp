@@ -286,6 +286,7 @@ struct gsh_grid_s {
   std::map<long, std::pair<long*, long>> cso;
   // Analysis work lists by (kernel family, lmax, n, real, per-group degree bounds).
   std::map<std::tuple<int, int, int, int, std::vector<int>>, WorkList> worklists;
+  hipStream_t aux = nullptr;  // first-use tables (see OutsideCapture)
   double* stage = nullptr;  // host-call staging
   size_t stage_bytes = 0;
   // Incremented whenever work or work2 is (re)allocated: a captured plan
@@ -436,6 +437,40 @@ int ensure_work2(gsh_grid_s* g, size_t bytes) {
   return GSH_OK;
 }
 
+// Tables that a call prepares on first use (work lists, chunk offsets,
+// checkpoints) are made while the caller may be capturing a stream into a graph:
+// the calling thread is out of the capture's restrictions meanwhile, and copies
+// and kernels run on a stream of the grid's own, waited for.
+struct OutsideCapture {
+  hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+  OutsideCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+  ~OutsideCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+};
+
+// The grid's own stream (caller is OutsideCapture).
+int ensure_aux(gsh_grid_s* g) {
+  if (!g->aux) GSH_HIP(hipStreamCreateWithFlags(&g->aux, hipStreamNonBlocking));
+  return GSH_OK;
+}
+
+// Device copy of h in a new allocation *d.
+template <typename T, typename D>
+int device_table(gsh_grid_s* g, const std::vector<T>& h, D** d) {
+  const OutsideCapture outside;
+  int st;
+  if ((st = ensure_aux(g))) return st;
+  void* p = nullptr;
+  const size_t bytes = h.size() * sizeof(T);
+  GSH_HIP(hipMalloc(&p, bytes));
+  if (hipMemcpyAsync(p, h.data(), bytes, hipMemcpyHostToDevice, g->aux) != hipSuccess ||
+      hipStreamSynchronize(g->aux) != hipSuccess) {
+    (void)hipFree(p);
+    return GSH_ERR_DEVICE;
+  }
+  *d = static_cast<D*>(p);
+  return GSH_OK;
+}
+
 // Chunk offsets of the split coefficient layout: order m (slot m - m_first)
 // owns ceil((lmax - l0 + 1) / 32) chunks of 32 degrees, l0 = max(|m|, |n|).
 // Split-block offsets per slot: one block per 32-degree chunk, or (sym, the
@@ -460,8 +495,8 @@ int ensure_cso(gsh_grid_s* g, int lmax, int n, int real, int sym, long** dev, lo
   }
   h[nslot] = acc;
   long* d = nullptr;
-  GSH_HIP(hipMalloc(&d, h.size() * sizeof(long)));
-  GSH_HIP(hipMemcpy(d, h.data(), h.size() * sizeof(long), hipMemcpyHostToDevice));
+  int st;
+  if ((st = device_table(g, h, &d))) return st;
   g->cso.emplace(key, std::make_pair(d, acc));
   *dev = d;
   *total = acc;
@@ -470,7 +505,7 @@ int ensure_cso(gsh_grid_s* g, int lmax, int n, int real, int sym, long** dev, lo
 
 // Checkpoints of every order of upper index n (gsh::rec_checkpoints): per
 // order, one row of ntheta states per pass k = 1 .. npass(L) - 1.
-int ensure_ck(gsh_grid_s* g, NData* d, int n, hipStream_t s) {
+int ensure_ck(gsh_grid_s* g, NData* d, int n) {
   if (d->ck) return GSH_OK;
   const int L = g->L, nt = g->ntheta();
   std::vector<long> off(2 * L + 1);
@@ -480,6 +515,9 @@ int ensure_ck(gsh_grid_s* g, NData* d, int n, hipStream_t s) {
     const int l0 = std::max(std::abs(m), std::abs(n));
     rows += std::max(0, (L - l0 + gsh::kCk) / gsh::kCk - 1);
   }
+  const OutsideCapture outside;
+  int st;
+  if ((st = ensure_aux(g))) return st;
   double2* ck = nullptr;
   long* ckoff = nullptr;
   unsigned short* kf = nullptr;
@@ -491,11 +529,9 @@ int ensure_ck(gsh_grid_s* g, NData* d, int n, hipStream_t s) {
     return status;
   };
   if (hipMalloc(&ck, std::max(rows, 1L) * nt * sizeof(double2)) != hipSuccess ||
-      hipMalloc(&ckoff, off.size() * sizeof(long)) != hipSuccess ||
       hipMalloc(&kf, off.size() * nrt * sizeof(unsigned short)) != hipSuccess)
     return release(GSH_ERR_OUT_OF_MEMORY);
-  if (hipMemcpy(ckoff, off.data(), off.size() * sizeof(long), hipMemcpyHostToDevice) != hipSuccess)
-    return release(GSH_ERR_DEVICE);
+  if ((st = device_table(g, off, &ckoff))) return release(st);
   LegParams p{};
   p.L = L;
   p.ntheta = nt;
@@ -511,7 +547,8 @@ int ensure_ck(gsh_grid_s* g, NData* d, int n, hipStream_t s) {
   p.skexp = d->skexp;
   p.kf_out = kf;
   p.nrt = nrt;
-  if (gsh::launch_rec_checkpoints(p, s) != hipSuccess || hipStreamSynchronize(s) != hipSuccess)
+  if (gsh::launch_rec_checkpoints(p, g->aux) != hipSuccess ||
+      hipStreamSynchronize(g->aux) != hipSuccess)
     return release(GSH_ERR_DEVICE);
   d->ck = ck;
   d->ckoff = ckoff;
@@ -613,8 +650,8 @@ int ensure_worklist(gsh_grid_s* g, int family, int lmax, int n, int real, int ng
   }
   WorkList w;
   w.per = static_cast<int>(per);
-  GSH_HIP(hipMalloc(&w.d, items.size() * sizeof(uint2)));
-  GSH_HIP(hipMemcpy(w.d, items.data(), items.size() * sizeof(uint2), hipMemcpyHostToDevice));
+  int st;
+  if ((st = device_table(g, items, &w.d))) return st;
   g->worklists.emplace(key, w);
   *out = w;
   return GSH_OK;
@@ -669,8 +706,8 @@ int ensure_synth_worklist(gsh_grid_s* g, int family, int lmax, int real, int ngr
   }
   WorkList w;
   w.per = static_cast<int>(items.size() / 8);
-  GSH_HIP(hipMalloc(&w.d, items.size() * sizeof(uint2)));
-  GSH_HIP(hipMemcpy(w.d, items.data(), items.size() * sizeof(uint2), hipMemcpyHostToDevice));
+  int st;
+  if ((st = device_table(g, items, &w.d))) return st;
   g->worklists.emplace(key, w);
   *out = w;
   return GSH_OK;
@@ -684,13 +721,29 @@ int ensure_synth_worklist(gsh_grid_s* g, int family, int lmax, int real, int ngr
 // first: the coefficients of neighbouring orders at a degree share cache
 // lines, and a unit's items (sub by sub, 8 orders each) run there together.
 // The weight of a degree is the share of rows at which it matters (sin t >
-// m / l).  gl[g] bounds the degrees of group g (empty: lmax); orders past it
-// have no items.
+// m / l).  Orders past the largest degree of a group's fields have no items.
+// The key holds what the items depend on and nothing else -- row blocks, and the
+// degree bound of each group -- so batches of as many groups share a list.
 int ensure_pair_worklist(gsh_grid_s* g, int dir, int lmax, int n, int pair, int ncol,
                          const gsh::PairTile& t, const std::vector<int>* f_lmax, WorkList* out) {
-  std::vector<int> shape{t.cols, t.nblk, t.vint, ncol};
-  if (f_lmax) shape.insert(shape.end(), f_lmax->begin(), f_lmax->end());
-  auto key = std::make_tuple(40 + dir, lmax, n, pair, shape);
+  // Largest degree of the group from virtual column v0 at order m (-1: the group
+  // has no column of the order), as the kernels' vcol and vcol_lmax.
+  auto bound = [&](int v0, int m) {
+    int col = v0 % ncol;
+    if (t.vint && pair)
+      col = v0 / 32 * 16;
+    else if (pair && m > 0 && v0 < ncol && v0 + t.cols > ncol)
+      col = 0;
+    else if (pair && m == 0 && v0 >= ncol)
+      return -1;
+    return f_lmax ? (*f_lmax)[std::min(col, ncol - 1) / 2] : lmax;
+  };
+  std::vector<int> shape{t.nblk};
+  for (int v0 = 0; v0 < t.vcols; v0 += t.cols) {
+    shape.push_back(bound(v0, 0));
+    shape.push_back(bound(v0, 1));
+  }
+  auto key = std::make_tuple(40 + dir, lmax, n, 0, shape);
   auto it = g->worklists.find(key);
   if (it != g->worklists.end()) {
     *out = it->second;
@@ -725,17 +778,7 @@ int ensure_pair_worklist(gsh_grid_s* g, int dir, int lmax, int n, int pair, int 
       std::vector<int> subs(b1 - b0, 0);
       int smax = 0;
       for (int m = b0; m < b1; m++) {
-        // the kernels' vcol and vcol_lmax
-        int col = v0;
-        if (t.vint && pair)
-          col = v0 / 32 * 16;
-        else if (pair && m > 0 && v0 < ncol && v0 + t.cols > ncol)
-          col = 0;
-        else if (pair && m == 0 && v0 >= ncol)
-          continue;
-        else
-          col = v0 % ncol;
-        const int lw = f_lmax ? (*f_lmax)[std::min(col, ncol - 1) / 2] : lmax;
+        const int lw = shape[1 + 2 * grp + (m > 0 ? 1 : 0)];
         const int l0 = std::max(m, std::abs(n));
         if (l0 > lw) continue;
         const int nu = (lw - l0 + 32) / 32;
@@ -773,8 +816,8 @@ int ensure_pair_worklist(gsh_grid_s* g, int dir, int lmax, int n, int pair, int 
   }
   WorkList w;
   w.per = static_cast<int>(per);
-  GSH_HIP(hipMalloc(&w.d, items.size() * sizeof(uint4)));
-  GSH_HIP(hipMemcpy(w.d, items.data(), items.size() * sizeof(uint4), hipMemcpyHostToDevice));
+  int st;
+  if ((st = device_table(g, items, &w.d))) return st;
   g->worklists.emplace(key, w);
   *out = w;
   return GSH_OK;
@@ -822,8 +865,8 @@ int ensure_split_worklist(gsh_grid_s* g, int lmax, int n, int real, int ntile, i
   while (items.size() % 8 != 0 || items.empty()) items.push_back(make_uint2(~0u, 0u));
   WorkList w;
   w.per = static_cast<int>(items.size() / 8);
-  GSH_HIP(hipMalloc(&w.d, items.size() * sizeof(uint2)));
-  GSH_HIP(hipMemcpy(w.d, items.data(), items.size() * sizeof(uint2), hipMemcpyHostToDevice));
+  int st;
+  if ((st = device_table(g, items, &w.d))) return st;
   g->worklists.emplace(key, w);
   *out = w;
   return GSH_OK;
@@ -1142,6 +1185,7 @@ int gsh_grid_destroy(gsh_grid_t g) {
   if (g->work2) (void)hipFree(g->work2);
   for (auto& kv : g->cso) (void)hipFree(kv.second.first);
   if (g->stage) (void)hipFree(g->stage);
+  if (g->aux) (void)hipStreamDestroy(g->aux);
   delete g;
   return GSH_OK;
 }
@@ -1247,7 +1291,7 @@ int run_inverse(gsh_grid_s* g, NData* d, int lmax, int n, int real, int precisio
     // parity (not in FP32, whose sums keep the order of the degrees).
     const int sym = n == 0 && precision == GSH_FP64 ? 1 : 0;
     p.pair = real ? 0 : 1;
-    if ((st = ensure_ck(g, d, n, s))) return st;
+    if ((st = ensure_ck(g, d, n))) return st;
     p.ck = d->ck;
     p.ckoff = d->ckoff;
     p.kf = d->kf;
@@ -1289,7 +1333,7 @@ int run_inverse(gsh_grid_s* g, NData* d, int lmax, int n, int real, int precisio
     p.items_per = w.per;
     const int ns = precision == GSH_BF16X6 ? 3 : 2;
     // The split-BF16 synthesis starts its recurrences at the checkpoints.
-    if ((st = ensure_ck(g, d, n, s))) return st;
+    if ((st = ensure_ck(g, d, n))) return st;
     p.ck = d->ck;
     p.ckoff = d->ckoff;
     p.kf = d->kf;
@@ -1394,7 +1438,7 @@ int run_forward(gsh_grid_s* g, NData* d, int lmax, int n, int real, int precisio
   q.fa32 = mixed ? 1 : 0;
   q.zero_pad = precision != GSH_FP64 ? 1 : 0;
   p.FA32 = mixed ? reinterpret_cast<const float*>(q.F) : nullptr;
-  if ((st = ensure_ck(g, d, n, s))) return st;
+  if ((st = ensure_ck(g, d, n))) return st;
   p.ck = d->ck;
   p.ckoff = d->ckoff;
   p.kf = d->kf;

@@ -234,3 +234,38 @@ def test_one_high_order_in_any_tile(torch, n, real):
         terms = [np.abs(oracle.wigner_block(L, L, n, t)[idx]).sum() for t in th]
         err = np.abs(f[i] - ref).max(axis=1)
         assert (err <= 301 * 2.0**-120 + 1e-12 * np.array(terms)).all()
+
+
+# A program warms up at one batch size and captures another into a graph: the
+# work list of the new shape is made during the capture, and every replay gives
+# the eager result, with eager work between.
+@pytest.mark.parametrize("precision", ["fp64", "fp32", "bf16x6"])
+@pytest.mark.parametrize("warm,batch", [(8, 3), (3, 40)])
+def test_first_call_at_a_batch_size_can_be_captured(torch, warm, batch, precision):
+    L, n, real = 160, 0, True
+    say(f"[pair] capture batch {batch} after {warm} {precision}")
+    g, eager = G.GaussLegendreGrid(L, 2), G.GaussLegendreGrid(L, 2)
+
+    def coeffs(seed, b, n=n, real=real):
+        return torch.from_numpy(G.random_coefficients(L, n, real=real, seed=seed, batch=b)).cuda()
+
+    # complex fields of another upper index size the scratch arrays for either batch
+    for b, k, r in ((max(warm, batch), 1, False), (warm, n, real)):
+        f = g.inverse(L, k, coeffs(SEED0, b, k, r), real=r, precision=precision)
+        g.forward(L, k, f, real=r, precision=precision)
+    c = coeffs(SEED0 + 1, batch)
+    f = torch.zeros((batch, L + 1, 2 * L), dtype=torch.float64, device="cuda")
+    a = torch.zeros_like(c)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        g.inverse(L, n, c, field=f, real=real, precision=precision)
+        g.forward(L, n, f, coeffs=a, real=real, precision=precision)
+    for rep in range(3):
+        c.copy_(coeffs(SEED0 + 2 + rep, batch))
+        graph.replay()
+        torch.cuda.synchronize()
+        fe = eager.inverse(L, n, c, real=real, precision=precision)
+        assert torch.equal(f, fe), rep
+        assert torch.equal(a, eager.forward(L, n, fe, real=real, precision=precision)), rep
+        torch.cuda.synchronize()
