@@ -70,3 +70,77 @@ def test_short_rings_against_extended_precision(torch, L, n, real):
             ref = og.forward(L, n, f[i], real=real)
             if np.linalg.norm(ref.astype(complex)) > 0:
                 assert rel(a[i], ref) <= 1e-14
+
+
+# The wavefront kernels (512, 1024 and 2048 points, more than 4 fields): partly
+# empty field groups (of 4 or 8 rings), odd counts of real fields (two to a ring),
+# truncation below the grid, and lmax = N / 2, whose last bin is stored apart.
+# FP64 parity as everywhere: 1e-12 of the oracle's norm.  Split BF16 moves FP32
+# bins: 2^-24 each and products of bf16x6, against FP64 1e-5.
+@pytest.mark.parametrize("L,lmax,n,real,batch", [
+    (256, 130, -2, False, 5), (256, 256, 1, False, 9), (256, 70, 2, True, 5),
+    (256, 256, 0, True, 17), (512, 512, 1, True, 7), (512, 301, 0, True, 5),
+    (512, 512, -1, False, 11), (512, 200, 0, False, 6), (1024, 1024, 0, True, 5),
+    (1024, 700, 1, True, 7), (1024, 1024, 2, False, 6), (1024, 515, 0, False, 5)])
+def test_wavefront_batches(torch, L, lmax, n, real, batch):
+    say(f"[wavefront] L={L} lmax={lmax} n={n} real={real} batch={batch}")
+    g = G.GaussLegendreGrid(L, 2)
+    og = oracle.OracleGrid(L, 2, table=False)
+    c = G.random_coefficients(lmax, n, real=real, seed=SEED0 + L + batch, grid_lmax=L, batch=batch)
+    cd = torch.from_numpy(c).cuda()
+    f = g.inverse(lmax, n, cd, real=real)
+    a = g.forward(lmax, n, f, real=real)
+    fh, ah = f.cpu().numpy(), a.cpu().numpy()
+    for i in (0, batch - 1):
+        assert rel(fh[i], og.inverse(lmax, n, c[i], real=real)) <= 1e-12
+        assert rel(ah[i], og.forward(lmax, n, fh[i], real=real)) <= 1e-12
+    fm = g.inverse(lmax, n, cd, real=real, precision="bf16x6")
+    am = g.forward(lmax, n, f, real=real, precision="bf16x6")
+    for x, y in ((fm, f), (am, a)):
+        for i in range(batch):
+            assert float((x[i] - y[i]).norm() / y[i].norm()) <= 1e-5
+
+
+# Both families transform the same bins: a batch of more than 4 fields and its
+# fields one by one differ by the FFTs' rounding, log2(2048) = 11 levels of
+# 1.1e-16, below 1e-14 of a field's norm (not bit for bit at these lengths).
+@pytest.mark.parametrize("L", [256, 512, 1024])
+@pytest.mark.parametrize("n,real", [(0, True), (2, False)])
+def test_batch_against_single_fields(torch, L, n, real):
+    say(f"[wavefront] batch against single L={L} n={n} real={real}")
+    g = G.GaussLegendreGrid(L, 2)
+    c = torch.from_numpy(G.random_coefficients(L, n, real=real, seed=SEED0, batch=9)).cuda()
+    f = g.inverse(L, n, c, real=real)
+    a = g.forward(L, n, f, real=real)
+    for i in range(9):
+        one = g.inverse(L, n, c[i:i + 1], real=real)[0]
+        assert float((f[i] - one).norm() / one.norm()) <= 1e-14
+        one = g.forward(L, n, f[i:i + 1], real=real)[0]
+        assert float((a[i] - one).norm() / one.norm()) <= 1e-14
+
+
+# Plans: the fields of a group in descending degree, so a pair of real fields in
+# one ring has two degrees, one of them N / 2, and groups fall on both sides of 4
+# fields.  Against the field alone: the FFT's rounding in FP64, FP32 bins (2^-24,
+# a plan may choose FP64 ones) in split BF16.
+@pytest.mark.parametrize("L", [256, 512, 1024])
+@pytest.mark.parametrize("real", [True, False])
+@pytest.mark.parametrize("precision,tol", [("fp64", 1e-14), ("bf16x6", 1e-6)])
+def test_uneven_plans(torch, L, real, precision, tol):
+    lmax = [L, L // 2, L, L - 24, 31, L, (7 * L) // 10] + [L, L - 1, 40] + [L]
+    n = [0] * 7 + [1] * 3 + [2]
+    say(f"[wavefront] uneven plan L={L} real={real} {precision}")
+    g = G.GaussLegendreGrid(L, 2)
+    plan = G.BatchPlan(g, lmax, n, real=real, precision=precision)
+    c = torch.zeros((len(n), plan.cmax), dtype=torch.complex128, device="cuda")
+    for i, (lm, k) in enumerate(zip(lmax, n)):
+        c[i, :G.coefficient_size(lm, k, real)] = torch.from_numpy(
+            G.random_coefficients(lm, k, real=real, seed=SEED0 + i, grid_lmax=L)).cuda()
+    f = plan.inverse(c)
+    a = plan.forward(f)
+    for i, (lm, k) in enumerate(zip(lmax, n)):
+        size = G.coefficient_size(lm, k, real)
+        one = g.inverse(lm, k, c[i:i + 1, :size].contiguous(), real=real, precision=precision)[0]
+        assert float((f[i] - one).norm() / one.norm()) <= tol, i
+        one = g.forward(lm, k, f[i:i + 1], real=real, precision=precision)[0]
+        assert float((a[i, :size] - one).norm() / one.norm()) <= tol, i
