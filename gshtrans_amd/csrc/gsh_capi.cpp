@@ -1245,14 +1245,30 @@ int bin_columns(int ncol, int precision) {
   while (cw < ncol && cw < 16) cw *= 2;
   return cw;
 }
-// Ring FFTs of a call.  The wavefront kernels (N = 512, 1024, 2048) move bins
-// for 8 complex rings (16 real ones) of a colatitude at a time; calls of at
-// most 4 fields, other lengths and o.fft = 2 take the ring kernels (a group of 8
-// would be half empty), and transforms of more than 4096 points the LDS
-// kernels.  The two families add in another order, so at these three lengths a
-// batch of more than 4 fields and one field alone agree to rounding.
+// Most fields of a call whose rings the ring kernels transform at the wavefront
+// kernels' lengths (N = 512, 1024, 2048; others always take the ring kernels, or
+// the LDS kernel above 4096 points).  The wavefront kernels move bins for 8
+// complex rings (16 real ones) of a colatitude at a time, so a group of few
+// fields is half empty; a ring alone reads and writes whole lines of 16 columns
+// for its own two where the bins come in such groups (cw; FP64 calls of up to 4
+// fields keep narrow ones).  With 16-column bins, ring and wavefront kernel:
+//   N = 512, FP32 bins, synthesis   1 field 14.7 / 10.0 us, 4 fields 14.9 / 10.5
+//   N = 1024, FP32 bins, synthesis  4 real fields 18.9 / 31.0 us, complex 25.8 / 34.4
+//   N = 2048, synthesis  2 fields 38 .. 76 / 57 .. 85 us, 3 real ones with FP32 bins
+//                        45 / 59, 3 others 66 .. 88 / 57 .. 88, 4 fields 58 .. 97 / 58 .. 92
+//   N = 2048, analysis   3 complex fields 128 / 143 us, 4 163 / 155; 4 real 76 / 82
+// The two add in another order, so at these lengths a batch above the count and
+// its fields one by one agree to rounding.
+int ring_fields(int N, int cw, bool anal, bool real, bool fp32_bins) {
+  if (cw < 16) return 4;
+  if (N == 512) return !anal && fp32_bins ? 0 : 4;
+  if (N == 1024) return 4;
+  if (anal) return real ? 4 : 3;
+  return real && fp32_bins ? 3 : 2;
+}
+// Ring FFTs of a call; o.fft = 2 asks for the ring kernels.
 hipError_t run_fft(const FFTParams& q, const RunOpts& o, bool anal, hipStream_t s) {
-  if (use_wave_fft(q, o) && q.nfield > 4 && q.cw == 16)
+  if (use_wave_fft(q, o) && q.nfield > ring_fields(q.N, q.cw, anal, q.real, q.fa32))
     return anal ? gsh::launch_fft_anal_wave(q, s) : gsh::launch_fft_synth_wave(q, s);
   if (gsh::ring_fft_supported(q.M)) return gsh::launch_fft_ring(q, anal, s);
   return anal ? gsh::launch_fft_anal(q, s) : gsh::launch_fft_synth(q, s);

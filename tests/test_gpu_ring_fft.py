@@ -144,3 +144,23 @@ def test_uneven_plans(torch, L, real, precision, tol):
         assert float((f[i] - one).norm() / one.norm()) <= tol, i
         one = g.forward(lm, k, f[i:i + 1], real=real, precision=precision)[0]
         assert float((a[i, :size] - one).norm() / one.norm()) <= tol, i
+
+
+# Few fields with bins in groups of 16 columns (every mode but FP64), on both
+# sides of each count at which the FFT family changes, against FP64: FP32 products
+# and bins of 2^-24 over sums of at most 1025 terms, below 1e-5.
+@pytest.mark.parametrize("L", [256, 512, 1024])
+@pytest.mark.parametrize("n,real", [(0, True), (2, False)])
+@pytest.mark.parametrize("precision", ["fp32", "bf16x6"])
+def test_few_fields_in_wide_bins(torch, L, n, real, precision):
+    say(f"[few fields] L={L} n={n} real={real} {precision}")
+    g = G.GaussLegendreGrid(L, 2)
+    c = torch.from_numpy(G.random_coefficients(L, n, real=real, seed=SEED0, batch=5)).cuda()
+    f = g.inverse(L, n, c, real=real)
+    a = g.forward(L, n, f, real=real)
+    for batch in (1, 2, 3, 4, 5):
+        fm = g.inverse(L, n, c[:batch], real=real, precision=precision)
+        am = g.forward(L, n, f[:batch], real=real, precision=precision)
+        for x, y in ((fm, f), (am, a)):
+            for i in range(batch):
+                assert float((x[i] - y[i]).norm() / y[i].norm()) <= 1e-5, (batch, i)
