@@ -1225,7 +1225,7 @@ struct RunOpts {
   std::vector<int> cg_lmax_host;  // the same on the host (work lists)
   const std::vector<int>* f_lmax_host = nullptr;  // f_lmax on the host
   int f32 = 0;                   // fields stored in FP32
-  int fft = 0;                   // 0: auto, 1: wavefront-per-ring kernel, 2: LDS kernel
+  int fft = 0;                   // 0, 1: run_fft's rule, 2: ring kernels of any length
   int anal_pass = 0;             // split-BF16 analysis degrees per pass: 64, 128 (0: auto)
   const void* field2 = nullptr;  // analysis of a pointwise expression: second operand
   int op = 0;                    // gsh::ExprOp applied as the analysis rings load
@@ -1848,7 +1848,7 @@ struct PlanGroup {
   int* d_cglmax = nullptr;
   NData* nd = nullptr;
   int synth_tiles = 0;  // FP64 / FP32 synthesis column tiles per wave, reported (0: not executed)
-  int fft_inv = 0;      // 1: wavefront FFT, 2: ring kernels of any length (0: not tuned)
+  int fft_inv = 0;      // 1: by run_fft's rule, 2: ring kernels of any length (0: not tuned)
   int fft_fwd = 0;
   int anal_pass = 0;    // split-BF16 analysis degrees per pass, 64 or 128 (0: not tuned)
 };
@@ -2008,10 +2008,12 @@ int run_plan(gsh_plan_s* P, int dir, const void* in, long istride, void* out, lo
 // takes the choices without timing.  Kept for the life of the process and,
 // when the environment variable GSH_TUNE_CACHE names a file, read from and
 // appended to that file (one "key tiles fft pass" line per shape;
-// unreadable lines are skipped).
+// unreadable lines are skipped).  The key's "r2" names the generation of the
+// kernels: lines without it were timed when choice 2 was another FFT, and are
+// not taken.
 std::mutex tune_mu;
-// Choices per shape: synthesis column tiles (reported only), FFT family,
-// analysis pass length.
+// Choices per shape: synthesis column tiles (written for the reader of the file
+// only: the launch's rule gives them), FFT family, analysis pass length.
 struct TuneChoice {
   int tiles = 0, fft = 0, pass = 0;
 };
@@ -2025,7 +2027,7 @@ std::string tune_key(const gsh_plan_s* P, const PlanGroup& G, int dir) {
     h *= 1099511628211ULL;
   }
   std::ostringstream k;
-  k << "gsh2:L" << P->g->L << ":k" << P->kind << ":p" << P->precision << ":s" << P->storage
+  k << "gsh2:r2:L" << P->g->L << ":k" << P->kind << ":p" << P->precision << ":s" << P->storage
     << ":d" << dir << ":n" << G.n << ":c" << G.count << ":h" << std::hex << h;
   return k.str();
 }
@@ -2066,6 +2068,27 @@ void tune_store(const std::string& key, const TuneChoice& v) {
   if (f) f << key << " " << v.tiles << " " << v.fft << " " << v.pass << "\n";
 }
 
+// Column tiles per wave of a group's FP64 / FP32 synthesis, as run_inverse
+// chooses them (0 for at most 8 fields: one tile always).
+int synth_column_tiles(const gsh_plan_s* P, const PlanGroup& G) {
+  if (G.count <= 8) return 0;
+  const int sym = G.n == 0 && P->precision == GSH_FP64 ? 1 : 0, nt = P->g->ntheta();
+  return gsh::pair_synth_tile(2 * G.count, P->kind == GSH_REAL ? 0 : 1, sym,
+                              P->precision == GSH_FP32, true, sym ? (nt + 1) / 2 : nt, G.lmax + 1)
+      .nj;
+}
+
+// Whether a group's launches with FFT choice 1 run the wavefront kernels (run_fft's
+// rule), and the family that choice `fft` runs (0: not tuned).
+bool takes_wave(const gsh_plan_s* P, const PlanGroup& G, int dir) {
+  const bool mixed = P->precision == GSH_BF16X6 || P->precision == GSH_BF16X3;
+  return P->g->d_twa && G.count > ring_fields(P->g->nphi(), bin_columns(2 * G.count, P->precision),
+                                              dir == 1, P->kind == GSH_REAL, mixed);
+}
+int fft_family(const gsh_plan_s* P, const PlanGroup& G, int dir, int fft) {
+  return fft == 1 && !takes_wave(P, G, dir) ? 2 : fft;
+}
+
 // Autotuner: per group, run each candidate (FFT family, and for the
 // split-BF16 analysis 64- or 128-degree passes) once to warm up and once timed
 // with events, and keep the fastest; a shape tuned before (this process, or
@@ -2090,9 +2113,11 @@ int tune_plan(gsh_plan_s* P, int dir, const void* in, long istride, void* out, l
   for (PlanGroup& G : P->groups) {
     const std::string key = tune_key(P, G, dir);
     TuneChoice known;
+    const bool fp = P->precision == GSH_FP64 || P->precision == GSH_FP32;
+    const int tiles = fp && dir == 0 ? synth_column_tiles(P, G) : 0;
     if (tune_lookup(key, &known)) {
       if (dir == 0) {
-        G.synth_tiles = known.tiles;
+        G.synth_tiles = tiles;
         G.fft_inv = known.fft;
       } else {
         G.fft_fwd = known.fft;
@@ -2101,11 +2126,12 @@ int tune_plan(gsh_plan_s* P, int dir, const void* in, long istride, void* out, l
       continue;
     }
     std::vector<TuneChoice> cands;
-    const bool wave_ok = P->g->d_twa != nullptr;
-    const bool fp = P->precision == GSH_FP64 || P->precision == GSH_FP32;
+    // Choice 1 where it differs from 2: the wavefront kernels, or (split-BF16
+    // synthesis) FP32 bins.
+    const bool two = P->g->d_twa && (takes_wave(P, G, dir) || (dir == 0 && !fp));
     const std::vector<int> passes =
         dir == 1 && !fp ? std::vector<int>{gsh::kPass, gsh::kWideAnalPass} : std::vector<int>{0};
-    for (int f : wave_ok ? std::vector<int>{1, 2} : std::vector<int>{2})
+    for (int f : two ? std::vector<int>{1, 2} : std::vector<int>{2})
       for (int pl : passes) cands.push_back(TuneChoice{0, f, pl});
     float best = 1e30f;
     TuneChoice pick = cands[0];
@@ -2131,13 +2157,7 @@ int tune_plan(gsh_plan_s* P, int dir, const void* in, long istride, void* out, l
       }
     }
     if (dir == 0) {
-      // Reported with the choices, not timed: the synthesis's column tiles.
-      if (fp && G.count > 8) {
-        const int pair = P->kind == GSH_REAL ? 0 : 1;
-        pick.tiles = gsh::pair_synth_tile(2 * G.count, pair, G.n == 0 && P->precision == GSH_FP64,
-                                          P->precision == GSH_FP32, true, P->g->ntheta(), G.lmax + 1)
-                         .nj;
-      }
+      pick.tiles = tiles;
       G.synth_tiles = pick.tiles;
       G.fft_inv = pick.fft;
     } else {
@@ -2350,8 +2370,8 @@ int gsh_plan_info(gsh_plan_t P, int* ngroups, int cap, int* n, int* lmax, int* c
     if (lmax) lmax[i] = G.lmax;
     if (count) count[i] = G.count;
     if (synth_tiles) synth_tiles[i] = G.synth_tiles;
-    if (fft_inverse) fft_inverse[i] = G.fft_inv;
-    if (fft_forward) fft_forward[i] = G.fft_fwd;
+    if (fft_inverse) fft_inverse[i] = fft_family(P, G, 0, G.fft_inv);
+    if (fft_forward) fft_forward[i] = fft_family(P, G, 1, G.fft_fwd);
   }
   return GSH_OK;
 }

@@ -164,3 +164,44 @@ def test_few_fields_in_wide_bins(torch, L, n, real, precision):
         for x, y in ((fm, f), (am, a)):
             for i in range(batch):
                 assert float((x[i] - y[i]).norm() / y[i].norm()) <= 1e-5, (batch, i)
+
+
+# A plan reports the FFT family that its groups run and the tiles of the launch's
+# own rule, also where a tuning file says otherwise, and does not take choices
+# that a file holds for an earlier generation of the kernels.
+def test_plan_reports_what_it_runs(torch, tmp_path, monkeypatch):
+    L, degrees = 512, [512, 500, 400]
+    lmax = degrees + [512 - 3 * i for i in range(9)] + [512] * 2
+    n = [0] * 3 + [1] * 9 + [2] * 2
+    cache = tmp_path / "tune.txt"
+    monkeypatch.setenv("GSH_TUNE_CACHE", str(cache))
+    g = G.GaussLegendreGrid(L, 2)
+    # the line of an earlier generation for the group of 3 (FNV-1a of its degrees)
+    h = 1469598103934665603
+    for l in degrees:
+        h = (h ^ l) * 1099511628211 % 2**64
+    key = f"L{L}:k{G.COMPLEX}:p{G.PRECISION['fp64']}:s{G.STORAGE['fp64']}:d0:n0:c3:h{h:x}"
+    cache.write_text(f"gsh2:{key} 1 1 0\n")
+
+    def run(path):
+        monkeypatch.setenv("GSH_TUNE_CACHE", str(path))
+        plan = G.BatchPlan(g, lmax, n)
+        c = torch.zeros((len(n), plan.cmax), dtype=torch.complex128, device="cuda")
+        plan.forward(plan.inverse(c))
+        info = {d["n"]: d for d in plan.info()}
+        plan.close()
+        return info
+
+    first = run(cache)
+    lines = [x.split() for x in cache.read_text().splitlines()[1:]]
+    say(f"[plan] {first} {lines}")
+    assert any(x[0].endswith(":" + key) for x in lines)  # timed, not taken from the old line
+    pinned = tmp_path / "pinned.txt"
+    pinned.write_text("\n".join(f"{k} {1 if t == '2' else 2} 1 {p}" for k, t, f, p in lines) + "\n")
+    second = run(pinned)
+    for info in (first, second):
+        for k in (0, 2):  # at most 4 fields
+            assert info[k]["fft_inverse"] == info[k]["fft_forward"] == 2
+    assert second[1]["fft_inverse"] == second[1]["fft_forward"] == 1
+    assert {k: d["synth_tiles"] for k, d in second.items()} == \
+        {k: d["synth_tiles"] for k, d in first.items()}
