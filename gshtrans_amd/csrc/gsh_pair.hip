@@ -880,9 +880,23 @@ PairTile pair_anal_tile(int ncol, int pair, bool uneven, int norder) {
     return t;
   }
   if (uneven && t.cols > 32) set_cols(t, 32);
-  while (t.cols > 16 &&
-         norder * ((norder + 255) / 256) * ((t.vcols + t.cols - 1) / t.cols) < kFewBlocks)
+  // 17 .. 24 and 33 .. 40 real fields: tiles of 64 and 128 would multiply a third
+  // and more of padding columns, tiles of 16 none (the sums are then as many as the
+  // recurrences repeated for them).  n = 1, 24 fields: lMax=256 52 -> 44 us, lMax=512
+  // 237 -> 205 us; 40 fields 95 -> 63 and 374 -> 333 us.  96 columns in tiles of 32
+  // gain at some degrees and lose at others: lMax=512, n = 2 376 -> 351 us, n = 0
+  // 236 -> 257 us.
+  if (!uneven && (t.vcols == 48 || t.vcols == 80)) set_cols(t, 16);
+  auto groups = [&](int cols) { return (t.vcols + cols - 1) / cols; };
+  auto few = [&] { return norder * ((norder + 255) / 256) * groups(t.cols) < kFewBlocks; };
+  // Fewer padding columns in the half as wide tile (96 columns at lMax=256, which
+  // stopped at 64: 94 -> 67 us).
+  auto leaner = [&](int cols) { return groups(cols / 2) * (cols / 2) < groups(cols) * cols; };
+  bool narrow = few();
+  while (narrow && t.cols > 16) {
     set_cols(t, t.cols / 2);
+    narrow = few() || (t.cols > 16 && leaner(t.cols));
+  }
   return t;
 }
 

@@ -269,3 +269,11 @@ def test_first_call_at_a_batch_size_can_be_captured(torch, warm, batch, precisio
         assert torch.equal(f, fe), rep
         assert torch.equal(a, eager.forward(L, n, fe, real=real, precision=precision)), rep
         torch.cuda.synchronize()
+
+
+# Analysis tiles chosen for their padding columns: 48 and 80 columns (17 .. 24 and
+# 33 .. 40 real fields) in tiles of 16, 96 of few workgroups in tiles of 32.
+@pytest.mark.parametrize("L,n,real,batch", [(256, 1, True, 24), (130, 0, True, 40), (256, 2, False, 20),
+                                            (256, 0, False, 24), (300, -1, False, 24)])
+def test_lean_analysis_tiles(torch, L, n, real, batch):
+    check(torch, L, L, n, real, batch)
