@@ -241,8 +241,8 @@ struct NData {
   int* skexp = nullptr;
   double4* rec = nullptr;  // {a, b, c, 0} per (m, l), see gsh_internal.h
   long* roff = nullptr;
-  // Recurrence checkpoints at the start of every analysis pass k >= 1
-  // (built on the first analysis with this upper index).
+  // Recurrence checkpoints, every kCk degrees of an order (built on the first
+  // transform with this upper index).
   double2* ck = nullptr;
   long* ckoff = nullptr;
   unsigned short* kf = nullptr;  // first checkpoint that matters per (order, 16 rows)
@@ -275,7 +275,7 @@ struct gsh_grid_s {
   double2* d_chirp = nullptr;  // Bluestein tables (ring length not a power of two)
   double2* d_hf = nullptr;
   double2* d_hb = nullptr;
-  int M = 0;                   // FFT length in LDS
+  int M = 0;                   // ring transform length (FFTParams::M)
   std::map<int, NData> ndata;
   double* work = nullptr;
   size_t work_bytes = 0;
@@ -1040,8 +1040,8 @@ int gsh_grid_create(int lmax, int nmax, int mrange, int nrange, gsh_grid_t* grid
   if (nrange != GSH_ALL && nrange != GSH_NONNEGATIVE && nrange != GSH_SINGLE)
     return GSH_ERR_INVALID_ARGUMENT;
   // Grids up to lMax = 2048 (the reference's constructor has no cap).  The
-  // LDS ring FFT transforms up to 8192 points, so every ring length up to
-  // 4096 runs, power of two or through Bluestein's convolution; past 2048 the
+  // ring FFTs transform up to 8192 points, so every ring length up to 4096
+  // runs, power of two or through Bluestein's convolution; past 2048 the
   // recurrence checkpoint table of one upper index, about (L + 1)^3 bytes,
   // grows from 8.6 GB (L = 2048) to 69 GB (L = 4096).
   if (lmax > kMaxGridDegree) return GSH_ERR_UNSUPPORTED;
@@ -1247,8 +1247,8 @@ int bin_columns(int ncol, int precision) {
 }
 // Most fields of a call whose rings the ring kernels transform at the wavefront
 // kernels' lengths (N = 512, 1024, 2048; others always take the ring kernels, or
-// the LDS kernel above 4096 points).  The wavefront kernels move bins for 8
-// complex rings (16 real ones) of a colatitude at a time, so a group of few
+// the LDS kernels where their convolution has 8192 points).  The wavefront kernels
+// move bins for 8 complex rings (16 real ones) of a colatitude at a time, so a group of few
 // fields is half empty; a ring alone reads and writes whole lines of 16 columns
 // for its own two where the bins come in such groups (cw; FP64 calls of up to 4
 // fields keep narrow ones).  With 16-column bins, ring and wavefront kernel:
@@ -1297,9 +1297,10 @@ int run_inverse(gsh_grid_s* g, NData* d, int lmax, int n, int real, int precisio
   q.fstride = fstride;
   q.f32 = o.f32;
   q.fmap = o.fmap;
-  // The split-BF16 synthesis hands its sums to the wavefront ring FFT in
-  // FP32 (half the bytes of F written and read; the products are FP32-
-  // accurate already).  The LDS ring FFT reads FP64 bins.
+  // The split-BF16 synthesis hands its sums to the ring FFT in FP32 at the
+  // wavefront kernels' ring lengths (half the bytes of F written and read; the
+  // products are FP32-accurate already), in FP64 at the others and where a plan
+  // chose the ring kernels.
   const bool f32bins = precision != GSH_FP64 && precision != GSH_FP32 && use_wave_fft(q, o);
   p.f32out = q.fa32 = f32bins ? 1 : 0;
   if (precision == GSH_FP64 || precision == GSH_FP32) {
@@ -1708,8 +1709,8 @@ int gsh_forward_expr(gsh_grid_t g, int lmax, int n, int value_kind, int op, int 
   o.op = op;
   o.src_cplx = src_cplx ? 1 : 0;
   o.scalar = make_double2(scalar_re, scalar_im);
-  // Re / Im of complex fields: the wavefront FFT reads two complex samples
-  // per real pair; the LDS kernels handle every form.
+  // Re / Im of complex fields: the ring FFTs read complex samples into real
+  // rings.
   return run_forward(g, d, lmax, n, real, precision, batch, field_a, field_stride,
                      static_cast<double*>(coeffs), coeff_stride, accumulate, 0, s, o);
 }

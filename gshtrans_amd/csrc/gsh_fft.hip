@@ -1,30 +1,23 @@
-// gsh_fft.hip -- batched longitude-ring FFTs for the Gauss-Legendre grid.
+// gsh_fft.hip -- ring FFTs of 2049 .. 4095 points, and the lMax = 0 branches.
 //
 // The reference runs one FFTW plan per ring (GaussLegendreGrid.h:147-174 for
 // the analysis, :266-319 for the synthesis): an unnormalised c2c/c2r backward
 // transform of the order bins F_m placed at k = m (m >= 0) and k = N + m
-// (m < 0), and an unnormalised c2c/r2c forward transform of each ring.  Here
-// each workgroup loads `rings` rings of N = 2L points into LDS (64 KiB of
-// complex values, 128 KiB for transforms of 8192 points), runs a Stockham radix-4 (+ one radix-2) autosort FFT in
-// place (values go through registers between barriers), and writes the rings
-// back.  A ring length that is not a power of two is transformed with
-// Bluestein's chirp-z identity jk = (j^2 + k^2 - (k-j)^2)/2: chirp multiply,
-// power-of-two FFT of length M >= 2N-1, multiply by the transformed chirp
-// filter, inverse FFT, chirp multiply (Bluestein 1970).  The synthesis kernel also assembles the bins from
-// the Legendre work buffer F[theta][slot][col]; the analysis kernel scatters
-// X_m * w_theta * 2 pi / N back into F for the Legendre contraction.
+// (m < 0), and an unnormalised c2c/r2c forward transform of each ring.
+// gsh_fft_ring.hip and gsh_fft_wave.hip transform in registers every ring whose
+// length is a power of two or at most 2048.  The other lengths (1024 < lMax <
+// 2048) take Bluestein's chirp-z identity jk = (j^2 + k^2 - (k-j)^2)/2 through a
+// convolution of 8192 points: one workgroup per ring keeps it in 128 KiB of LDS
+// and runs Stockham autosort passes of radix 4 (and one of radix 2) in place,
+// values going through registers between barriers.  Chirp multiply, FFT, multiply
+// by the transformed chirp filter, inverse FFT, chirp multiply (Bluestein 1970).
 #include "gsh_internal.h"
 
 namespace gsh {
 namespace {
 
 constexpr int kFFTThreads = 256;
-// Complex values per workgroup: CAP = 4096 (64 KiB of LDS) holds every ring
-// of up to 4096 points, or its Bluestein convolution, several rings at a
-// time; CAP = 8192 (128 KiB) takes the 8192-point transforms of the longer
-// rings, one at a time.
-constexpr int kFFTElems = 4096;
-constexpr int kFFTElemsMax = 8192;
+constexpr int kFFTPoints = 8192;  // of the convolution, the ring zero-padded to them
 
 __device__ __forceinline__ double2 cmul(double2 a, double2 b) {
   return make_double2(a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x);
@@ -40,31 +33,24 @@ __device__ __forceinline__ double2 cmuli(double2 a, int s) {
   return s > 0 ? make_double2(-a.y, a.x) : make_double2(a.y, -a.x);
 }
 
-// Stockham autosort passes over `rings` rings of length N held in buf
-// (ring q at buf[q*N]).  sign = -1 forward, +1 backward.
-template <int SIGN, int CAP>
-__device__ void stockham(double2* buf, int N, int rings, const double2* __restrict__ tw) {
-  int logN = 31 - __clz(N);
+// Stockham autosort passes over buf.  SIGN = -1 forward, +1 backward.
+template <int SIGN>
+__device__ void stockham(double2* buf, const double2* __restrict__ tw) {
+  constexpr int M = kFFTPoints;
+  constexpr int quarter = M / 4, half = M / 2;
   int Ns = 1;
   // radix-4 passes
-  while (logN >= 2) {
-    const int quarter = N >> 2;
-    const int total = rings * quarter;  // butterflies
-    constexpr int kPer = CAP / 4 / kFFTThreads;
+  while (4 * Ns <= M) {
+    constexpr int kPer = quarter / kFFTThreads;
     double2 v[kPer][4];
-    int dst[kPer];
 #pragma unroll
     for (int i = 0; i < kPer; i++) {
-      const int bi = threadIdx.x + i * kFFTThreads;
-      dst[i] = -1;
-      if (bi >= total) continue;
-      const int q = bi / quarter;
-      const int j = bi - q * quarter;
+      const int j = threadIdx.x + i * kFFTThreads;
       const int k = j & (Ns - 1);
-      const double2* x = buf + q * N;
-      double2 a0 = x[j], a1 = x[j + quarter], a2 = x[j + 2 * quarter], a3 = x[j + 3 * quarter];
+      double2 a0 = buf[j], a1 = buf[j + quarter], a2 = buf[j + 2 * quarter],
+              a3 = buf[j + 3 * quarter];
       if (Ns > 1) {
-        const int step = N / (Ns * 4);
+        const int step = M / (Ns * 4);
         double2 w1 = tw[k * step], w2 = tw[2 * k * step], w3 = tw[3 * k * step];
         if (SIGN > 0) {
           w1.y = -w1.y;
@@ -81,106 +67,78 @@ __device__ void stockham(double2* buf, int N, int rings, const double2* __restri
       v[i][1] = cadd(t1, t3);
       v[i][2] = csub(t0, t2);
       v[i][3] = csub(t1, t3);
-      dst[i] = q * N + (j / Ns) * Ns * 4 + k;
     }
     __syncthreads();
 #pragma unroll
     for (int i = 0; i < kPer; i++) {
-      if (dst[i] < 0) continue;
-      buf[dst[i]] = v[i][0];
-      buf[dst[i] + Ns] = v[i][1];
-      buf[dst[i] + 2 * Ns] = v[i][2];
-      buf[dst[i] + 3 * Ns] = v[i][3];
+      const int j = threadIdx.x + i * kFFTThreads;
+      double2* y = buf + (j / Ns) * Ns * 4 + (j & (Ns - 1));
+      y[0] = v[i][0];
+      y[Ns] = v[i][1];
+      y[2 * Ns] = v[i][2];
+      y[3 * Ns] = v[i][3];
     }
     __syncthreads();
     Ns *= 4;
-    logN -= 2;
   }
-  if (logN == 1) {
-    const int half = N >> 1;
-    const int total = rings * half;
-    constexpr int kPer = CAP / 2 / kFFTThreads;
-    double2 v[kPer][2];
-    int dst[kPer];
+  // the last pass, radix 2: Ns = M / 2
+  constexpr int kPer = half / kFFTThreads;
+  double2 v[kPer][2];
 #pragma unroll
-    for (int i = 0; i < kPer; i++) {
-      const int bi = threadIdx.x + i * kFFTThreads;
-      dst[i] = -1;
-      if (bi >= total) continue;
-      const int q = bi / half;
-      const int j = bi - q * half;
-      const int k = j & (Ns - 1);
-      const double2* x = buf + q * N;
-      double2 a0 = x[j], a1 = x[j + half];
-      if (Ns > 1) {
-        double2 w1 = tw[k * (N / (Ns * 2))];
-        if (SIGN > 0) w1.y = -w1.y;
-        a1 = cmul(a1, w1);
-      }
-      v[i][0] = cadd(a0, a1);
-      v[i][1] = csub(a0, a1);
-      dst[i] = q * N + (j / Ns) * Ns * 2 + k;
-    }
-    __syncthreads();
-#pragma unroll
-    for (int i = 0; i < kPer; i++) {
-      if (dst[i] < 0) continue;
-      buf[dst[i]] = v[i][0];
-      buf[dst[i] + Ns] = v[i][1];
-    }
-    __syncthreads();
+  for (int i = 0; i < kPer; i++) {
+    const int j = threadIdx.x + i * kFFTThreads;
+    double2 w1 = tw[j];
+    if (SIGN > 0) w1.y = -w1.y;
+    const double2 a0 = buf[j], a1 = cmul(buf[j + half], w1);
+    v[i][0] = cadd(a0, a1);
+    v[i][1] = csub(a0, a1);
   }
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < kPer; i++) {
+    const int j = threadIdx.x + i * kFFTThreads;
+    buf[j] = v[i][0];
+    buf[j + half] = v[i][1];
+  }
+  __syncthreads();
 }
 
 __device__ __forceinline__ double2 cconj(double2 a) { return make_double2(a.x, -a.y); }
 
-// Unnormalised DFT of length N of each ring (ring q at buf[q*M], zero from N
-// to M when Bluestein is used).  SIGN = -1 forward, +1 backward.
-template <int SIGN, int CAP>
+// Unnormalised DFT of the ring in buf (N points, zero from there on).
+// SIGN = -1 forward, +1 backward.
+template <int SIGN>
 __device__ void ring_dft(double2* buf, const FFTParams& p) {
-  const int N = p.N, M = p.M, R = p.rings;
-  if (M == N) {
-    stockham<SIGN, CAP>(buf, N, R, p.tw);
-    return;
-  }
-  for (int idx = threadIdx.x; idx < R * N; idx += kFFTThreads) {
-    const int q = idx / N, j = idx - q * N;
-    const double2 w = SIGN < 0 ? p.chirp[j] : cconj(p.chirp[j]);
-    buf[q * M + j] = cmul(buf[q * M + j], w);
-  }
-  __syncthreads();
-  stockham<-1, CAP>(buf, M, R, p.tw);
+  auto chirp = [&] {
+    for (int j = threadIdx.x; j < p.N; j += kFFTThreads) {
+      const double2 w = SIGN < 0 ? p.chirp[j] : cconj(p.chirp[j]);
+      buf[j] = cmul(buf[j], w);
+    }
+    __syncthreads();
+  };
+  chirp();
+  stockham<-1>(buf, p.tw);
   const double2* h = SIGN < 0 ? p.hf : p.hb;
-  for (int idx = threadIdx.x; idx < R * M; idx += kFFTThreads)
-    buf[idx] = cmul(buf[idx], h[idx & (M - 1)]);
+  for (int j = threadIdx.x; j < kFFTPoints; j += kFFTThreads) buf[j] = cmul(buf[j], h[j]);
   __syncthreads();
-  stockham<+1, CAP>(buf, M, R, p.tw);
-  for (int idx = threadIdx.x; idx < R * N; idx += kFFTThreads) {
-    const int q = idx / N, j = idx - q * N;
-    const double2 w = SIGN < 0 ? p.chirp[j] : cconj(p.chirp[j]);
-    buf[q * M + j] = cmul(buf[q * M + j], w);
-  }
-  __syncthreads();
+  stockham<+1>(buf, p.tw);
+  chirp();
 }
 
-// Synthesis: bins from F, backward FFT, write field rings.
-template <int CAP>
+// Synthesis of field f at colatitude theta: bins from F, backward FFT, write
+// the ring.
 __global__ __launch_bounds__(kFFTThreads) void fft_synth(FFTParams p) {
-  __shared__ double2 buf[CAP];
-  const int theta = blockIdx.x / p.nfg;
-  const int fg = blockIdx.x % p.nfg;
-  const int N = p.N, M = p.M, R = p.rings;
+  __shared__ double2 buf[kFFTPoints];
+  const int theta = blockIdx.x / p.nfield;
+  const int f = blockIdx.x % p.nfield;
+  const int N = p.N;
   const int cw = p.cw, ncg = (p.ncol + cw - 1) / cw;
-  // Fill: consecutive threads read consecutive fields of one bin.
-  for (int idx = threadIdx.x; idx < R * M; idx += kFFTThreads) {
-    const int q = idx % R;
-    const int k = idx / R;
-    const int f = fg * R + q;
+  // slot s of this field at Fp[cw s]
+  const double* Fp = p.F + f_index(theta, 0, 2 * f, p.nslot, ncg, cw);
+  const int lf = ring_lmax(p, f);
+  for (int k = threadIdx.x; k < kFFTPoints; k += kFFTThreads) {
     double2 X = make_double2(0.0, 0.0);
-    if (f < p.nfield && k < N) {
-      // slot s of this field at Fp[cw s]
-      const double* Fp = p.F + f_index(theta, 0, 2 * f, p.nslot, ncg, cw);
-      const int lf = ring_lmax(p, f);
+    if (k < N) {
       if (!p.real) {
         if (k <= lf) {
           const int s = k - p.m_first;
@@ -201,17 +159,14 @@ __global__ __launch_bounds__(kFFTThreads) void fft_synth(FFTParams p) {
         }
       }
     }
-    buf[q * M + k] = X;
+    buf[k] = X;
   }
   __syncthreads();
-  ring_dft<+1, CAP>(buf, p);
-  for (int idx = threadIdx.x; idx < R * N; idx += kFFTThreads) {
-    const int q = idx / N;
-    const int j = idx - q * N;
-    const int f = fg * R + q;
-    if (f >= p.nfield) continue;
-    const long o = (long)(p.fmap ? p.fmap[f] : f) * p.fstride + (long)theta * N + j;
-    const double2 x = buf[q * M + j];
+  ring_dft<+1>(buf, p);
+  const long ring = (long)(p.fmap ? p.fmap[f] : f) * p.fstride + (long)theta * N;
+  for (int j = threadIdx.x; j < N; j += kFFTThreads) {
+    const long o = ring + j;
+    const double2 x = buf[j];
     if (p.real && p.f32)
       static_cast<float*>(p.fout)[o] = (float)x.x;
     else if (p.real)
@@ -223,20 +178,18 @@ __global__ __launch_bounds__(kFFTThreads) void fft_synth(FFTParams p) {
   }
 }
 
-// Analysis: load rings, forward FFT, scatter weighted bins into F.
-template <int CAP>
+// Analysis of field f at colatitude theta: load the ring, forward FFT, scatter
+// weighted bins into F.
 __global__ __launch_bounds__(kFFTThreads) void fft_anal(FFTParams p) {
-  __shared__ double2 buf[CAP];
-  const int theta = blockIdx.x / p.nfg;
-  const int fg = blockIdx.x % p.nfg;
-  const int N = p.N, M = p.M, R = p.rings;
-  for (int idx = threadIdx.x; idx < R * M; idx += kFFTThreads) {
-    const int q = idx / M;
-    const int j = idx - q * M;
-    const int f = fg * R + q;
+  __shared__ double2 buf[kFFTPoints];
+  const int theta = blockIdx.x / p.nfield;
+  const int f = blockIdx.x % p.nfield;
+  const int N = p.N;
+  const long ring = (long)(p.fmap ? p.fmap[f] : f) * p.fstride + (long)theta * N;
+  for (int j = threadIdx.x; j < kFFTPoints; j += kFFTThreads) {
     double2 x = make_double2(0.0, 0.0);
-    if (f < p.nfield && j < N) {
-      const long o = (long)(p.fmap ? p.fmap[f] : f) * p.fstride + (long)theta * N + j;
+    if (j < N) {
+      const long o = ring + j;
       auto load = [&](const void* b) {
         if (p.real && p.f32) return make_double2(static_cast<const float*>(b)[o], 0.0);
         if (p.real) return make_double2(static_cast<const double*>(b)[o], 0.0);
@@ -258,20 +211,17 @@ __global__ __launch_bounds__(kFFTThreads) void fft_anal(FFTParams p) {
         }
       }
     }
-    buf[idx] = x;
+    buf[j] = x;
   }
   __syncthreads();
-  ring_dft<-1, CAP>(buf, p);
+  ring_dft<-1>(buf, p);
   const double w = p.wq[theta];
-  for (int idx = threadIdx.x; idx < R * p.nslot; idx += kFFTThreads) {
-    const int q = idx % R;
-    const int s = idx / R;
-    const int f = fg * R + q;
-    if (f >= p.nfield) continue;
+  const int lf = ring_lmax(p, f);
+  for (int s = threadIdx.x; s < p.nslot; s += kFFTThreads) {
     const int m = s + p.m_first;
-    if (abs(m) > ring_lmax(p, f)) continue;
+    if (abs(m) > lf) continue;
     const int k = m >= 0 ? m : N + m;
-    double2 X = buf[q * M + k];
+    double2 X = buf[k];
     if (p.adjoint && p.real) {
       // c2r bin weights: 2 for 0 < k < N/2, real part only at k = 0, N/2
       if (k == 0 || 2 * k == N) X.y = 0.0;
@@ -339,18 +289,10 @@ __global__ void lmax0_kernel(int mode, int real, int nfield, const double* in, l
 
 }  // namespace
 
-hipError_t launch_fft_synth(const FFTParams& p0, hipStream_t s) {
-  FFTParams p = p0;
-  if (p.M > kFFTElemsMax) return hipErrorInvalidValue;
+hipError_t launch_fft_synth(const FFTParams& p, hipStream_t s) {
+  if (p.M != kFFTPoints || p.N > p.M / 2) return hipErrorInvalidValue;
   if (p.fa32) return hipErrorInvalidValue;  // FP32 bins: wavefront kernels only
-  const bool big = p.M > kFFTElems;
-  p.rings = (big ? kFFTElemsMax : kFFTElems) / p.M;
-  p.nfg = (p.nfield + p.rings - 1) / p.rings;
-  const dim3 grid((long)p.ntheta * p.nfg);
-  if (big)
-    hipLaunchKernelGGL((fft_synth<kFFTElemsMax>), grid, dim3(kFFTThreads), 0, s, p);
-  else
-    hipLaunchKernelGGL((fft_synth<kFFTElems>), grid, dim3(kFFTThreads), 0, s, p);
+  hipLaunchKernelGGL(fft_synth, dim3((long)p.ntheta * p.nfield), dim3(kFFTThreads), 0, s, p);
   return hipGetLastError();
 }
 
@@ -358,15 +300,8 @@ hipError_t launch_fft_anal(const FFTParams& p0, hipStream_t s) {
   FFTParams p = p0;
   p.n_cg = (p.ncol + p.cw - 1) / p.cw;
   p.nquad = (p.ntheta + 3) / 4;
-  if (p.M > kFFTElemsMax) return hipErrorInvalidValue;
-  const bool big = p.M > kFFTElems;
-  p.rings = (big ? kFFTElemsMax : kFFTElems) / p.M;
-  p.nfg = (p.nfield + p.rings - 1) / p.rings;
-  const dim3 grid((long)p.ntheta * p.nfg);
-  if (big)
-    hipLaunchKernelGGL((fft_anal<kFFTElemsMax>), grid, dim3(kFFTThreads), 0, s, p);
-  else
-    hipLaunchKernelGGL((fft_anal<kFFTElems>), grid, dim3(kFFTThreads), 0, s, p);
+  if (p.M != kFFTPoints || p.N > p.M / 2) return hipErrorInvalidValue;
+  hipLaunchKernelGGL(fft_anal, dim3((long)p.ntheta * p.nfield), dim3(kFFTThreads), 0, s, p);
   return hipGetLastError();
 }
 

@@ -1,10 +1,10 @@
 // gsh_fft_wave.hip -- register-resident ring FFTs, one wavefront per ring,
 // for ring lengths N = 64 R with R in {8, 16, 32} (L = 256, 512, 1024).
 //
-// Same transforms as gsh_fft.hip (GaussLegendreGrid.h:147-174 analysis,
-// :266-319 synthesis: unnormalised DFTs of the longitude rings, bins k = m for
-// m >= 0 and k = N + m for m < 0, c2r/r2c semantics for real fields), laid
-// out for HBM: every ring is read and written as R rows of 64 consecutive
+// Same transforms as gsh_fft_ring.hip and gsh_fft.hip (GaussLegendreGrid.h:
+// 147-174 analysis, :266-319 synthesis: unnormalised DFTs of the longitude rings,
+// bins k = m for m >= 0 and k = N + m for m < 0, c2r/r2c semantics for real
+// fields), laid out for HBM: every ring is read and written as R rows of 64 consecutive
 // points (1 KiB per wavefront instruction for complex rings), and the order
 // bins are gathered from / scattered to the Legendre work buffers with whole
 // 128-byte lines per workgroup (8 wavefronts = 8 complex or 16 real fields of

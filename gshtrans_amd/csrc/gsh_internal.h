@@ -1,5 +1,5 @@
 // gsh_internal.h -- shared declarations between the host layer (gsh_capi.cpp)
-// and the HIP kernels (gsh_legendre.hip, gsh_fft.hip).
+// and the HIP kernels (gsh_*.hip).
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -246,13 +246,13 @@ __device__ inline double expr_real(int op, double a, double b, double s) {
 // Parameters of one ring-FFT launch.
 struct FFTParams {
   int N;            // ring length 2L
-  int M;            // transform length in LDS: N if N is a power of two, else
-                    // the Bluestein convolution length (power of two >= 2N-1)
+  int M;            // transform length: N if N is a power of two from 64 on, else
+                    // the Bluestein convolution length (power of two >= 2N-1, at
+                    // least 64)
   int L, ntheta, lmax, nslot, ncol, nfield, real, m_first;
-  int rings;        // rings per workgroup, rings * M <= 4096
-  int nfg;          // field groups
-  int cw;           // columns per group of the bins F / FA: 16, or for the ring
-                    // kernels (gsh_fft_ring.hip) the power of two >= ncol below it
+  int nfg;          // field groups (wavefront kernels)
+  int cw;           // columns per group of the bins F / FA: 16, or the power of two
+                    // >= ncol below it (not for the wavefront kernels)
   int n_cg;         // analysis: column groups, ceil(ncol / cw)
   int nquad;        // analysis: colatitude quads
   int zero_pad;     // analysis: zero the padding rows of the last quad (the FP64
@@ -267,8 +267,8 @@ struct FFTParams {
                       // bin weights (2 for 0 < k < N/2, Re only at 0, N/2)
   double* F;          // bins: FA (analysis) or F (synthesis); float elements
                       // when fa32
-  int fa32;           // bins in FP32 (split-BF16 modes; the synthesis only
-                      // through the wavefront kernels)
+  int fa32;           // bins in FP32 (split-BF16 modes; the synthesis only at the
+                      // wavefront kernels' ring lengths)
   const void* fin;    // analysis input field
   const void* fin2;   // analysis of a pointwise expression of two fields: the
                       // second operand (same layout as fin), or null
