@@ -170,12 +170,24 @@ __device__ __forceinline__ int wave_min(int v) {
 
 // Narrow tiles multiply for a few hundred cycles per chunk, which hides
 // neither a load nor the barrier: they keep one D buffer (two barriers per
-// chunk) and run four workgroups per CU instead of two.
+// chunk) and run three or four workgroups per CU instead of two.
 constexpr int nbuf(int kind, int tiles) { return kind == 2 || tiles <= 2 ? 1 : 2; }
 // Workgroups per CU (waves per SIMD) that the registers are cut to.
 constexpr int waves(int kind, int tiles, int nj) {
   return nbuf(kind, tiles) == 2 ? 2 : kind != 2 && nj == 2 ? 3 : 4;
 }
+// The same for the synthesis: waves of one column tile keep one D buffer too
+// (32 and 64 columns, two buffers and two workgroups: lMax=1000, n=2, 16 and 32
+// real fields 817 and 1356 us, one and three 697 and 1174 us).
+constexpr int synth_nbuf(int kind, int sym, int tiles, int nj) {
+  return !sym && nj == 1 ? 1 : nbuf(kind, tiles);
+}
+constexpr int synth_waves(int kind, int sym, int tiles, int nj) {
+  if (sym || nj == 2 || tiles <= 2 || kind == 2) return waves(kind, tiles, sym ? 2 : nj);
+  return kind == 0 ? 3 : tiles <= 4 ? 4 : 2;
+}
+// Row groups of a synthesis workgroup's four waves.
+constexpr int row_groups(int rt) { return rt == 2 ? 4 : rt <= 4 ? 2 : 1; }
 
 // ---------------------------------------------------------------------------
 // Synthesis.  An item is (m, row block, group of virtual columns); the 4
@@ -189,16 +201,23 @@ constexpr int waves(int kind, int tiles, int nj) {
 // Beside the MFMAs every vector instruction costs about 3 of an MFMA's 72
 // cycles (measured, two waves per SIMD), so the coefficient loads step one
 // byte offset per 4 degrees and mask nothing until a column's last degrees.
+// A load of B operands is 32 pieces of 16 bytes (4 degrees of 8 fields), 32
+// cycles of the CU's address path, so it has to serve many row tiles: waves of 4
+// row tiles x 1 column tile for 32 columns and of 8 x 1 for 64, where 2 x 2 and
+// 4 x 2 fetched each operand twice (lMax=1000, n=2, 16 real fields 904 -> 697 us, 32
+// fields 1340 -> 1174 us; 64 fields in two groups of 64 columns take 2305 us, 2378
+// in one of 8 x 2).  FP32, whose products take half the time, gains from the
+// shared production of 128 columns (lMax=1000, 64 complex fields 3180 us, 3240).
 // Bound: FP64 MFMA, 47 of 71 TFLOP/s of the products issued.  lMax=1024, 64
 // fields: 7.21 -> 4.95 ms (complex, n=2) and 3.55 -> 1.56 ms (real, n=0) against
 // a kernel that ran the recurrence of every order for every 32 columns; FP32
 // 3.98 -> 2.52 ms, the mean of both.
 // ---------------------------------------------------------------------------
 template <int KIND, int SYM, int RT, int NJ>
-__global__ __launch_bounds__(256, waves(KIND, RT, SYM ? 2 : NJ)) void leg_synth_p(LegParams p) {
+__global__ __launch_bounds__(256, synth_waves(KIND, SYM, RT, NJ)) void leg_synth_p(LegParams p) {
   typedef Mma<KIND> M;
   typedef typename M::elem E;
-  constexpr int WR = RT == 2 ? 4 : RT <= 4 ? 2 : 1;
+  constexpr int WR = row_groups(RT);
   constexpr int WC = 4 / WR;
   constexpr int TW = RT * WR;      // row tiles of a block without the extra one
   constexpr int NH = 2;            // 16-degree segments of a chunk
@@ -208,7 +227,7 @@ __global__ __launch_bounds__(256, waves(KIND, RT, SYM ? 2 : NJ)) void leg_synth_
   constexpr int SP = 152;
   constexpr int NB = SYM ? 2 : NJ; // accumulators per row tile
   constexpr int NC = SYM ? 1 : NJ; // column tiles per wave
-  constexpr int NBUF = nbuf(KIND, RT);
+  constexpr int NBUF = synth_nbuf(KIND, SYM, RT, NJ);
   __shared__ E D[NBUF][SC * SP];
   __shared__ uint4 rs[2][2 * SC];
   const int tid = threadIdx.x, lane = tid & 63;
@@ -819,15 +838,16 @@ hipError_t go_anal(const LegParams& p, hipStream_t s) {
 // kFewBlocks workgroups takes narrower tiles (and no 9th row tile): a wave
 // then has fewer MFMAs between two barriers, and idle CUs repeat the recurrence
 // for the other columns.  lMax=256, complex: 8 fields (514 workgroups of 32
-// columns) 44.0 -> 39.8 us synthesis, 39.2 -> 34.1 us analysis with n=1, 33.8 ->
-// 30.1 and 28.1 -> 24.2 us with n=0; lMax=384 (1155 of them) no gain, 69.7 ->
-// 80.7 us analysis.
+// columns) 39.2 -> 34.1 us analysis with n=1, 33.8 -> 30.1 (synthesis) and 28.1 ->
+// 24.2 us with n=0; lMax=384 (1155 of them) no gain, 69.7 -> 80.7 us analysis.
 constexpr int kFewBlocks = 600;
 static void set_cols(PairTile& t, int cols) {
   t.cols = cols;
   t.nj = cols == 16 ? 1 : 2;
   t.rt = cols <= 32 ? 2 : cols / 16;
 }
+// Columns that groups of cols multiply for v of them.
+static int padded(int v, int cols) { return (v + cols - 1) / cols * cols; }
 static PairTile pair_tile(int ncol, int pair, bool f32m) {
   PairTile t;
   const int V = ncol * (pair ? 2 : 1);
@@ -843,29 +863,51 @@ static PairTile pair_tile(int ncol, int pair, bool f32m) {
 PairTile pair_synth_tile(int ncol, int pair, int sym, bool f32m, bool uneven, int nr, int norder) {
   PairTile t = pair_tile(ncol, pair, f32m);
   const int rtt = (nr + 15) / 16;
-  // Blocks of tw row tiles, each with room for one more.
-  auto blocks = [rtt](int tw) { return std::max(1, (rtt + tw) / (tw + 1)); };
-  t.nblk = blocks(8);
+  // Row tiles of the busiest waves of n row blocks: rt each, one more in a block
+  // with room for an extra one (of all its waves only those of the last row group
+  // have it: lMax=1000, whose 63 tiles fit 7 blocks of 9, 10 real fields of n=2 841
+  // us in 7 blocks, 786 in 8).
+  auto row_cost = [rtt](int rt, int n) {
+    return n * rt + std::max(0, rtt - n * rt * row_groups(rt));
+  };
+  auto full_blocks = [rtt](int rt) {
+    const int tw = rt * row_groups(rt);
+    return (rtt + tw - 1) / tw;
+  };
+  auto row_blocks = [&](int rt) {
+    int n = full_blocks(rt);
+    for (int k = n - 1; k > 0 && k * (rt * row_groups(rt) + 1) >= rtt; k--)
+      if (row_cost(rt, k) <= row_cost(rt, n)) n = k;
+    return n;
+  };
   if (t.kind == 2) {
     t.nj = 1;
-    if (t.vcols > 4) t.rt = 4;
+    t.rt = t.vcols > 4 ? 4 : 2;
     t.cols = t.vcols > 4 ? 8 : 4;
+    t.nblk = row_blocks(t.rt);
     return t;
   }
-  if (uneven && t.cols > 64) set_cols(t, 64);
-  auto few = [&] { return norder * t.nblk * ((t.vcols + t.cols - 1) / t.cols) < kFewBlocks; };
-  if (few()) t.nblk = std::max(1, (rtt + 7) / 8);
-  while (t.cols > 16 && few()) set_cols(t, t.cols / 2);
-  if (sym) {  // both parities in a wave: one column tile
-    t.cols = std::min(t.cols, 64);
-    t.rt = t.cols / 8;
-    t.nj = 1;
-  }
+  // Fewer padding columns in groups of 32 are worth more A operands read (64
+  // columns in them, lMax=1000: 1356 us, 1174 in one group; 80 columns 1956 and
+  // 2265, 96 columns 2047 and 2294; 160 columns 3595 and 3560).
+  int cols = t.vcols <= 16 ? 16 : t.vcols <= 32 ? 32 : 64;
+  if (!sym && cols == 64 && 5 * padded(t.vcols, 32) <= 4 * padded(t.vcols, 64)) cols = 32;
+  if (t.kind == 1 && !uneven && t.vcols > 64 && padded(t.vcols, 128) == padded(t.vcols, 64)) cols = 128;
+  auto set = [&](int c) {
+    t.cols = c;
+    t.nj = c == 128 ? 2 : 1;
+    t.rt = c == 16 ? 2 : c == 32 ? 4 : 8;
+  };
+  set(cols);
+  auto few = [&] { return norder * t.nblk * (padded(t.vcols, t.cols) / t.cols) < kFewBlocks; };
+  t.nblk = row_blocks(t.rt);
+  if (few()) t.nblk = full_blocks(t.rt);
+  while (t.cols > 16 && few()) set(t.cols / 2);
   if (t.kind == 0 && t.rt >= 4) {
-    const int n6 = blocks(6), n8 = t.nblk;
-    const int c6 = std::max(6 * n6, rtt), c8 = std::max(8 * n8, rtt);
-    if (c6 < c8) {
-      t.rt = t.rt == 8 ? 6 : 3;
+    const int r6 = t.rt == 8 ? 6 : 3;
+    const int n6 = row_blocks(r6);
+    if (row_cost(r6, n6) < row_cost(t.rt, t.nblk)) {
+      t.rt = r6;
       t.nblk = n6;
     }
   }
@@ -907,9 +949,8 @@ hipError_t launch_leg_synth_pair(const LegParams& p0, const PairTile& t, int sym
   p.vint = t.vint;
   if (t.kind == 1) {
     if (sym) return hipErrorInvalidValue;
-    if (t.rt == 8) return go_synth<1, 0, 8, 2>(p, s);
-    if (t.rt == 4) return go_synth<1, 0, 4, 2>(p, s);
-    return t.nj == 2 ? go_synth<1, 0, 2, 2>(p, s) : go_synth<1, 0, 2, 1>(p, s);
+    if (t.rt == 8) return t.nj == 2 ? go_synth<1, 0, 8, 2>(p, s) : go_synth<1, 0, 8, 1>(p, s);
+    return t.rt == 4 ? go_synth<1, 0, 4, 1>(p, s) : go_synth<1, 0, 2, 1>(p, s);
   }
   if (t.kind == 2) {
     if (sym) return t.rt == 2 ? go_synth<2, 1, 2, 1>(p, s) : go_synth<2, 1, 4, 1>(p, s);
@@ -923,11 +964,11 @@ hipError_t launch_leg_synth_pair(const LegParams& p0, const PairTile& t, int sym
       default: return go_synth<0, 1, 2, 1>(p, s);
     }
   switch (t.rt) {
-    case 8: return go_synth<0, 0, 8, 2>(p, s);
-    case 6: return go_synth<0, 0, 6, 2>(p, s);
-    case 4: return go_synth<0, 0, 4, 2>(p, s);
-    case 3: return go_synth<0, 0, 3, 2>(p, s);
-    default: return t.nj == 2 ? go_synth<0, 0, 2, 2>(p, s) : go_synth<0, 0, 2, 1>(p, s);
+    case 8: return go_synth<0, 0, 8, 1>(p, s);
+    case 6: return go_synth<0, 0, 6, 1>(p, s);
+    case 4: return go_synth<0, 0, 4, 1>(p, s);
+    case 3: return go_synth<0, 0, 3, 1>(p, s);
+    default: return go_synth<0, 0, 2, 1>(p, s);
   }
 }
 

@@ -277,3 +277,24 @@ def test_first_call_at_a_batch_size_can_be_captured(torch, warm, batch, precisio
                                             (256, 0, False, 24), (300, -1, False, 24)])
 def test_lean_analysis_tiles(torch, L, n, real, batch):
     check(torch, L, L, n, real, batch)
+
+
+# Synthesis tiles of launches with workgroups enough for 32 and 64 columns: rows of
+# 19 and 20 tiles of 16 (blocks of 6, 7 and 8 tiles), 32 columns (full, and 80 and 96
+# in groups of 32), 64 columns (40 to 64 of them used, one to three groups); FP32 with
+# groups of 32, 64 and 128.  A field of a batch has the bits that it has alone.
+@pytest.mark.parametrize("L", [288, 303, 304])
+@pytest.mark.parametrize("n,real,batch", [(1, True, 16), (1, True, 20), (-2, False, 20), (2, True, 45),
+                                          (1, False, 32), (-1, False, 45)])
+def test_synthesis_tiles(torch, L, n, real, batch):
+    check(torch, L, L, n, real, batch)
+    g = G.GaussLegendreGrid(L, 2)
+    c = torch.from_numpy(G.random_coefficients(L, n, real=real, seed=SEED0 + L, grid_lmax=L,
+                                               batch=batch)).cuda()
+    f = g.inverse(L, n, c, real=real)
+    s = g.inverse(L, n, c, real=real, precision="fp32")
+    for i in (0, batch // 2, batch - 1):
+        one = c[i:i + 1].contiguous()
+        assert torch.equal(f[i:i + 1], g.inverse(L, n, one, real=real)), i
+        assert torch.equal(s[i:i + 1], g.inverse(L, n, one, real=real, precision="fp32")), i
+        assert rel(s[i].cpu().numpy(), f[i].cpu().numpy()) <= 3e-6, i
