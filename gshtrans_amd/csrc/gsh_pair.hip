@@ -929,7 +929,16 @@ PairTile pair_anal_tile(int ncol, int pair, bool uneven, int norder) {
   // gain at some degrees and lose at others: lMax=512, n = 2 376 -> 351 us, n = 0
   // 236 -> 257 us.
   if (!uneven && (t.vcols == 48 || t.vcols == 80)) set_cols(t, 16);
+  // The same past 128: 144 or 160 columns in groups of 32, 176 or 192 in groups
+  // of 64, which take 1.3 and 1.2 times as long a column as groups of 128.  36 .. 48
+  // complex fields, n=2: lMax=256 131 -> 101 (40) us, lMax=1000 3917 -> 3247 (40) and
+  // 3964 -> 3610 (48) us.
   auto groups = [&](int cols) { return (t.vcols + cols - 1) / cols; };
+  if (!uneven && t.cols == 128) {
+    const int w[3] = {26 * padded(t.vcols, 32), 24 * padded(t.vcols, 64), 19 * padded(t.vcols, 128)};
+    const int k = static_cast<int>(std::min_element(w, w + 3) - w);
+    set_cols(t, 32 << k);
+  }
   auto few = [&] { return norder * ((norder + 255) / 256) * groups(t.cols) < kFewBlocks; };
   // Fewer padding columns in the half as wide tile (96 columns at lMax=256, which
   // stopped at 64: 94 -> 67 us).

@@ -298,3 +298,11 @@ def test_synthesis_tiles(torch, L, n, real, batch):
         assert torch.equal(f[i:i + 1], g.inverse(L, n, one, real=real)), i
         assert torch.equal(s[i:i + 1], g.inverse(L, n, one, real=real, precision="fp32")), i
         assert rel(s[i].cpu().numpy(), f[i].cpu().numpy()) <= 3e-6, i
+
+
+# Analysis tiles past 128 columns: 144 and 160 in groups of 32, 176 and 192 in groups
+# of 64, 256 in groups of 128.
+@pytest.mark.parametrize("n,real,batch", [(1, True, 72), (-2, False, 40), (0, False, 36), (1, False, 48),
+                                          (0, True, 88), (2, False, 64)])
+def test_wide_analysis_tiles(torch, n, real, batch):
+    check(torch, 260, 260, n, real, batch)
