@@ -132,8 +132,9 @@ int gsh_grid_destroy(gsh_grid_t grid);
 int gsh_grid_info(gsh_grid_t grid, int* lmax, int* nmax, int* min_upper_index,
                   int* ntheta, int* nphi);
 int gsh_grid_colatitudes(gsh_grid_t grid, double* theta, double* weight);
-/* Build the per-upper-index device data (seeds, recurrence coefficients)
- * ahead of the first transform; transforms build it on demand otherwise. */
+/* Build the per-upper-index device data (seeds, recurrence coefficients and,
+ * where the device has room for them, checkpoints) ahead of the first
+ * transform; transforms build it on demand otherwise. */
 int gsh_grid_prepare(gsh_grid_t grid, int n);
 
 /* ---- transforms on device memory -------------------------------------- */

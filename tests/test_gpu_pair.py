@@ -306,3 +306,22 @@ def test_synthesis_tiles(torch, L, n, real, batch):
                                           (0, True, 88), (2, False, 64)])
 def test_wide_analysis_tiles(torch, n, real, batch):
     check(torch, 260, 260, n, real, batch)
+
+
+# A prepared upper index has every table that depends on it alone: what a first call
+# still allocates is its work lists and, growing with the call, the grid's bins.
+@pytest.mark.parametrize("precision", ["fp64", "fp32", "bf16x6"])
+def test_prepare_builds_the_checkpoints(torch, precision):
+    L = 512
+    g = G.GaussLegendreGrid(L, 1)
+    before = torch.cuda.mem_get_info()[0]
+    g.prepare(1)
+    table = before - torch.cuda.mem_get_info()[0]
+    # 16-byte states at L + 1 colatitudes every 16 degrees of the orders m >= 0
+    states = sum(max(0, (L - max(m, 1)) // 16) for m in range(L + 1))
+    assert table >= 16 * (L + 1) * states
+    c = torch.from_numpy(G.random_coefficients(L, 1, seed=SEED0, batch=1)).cuda()
+    f = g.inverse(L, 1, c, precision=precision)
+    g2 = G.GaussLegendreGrid(L, 1)  # not prepared
+    assert torch.equal(f, g2.inverse(L, 1, c, precision=precision))
+    assert torch.equal(g.forward(L, 1, f, precision=precision), g2.forward(L, 1, f, precision=precision))
