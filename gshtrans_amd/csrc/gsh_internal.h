@@ -295,6 +295,7 @@ struct PairTile {
   int kind = 0;  // matrix instruction (Mma in gsh_pair.hip)
   int rt = 8;    // row (synthesis) or degree (analysis) tiles per wave
   int nj = 1;    // column tiles per wave
+  int wr = 1;    // synthesis: row groups of a workgroup (4 / wr column groups)
   int cols = 0;  // virtual columns per workgroup
   int vcols = 0; // virtual columns of an order m > 0
   int vint = 0;  // see LegParams

@@ -186,16 +186,15 @@ constexpr int synth_waves(int kind, int sym, int tiles, int nj) {
   if (sym || nj == 2 || tiles <= 2 || kind == 2) return waves(kind, tiles, sym ? 2 : nj);
   return kind == 0 ? 3 : tiles <= 4 ? 4 : 2;
 }
-// Row groups of a synthesis workgroup's four waves.
-constexpr int row_groups(int rt) { return rt == 2 ? 4 : rt <= 4 ? 2 : 1; }
 
 // ---------------------------------------------------------------------------
 // Synthesis.  An item is (m, row block, group of virtual columns); the 4
 // waves share the D values of (32 degrees) x (RT WR + 1 row tiles) and split
 // the tile: WR row groups of RT row tiles x WC column groups of NJ column
 // tiles.  Wave w produces degrees 16 (w / 2) .. + 15 of each chunk for 64
-// rows; the last row group takes one row tile more where the block has it
-// (ntheta = 2^k + 1 would otherwise leave a block of one row).  SYM: one
+// rows (blocks of 16 row tiles: chunks of 16 degrees, 64 rows each wave); the
+// last row group takes one row tile more where the block has it (ntheta = 2^k
+// + 1 would otherwise leave a block of one row).  SYM: one
 // column tile per wave, the even and odd degrees in accumulators of their own.
 //
 // Beside the MFMAs every vector instruction costs about 3 of an MFMA's 72
@@ -213,18 +212,19 @@ constexpr int row_groups(int rt) { return rt == 2 ? 4 : rt <= 4 ? 2 : 1; }
 // a kernel that ran the recurrence of every order for every 32 columns; FP32
 // 3.98 -> 2.52 ms, the mean of both.
 // ---------------------------------------------------------------------------
-template <int KIND, int SYM, int RT, int NJ>
+template <int KIND, int SYM, int RT, int NJ, int WR>
 __global__ __launch_bounds__(256, synth_waves(KIND, SYM, RT, NJ)) void leg_synth_p(LegParams p) {
   typedef Mma<KIND> M;
   typedef typename M::elem E;
-  constexpr int WR = row_groups(RT);
   constexpr int WC = 4 / WR;
   constexpr int TW = RT * WR;      // row tiles of a block without the extra one
-  constexpr int NH = 2;            // 16-degree segments of a chunk
+  constexpr int NH = TW <= 8 ? 2 : 1;  // 16-degree segments of a chunk
   constexpr int SC = kCk * NH;     // degrees per chunk
-  // Elements per degree row in LDS: 9 row tiles, padded so that the A operands
-  // of both forms spread over all banks.
-  constexpr int SP = 152;
+  constexpr int PW = 4 / NH;       // waves that produce a segment, 64 rows each
+  static_assert(16 * TW <= 64 * PW, "every row of a block is produced");
+  // Elements per degree row in LDS: 9 (17) row tiles, padded so that the A
+  // operands of both forms spread over all banks.
+  constexpr int SP = TW <= 8 ? 152 : 280;
   constexpr int NB = SYM ? 2 : NJ; // accumulators per row tile
   constexpr int NC = SYM ? 1 : NJ; // column tiles per wave
   constexpr int NBUF = synth_nbuf(KIND, SYM, RT, NJ);
@@ -267,6 +267,7 @@ __global__ __launch_bounds__(256, synth_waves(KIND, SYM, RT, NJ)) void leg_synth
   // First checkpoint that counts at any of the block's rows.
   const unsigned short* kfm = p.kf + (long)(m + p.L) * p.nrt;
   int ks = wave_min(kfm[tile0 + min(lane & 15, ntile - 1)]);
+  if (TW > 15) ks = min(ks, ld_uniform_u16(kfm, tile0 + ntile - 1));  // the 17th tile
   ks = min(ks, max(0, lwg - l0 + kCk) / kCk);
   const int ls = l0 + kCk * ks;
   const int nchunk = ls > lwg ? 0 : (lwg - ls + SC) / SC;
@@ -345,10 +346,10 @@ __global__ __launch_bounds__(256, synth_waves(KIND, SYM, RT, NJ)) void leg_synth
   }
 
   // Production: wave -> (16-degree segment, 64 rows), and for the extra row
-  // tile lanes 0..15 of waves 0 and 2.
-  const int seg = wave >> 1;
-  const int prow = 64 * (wave & 1) + lane;
-  const bool xprod = ext && TW == 8 && !(wave & 1);
+  // tile lanes 0..15 of the segment's first wave.
+  const int seg = wave / PW;
+  const int prow = 64 * (wave % PW) + lane;
+  const bool xprod = ext && 16 * TW == 64 * PW && wave % PW == 0;
   constexpr int XR = 16 * TW;  // first row of the extra tile
   const int t = 16 * tile0 + prow, tx = 16 * tile0 + XR + (lane & 15);
   const bool tv = t < nr, txv = xprod && lane < 16 && tx < nr;
@@ -359,7 +360,7 @@ __global__ __launch_bounds__(256, synth_waves(KIND, SYM, RT, NJ)) void leg_synth
   int kt[5];
 #pragma unroll
   for (int i = 0; i < 4; i++)
-    kt[i] = ld_uniform_u16(kfm, min(tile0 + 4 * (wave & 1) + i, p.nrt - 1));
+    kt[i] = ld_uniform_u16(kfm, min(tile0 + 4 * (wave % PW) + i, p.nrt - 1));
   kt[4] = ld_uniform_u16(kfm, min(tile0 + TW, p.nrt - 1));
   const unsigned long long rows = __ballot(tv), rowsx = __ballot(txv);
   const double* seedm = p.seeds + (long)(m + p.L) * nt;
@@ -814,9 +815,9 @@ __global__ __launch_bounds__(256, waves(KIND, LT, NJ)) void leg_anal_p(LegParams
   }
 }
 
-template <int KIND, int SYM, int RT, int NJ>
+template <int KIND, int SYM, int RT, int NJ, int WR>
 hipError_t go_synth(const LegParams& p, hipStream_t s) {
-  hipLaunchKernelGGL((leg_synth_p<KIND, SYM, RT, NJ>), dim3(8 * p.items_per), dim3(256), 0, s, p);
+  hipLaunchKernelGGL((leg_synth_p<KIND, SYM, RT, NJ, WR>), dim3(8 * p.items_per), dim3(256), 0, s, p);
   return hipGetLastError();
 }
 template <int KIND, int SYM, int LT, int NJ>
@@ -863,28 +864,24 @@ static PairTile pair_tile(int ncol, int pair, bool f32m) {
 PairTile pair_synth_tile(int ncol, int pair, int sym, bool f32m, bool uneven, int nr, int norder) {
   PairTile t = pair_tile(ncol, pair, f32m);
   const int rtt = (nr + 15) / 16;
-  // Row tiles of the busiest waves of n row blocks: rt each, one more in a block
-  // with room for an extra one (of all its waves only those of the last row group
-  // have it: lMax=1000, whose 63 tiles fit 7 blocks of 9, 10 real fields of n=2 841
-  // us in 7 blocks, 786 in 8).
-  auto row_cost = [rtt](int rt, int n) {
-    return n * rt + std::max(0, rtt - n * rt * row_groups(rt));
-  };
-  auto full_blocks = [rtt](int rt) {
-    const int tw = rt * row_groups(rt);
-    return (rtt + tw - 1) / tw;
-  };
-  auto row_blocks = [&](int rt) {
-    int n = full_blocks(rt);
-    for (int k = n - 1; k > 0 && k * (rt * row_groups(rt) + 1) >= rtt; k--)
-      if (row_cost(rt, k) <= row_cost(rt, n)) n = k;
+  // Row tiles of the busiest waves of n row blocks of wr row groups: rt each, one
+  // more in a block with room for an extra one (of all its waves only those of the
+  // last row group have it: lMax=1000, whose 63 tiles fit 7 blocks of 9, 10 real
+  // fields of n=2 841 us in 7 blocks, 786 in 8).
+  auto row_cost = [rtt](int rt, int wr, int n) { return n * rt + std::max(0, rtt - n * rt * wr); };
+  auto full_blocks = [rtt](int rt, int wr) { return (rtt + rt * wr - 1) / (rt * wr); };
+  auto row_blocks = [&](int rt, int wr) {
+    int n = full_blocks(rt, wr);
+    for (int k = n - 1; k > 0 && k * (rt * wr + 1) >= rtt; k--)
+      if (row_cost(rt, wr, k) <= row_cost(rt, wr, n)) n = k;
     return n;
   };
   if (t.kind == 2) {
     t.nj = 1;
     t.rt = t.vcols > 4 ? 4 : 2;
+    t.wr = t.vcols > 4 ? 2 : 4;
     t.cols = t.vcols > 4 ? 8 : 4;
-    t.nblk = row_blocks(t.rt);
+    t.nblk = row_blocks(t.rt, t.wr);
     return t;
   }
   // Fewer padding columns in groups of 32 are worth more A operands read (64
@@ -897,18 +894,30 @@ PairTile pair_synth_tile(int ncol, int pair, int sym, bool f32m, bool uneven, in
     t.cols = c;
     t.nj = c == 128 ? 2 : 1;
     t.rt = c == 16 ? 2 : c == 32 ? 4 : 8;
+    t.wr = c == 16 ? 4 : c == 32 ? 2 : 1;
   };
   set(cols);
-  auto few = [&] { return norder * t.nblk * (padded(t.vcols, t.cols) / t.cols) < kFewBlocks; };
-  t.nblk = row_blocks(t.rt);
-  if (few()) t.nblk = full_blocks(t.rt);
-  while (t.cols > 16 && few()) set(t.cols / 2);
+  auto few = [&](int nblk) { return norder * nblk * (padded(t.vcols, t.cols) / t.cols) < kFewBlocks; };
+  t.nblk = row_blocks(t.rt, t.wr);
+  if (few(t.nblk)) t.nblk = full_blocks(t.rt, t.wr);
+  while (t.cols > 16 && few(t.nblk)) set(t.cols / 2);
   if (t.kind == 0 && t.rt >= 4) {
     const int r6 = t.rt == 8 ? 6 : 3;
-    const int n6 = row_blocks(r6);
-    if (row_cost(r6, n6) < row_cost(t.rt, t.nblk)) {
+    const int n6 = row_blocks(r6, t.wr);
+    if (row_cost(r6, t.wr, n6) < row_cost(t.rt, t.wr, t.nblk)) {
       t.rt = r6;
       t.nblk = n6;
+    }
+  }
+  // FP32, at most 16 columns: blocks of 16 row tiles use each coefficient twice as
+  // often (lMax=1024, 8 real fields 410 -> 364 us, 1 field 356 -> 352), where enough of
+  // them are left (lMax=800, 2403 workgroups: 222 -> 213 and 190 -> 212 us).  FP64, with
+  // products twice as long, gains nothing (489 and 500 us).
+  if (t.kind == 1 && t.cols == 16) {
+    const int n4 = row_blocks(4, 4);
+    if (norder * n4 >= 5 * kFewBlocks && row_cost(4, 4, n4) <= row_cost(2, 4, t.nblk)) {
+      t.rt = 4;
+      t.nblk = n4;
     }
   }
   return t;
@@ -958,26 +967,27 @@ hipError_t launch_leg_synth_pair(const LegParams& p0, const PairTile& t, int sym
   p.vint = t.vint;
   if (t.kind == 1) {
     if (sym) return hipErrorInvalidValue;
-    if (t.rt == 8) return t.nj == 2 ? go_synth<1, 0, 8, 2>(p, s) : go_synth<1, 0, 8, 1>(p, s);
-    return t.rt == 4 ? go_synth<1, 0, 4, 1>(p, s) : go_synth<1, 0, 2, 1>(p, s);
+    if (t.rt == 8) return t.nj == 2 ? go_synth<1, 0, 8, 2, 1>(p, s) : go_synth<1, 0, 8, 1, 1>(p, s);
+    if (t.rt == 4) return t.wr == 4 ? go_synth<1, 0, 4, 1, 4>(p, s) : go_synth<1, 0, 4, 1, 2>(p, s);
+    return go_synth<1, 0, 2, 1, 4>(p, s);
   }
   if (t.kind == 2) {
-    if (sym) return t.rt == 2 ? go_synth<2, 1, 2, 1>(p, s) : go_synth<2, 1, 4, 1>(p, s);
-    return t.rt == 2 ? go_synth<2, 0, 2, 1>(p, s) : go_synth<2, 0, 4, 1>(p, s);
+    if (sym) return t.rt == 2 ? go_synth<2, 1, 2, 1, 4>(p, s) : go_synth<2, 1, 4, 1, 2>(p, s);
+    return t.rt == 2 ? go_synth<2, 0, 2, 1, 4>(p, s) : go_synth<2, 0, 4, 1, 2>(p, s);
   }
   if (sym) switch (t.rt) {
-      case 8: return go_synth<0, 1, 8, 1>(p, s);
-      case 6: return go_synth<0, 1, 6, 1>(p, s);
-      case 4: return go_synth<0, 1, 4, 1>(p, s);
-      case 3: return go_synth<0, 1, 3, 1>(p, s);
-      default: return go_synth<0, 1, 2, 1>(p, s);
+      case 8: return go_synth<0, 1, 8, 1, 1>(p, s);
+      case 6: return go_synth<0, 1, 6, 1, 1>(p, s);
+      case 4: return go_synth<0, 1, 4, 1, 2>(p, s);
+      case 3: return go_synth<0, 1, 3, 1, 2>(p, s);
+      default: return go_synth<0, 1, 2, 1, 4>(p, s);
     }
   switch (t.rt) {
-    case 8: return go_synth<0, 0, 8, 1>(p, s);
-    case 6: return go_synth<0, 0, 6, 1>(p, s);
-    case 4: return go_synth<0, 0, 4, 1>(p, s);
-    case 3: return go_synth<0, 0, 3, 1>(p, s);
-    default: return go_synth<0, 0, 2, 1>(p, s);
+    case 8: return go_synth<0, 0, 8, 1, 1>(p, s);
+    case 6: return go_synth<0, 0, 6, 1, 1>(p, s);
+    case 4: return go_synth<0, 0, 4, 1, 2>(p, s);
+    case 3: return go_synth<0, 0, 3, 1, 2>(p, s);
+    default: return go_synth<0, 0, 2, 1, 4>(p, s);
   }
 }
 

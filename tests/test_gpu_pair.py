@@ -325,3 +325,22 @@ def test_prepare_builds_the_checkpoints(torch, precision):
     g2 = G.GaussLegendreGrid(L, 1)  # not prepared
     assert torch.equal(f, g2.inverse(L, 1, c, precision=precision))
     assert torch.equal(g.forward(L, 1, f, precision=precision), g2.forward(L, 1, f, precision=precision))
+
+
+# FP32 synthesis of at most 16 columns in blocks of 16 and 17 row tiles (lMax=1024: 65
+# tiles, the last block with the extra one; lMax=900, where the last block is short),
+# to the bits of the same fields in a wider batch, whose tiles are others.
+@pytest.mark.parametrize("L,lmax,n,real", [(1023, 1023, 0, True), (1000, 1000, 2, False),
+                                           (900, 900, -1, True), (1023, 899, 1, False)])
+def test_fp32_synthesis_of_tall_blocks(torch, L, lmax, n, real):
+    say(f"[tall] L={L} lmax={lmax} n={n} real={real}")
+    g = G.GaussLegendreGrid(L, 2)
+    few = 8 if real else 4
+    c = torch.from_numpy(G.random_coefficients(lmax, n, real=real, seed=SEED0 + L, grid_lmax=L,
+                                               batch=few + 1)).cuda()
+    wide = g.inverse(lmax, n, c, real=real, precision="fp32")
+    assert torch.equal(g.inverse(lmax, n, c[:few].contiguous(), real=real, precision="fp32"), wide[:few])
+    assert torch.equal(g.inverse(lmax, n, c[:1].contiguous(), real=real, precision="fp32"), wide[:1])
+    exact = g.inverse(lmax, n, c, real=real)
+    for i in (0, few):
+        assert rel(wide[i].cpu().numpy(), exact[i].cpu().numpy()) <= 3e-6, i
