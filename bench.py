@@ -53,16 +53,16 @@ FAMILY_KERNELS = {
     "legendre_analysis": {"fp64": r"leg_anal_p<0, \d, 8, 2>", "fp32": r"leg_anal_f32<4>",
                           "bf16x3": r"leg_anal_bf16_(ws<2, \d>|pm<2>)",
                           "bf16x6": r"leg_anal_bf16_(ws<3, \d>|pm<3>)"},
-    "legendre_synthesis": {"fp64": r"leg_synth_p<0, \d, 8, \d>",
-                           "fp32": r"leg_synth_p<1, 0, 8, 2>",
+    "legendre_synthesis": {"fp64": r"leg_synth_p<0, \d, 8, 1, 1>",
+                           "fp32": r"leg_synth_p<1, 0, 8, 2, 1>",
                            "bf16x3": r"leg_synth_bf16_(s<2, \d>|pm<2>)",
                            "bf16x6": r"leg_synth_bf16_(s<3, \d>|pm<3>)"},
-    # FA in FP64 (fp64, fp32) or FP32 (split-BF16 modes): last template argument
-    "fft_analysis": {"fp64": r"fft_anal_w<32, \d, 0, 0(, \d)?>", "fp32": r"fft_anal_w<32, \d, 0, 0(, \d)?>",
-                     "bf16x3": r"fft_anal_w<32, \d, 0, 1(, \d)?>", "bf16x6": r"fft_anal_w<32, \d, 0, 1(, \d)?>"},
-    # F in FP64 (fp64, fp32) or FP32 (split-BF16 modes): last template argument
-    "fft_synthesis": {"fp64": r"fft_synth_w<32, \d, 0, 0(, \d)?>", "fp32": r"fft_synth_w<32, \d, 0, 0(, \d)?>",
-                      "bf16x3": r"fft_synth_w<32, \d, 0, 1(, \d)?>", "bf16x6": r"fft_synth_w<32, \d, 0, 1(, \d)?>"},
+    # FA in FP64 (fp64, fp32) or FP32 (split-BF16 modes): the argument before the last
+    "fft_analysis": {"fp64": r"fft_anal_w<32, \d, 0, 0, \d>", "fp32": r"fft_anal_w<32, \d, 0, 0, \d>",
+                     "bf16x3": r"fft_anal_w<32, \d, 0, 1, \d>", "bf16x6": r"fft_anal_w<32, \d, 0, 1, \d>"},
+    # F in FP64 (fp64, fp32) or FP32 (split-BF16 modes): the argument before the last
+    "fft_synthesis": {"fp64": r"fft_synth_w<32, \d, 0, 0, \d>", "fp32": r"fft_synth_w<32, \d, 0, 0, \d>",
+                      "bf16x3": r"fft_synth_w<32, \d, 0, 1, \d>", "bf16x6": r"fft_synth_w<32, \d, 0, 1, \d>"},
     "coef_split": {"bf16x3": r"coef_split<2, \d, \d>", "bf16x6": r"coef_split<3, \d, \d>"},
 }
 HEADLINE = "bf16x6"            # <= 1e-7 relative L2 against FP64

@@ -15,8 +15,8 @@
 // instructions share one pipe (a half-and-half mix of both runs at the sum of
 // their times, 61 of 68 TFLOP/s), so every recurrence step is paid in MFMA
 // time.  The four waves of a workgroup therefore share the recurrence values
-// through LDS: each value is computed once for up to 128 virtual columns
-// (3 FP64 instructions against 128 multiply-adds), 16 degrees at a time from
+// through LDS: each value is computed once for up to 64 (synthesis) or 128 virtual
+// columns (3 FP64 instructions against as many multiply-adds), 16 degrees at a time from
 // the checkpoint table, one chunk ahead of the MFMAs that use it.
 //
 // Near the poles d^l_{mn} is evanescent for l < m / sin t.  Values of the 16
@@ -208,9 +208,9 @@ constexpr int synth_waves(int kind, int sym, int tiles, int nj) {
 // in one of 8 x 2).  FP32, whose products take half the time, gains from the
 // shared production of 128 columns (lMax=1000, 64 complex fields 3180 us, 3240).
 // Bound: FP64 MFMA, 47 of 71 TFLOP/s of the products issued.  lMax=1024, 64
-// fields: 7.21 -> 4.95 ms (complex, n=2) and 3.55 -> 1.56 ms (real, n=0) against
+// fields: 7.21 -> 4.97 ms (complex, n=2) and 3.55 -> 1.56 ms (real, n=0) against
 // a kernel that ran the recurrence of every order for every 32 columns; FP32
-// 3.98 -> 2.52 ms, the mean of both.
+// 3.98 -> 2.50 ms, the mean of both.
 // ---------------------------------------------------------------------------
 template <int KIND, int SYM, int RT, int NJ, int WR>
 __global__ __launch_bounds__(256, synth_waves(KIND, SYM, RT, NJ)) void leg_synth_p(LegParams p) {

@@ -106,10 +106,17 @@ enum gsh_value_kind { GSH_REAL = 0, GSH_COMPLEX = 1 };
 /* Arithmetic of the Legendre contraction.  The Wigner recurrence, its seeds,
  * the quadrature weights and the FFT arithmetic are FP64 in every mode; the
  * split-BF16 modes hand the order bins between the Legendre sums and the
- * wavefront ring FFT (ring lengths 512, 1024, 2048) over in FP32. */
+ * wavefront ring FFT (ring lengths 512, 1024, 2048) over in FP32.
+ *
+ * FP64, the FP32 synthesis and most split-BF16 kernels leave out Wigner values
+ * that stay below 2^-120 at 16 neighbouring colatitudes from an order's lowest
+ * degree on (near the poles): at most 2^-120 times the sum of |coefficients| of
+ * absolute error, so a field of high orders alone may have zeros there.  Inf
+ * and NaN of what is left out still reach the result. */
 enum gsh_precision {
   GSH_FP64 = 0,   /* FP64 MFMA, the reference's arithmetic                 */
-  GSH_FP32 = 1,   /* FP32 MFMA on FP32-rounded operands                     */
+  GSH_FP32 = 1,   /* FP32 MFMA on FP32-rounded operands (faster than FP64
+                     for syntheses of n != 0 only)                          */
   GSH_BF16X3 = 2, /* 2-way BF16 split, 3 products, FP32 accumulation        */
   GSH_BF16X6 = 3  /* 3-way BF16 split, 6 products, FP32 accumulation with
                      periodic FP64 flush                                     */
@@ -138,7 +145,10 @@ int gsh_grid_colatitudes(gsh_grid_t grid, double* theta, double* weight);
 int gsh_grid_prepare(gsh_grid_t grid, int n);
 
 /* ---- transforms on device memory -------------------------------------- */
-/* Synthesis: field = S_n(coeffs) for `batch` fields. */
+/* Synthesis: field = S_n(coeffs) for `batch` fields.  A field's FP64 and FP32
+ * results have the same bits in every batch, except at lmax_grid = 256, 512 and
+ * 1024, where batches of more than 2 to 4 fields take ring FFTs that add in
+ * another order (the same to rounding). */
 int gsh_inverse(gsh_grid_t grid, int lmax, int n, int value_kind, int precision,
                 int storage, int batch, const void* coeffs, long coeff_stride,
                 void* field, long field_stride, void* stream);
