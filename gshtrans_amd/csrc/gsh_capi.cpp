@@ -244,6 +244,7 @@ struct NData {
   // Recurrence checkpoints, every kCk degrees of an order (built on the first
   // transform with this upper index).
   double2* ck = nullptr;
+  double2* ckn = nullptr;  // of the orders m < 0 (built on the first call that reads them)
   long* ckoff = nullptr;
   unsigned short* kf = nullptr;  // first checkpoint that matters per (order, 16 rows)
 };
@@ -495,34 +496,39 @@ int ensure_cso(gsh_grid_s* g, int lmax, int n, int real, int sym, long** dev, lo
   return GSH_OK;
 }
 
-// Checkpoints of every order of upper index n (gsh::rec_checkpoints): per
-// order, one row of ntheta states per pass k = 1 .. npass(L) - 1.
-int ensure_ck(gsh_grid_s* g, NData* d, int n) {
-  if (d->ck) return GSH_OK;
-  const int L = g->L, nt = g->ntheta();
+// Checkpoints of the orders of upper index n (gsh::rec_checkpoints): per order, a
+// row of ntheta states for every kCk degrees after its first.  Real fields, FP64
+// and every kernel that pairs orders m and -m read those of m >= 0 only; neg: the
+// caller's kernels read the others too, half of about (L + 1)^3 bytes each.
+int ensure_ck(gsh_grid_s* g, NData* d, int n, bool neg) {
+  if (d->ck && (d->ckn || !neg)) return GSH_OK;
+  const int L = g->L, nt = g->ntheta(), nrt = (nt + 15) / 16;
   std::vector<long> off(2 * L + 1);
-  long rows = 0;
+  long rows[2] = {0, 0};  // m >= 0, m < 0
   for (int m = -L; m <= L; m++) {
-    off[m + L] = rows;
     const int l0 = std::max(std::abs(m), std::abs(n));
-    rows += std::max(0, (L - l0 + gsh::kCk) / gsh::kCk - 1);
+    off[m + L] = rows[m < 0];
+    rows[m < 0] += std::max(0, (L - l0 + gsh::kCk) / gsh::kCk - 1);
   }
   const OutsideCapture outside;
   int st;
-  double2* ck = nullptr;
-  long* ckoff = nullptr;
-  unsigned short* kf = nullptr;
-  const int nrt = (nt + 15) / 16;
+  double2* ck[2] = {nullptr, nullptr};
   auto release = [&](int status) {
-    if (ck) (void)hipFree(ck);
-    if (ckoff) (void)hipFree(ckoff);
-    if (kf) (void)hipFree(kf);
+    for (double2* c : ck)
+      if (c) (void)hipFree(c);
     return status;
   };
-  if (hipMalloc(&ck, std::max(rows, 1L) * nt * sizeof(double2)) != hipSuccess ||
-      hipMalloc(&kf, off.size() * nrt * sizeof(unsigned short)) != hipSuccess)
-    return release(GSH_ERR_OUT_OF_MEMORY);
-  if ((st = device_table(g, off, &ckoff))) return release(st);
+  if (!d->ckoff && (st = device_table(g, off, &d->ckoff))) return st;
+  if (!d->kf && hipMalloc(&d->kf, off.size() * nrt * sizeof(unsigned short)) != hipSuccess) {
+    d->kf = nullptr;
+    return GSH_ERR_OUT_OF_MEMORY;
+  }
+  for (int h = 0; h < (neg ? 2 : 1); h++)
+    if (!(h ? d->ckn : d->ck) &&
+        hipMalloc(&ck[h], std::max(rows[h], 1L) * nt * sizeof(double2)) != hipSuccess) {
+      ck[h] = nullptr;
+      return release(GSH_ERR_OUT_OF_MEMORY);
+    }
   LegParams p{};
   p.L = L;
   p.ntheta = nt;
@@ -532,19 +538,31 @@ int ensure_ck(gsh_grid_s* g, NData* d, int n) {
   p.seeds = d->seeds;
   p.rec = d->rec;
   p.roff = d->roff;
-  p.ck = ck;
-  p.ckoff = ckoff;
+  p.ck = ck[0];
+  p.ckn = ck[1];
+  p.ckoff = d->ckoff;
   p.sseed = d->sseed;
   p.skexp = d->skexp;
-  p.kf_out = kf;
+  p.kf_out = d->kf;
   p.nrt = nrt;
-  if (gsh::launch_rec_checkpoints(p, g->aux) != hipSuccess ||
-      hipStreamSynchronize(g->aux) != hipSuccess)
-    return release(GSH_ERR_DEVICE);
-  d->ck = ck;
-  d->ckoff = ckoff;
-  d->kf = kf;
+  for (int h = 0; h < 2; h++) {
+    if (!ck[h]) continue;
+    p.m_first = h ? -L : 0;
+    if (gsh::launch_rec_checkpoints(p, h ? L : L + 1, g->aux) != hipSuccess)
+      return release(GSH_ERR_DEVICE);
+  }
+  if (hipStreamSynchronize(g->aux) != hipSuccess) return release(GSH_ERR_DEVICE);
+  if (ck[0]) d->ck = ck[0];
+  if (ck[1]) d->ckn = ck[1];
   return GSH_OK;
+}
+// The tables in a launch's parameters.
+void use_ck(const NData* d, LegParams* p) {
+  p->ck = d->ck;
+  p->ckn = d->ckn;
+  p->ckoff = d->ckoff;
+  p->kf = d->kf;
+  p->nrt = (p->ntheta + 15) / 16;
 }
 
 constexpr int kMaxGridDegree = 2048;
@@ -756,8 +774,8 @@ int ensure_pair_worklist(gsh_grid_s* g, int dir, int lmax, int n, int pair, int 
       if (m >= 0) {
         ckrow[m] = row;
         rec0[m] = ent;
+        row += std::max(0, (L - l0 + gsh::kCk) / gsh::kCk - 1);
       }
-      row += std::max(0, (L - l0 + gsh::kCk) / gsh::kCk - 1);
       ent += L - l0 + 1 + gsh::kRecPad;
     }
   }
@@ -1153,6 +1171,7 @@ int gsh_grid_destroy(gsh_grid_t g) {
     (void)hipFree(kv.second.rec);
     (void)hipFree(kv.second.roff);
     if (kv.second.ck) (void)hipFree(kv.second.ck);
+    if (kv.second.ckn) (void)hipFree(kv.second.ckn);
     if (kv.second.ckoff) (void)hipFree(kv.second.ckoff);
     if (kv.second.kf) (void)hipFree(kv.second.kf);
     if (kv.second.sseed) (void)hipFree(kv.second.sseed);
@@ -1209,7 +1228,7 @@ int gsh_grid_prepare(gsh_grid_t g, int n) {
   // The checkpoints too, which every transform reads (lMax=512: the first synthesis
   // of 24 FP32 maps 619 -> 354 us).  A device without room for them has prepared what
   // it can: the first transform tries again.
-  if ((st = ensure_ck(g, d, n)) == GSH_ERR_OUT_OF_MEMORY) {
+  if ((st = ensure_ck(g, d, n, false)) == GSH_ERR_OUT_OF_MEMORY) {
     (void)hipGetLastError();
     st = GSH_OK;
   }
@@ -1309,11 +1328,8 @@ int run_inverse(gsh_grid_s* g, NData* d, int lmax, int n, int real, int precisio
     // parity (not in FP32, whose sums keep the order of the degrees).
     const int sym = n == 0 && precision == GSH_FP64 ? 1 : 0;
     p.pair = real ? 0 : 1;
-    if ((st = ensure_ck(g, d, n))) return st;
-    p.ck = d->ck;
-    p.ckoff = d->ckoff;
-    p.kf = d->kf;
-    p.nrt = (p.ntheta + 15) / 16;
+    if ((st = ensure_ck(g, d, n, false))) return st;
+    use_ck(d, &p);
     const gsh::PairTile t = gsh::pair_synth_tile(p.ncol, p.pair, sym, precision == GSH_FP32,
                                                  o.f_lmax != nullptr, sym ? (p.ntheta + 1) / 2 : p.ntheta,
                                                  lmax + 1);
@@ -1351,11 +1367,8 @@ int run_inverse(gsh_grid_s* g, NData* d, int lmax, int n, int real, int precisio
     p.items_per = w.per;
     const int ns = precision == GSH_BF16X6 ? 3 : 2;
     // The split-BF16 synthesis starts its recurrences at the checkpoints.
-    if ((st = ensure_ck(g, d, n))) return st;
-    p.ck = d->ck;
-    p.ckoff = d->ckoff;
-    p.kf = d->kf;
-    p.nrt = (p.ntheta + 15) / 16;
+    if ((st = ensure_ck(g, d, n, sym && !real))) return st;
+    use_ck(d, &p);
     long* cso = nullptr;
     long nchunks = 0;
     if ((st = ensure_cso(g, lmax, n, real, sym, &cso, &nchunks))) return st;
@@ -1456,17 +1469,26 @@ int run_forward(gsh_grid_s* g, NData* d, int lmax, int n, int real, int precisio
   q.fa32 = mixed ? 1 : 0;
   q.zero_pad = precision != GSH_FP64 ? 1 : 0;
   p.FA32 = mixed ? reinterpret_cast<const float*>(q.F) : nullptr;
-  if ((st = ensure_ck(g, d, n))) return st;
-  p.ck = d->ck;
-  p.ckoff = d->ckoff;
-  p.kf = d->kf;
-  p.nrt = (p.ntheta + 15) / 16;
+  // Upper index 0 runs over the northern colatitudes only in the split-BF16 modes
+  // (the Gauss-Legendre nodes are symmetric about the equator and d^l_{m0} has
+  // parity (-1)^(l+m) under theta -> pi - theta).  Complex fields of other
+  // upper indices run orders m and -m together in 64-degree passes
+  // (d^l_{-m,n}(theta) = (-1)^(l+n) d^l_{m,n}(pi - theta)) by default;
+  // everything else defaults to 128-degree passes.  o.anal_pass (64 or 128,
+  // 0 for the default) overrides.
+  const bool sym = n == 0;
+  const bool pm_ok = !real && !sym;
+  const int apass = o.anal_pass ? o.anal_pass : pm_ok ? gsh::kPass : kDefaultAnalPass;
+  const bool wide = apass == gsh::kWideAnalPass;
+  const bool pm = pm_ok && !wide;
+  const bool neg = !real && (precision == GSH_FP32 || (mixed && !pm));
+  if ((st = ensure_ck(g, d, n, neg))) return st;
+  use_ck(d, &p);
   const int ncg16 = (ncol + 15) / 16;
   GSH_HIP(timed(g, GSH_KERNEL_FFT_ANALYSIS, s, [&] {
     return run_fft(q, o, true, s);
   }));
   if (precision == GSH_FP64) {
-    const int sym = n == 0 ? 1 : 0;
     p.pair = real ? 0 : 1;
     const gsh::PairTile t = gsh::pair_anal_tile(p.ncol, p.pair, o.f_lmax != nullptr, lmax + 1);
     WorkList w;
@@ -1488,18 +1510,6 @@ int run_forward(gsh_grid_s* g, NData* d, int lmax, int n, int real, int precisio
     }));
     return GSH_OK;
   }
-  // Upper index 0 runs over the northern colatitudes only (the
-  // Gauss-Legendre nodes are symmetric about the equator and d^l_{m0} has
-  // parity (-1)^(l+m) under theta -> pi - theta).  Complex fields of other
-  // upper indices run orders m and -m together in 64-degree passes
-  // (d^l_{-m,n}(theta) = (-1)^(l+n) d^l_{m,n}(pi - theta)) by default;
-  // everything else defaults to 128-degree passes.  o.anal_pass (64 or 128,
-  // 0 for the default) overrides.
-  const bool sym = n == 0;
-  const bool pm_ok = !real && !sym;
-  const int apass = o.anal_pass ? o.anal_pass : pm_ok ? gsh::kPass : kDefaultAnalPass;
-  const bool wide = apass == gsh::kWideAnalPass;
-  const bool pm = pm_ok && !wide;
   {
     // 128-column super-groups of the split-BF16 kernel.
     const int nsg = (ncg16 + 7) / 8;

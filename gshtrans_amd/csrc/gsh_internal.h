@@ -106,8 +106,10 @@ struct LegParams {
   int items_per;
   // Recurrence checkpoints: state (e_l, e_{l-1}) at l = l0 + kCk k of order
   // m, k >= 1, colatitude t: ck[(ckoff[m + L] + k - 1) * ntheta + t], for
-  // every l0 + kCk k <= L.
+  // every l0 + kCk k <= L.  Orders m < 0 are in a table of their own, ckn (same
+  // index; null where no kernel of the launch reads them): see ck_rows.
   const double2* ck;
+  const double2* ckn;
   const long* ckoff;
   // Split-BF16 synthesis of the tail_rows colatitudes tail_t0 .. (0: none),
   // from the d values tail_dv[r * tail_dstride + 32 block + j] of the degree
@@ -164,6 +166,11 @@ __host__ __device__ inline long f_index(int theta, int slot, int col, int nslot,
 template <class T>
 __device__ __forceinline__ T ld_uniform(const T* p, long i) {
   return ((const __attribute__((address_space(4))) T*)p)[i];
+}
+
+// Checkpoints of order m: state k at ck_rows(p, m)[(k - 1) * ntheta + t].
+__device__ __forceinline__ const double2* ck_rows(const LegParams& p, int m) {
+  return (m < 0 ? p.ckn : p.ck) + ld_uniform(p.ckoff, m + p.L) * (long)p.ntheta;
 }
 
 // Work item of this workgroup.  Workgroups are dispatched to the device's 8
@@ -307,9 +314,9 @@ hipError_t launch_leg_synth_pair(const LegParams& p, const PairTile& t, int sym,
 hipError_t launch_leg_anal_pair(const LegParams& p, const PairTile& t, int sym, hipStream_t s);
 // Values below this at every row of a tile are left out of the FP64 sums.
 constexpr double kNegligible = 0x1p-120;
-// Recurrence checkpoints of every order of upper index p.n (uses L, ntheta,
-// nabs, cosv, seeds, rec, roff, ck, ckoff).
-hipError_t launch_rec_checkpoints(const LegParams& p, hipStream_t s);
+// Recurrence checkpoints of the norder orders from p.m_first on, of upper index
+// p.n (uses L, ntheta, nabs, cosv, seeds, rec, roff, ck or ckn, ckoff, kf_out).
+hipError_t launch_rec_checkpoints(const LegParams& p, int norder, hipStream_t s);
 hipError_t launch_fft_synth(const FFTParams& p, hipStream_t s);
 hipError_t launch_fft_anal(const FFTParams& p, hipStream_t s);
 // Wavefront-per-ring FFTs (gsh_fft_wave.hip) for N in {512, 1024, 2048}.

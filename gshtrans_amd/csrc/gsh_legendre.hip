@@ -103,8 +103,7 @@ __global__ __launch_bounds__(256) void leg_anal_f32(LegParams p) {
   __syncthreads();
   const d4* rl = reinterpret_cast<const d4*>(&rsa[0]);  // entry lc + 1 + j
   // Recurrence state at degree lc: the seed for pass 0, else the checkpoint.
-  const double2* ckp =
-      p.ck + (ld_uniform(p.ckoff, m + p.L) + (kPass / kCk) * pass - 1) * (long)p.ntheta;
+  const double2* ckp = ck_rows(p, m) + ((kPass / kCk) * pass - 1) * (long)p.ntheta;
   auto state = [&](int t, double& e0_, double& e1_) {
     if (pass == 0) {
       e0_ = p.seeds[(long)(m + p.L) * p.ntheta + t];
@@ -248,7 +247,7 @@ hipError_t launch_anal(const LegParams& p, hipStream_t s) {
   return hipGetLastError();
 }
 
-// Recurrence checkpoints: order m (blockIdx.y = m + L) runs its recurrence
+// Recurrence checkpoints: order m = m_first + blockIdx.y runs its recurrence
 // for 256 colatitudes per workgroup from the seed at l0 and stores the state
 // (e_l, e_{l-1}) at l = l0 + kCk k, k = 1 .. nck - 1, with the same
 // arithmetic as the transform kernels.  The coefficients are staged in LDS
@@ -263,8 +262,8 @@ hipError_t launch_anal(const LegParams& p, hipStream_t s) {
 // accurate once the order's values rise toward significance.  Lanes with
 // k = 0 take exactly the steps of the transform kernels.
 __global__ __launch_bounds__(256) void rec_checkpoints(LegParams p) {
-  const int mi = blockIdx.y;
-  const int m = mi - p.L;
+  const int m = p.m_first + blockIdx.y;
+  const int mi = m + p.L;
   const int l0 = max(abs(m), p.nabs);
   const int nt = p.ntheta;
   const int t = blockIdx.x * 256 + threadIdx.x;
@@ -277,7 +276,7 @@ __global__ __launch_bounds__(256) void rec_checkpoints(LegParams p) {
   const int nck = (p.L - l0 + kCk) / kCk;
   __shared__ uint4 rs[128];
   const uint4* recq = reinterpret_cast<const uint4*>(p.rec + (ld_uniform(p.roff, mi) - l0));
-  double2* out = const_cast<double2*>(p.ck) + ld_uniform(p.ckoff, mi) * (long)nt;
+  double2* out = const_cast<double2*>(ck_rows(p, m));
   // Entries up to L + kRecPad exist, so staging 64 entries past any
   // checkpoint's start stays in bounds.
   for (int k = 1; k < nck; k++) {
@@ -328,14 +327,13 @@ __global__ __launch_bounds__(256) void rec_checkpoints(LegParams p) {
 
 }  // namespace
 
-hipError_t launch_rec_checkpoints(const LegParams& p, hipStream_t s) {
-  hipLaunchKernelGGL(rec_checkpoints, dim3((p.ntheta + 255) / 256, 2 * p.L + 1), dim3(256), 0, s,
-                     p);
+hipError_t launch_rec_checkpoints(const LegParams& p, int norder, hipStream_t s) {
+  hipLaunchKernelGGL(rec_checkpoints, dim3((p.ntheta + 255) / 256, norder), dim3(256), 0, s, p);
   return hipGetLastError();
 }
 
 hipError_t launch_leg_anal_f32(const LegParams& p0, hipStream_t s) {
-  if (!p0.ck || !p0.ckoff) return hipErrorInvalidValue;  // checkpoint table required
+  if (!p0.ck || !p0.ckoff || (!p0.real && !p0.ckn)) return hipErrorInvalidValue;  // tables required
   LegParams p = p0;
   p.n_cg = (p.ncol + 15) / 16;
   p.nquad = (p.ntheta + 3) / 4;

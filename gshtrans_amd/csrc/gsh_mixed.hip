@@ -375,7 +375,7 @@ __global__ __launch_bounds__(512) void leg_synth_bf16(LegParams p) {
   // An order without checkpoints (nck < 2, so a single chunk) reads entry 0
   // of the table instead and never uses it.
   const double2* ckm =
-      (nck > 1 ? p.ck + ld_uniform(p.ckoff, m + p.L) * (long)nt : p.ck) + tpc;
+      (nck > 1 ? ck_rows(p, m) : p.ck) + tpc;
   auto ck_state = [&](int k) { return ckm[(long)(nck > 1 ? min(k, nck - 1) - 1 : 0) * nt]; };
   double pe0, pe1;
   {
@@ -614,7 +614,7 @@ __global__ __launch_bounds__(512) void leg_synth_bf16_s(LegParams p) {
   // State at checkpoint k >= 1; past L it clamps to the last checkpoint.  An
   // order without checkpoints reads entry 0 of the table and never uses it.
   const double2* ckm =
-      (nck > 1 ? p.ck + ld_uniform(p.ckoff, m + p.L) * (long)nt : p.ck) + tpc;
+      (nck > 1 ? ck_rows(p, m) : p.ck) + tpc;
   auto ck_state = [&](int k) { return ckm[(long)(nck > 1 ? min(k, nck - 1) - 1 : 0) * nt]; };
   double pe0, pe1;
   {
@@ -858,7 +858,7 @@ __global__ __launch_bounds__(512) void leg_synth_bf16_pm(LegParams p) {
   const double pcs = p.cosv[tpc];
   const int nck = (p.L - l0 + kCk) / kCk;  // checkpoints 1 .. nck-1 exist
   const double2* ckm =
-      (nck > 1 ? p.ck + ld_uniform(p.ckoff, m + p.L) * (long)nt : p.ck) + tpc;
+      (nck > 1 ? ck_rows(p, m) : p.ck) + tpc;
   auto ck_state = [&](int k) { return ckm[(long)(nck > 1 ? min(k, nck - 1) - 1 : 0) * nt]; };
   double pe0, pe1;
   {
@@ -1087,7 +1087,7 @@ __global__ __launch_bounds__(512) void leg_anal_bf16(LegParams p) {
   const int bh = wave & 1, q = wave >> 1;
   const int nck = (p.L - l0 + kCk) / kCk;  // checkpoints 1 .. nck-1 exist
   const int kq = min((kPass / kCk) * pass + q, nck - 1);
-  const double2* ckp = kq == 0 ? p.ck : p.ck + (ld_uniform(p.ckoff, m + p.L) + kq - 1) * (long)nt;
+  const double2* ckp = kq == 0 ? p.ck : ck_rows(p, m) + (kq - 1) * (long)nt;
   const double* sdp = p.seeds + (long)(m + p.L) * nt;
   // The state and cosine of group g's colatitude are loaded into registers
   // one group before they are used, after the previous production (so the
@@ -1333,7 +1333,7 @@ __global__ __launch_bounds__(512) void leg_anal_bf16_pm(LegParams p) {
   const int bh = wave & 1, q = wave >> 1;
   const int nck = (p.L - l0 + kCk) / kCk;
   const int kq = min((kPass / kCk) * pass + q, nck - 1);
-  const double2* ckp = kq == 0 ? p.ck : p.ck + (ld_uniform(p.ckoff, m + p.L) + kq - 1) * (long)nt;
+  const double2* ckp = kq == 0 ? p.ck : ck_rows(p, m) + (kq - 1) * (long)nt;
   const double* sdp = p.seeds + (long)(m + p.L) * nt;
   double nx_seed, nx_cs;
   double2 nx_ck;
@@ -1587,7 +1587,7 @@ __global__ __launch_bounds__(512) void leg_anal_bf16_s(LegParams p) {
   const int bh = wave & 1, q = wave >> 1;
   const int nck = (p.L - l0 + kCk) / kCk;  // checkpoints 1 .. nck-1 exist
   const int kq = min((kPass / kCk) * pass + q, nck - 1);
-  const double2* ckp = kq == 0 ? p.ck : p.ck + (ld_uniform(p.ckoff, m + p.L) + kq - 1) * (long)nt;
+  const double2* ckp = kq == 0 ? p.ck : ck_rows(p, m) + (kq - 1) * (long)nt;
   const double* sdp = p.seeds + (long)(m + p.L) * nt;
   // The state and cosine of group g's colatitude are loaded into registers
   // one group before they are used, after the previous production (so the
@@ -1863,7 +1863,7 @@ __global__ __launch_bounds__(512) void leg_anal_bf16_w(LegParams p) {
   // from checkpoint kq (the seed for kq = 0; past L clamped to the last).
   const int nck = (p.L - l0 + kCk) / kCk;  // checkpoints 1 .. nck-1 exist
   const int kq = min((kWidePass / kCk) * pass + wave, nck - 1);
-  const double2* ckp = kq == 0 ? p.ck : p.ck + (ld_uniform(p.ckoff, m + p.L) + kq - 1) * (long)nt;
+  const double2* ckp = kq == 0 ? p.ck : ck_rows(p, m) + (kq - 1) * (long)nt;
   const double* sdp = p.seeds + (long)(m + p.L) * nt;
   double nx_seed, nx_cs;
   double2 nx_ck;
@@ -2077,7 +2077,7 @@ __global__ __launch_bounds__(512) void leg_anal_bf16_ws(LegParams p) {
   // from checkpoint kq (the seed for kq = 0; past L clamped to the last).
   const int nck = (p.L - l0 + kCk) / kCk;  // checkpoints 1 .. nck-1 exist
   const int kq = min((kWidePass / kCk) * pass + wave, nck - 1);
-  const double2* ckp = kq == 0 ? p.ck : p.ck + (ld_uniform(p.ckoff, m + p.L) + kq - 1) * (long)nt;
+  const double2* ckp = kq == 0 ? p.ck : ck_rows(p, m) + (kq - 1) * (long)nt;
   const double* sdp = p.seeds + (long)(m + p.L) * nt;
   double nx_seed, nx_cs;
   double2 nx_ck;
@@ -2307,7 +2307,7 @@ __global__ __launch_bounds__(64) void tail_dvals(LegParams p, double* dv) {
   const int nck = (p.L - l0 + kCk) / kCk;  // checkpoints 1 .. nck-1 exist
   const double cs = p.cosv[t];
   const d4* rl = reinterpret_cast<const d4*>(p.rec + (ld_uniform(p.roff, m + p.L) - l0));
-  const double2* ckm = p.ck + ld_uniform(p.ckoff, m + p.L) * (long)p.ntheta + t;
+  const double2* ckm = ck_rows(p, m) + t;
   double* out = dv + blockIdx.y * p.tail_dstride + ld_uniform(p.cso, slot) * 32;
   // Entry of degree l0 + d: d itself, or in the parity layout block
   // 2 (d / 64) + k (k = (d + l0 + m) % 2), entry (d % 64) / 2.
@@ -2378,7 +2378,8 @@ hipError_t launch_coef_split(const LegParams& p, int ns, hipStream_t s) {
 }
 
 hipError_t launch_leg_synth_bf16(const LegParams& p0, int ns, hipStream_t s) {
-  if (!p0.ck || !p0.ckoff || !p0.kf) return hipErrorInvalidValue;  // checkpoint tables required
+  if (!p0.ck || !p0.ckoff || !p0.kf || (!p0.real && !p0.pm && !p0.ckn))
+    return hipErrorInvalidValue;  // checkpoint tables required
   LegParams p = p0;
   p.n_tsb = (p.ntheta + 255) / 256;
   p.n_cg = (p.ntile + 7) / 8;  // column super-groups of 8 tiles
@@ -2415,7 +2416,8 @@ hipError_t launch_leg_synth_bf16(const LegParams& p0, int ns, hipStream_t s) {
 }
 
 hipError_t launch_tail_dvals(const LegParams& p, hipStream_t s) {
-  if (p.tail_rows < 1 || p.tail_rows > kSynthTailRows || !p.tail_dv || !p.ck || !p.ckoff)
+  if (p.tail_rows < 1 || p.tail_rows > kSynthTailRows || !p.tail_dv || !p.ck || !p.ckoff ||
+      (!p.real && !p.pm && !p.ckn))
     return hipErrorInvalidValue;
   hipLaunchKernelGGL(tail_dvals, dim3(p.nslot, p.tail_rows), dim3(64), 0, s, p,
                      const_cast<double*>(p.tail_dv));
@@ -2469,7 +2471,8 @@ hipError_t launch_anal_bf16_w(const LegParams& p0, hipStream_t s, bool sym) {
 }
 
 hipError_t launch_leg_anal_bf16(const LegParams& p, int ns, hipStream_t s, int form) {
-  if (!p.ck || !p.ckoff || !p.kf) return hipErrorInvalidValue;  // checkpoint tables required
+  if (!p.ck || !p.ckoff || !p.kf || (!p.real && form != 4 && !p.ckn))
+    return hipErrorInvalidValue;  // checkpoint tables required
   if (!p.FA32) return hipErrorInvalidValue;             // FP32 bins required
   if ((form == 2 || form == 3) && p.nabs != 0) return hipErrorInvalidValue;  // n = 0 only
   if (form == 4) {  // orders m and -m together: complex fields

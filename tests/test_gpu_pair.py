@@ -344,3 +344,35 @@ def test_fp32_synthesis_of_tall_blocks(torch, L, lmax, n, real):
     exact = g.inverse(lmax, n, c, real=real)
     for i in (0, few):
         assert rel(wide[i].cpu().numpy(), exact[i].cpu().numpy()) <= 3e-6, i
+
+
+# The checkpoints of orders m < 0 are built by the first call that reads them: FP64
+# holds half a table, and what other modes compute does not depend on the order in
+# which the two halves came.
+@pytest.mark.parametrize("n,mode", [(0, "bf16x6"), (0, "fp32"), (1, "fp32"), (-2, "bf16x3")])
+def test_checkpoints_of_negative_orders(torch, n, mode):
+    L = 400
+    def both(g, precision):
+        f = g.inverse(L, n, c, precision=precision)
+        return f, g.forward(L, n, f, precision=precision)
+    c = torch.from_numpy(G.random_coefficients(L, n, seed=SEED0, batch=2)).cuda()
+    states = 16 * (L + 1) * sum(max(0, (L - max(m, abs(n))) // 16) for m in range(L + 1))
+    g = G.GaussLegendreGrid(L, 2)
+    before = torch.cuda.mem_get_info()[0]
+    g.prepare(n)
+    # seeds and recurrence coefficients: 20 and 32 bytes for each of (2 L + 1)(L + 1) and
+    # about L^2 + 64 (2 L + 1) entries, and allocation granules
+    others = 20 * (2 * L + 1) * (L + 1) + 32 * (L * L + 66 * (2 * L + 1)) + (16 << 20)
+    assert before - torch.cuda.mem_get_info()[0] <= states + others
+    first = both(g, "fp64")
+    second = both(g, mode)
+    for x, y in zip(both(g, "fp64"), first):
+        assert torch.equal(x, y)
+    g2 = G.GaussLegendreGrid(L, 2)
+    for x, y in zip(both(g2, mode), second):
+        assert torch.equal(x, y)
+    for x, y in zip(both(g2, "fp64"), first):
+        assert torch.equal(x, y)
+    og = oracle.OracleGrid(L, 2, table=False)
+    tol = {"fp32": 3e-6, "bf16x6": 1e-7, "bf16x3": 3e-5}[mode]
+    assert rel(second[0][1].cpu().numpy(), og.inverse(L, n, c[1].cpu().numpy(), real=False)) <= tol
