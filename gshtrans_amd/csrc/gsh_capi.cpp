@@ -287,7 +287,7 @@ struct gsh_grid_s {
   std::map<long, std::pair<long*, long>> cso;
   // Analysis work lists by (kernel family, lmax, n, real, per-group degree bounds).
   std::map<std::tuple<int, int, int, int, std::vector<int>>, WorkList> worklists;
-  hipStream_t aux = nullptr;  // first-use tables (see OutsideCapture)
+  hipStream_t aux = nullptr;  // first-use tables (see OutsideCapture; take_aux)
   double* stage = nullptr;  // host-call staging
   size_t stage_bytes = 0;
   // Incremented whenever work or work2 is (re)allocated: a captured plan
@@ -441,12 +441,33 @@ int ensure_work2(gsh_grid_s* g, size_t bytes) {
 // Tables that a call prepares on first use (work lists, chunk offsets,
 // checkpoints) are made while the caller may be capturing a stream into a graph:
 // the calling thread is out of the capture's restrictions meanwhile, and copies
-// and kernels run on a stream of the grid's own, waited for.
+// and kernels run on a stream that no caller captures, waited for.
 struct OutsideCapture {
   hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
   OutsideCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
   ~OutsideCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
 };
+
+// That stream, one for all grids of a device: making and destroying one for each
+// takes 90 us, a tenth of the life of a small grid.  It lives as long as a grid
+// of the device does.
+std::mutex aux_mu;
+std::map<int, std::pair<hipStream_t, int>> aux_streams;  // device -> stream, grids
+hipStream_t take_aux(int device) {
+  std::lock_guard<std::mutex> lock(aux_mu);
+  auto& a = aux_streams[device];
+  if (!a.first && hipStreamCreateWithFlags(&a.first, hipStreamNonBlocking) != hipSuccess)
+    return a.first = nullptr;
+  a.second++;
+  return a.first;
+}
+void drop_aux(int device) {
+  std::lock_guard<std::mutex> lock(aux_mu);
+  auto& a = aux_streams[device];
+  if (--a.second > 0) return;
+  (void)hipStreamDestroy(a.first);
+  aux_streams.erase(device);
+}
 
 // Device copy of h in a new allocation *d.
 template <typename T, typename D>
@@ -1149,10 +1170,10 @@ int gsh_grid_create(int lmax, int nmax, int mrange, int nrange, gsh_grid_t* grid
     GSH_HIP(hipMemcpy(g->d_one, one.data(), one.size() * sizeof(double), hipMemcpyHostToDevice));
   }
   GSH_HIP(hipMemcpy(g->d_tw, tw.data(), tw.size() * sizeof(double2), hipMemcpyHostToDevice));
-  GSH_HIP(hipStreamCreateWithFlags(&g->aux, hipStreamNonBlocking));
   // Address of this device's copy of the allocation-free entry point's
   // scratch array (looked up once per device, with the device current).
   GSH_HIP(gsh::noalloc_scratch_init(dev));
+  if (!(g->aux = take_aux(dev))) return GSH_ERR_DEVICE;
   *grid = g.release();
   return GSH_OK;
 }
@@ -1196,7 +1217,7 @@ int gsh_grid_destroy(gsh_grid_t g) {
   if (g->work2) (void)hipFree(g->work2);
   for (auto& kv : g->cso) (void)hipFree(kv.second.first);
   if (g->stage) (void)hipFree(g->stage);
-  if (g->aux) (void)hipStreamDestroy(g->aux);
+  drop_aux(g->device);
   delete g;
   return GSH_OK;
 }

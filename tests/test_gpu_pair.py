@@ -376,3 +376,41 @@ def test_checkpoints_of_negative_orders(torch, n, mode):
     og = oracle.OracleGrid(L, 2, table=False)
     tol = {"fp32": 3e-6, "bf16x6": 1e-7, "bf16x3": 3e-5}[mode]
     assert rel(second[0][1].cpu().numpy(), og.inverse(L, n, c[1].cpu().numpy(), real=False)) <= tol
+
+
+# Grids made, used and closed by several threads at once share the stream that builds
+# their tables; the results are those of a grid alone.
+def test_grids_of_several_threads(torch):
+    import threading
+    cases = [(16, 1, False), (33, 0, True), (64, 2, False), (47, -1, True)]
+    coeffs = [torch.from_numpy(G.random_coefficients(L, n, real=real, seed=SEED0 + L, batch=2)).cuda()
+              for L, n, real in cases]
+
+    def use(k):
+        L, n, real = cases[k]
+        g = G.GaussLegendreGrid(L, 2)
+        f = g.inverse(L, n, coeffs[k], real=real)
+        a = g.forward(L, n, f, real=real)
+        torch.cuda.synchronize()
+        g.close()
+        return f, a
+
+    alone = [use(k) for k in range(len(cases))]
+    got, errors = {}, []
+
+    def work(k):
+        try:
+            for rep in range(4):
+                got[k, rep] = use((k + rep) % len(cases))
+        except Exception as e:  # reported by the main thread
+            errors.append(e)
+
+    threads = [threading.Thread(target=work, args=(k,)) for k in range(len(cases))]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not errors, errors
+    for (k, rep), (f, a) in got.items():
+        assert torch.equal(f, alone[(k + rep) % len(cases)][0]), (k, rep)
+        assert torch.equal(a, alone[(k + rep) % len(cases)][1]), (k, rep)
