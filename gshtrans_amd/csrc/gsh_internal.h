@@ -106,10 +106,8 @@ struct LegParams {
   int items_per;
   // Recurrence checkpoints: state (e_l, e_{l-1}) at l = l0 + kCk k of order
   // m, k >= 1, colatitude t: ck[(ckoff[m + L] + k - 1) * ntheta + t], for
-  // every l0 + kCk k <= L.  Orders m < 0 are in a table of their own, ckn (same
-  // index; null where no kernel of the launch reads them): see ck_rows.
+  // every l0 + kCk k <= L.  Orders m < 0 are in a table of their own, ckn below.
   const double2* ck;
-  const double2* ckn;
   const long* ckoff;
   // Split-BF16 synthesis of the tail_rows colatitudes tail_t0 .. (0: none),
   // from the d values tail_dv[r * tail_dstride + 32 block + j] of the degree
@@ -142,6 +140,9 @@ struct LegParams {
   const unsigned short* kf;
   unsigned short* kf_out;
   int nrt;  // row tiles, ceil(ntheta / 16)
+  // ck of the orders m < 0 (same index; null where no kernel of the launch reads
+  // them): see ck_rows.  Last, so that what every kernel reads shares lines.
+  const double2* ckn;
 };
 
 // Truncation degree and caller index of column field f.

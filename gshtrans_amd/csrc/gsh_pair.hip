@@ -90,10 +90,6 @@ struct Mma<2> {
   static __device__ __forceinline__ void add(acc& c, double v) { c += v; }
 };
 
-__device__ __forceinline__ int ld_uniform_u16(const unsigned short* a, int i) {
-  return __builtin_amdgcn_readfirstlane((int)a[i]);
-}
-
 // One recurrence step with uniform coefficients {a, b, c} and per-lane cos.
 __device__ __forceinline__ void rec_step(double2 ab, double c, double cs, double& e0, double& e1) {
   const double t = fma(ab.x, cs, -ab.y);
@@ -266,8 +262,9 @@ __global__ __launch_bounds__(256, synth_waves(KIND, SYM, RT, NJ)) void leg_synth
 
   // First checkpoint that counts at any of the block's rows.
   const unsigned short* kfm = p.kf + (long)(m + p.L) * p.nrt;
-  int ks = wave_min(kfm[tile0 + min(lane & 15, ntile - 1)]);
-  if (TW > 15) ks = min(ks, ld_uniform_u16(kfm, tile0 + ntile - 1));  // the 17th tile
+  const int kfl = kfm[tile0 + min(lane & 31, ntile - 1)];  // lane i: row tile i
+  int ks = wave_min(kfl);  // tiles 0 .. 15
+  if (TW > 15) ks = min(ks, __builtin_amdgcn_readlane(kfl, 16));
   ks = min(ks, max(0, lwg - l0 + kCk) / kCk);
   const int ls = l0 + kCk * ks;
   const int nchunk = ls > lwg ? 0 : (lwg - ls + SC) / SC;
@@ -356,23 +353,26 @@ __global__ __launch_bounds__(256, synth_waves(KIND, SYM, RT, NJ)) void leg_synth
   const double cs = tv ? p.cosv[t] : 0.0, csx = txv ? p.cosv[tx] : 0.0;
   const int nck = (p.L - l0 + kCk) / kCk;  // checkpoints 1 .. nck - 1 exist
   // First checkpoints that count at the wave's four row tiles and at the extra
-  // one, in scalar registers (a per-lane copy of them costs the widest tiles 3%).
+  // one, in scalar registers (a per-lane copy of them costs the widest tiles 3%,
+  // loads of their own 0.2 us of a small launch); from kmax on all of them count.
   int kt[5];
 #pragma unroll
-  for (int i = 0; i < 4; i++)
-    kt[i] = ld_uniform_u16(kfm, min(tile0 + 4 * (wave % PW) + i, p.nrt - 1));
-  kt[4] = ld_uniform_u16(kfm, min(tile0 + TW, p.nrt - 1));
+  for (int i = 0; i < 4; i++) kt[i] = __builtin_amdgcn_readlane(kfl, 4 * (wave % PW) + i);
+  kt[4] = __builtin_amdgcn_readlane(kfl, TW);
+  const int kmax = max(max(max(kt[0], kt[1]), max(kt[2], kt[3])), kt[4]);
   const unsigned long long rows = __ballot(tv), rowsx = __ballot(txv);
   const double* seedm = p.seeds + (long)(m + p.L) * nt;
   const double2* ckm = p.ck + (long)it.z * nt;
   auto state = [&](int c, bool extra, int row) -> double2 {
     const int k = ks + NH * c + seg;
     unsigned long long live = k < nck ? extra ? rowsx : rows : 0;
-    if (extra) {
-      live = k < kt[4] ? 0 : live;
-    } else {
+    if (k < kmax) {
+      if (extra) {
+        live = k < kt[4] ? 0 : live;
+      } else {
 #pragma unroll
-      for (int i = 0; i < 4; i++) live &= k < kt[i] ? ~(0xffffull << (16 * i)) : ~0ull;
+        for (int i = 0; i < 4; i++) live &= k < kt[i] ? ~(0xffffull << (16 * i)) : ~0ull;
+      }
     }
     double2 s = make_double2(0.0, 0.0);
     if (__builtin_amdgcn_inverse_ballot_w64(live)) {
