@@ -1245,6 +1245,7 @@ int gsh_grid_prepare(gsh_grid_t g, int n) {
   std::lock_guard<std::mutex> lock(g->mu);
   NData* d;
   int st;
+  GSH_HIP(hipSetDevice(g->device));
   if ((st = ensure_ndata(g, n, &d)) || g->L == 0) return st;
   // The checkpoints too, which every transform reads (lMax=512: the first synthesis
   // of 24 FP32 maps 619 -> 354 us).  A device without room for them has prepared what
